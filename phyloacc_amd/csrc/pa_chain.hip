@@ -47,18 +47,16 @@ struct Ctx {
     const GBL uint8_t *codes;
     const GBL int32_t *wts, *site;
     // workgroup scratch in HBM
-    GBL V4<R> *parts;      // [2][I][Ppad]
-    GBL int32_t *exps;     // [2][I][Ppad]
+    GBL char *parts;       // partials and exponents by block of 64 patterns (block_bytes)
     GBL double *plin;      // [3][N][16]  P_{j->i} at [j*4+i]
     GBL double *logt;      // [3][N][16]  log P_{j->i} at [i*4+j]
     GBL uint32_t *amb;     // [S][24]
     const GBL double *dist2;   // [N] branch lengths (element node table)
     // LDS arrays
-    LDS int16_t *par, *nodes, *inodes, *up, *upoff, *down, *downoff, *tz;
+    LDS int16_t *par, *nodes, *inodes, *porder, *up, *upoff, *down, *downoff, *tz;
     LDS uint32_t *desc;    // [I][4] static pruning descriptor of each internal node (node_desc)
-    LDS int32_t *plist;    // [I] nodes a pass visits, level order: s | level << 16
+    LDS uint32_t *steps;   // [I][4] the steps of a pass (build_steps)
     LDS uint8_t *flags, *fixZ, *dirty, *cur, *changed;
-    LDS uint8_t *pb;       // [N] per-pass buffer / matrix bits (pass_bits); shares storage with changed
     LDS int8_t *Z, *maxZ;
     LDS double *E, *beta;
     LDS R *PTc, *PTp;      // [N][16], PT[i*4+j] = P_{j->i}
@@ -69,7 +67,7 @@ struct Ctx {
     double TMf[9], TMn[9];  // log_TM_Int for fixZ / free nodes, [i*3+j] = log P(child i | parent j)
     double red[16];
     unsigned long long bytes;   // algorithmic HBM bytes of this element's passes (see prune / sample_sites)
-    int accept_n, accept_c, max_m, skip, accept, fail, work, nch, n_vis;   // fail: PA_F_* bits
+    int accept_n, accept_c, max_m, skip, accept, fail, work, nch, n_steps, last_step;   // fail: PA_F_* bits
 };
 
 template <typename R>
@@ -97,8 +95,8 @@ __host__ __device__ size_t smem_arrays(int N, int S, int BS, LDS char *base, CP<
     PA_TAKE(PTc, R, 16 * N);
     // Phases that never overlap share storage:
     //   A: per-thread ancestral states (sample_sites) | emissions and Z
-    //      messages (emissions, update_Z) | Z-transition counts
-    //      (sample_transition);
+    //      messages (emissions, update_Z) | the steps of a pass (prune) |
+    //      Z-transition counts (sample_transition);
     //   B: per-branch transition counters (sample_sites, emissions) |
     //      proposal matrices (rate updates).  sample_sites clears the
     //      counters before it counts.
@@ -116,16 +114,17 @@ __host__ __device__ size_t smem_arrays(int N, int S, int BS, LDS char *base, CP<
             c->beta = (LDS double *)(base + o) + 3 * N;
             c->tgs = (LDS uint8_t *)(base + o);
             c->cnt9 = (LDS uint32_t *)(base + o);
+            c->steps = (LDS uint32_t *)(base + o);
         }
         o += szA;
     }
     o = al(o, 16);      // descriptors are read as 16-byte vectors
     if constexpr (BIND) c->desc = (LDS uint32_t *)(base + o);
     o += (size_t)16 * (I > 0 ? I : 1);
-    PA_TAKE(plist, int32_t, I > 0 ? I : 1);
     PA_TAKE(par, int16_t, N);
     PA_TAKE(nodes, int16_t, N);
     PA_TAKE(inodes, int16_t, N);
+    PA_TAKE(porder, int16_t, I > 0 ? I : 1);
     PA_TAKE(up, int16_t, N);
     PA_TAKE(upoff, int16_t, N + 1);
     PA_TAKE(down, int16_t, N);
@@ -136,7 +135,6 @@ __host__ __device__ size_t smem_arrays(int N, int S, int BS, LDS char *base, CP<
     PA_TAKE(dirty, uint8_t, N);
     PA_TAKE(cur, uint8_t, N);
     PA_TAKE(changed, uint8_t, N);
-    if constexpr (BIND) c->pb = c->changed;   // changed lives inside update_Z, pb inside prune
     PA_TAKE(Z, int8_t, N);
     PA_TAKE(maxZ, int8_t, N);
 #undef PA_TAKE
@@ -155,16 +153,15 @@ size_t chain_smem_bytes(int N, int S, int BS, int fp64)
            (fp64 ? sizeof(Ctx<double>) : sizeof(Ctx<float>)) + sizeof(ModelDev);
 }
 
-// Byte offset of the exponents behind the partials of an element of Ppad
-// padded patterns ([2][I][Ppad] 4-vectors of R).
-__host__ __device__ inline size_t chain_exps_off(int N, int S, int Ppad, int rs)
-{
-    return al((size_t)2 * (N - S) * Ppad * 4 * rs, 256);
-}
+// Partials of an element, by block of 64 patterns: two buffers of I node
+// slots of 64 4-vectors of R, then as many slots of 64 exponents (slot =
+// buffer * I + node - S).  A wave's block is one contiguous region, so every
+// address in a pass is a scalar base and a small offset.
+__host__ __device__ inline int block_bytes(int I, int rs) { return 2 * I * 64 * (4 * rs + 4); }
 
 size_t chain_part_bytes(int N, int S, int Ppad, int fp64)
 {
-    return chain_exps_off(N, S, Ppad, fp64 ? 8 : 4) + al((size_t)2 * (N - S) * Ppad * 4, 256);
+    return al((size_t)(Ppad / 64) * (size_t)block_bytes(N - S, fp64 ? 8 : 4), 256);
 }
 
 // Per-workgroup HBM scratch layout (bytes), shared with the host: the rate
@@ -180,6 +177,41 @@ size_t slot_scratch_bytes(int N, int S, int Pcap, int fp64, size_t *off)
 }
 
 // ------------------------------------------------------------------ helpers
+
+// A region of memory as a raw buffer: loads and stores take a lane's byte
+// offset and a scalar one, and an access outside the region is dropped (a
+// load gives 0).
+typedef __amdgpu_buffer_rsrc_t Buf;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+template <typename T>
+__device__ __forceinline__ Buf make_buf(T *base, int bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(T *)base, 0, bytes, 0x00027000);
+}
+template <typename R>
+__device__ __forceinline__ V4<R> buf_ld4(Buf b, uint32_t lane_off, uint32_t off)
+{
+    if constexpr (sizeof(R) == 4) {
+        return __builtin_bit_cast(V4<R>, __builtin_amdgcn_raw_buffer_load_b128(b, lane_off, off, 0));
+    } else {
+        struct { u32x4 lo, hi; } v = {__builtin_amdgcn_raw_buffer_load_b128(b, lane_off, off, 0),
+                                      __builtin_amdgcn_raw_buffer_load_b128(b, lane_off + 16, off, 0)};
+        return __builtin_bit_cast(V4<R>, v);
+    }
+}
+template <typename R>
+__device__ __forceinline__ void buf_st4(Buf b, const V4<R> &v, uint32_t lane_off, uint32_t off)
+{
+    if constexpr (sizeof(R) == 4) {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), b, lane_off, off, 0);
+    } else {
+        struct P { u32x4 lo, hi; };
+        const P p = __builtin_bit_cast(P, v);
+        __builtin_amdgcn_raw_buffer_store_b128(p.lo, b, lane_off, off, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(p.hi, b, lane_off + 16, off, 0);
+    }
+}
 
 __device__ __forceinline__ void lds_add(LDS uint32_t *p, uint32_t v)
 {
@@ -247,25 +279,8 @@ __device__ __noinline__ void refresh_PTc(CP<R> c, int only_cls)
 
 enum { PR_FULL = 0, PR_DIRTY = 1, PR_PROP = 2 };
 
-// Where one child of a node comes from in a pass: a leaf's code row, an
-// internal child's partial / exponent rows (offsets into the slot arrays), or
-// a cherry's two leaf code rows; and the branch matrices that apply.  Every
-// field is the same on all lanes (scalar registers).
-enum { KD_LEAF = 0, KD_STORED = 1, KD_CHERRY = 2, KD_KIND = 3, KD_MISS = 4, KD_MISS_A = 8, KD_MISS_B = 16 };
-
-template <typename R>
-struct KidDesc {
-    int bits;             // kind (KD_KIND), the child missing, a cherry's leaves missing
-    int off, offB;        // code row / partial offset; cherry: code rows of its two leaves
-    const LDS R *src;     // the child's branch matrix
-    const LDS R *sA, *sB; // cherry: its leaves' branch matrices
-};
-
-template <typename R>
-struct NodeDesc {
-    int dst;              // 2 * (offset of the node's partial / exponent rows in the written buffer) + missing
-    KidDesc<R> k[2];
-};
+// Kind of a node's child (node_desc): a leaf, a stored internal node, a cherry.
+enum { KD_LEAF = 0, KD_STORED = 1, KD_CHERRY = 2 };
 
 // Static pruning descriptor of an internal node, built when the element is
 // bound (node_desc): word 0 = its children x0 | x1 << 16; words 1 and 2 = the
@@ -275,72 +290,329 @@ struct NodeDesc {
 enum { DB_KIND1_SHIFT = 2, DB_MISS0 = 1 << 4, DB_MISS1 = 1 << 5, DB_MISS_A0 = 1 << 6, DB_MISS_B0 = 1 << 7,
        DB_MISS_A1 = 1 << 8, DB_MISS_B1 = 1 << 9, DB_MISS = 1 << 10 };
 
-// Per-pass bits of node y (pass_bits): PB_BUF = the buffer holding y's
-// partial in this pass (read as a child, written as a visited node);
-// PB_PROP = y's branch takes the proposal matrix.
-enum { PB_BUF = 1, PB_PROP = 2 };
+// One step of a pass: an internal node the pass visits, or a cherry whose
+// parent it visits.  Four words:
+//   w0: type | SB_* bits | child A's slot << 14 | the node's slot, in the buffer it is written to, << 23
+//   w1, w2: the code row offsets of children A and B (row 0 for a child that is no leaf)
+//   w3: the children's matrices A | B << 10 (the node's id, + N for a proposal matrix) | child B's slot << 20
+// A child comes from its leaf code (L), its stored partial (S), or the result
+// of the step just before (P) or the one before that (P2), which the thread
+// still holds in registers.  The types are the combinations that occur when
+// nothing is missing, so each is straight code; ST_GEN takes any sources and
+// missing nodes.  The two children's order does not matter: their messages
+// are multiplied.
+enum { SK_LEAF = 0, SK_STORED = 1, SK_PREV = 2, SK_PREV2 = 3 };
+enum { ST_LL = 0, ST_PL = 1, ST_PP2 = 2, ST_SL = 3, ST_SP = 4, ST_SS = 5, ST_GEN = 6 };
+enum { SB_TYPE = 7, SB_STORED_A = 1 << 3, SB_STORED_B = 1 << 4, SB_CHERRY = 1 << 5, SB_MISS = 1 << 6, SB_MISS_A = 1 << 7,
+       SB_MISS_B = 1 << 8, SB_KIND_A_SHIFT = 9, SB_KIND_B_SHIFT = 11, SB_SLOT_A_SHIFT = 14, SB_SLOT_SHIFT = 23,
+       SB_MAT_MASK = 0x3ff, SB_MAT_B_SHIFT = 10, SB_SLOT_B_SHIFT = 20 };
+static_assert(MAXN <= 512, "slots (below 2 I <= N) in nine bits, matrices (below 2 N) in ten");
 
-template <typename R>
-__device__ __forceinline__ KidDesc<R> kid_from(int kind, int miss, int missA, int missB, int x, int px, int yA, int pA,
-                                               int yB, int pB, const LDS R *PTc, const LDS R *PTp, int S, int Ppad,
-                                               int bufI)
-{
-    KidDesc<R> d;
-    d.src = ((px & PB_PROP) ? PTp : PTc) + 16 * x;
-    d.offB = 0;
-    d.sA = d.sB = PTc;
-    if (kind == KD_LEAF) {
-        d.bits = KD_LEAF | (miss ? KD_MISS : 0);
-        d.off = x * Ppad;
-    } else if (kind == KD_CHERRY) {
-        d.bits = KD_CHERRY | (miss ? KD_MISS : 0) | (missA ? KD_MISS_A : 0) | (missB ? KD_MISS_B : 0);
-        d.off = yA * Ppad;
-        d.offB = yB * Ppad;
-        d.sA = ((pA & PB_PROP) ? PTp : PTc) + 16 * yA;
-        d.sB = ((pB & PB_PROP) ? PTp : PTc) + 16 * yB;
-    } else {
-        d.bits = KD_STORED | (miss ? KD_MISS : 0);
-        d.off = (px & PB_BUF) * bufI + (x - S) * Ppad;
-    }
-    return d;
-}
-
-template <typename R>
-__device__ __forceinline__ ChildIn<R> kid_load(const KidDesc<R> &d, const GBL uint8_t *codes, const GBL V4<R> *parts,
-                                               const GBL int32_t *exps, int p)
-{
-    // a missing child contributes nothing, but its gap state still decides
-    // whether the parent is all-gap at this pattern, so its code / exponent
-    // is read either way; a cherry's two codes are packed into x
-    ChildIn<R> in;
-    in.v.x = in.v.y = in.v.z = in.v.w = (R)0;
-    const int kind = d.bits & KD_KIND;
-    if (kind == KD_LEAF) {
-        in.x = codes[d.off + p];
-    } else if (kind == KD_CHERRY) {
-        in.x = codes[d.off + p] | (codes[d.offB + p] << 8);
-    } else {
-        in.x = exps[d.off + p];
-        if (!(d.bits & KD_MISS)) in.v = ld4<R>(parts + d.off + p);
-    }
-    return in;
-}
-
-// Pattern-loop shapes the autotuner picks among.  U: visited nodes pruned
-// together per round (all their loads are issued before the first is used);
-// K: internal nodes whose partials one sampling chunk loads before drawing.
-// Shape 0 is the default: two nodes in FP32 and one in FP64 fit the
-// 128-register budget of the chain kernel without spilling in the pattern
-// loop (groups of 3 spill and ran 3 % slower on the 50,000-element
-// 43-species workload).
+// Pattern-loop shapes the autotuner picks among.  U: patterns a thread takes
+// through a pass together (they share each step's matrices); K: internal
+// nodes whose partials one sampling chunk loads before drawing.  Shape 0 is
+// the default: two patterns in FP32 and one in FP64 fit the 128-register
+// budget of the chain kernel.
 template <typename R, int SH>
 struct Shape;
-template <> struct Shape<float, 0> { static constexpr int U = 2, K = 4; };
+template <> struct Shape<float, 0> { static constexpr int U = 1, K = 4; };
 template <> struct Shape<float, 1> { static constexpr int U = 1, K = 4; };
 template <> struct Shape<float, 2> { static constexpr int U = 2, K = 8; };
 template <> struct Shape<double, 0> { static constexpr int U = 1, K = 2; };
 template <> struct Shape<double, 1> { static constexpr int U = 2, K = 2; };
 template <> struct Shape<double, 2> { static constexpr int U = 1, K = 4; };
+
+// The steps of a pass, written by one wave: a ballot per 64 internal nodes
+// (in pruning order) places them, and each lane encodes its own node.  A
+// child that is the list's previous (or second previous) entry is taken from
+// registers.
+template <typename R>
+__device__ __forceinline__ void build_steps(CP<R> c, int mode, int cls)
+{
+    const int lane = threadIdx.x;
+    const bool prop = mode == PR_PROP;
+    const int S = uni(c->S), N = uni(c->N), I = uni(c->I), n_int = uni(c->n_int), Ppad = uni(c->Ppad);
+    const LDS int16_t *porder = uni_ptr(c->porder), *par = uni_ptr(c->par);
+    const LDS uint8_t *flags = uni_ptr(c->flags), *dirty = uni_ptr(c->dirty), *cur = uni_ptr(c->cur);
+    const LDS int8_t *Z = uni_ptr(c->Z);
+    const LDS uint32_t *desc = uni_ptr(c->desc);
+    LDS uint32_t *steps = uni_ptr(c->steps);
+    int base = 0, last1 = -1, last2 = -1, n_node = 0, n_leaf = 0, n_cherry = 0;
+    for (int q0 = 0; q0 < n_int; q0 += 64) {
+        const int q = q0 + lane;
+        bool v = false;
+        int s = 0, f = 0, leaves = 0, cherries = 0;
+        if (q < n_int) {
+            s = porder[q];
+            f = flags[s];
+            // a cherry is a step of its parent's visit
+            const int t = (f & NF_CHERRY) ? par[s] : s;
+            v = mode == PR_FULL || (dirty[t] && !(flags[t] & NF_MISSING));
+        }
+        const unsigned long long bal = __ballot(v);
+        const unsigned long long below = bal & ((1ull << lane) - 1);
+        const int l1 = below ? 63 - __clzll(below) : -1;
+        const unsigned long long below2 = l1 >= 0 ? below ^ (1ull << l1) : 0;
+        const int l2 = below2 ? 63 - __clzll(below2) : -1;
+        const int s1 = __shfl(s, l1 < 0 ? 0 : l1, 64), s2 = __shfl(s, l2 < 0 ? 0 : l2, 64);
+        const int n1 = l1 >= 0 ? s1 : last1, n2 = l2 >= 0 ? s2 : (l1 >= 0 ? last1 : last2);
+        if (v) {
+            const LDS uint32_t *dd = desc + 4 * (s - S);
+            const uint32_t d0 = dd[0], d3 = dd[3];
+            int kind[2], miss[2], m[2], row[2] = {0, 0}, slot[2] = {0, 0};
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int x = j ? (int)(d0 >> 16) : (int)(d0 & 0xffff);
+                const int k = j ? (d3 >> DB_KIND1_SHIFT) & 3 : d3 & 3;
+                m[j] = x + ((prop && Z[x] == cls) ? N : 0);
+                miss[j] = (d3 & (j ? DB_MISS1 : DB_MISS0)) ? 1 : 0;
+                if (k == KD_LEAF) {
+                    kind[j] = SK_LEAF;
+                    row[j] = x * Ppad;
+                } else {
+                    const int cx = cur[x];
+                    kind[j] = x == n1 ? SK_PREV : (x == n2 ? SK_PREV2 : SK_STORED);
+                    slot[j] = ((prop && dirty[x]) ? 1 - cx : cx) * I + x - S;
+                }
+                leaves |= (k == KD_LEAF) << j;
+                cherries |= (k == KD_CHERRY) << j;
+            }
+            // child A: a stored node before the previous result, that before the one before it, a leaf last
+            const int rank = 0x2103;      // a nibble per kind
+            const int a = ((rank >> (4 * kind[1])) & 15) < ((rank >> (4 * kind[0])) & 15) ? 1 : 0;
+            const int ka = a ? kind[1] : kind[0], kb = a ? kind[0] : kind[1];
+            const int ma = a ? miss[1] : miss[0], mb = a ? miss[0] : miss[1];
+            int type = ST_GEN;
+            if (!(d3 & DB_MISS) && !ma && !mb) {
+                if (ka == SK_LEAF) type = ST_LL;
+                else if (ka == SK_PREV) type = kb == SK_LEAF ? ST_PL : (kb == SK_PREV2 ? ST_PP2 : ST_GEN);
+                else if (ka == SK_STORED) type = kb == SK_LEAF ? ST_SL : (kb == SK_PREV ? ST_SP : (kb == SK_STORED ? ST_SS : ST_GEN));
+            }
+            const int cs = cur[s];
+            const int dst = (prop ? 1 - cs : cs) * I + s - S;
+            LDS uint32_t *w = steps + 4 * (base + __popcll(below));
+            w[0] = (uint32_t)type | (ka == SK_STORED ? SB_STORED_A : 0) | (kb == SK_STORED ? SB_STORED_B : 0) |
+                   ((f & NF_CHERRY) ? SB_CHERRY : 0) | ((d3 & DB_MISS) ? SB_MISS : 0) | (ma ? SB_MISS_A : 0) |
+                   (mb ? SB_MISS_B : 0) | ((uint32_t)ka << SB_KIND_A_SHIFT) | ((uint32_t)kb << SB_KIND_B_SHIFT) |
+                   ((uint32_t)(a ? slot[1] : slot[0]) << SB_SLOT_A_SHIFT) | ((uint32_t)dst << SB_SLOT_SHIFT);
+            w[1] = (uint32_t)(a ? row[1] : row[0]);
+            w[2] = (uint32_t)(a ? row[0] : row[1]);
+            w[3] = (uint32_t)(a ? m[1] : m[0]) | ((uint32_t)(a ? m[0] : m[1]) << SB_MAT_B_SHIFT) |
+                   ((uint32_t)(a ? slot[0] : slot[1]) << SB_SLOT_B_SHIFT);
+        }
+        const int cnt = __popcll(bal);
+        if (cnt) {
+            const int h1 = 63 - __clzll(bal);
+            const unsigned long long rest = bal ^ (1ull << h1);
+            const int t1 = __shfl(s, h1, 64);
+            const int t2 = __shfl(s, rest ? 63 - __clzll(rest) : 0, 64);
+            last2 = cnt > 1 ? t2 : last1;
+            last1 = t1;
+        }
+        base += cnt;
+        const unsigned long long nodes = __ballot(v && !(f & NF_CHERRY));
+        n_node += __popcll(nodes);
+        n_leaf += __popcll(nodes & __ballot(leaves & 1)) + __popcll(nodes & __ballot(leaves & 2));
+        n_cherry += __popcll(nodes & __ballot(cherries & 1)) + __popcll(nodes & __ballot(cherries & 2));
+    }
+    if (lane == 0) {
+        c->n_steps = base;
+        c->last_step = last1;
+        // counted bytes, node by node: write partial + exponent; read each child's partial + exponent, its leaf
+        // code, or a cherry's two codes; then the root's partial, exponent and weight
+        const unsigned long long W = 4 * sizeof(R) + 4;
+        c->bytes += (unsigned long long)c->P * (n_node * W + n_leaf + 2 * n_cherry + (2 * n_node - n_leaf - n_cherry) * W + W + 4);
+    }
+}
+
+// The scalar arguments of a pass's pattern loop.
+template <typename R>
+struct PassArgs {
+    const LDS uint32_t *steps;
+    const LDS R *PT;             // [2N][16]: the current matrices, then the proposal's
+    Buf codes;
+    int n, I, amb;
+};
+
+// One child's message at one pattern, or ones where it holds no base; adds
+// its exponent and reports the gap.
+template <typename R, int K>
+__device__ __forceinline__ void message(const LDS R *PT, int amb, int code, const ChildIn<R> &in, V4<R> &o, int &e, bool &gap)
+{
+    if constexpr (K == SK_LEAF) {
+        gap = code == PA_GAP_CODE || code == PA_OTHER_CODE;
+        o = ld4<R>((const LDS V4<R> *)(PT + 4 * (code & 3)));
+        if (amb && code > PA_OTHER_CODE) {
+            o.x = o.y = o.z = o.w = (R)1;
+            leaf_mul<R>(PT, code, o.x, o.y, o.z, o.w);
+        }
+        o.x = gap ? (R)1 : o.x; o.y = gap ? (R)1 : o.y; o.z = gap ? (R)1 : o.z; o.w = gap ? (R)1 : o.w;
+    } else {
+        gap = in.x == GAPT;
+        int x = in.x;
+        const V4<R> v = in.v;
+        const V4<R> m0 = ld4<R>((const LDS V4<R> *)(PT + 0)), m1 = ld4<R>((const LDS V4<R> *)(PT + 4));
+        const V4<R> m2 = ld4<R>((const LDS V4<R> *)(PT + 8)), m3 = ld4<R>((const LDS V4<R> *)(PT + 12));
+        o.x = m0.x * v.x + m1.x * v.y + m2.x * v.z + m3.x * v.w;
+        o.y = m0.y * v.x + m1.y * v.y + m2.y * v.z + m3.y * v.w;
+        o.z = m0.z * v.x + m1.z * v.y + m2.z * v.z + m3.z * v.w;
+        o.w = m0.w * v.x + m1.w * v.y + m2.w * v.z + m3.w * v.w;
+        if (__ballot(gap)) {
+            // rare: some lane's subtree holds only gaps
+            o.x = gap ? (R)1 : o.x; o.y = gap ? (R)1 : o.y; o.z = gap ? (R)1 : o.z; o.w = gap ? (R)1 : o.w;
+            x = gap ? 0 : x;
+        }
+        e += x;
+    }
+}
+
+// A node from its children's messages: their product, rescaled by a power of two.
+template <typename R>
+__device__ __forceinline__ ChildIn<R> combine(const V4<R> &a, const V4<R> &b, int e, bool gap)
+{
+    const R x = a.x * b.x, y = a.y * b.y, z = a.z * b.z, w = a.w * b.w;
+    const R mx = fmax(fmax(x, y), fmax(z, w));
+    int kx = 0;
+    frexp(mx, &kx);
+    ChildIn<R> r;
+    r.v.x = ldexp(x, -kx); r.v.y = ldexp(y, -kx); r.v.z = ldexp(z, -kx); r.v.w = ldexp(w, -kx);
+    r.x = gap ? GAPT : e + kx;
+    return r;
+}
+
+// Byte offsets of a slot's partials and exponents within a pattern block.
+template <typename R>
+__device__ __forceinline__ uint32_t part_off(uint32_t slot) { return slot * (64 * (uint32_t)sizeof(V4<R>)); }
+template <typename R>
+__device__ __forceinline__ uint32_t exp_off(uint32_t slot, int I) { return (uint32_t)(2 * I) * (64 * (uint32_t)sizeof(V4<R>)) + slot * 256; }
+
+// Slot's partial and exponent of this lane's pattern, from the block's buffer.
+template <typename R>
+__device__ __forceinline__ ChildIn<R> slot_load(Buf blk, uint32_t slot, uint32_t lane, int I)
+{
+    ChildIn<R> in;
+    in.v = buf_ld4<R>(blk, lane * (uint32_t)sizeof(V4<R>), part_off<R>(slot));
+    in.x = (int)__builtin_amdgcn_raw_buffer_load_b32(blk, lane * 4, exp_off<R>(slot, I), 0);
+    return in;
+}
+
+// Takes one pattern a lane (pattern p, of the block at base) through every
+// step and returns the last step's partial and exponent.  The inputs of step
+// k + 2 are loaded while step k is computed and its words are read a step
+// before that, so neither a memory nor an LDS round trip stands between two
+// steps.  All lanes run (patterns are padded to whole waves).  Every step
+// issues the same code loads and stores, whether it needs them or not, since
+// a step's wait for its loads counts the memory operations issued after them:
+// a child that is no leaf loads row 0's code, and a cherry, which is kept in
+// registers only, stores through a buffer of no bytes (the hardware drops
+// accesses outside a buffer).
+template <typename R>
+__device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL char *base, int blk_bytes, uint32_t p)
+{
+    const int n = A.n;
+    const uint32_t lane = threadIdx.x & 63;
+    const Buf blk = make_buf(base, blk_bytes);
+    ChildIn<R> inA[2], inB[2], res[2];
+    int cdA[2], cdB[2];
+    uint32_t w[2][4], nw[4];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        res[j].x = GAPT;
+        res[j].v.x = res[j].v.y = res[j].v.z = res[j].v.w = (R)0;
+        inA[j] = inB[j] = res[j];
+        cdA[j] = cdB[j] = 0;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) nw[i] = A.steps[i];
+    // words and inputs of step k into set j
+    auto fetch = [&](auto J, int k) __attribute__((always_inline)) {
+        constexpr int j = decltype(J)::value;
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[j][i] = (uint32_t)uni((int)nw[i]);
+        const LDS uint32_t *nx = A.steps + 4 * (k + 1 < n ? k + 1 : k);
+#pragma unroll
+        for (int i = 0; i < 4; i++) nw[i] = nx[i];
+        const uint32_t w0 = w[j][0];
+        if (w0 & SB_STORED_A) inA[j] = slot_load<R>(blk, (w0 >> SB_SLOT_A_SHIFT) & 511, lane, A.I);
+        if (w0 & SB_STORED_B) inB[j] = slot_load<R>(blk, w[j][3] >> SB_SLOT_B_SHIFT, lane, A.I);
+        cdA[j] = __builtin_amdgcn_raw_buffer_load_b8(A.codes, p, w[j][1], 0);
+        cdB[j] = __builtin_amdgcn_raw_buffer_load_b8(A.codes, p, w[j][2], 0);
+    };
+    auto step = [&](auto J, int k) __attribute__((always_inline)) {
+        constexpr int j = decltype(J)::value;
+        const uint32_t w0 = w[j][0];
+        const int type = w0 & SB_TYPE;
+        const LDS R *PA = A.PT + 16 * (w[j][3] & SB_MAT_MASK), *PB = A.PT + 16 * ((w[j][3] >> SB_MAT_B_SHIFT) & SB_MAT_MASK);
+        int e = 0;
+        bool ga, gb;
+        V4<R> a, b;
+        ChildIn<R> out;
+        if (type == ST_PL) {
+            message<R, SK_PREV>(PA, 0, 0, res[j ^ 1], a, e, ga);
+            message<R, SK_LEAF>(PB, A.amb, cdB[j], inB[j], b, e, gb);
+            out = combine<R>(a, b, e, ga && gb);
+        } else if (type == ST_LL) {
+            message<R, SK_LEAF>(PA, A.amb, cdA[j], inA[j], a, e, ga);
+            message<R, SK_LEAF>(PB, A.amb, cdB[j], inB[j], b, e, gb);
+            out = combine<R>(a, b, e, ga && gb);
+        } else if (type == ST_PP2) {
+            message<R, SK_PREV>(PA, 0, 0, res[j ^ 1], a, e, ga);
+            message<R, SK_PREV2>(PB, 0, 0, res[j], b, e, gb);
+            out = combine<R>(a, b, e, ga && gb);
+        } else if (type == ST_SP) {
+            message<R, SK_STORED>(PA, 0, 0, inA[j], a, e, ga);
+            message<R, SK_PREV>(PB, 0, 0, res[j ^ 1], b, e, gb);
+            out = combine<R>(a, b, e, ga && gb);
+        } else if (type == ST_SL) {
+            message<R, SK_STORED>(PA, 0, 0, inA[j], a, e, ga);
+            message<R, SK_LEAF>(PB, A.amb, cdB[j], inB[j], b, e, gb);
+            out = combine<R>(a, b, e, ga && gb);
+        } else if (type == ST_SS) {
+            message<R, SK_STORED>(PA, 0, 0, inA[j], a, e, ga);
+            message<R, SK_STORED>(PB, 0, 0, inB[j], b, e, gb);
+            out = combine<R>(a, b, e, ga && gb);
+        } else {
+            // any sources, missing nodes: a missing child contributes nothing, but its gap state still
+            // decides whether the parent is all-gap at this pattern
+            const int ka = (w0 >> SB_KIND_A_SHIFT) & 3, kb = (w0 >> SB_KIND_B_SHIFT) & 3;
+            auto source = [&](int kind, const ChildIn<R> &ld, int code) __attribute__((always_inline)) {
+                const ChildIn<R> r1 = res[j ^ 1], r2 = res[j];
+                ChildIn<R> ci;
+                ci.x = kind == SK_PREV ? r1.x : (kind == SK_PREV2 ? r2.x : (kind == SK_LEAF ? code : ld.x));
+                ci.v.x = kind == SK_PREV ? r1.v.x : (kind == SK_PREV2 ? r2.v.x : ld.v.x);
+                ci.v.y = kind == SK_PREV ? r1.v.y : (kind == SK_PREV2 ? r2.v.y : ld.v.y);
+                ci.v.z = kind == SK_PREV ? r1.v.z : (kind == SK_PREV2 ? r2.v.z : ld.v.z);
+                ci.v.w = kind == SK_PREV ? r1.v.w : (kind == SK_PREV2 ? r2.v.w : ld.v.w);
+                return ci;
+            };
+            a.x = a.y = a.z = a.w = b.x = b.y = b.z = b.w = (R)1;
+            child_apply<R>(ka == SK_LEAF, w0 & SB_MISS_A, PA, source(ka, inA[j], cdA[j]), a.x, a.y, a.z, a.w, e, ga);
+            child_apply<R>(kb == SK_LEAF, w0 & SB_MISS_B, PB, source(kb, inB[j], cdB[j]), b.x, b.y, b.z, b.w, e, gb);
+            out = combine<R>(a, b, e, ga && gb);
+            if ((w0 & SB_MISS) && !(ga && gb)) out.x = 0;
+        }
+        if (k + 2 < n) fetch(J, k + 2);
+        res[j] = out;
+        const uint32_t d = w0 >> SB_SLOT_SHIFT;
+        const Buf to = make_buf(base, (w0 & SB_CHERRY) ? 0 : blk_bytes);
+        buf_st4<R>(to, out.v, lane * (uint32_t)sizeof(V4<R>), part_off<R>(d));
+        __builtin_amdgcn_raw_buffer_store_b32((uint32_t)out.x, to, lane * 4, exp_off<R>(d, A.I), 0);
+    };
+    fetch(std::integral_constant<int, 0>(), 0);
+    if (n > 1) fetch(std::integral_constant<int, 1>(), 1);
+    for (int k = 0; k < n; k += 2) {
+        step(std::integral_constant<int, 0>(), k);
+        if (k + 1 < n) step(std::integral_constant<int, 1>(), k + 1);
+    }
+    const bool odd = (n - 1) & 1;
+    ChildIn<R> r;
+    r.x = odd ? res[1].x : res[0].x;
+    r.v.x = odd ? res[1].v.x : res[0].v.x;
+    r.v.y = odd ? res[1].v.y : res[0].v.y;
+    r.v.z = odd ? res[1].v.z : res[0].v.z;
+    r.v.w = odd ? res[1].v.w : res[0].v.w;
+    return r;
+}
 
 // One pruning pass (BPP_C::Update_Tg(tosample=false), src/PhyloAcc-ST/bpp_c.cpp:644-671,
 // and log_f_Xz, bpp_c.cpp:860-928).  FULL: every internal node of the tree
@@ -351,174 +623,68 @@ template <> struct Shape<double, 2> { static constexpr int U = 1, K = 4; };
 // used.  Returns the element's log-likelihood (FP64), identical on every
 // thread.
 //
-// Nodes are taken by tree level (the element's height-ordered list), so the
-// nodes of one round never depend on each other: a round takes up to U
-// visited nodes of one level and, for each pattern block, issues the loads
-// of all their children before computing any of them.  A pass then costs
-// about one memory round trip per round instead of one per node.  A thread
-// owns the patterns p = tid (mod BS) of every node, so it only reads partials
-// it wrote itself and the pass needs no barrier between rounds.  The pass
-// first lists the nodes it visits (one ballot per 64 nodes of a level) and
-// every node's buffer and matrix bits, so a round's scalar set-up is a few
-// independent LDS reads: its list entries, its nodes' static descriptors
-// (node_desc) and their children's bits.
+// A pass is a chain of nodes, and what bounds it is the time of one link.
+// The steps are therefore in post-order with the larger subtree of every fork
+// first (pruning order), so that a node mostly follows its child: the
+// child's partial is still in registers, a cherry's always is, and only the
+// larger side of a fork of stored nodes is read back.  Each step's nodes,
+// sources and matrices come as two words (build_steps) that are read ahead of
+// their use, and the inputs of the step after next are in flight.  (By tree
+// level, with each node's descriptor read when its turn came, a step waited
+// for three dependent LDS round trips and the loads of both children.)
+// A thread owns the patterns p = tid (mod BS) of every node, so the pass
+// needs no barrier between steps.  The root's FP64 log sum is a deterministic
+// block reduction.
 template <typename R, int BS, int SH>
 __device__ __noinline__ double prune(MP M, CP<R> c, int mode, int cls)
 {
     const int tid = threadIdx.x;
-    const int P = uni(c->P), Ppad = uni(c->Ppad), S = uni(c->S), n_up = uni(c->n_up);
-    const int bufI = uni(c->I) * Ppad;
-    GBL V4<R> *parts = uni_ptr(c->parts);
-    GBL int32_t *exps = uni_ptr(c->exps);
-    const GBL uint8_t *codes = uni_ptr(c->codes);
-    const LDS R *PTc = uni_ptr(c->PTc), *PTp = uni_ptr(c->PTp);
-    constexpr int U = Shape<R, SH>::U;
-    unsigned long long bytes = 0;
-    const LDS uint8_t *flags = uni_ptr(c->flags), *dirty = uni_ptr(c->dirty), *cur = uni_ptr(c->cur);
-    const LDS int32_t *plist = uni_ptr(c->plist);
-    // pass set-up: every node's buffer and matrix bits, and the list of
-    // nodes the pass visits in level order (one wave compacts it by ballot)
-    {
-        const bool prop = mode == PR_PROP;
-        const LDS int16_t *nodes = uni_ptr(c->nodes), *up = uni_ptr(c->up), *upoff = uni_ptr(c->upoff);
-        const LDS int8_t *Zs = uni_ptr(c->Z);
-        LDS uint8_t *pbw = uni_ptr(c->pb);
-        LDS int32_t *plw = uni_ptr(c->plist);
-        const int n_nodes = uni(c->n_nodes);
-        for (int q = tid; q < n_nodes; q += BS) {
-            const int y = nodes[q];
-            const int cu = cur[y];
-            pbw[y] = (uint8_t)(((prop && dirty[y]) ? 1 - cu : cu) | ((prop && Zs[y] == cls) ? PB_PROP : 0));
-        }
-        if (tid < 64) {
-            int base = 0;
-            for (int h = 0; h < n_up; h++) {
-                const int qa = h == 0 ? 0 : upoff[h - 1], qb = upoff[h];
-                for (int q0 = qa; q0 < qb; q0 += 64) {
-                    const int q = q0 + tid;
-                    bool v = false;
-                    int y = 0;
-                    if (q < qb) {
-                        y = up[q];
-                        const int f = flags[y];
-                        v = !(f & NF_CHERRY) && (mode == PR_FULL || (dirty[y] && !(f & NF_MISSING)));
-                    }
-                    const unsigned long long bal = __ballot(v);
-                    if (v) plw[base + __popcll(bal & ((1ull << tid) - 1))] = y | (h << 16);
-                    base += __popcll(bal);
-                }
-            }
-            if (tid == 0) c->n_vis = base;
-        }
-        __syncthreads();
-    }
-    const int n_vis = uni(c->n_vis);
-    const LDS uint8_t *pb = uni_ptr(c->pb);
-    const LDS uint32_t *desc = uni_ptr(c->desc);
-    for (int k = 0; k < n_vis;) {
-        {
-            // up to U consecutive visited nodes of one level
-            int ent[U], sel[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) ent[u] = (k + u < n_vis) ? uni(plist[k + u]) : -1;
-            int used = 1;
-            sel[0] = ent[0] & 0xffff;
-#pragma unroll
-            for (int u = 1; u < U; u++) {
-                sel[u] = -1;
-                if (used == u && ent[u] >= 0 && (ent[u] >> 16) == (ent[0] >> 16)) { sel[u] = ent[u] & 0xffff; used++; }
-            }
-            k += used;
-            NodeDesc<R> nd[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (sel[u] < 0) continue;
-                const int s = sel[u];
-                const LDS uint32_t *dd = desc + 4 * (s - S);
-                const uint32_t w0 = uni(dd[0]), w1 = uni(dd[1]), w2 = uni(dd[2]), w3 = uni(dd[3]);
-                const int x0 = w0 & 0xffff, x1 = w0 >> 16;
-                const int yA0 = w1 & 0xffff, yB0 = w1 >> 16, yA1 = w2 & 0xffff, yB1 = w2 >> 16;
-                const int ps = uni(pb[s]), p0 = uni(pb[x0]), p1 = uni(pb[x1]);
-                const int pA0 = uni(pb[yA0]), pB0 = uni(pb[yB0]), pA1 = uni(pb[yA1]), pB1 = uni(pb[yB1]);
-                nd[u].dst = 2 * ((ps & PB_BUF) * bufI + (s - S) * Ppad) + ((w3 & DB_MISS) ? 1 : 0);
-                nd[u].k[0] = kid_from<R>(w3 & 3, w3 & DB_MISS0, w3 & DB_MISS_A0, w3 & DB_MISS_B0, x0, p0, yA0, pA0, yB0,
-                                         pB0, PTc, PTp, S, Ppad, bufI);
-                nd[u].k[1] = kid_from<R>((w3 >> DB_KIND1_SHIFT) & 3, w3 & DB_MISS1, w3 & DB_MISS_A1, w3 & DB_MISS_B1, x1,
-                                         p1, yA1, pA1, yB1, pB1, PTc, PTp, S, Ppad, bufI);
-                // write partial + exponent; read each child's partial + exponent, its leaf code, or a cherry's two codes
-                bytes += (unsigned long long)P * (4 * sizeof(R) + 4);
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-                    bytes += (unsigned long long)P * ((nd[u].k[j].bits & KD_KIND) == KD_LEAF ? 1 : (nd[u].k[j].bits & KD_KIND) == KD_CHERRY ? 2 : 4 * sizeof(R) + 4);
-            }
-            for (int p = tid; p < P; p += BS) {
-                ChildIn<R> in[U][2];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    if (sel[u] < 0) continue;
-                    in[u][0] = kid_load<R>(nd[u].k[0], codes, parts, exps, p);
-                    in[u][1] = kid_load<R>(nd[u].k[1], codes, parts, exps, p);
-                }
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    // one node at a time: keeps the scheduler from hoisting
-                    // every node's matrices into registers at once
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (sel[u] < 0) continue;
-                    R a0 = 1, a1 = 1, a2 = 1, a3 = 1;
-                    int e = 0;
-                    bool g[2];
-#pragma unroll
-                    for (int j = 0; j < 2; j++) {
-                        const KidDesc<R> &d = nd[u].k[j];
-                        const int kind = d.bits & KD_KIND;
-                        const bool miss = d.bits & KD_MISS;
-                        ChildIn<R> cin = in[u][j];
-                        if (kind == KD_CHERRY)
-                            cin = cherry_in<R>(d.sA, d.sB, d.bits & KD_MISS_A, d.bits & KD_MISS_B, miss, cin.x & 255, cin.x >> 8);
-                        child_apply<R>(kind == KD_LEAF, miss, d.src, cin, a0, a1, a2, a3, e, g[j]);
-                    }
-                    const int dst = nd[u].dst >> 1;
-                    GBL int32_t *dste = exps + dst;
-                    if (g[0] && g[1]) {
-                        dste[p] = GAPT;
-                    } else if (nd[u].dst & 1) {
-                        dste[p] = 0;
-                    } else {
-                        const R mx = fmax(fmax(a0, a1), fmax(a2, a3));
-                        int kx = 0;
-                        frexp(mx, &kx);
-                        a0 = ldexp(a0, -kx); a1 = ldexp(a1, -kx); a2 = ldexp(a2, -kx); a3 = ldexp(a3, -kx);
-                        st4<R>(parts + dst + p, a0, a1, a2, a3);
-                        dste[p] = e + kx;
-                    }
-                }
-            }
-        }
-    }
-    if (tid == 0) c->bytes += bytes;
-    // root: log sum_j pi_j L_j + exponent * ln 2; all-gap columns contribute 0
+    const int P = uni(c->P);
+    if (tid < 64) build_steps<R>(c, mode, cls);
+    __syncthreads();
+    PassArgs<R> A;
+    A.n = uni(c->n_steps);
+    A.I = uni(c->I);
+    A.amb = uni(c->has_amb);
+    A.steps = uni_ptr(c->steps);
+    A.PT = uni_ptr(c->PTc);
+    A.codes = make_buf(uni_ptr(c->codes), (int)std::min<int64_t>((int64_t)uni(c->S) * uni(c->Ppad), INT32_MAX));
+    GBL char *parts = uni_ptr(c->parts);
+    const int blkB = block_bytes(A.I, sizeof(R));
     const int r = uni(c->root);
+    const GBL int32_t *wts = uni_ptr(c->wts);
+    const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
+    // the root is the last step of every pass that visits it
+    const bool in_regs = A.n > 0 && uni(c->last_step) == r && !(uni(c->flags[r]) & NF_MISSING);
+    const int rc = uni(c->cur[r]), rb = (mode == PR_PROP && uni(c->dirty[r])) ? 1 - rc : rc;
     double acc = 0;
-    if (r >= S) {
-        const int rb = uni(pb[r]) & PB_BUF;
-        const GBL V4<R> *rp = parts + rb * bufI + (size_t)(r - S) * Ppad;
-        const GBL int32_t *re = exps + rb * bufI + (size_t)(r - S) * Ppad;
-        const GBL int32_t *wts = uni_ptr(c->wts);
-        const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
-        if (tid == 0) c->bytes += (unsigned long long)P * (4 * sizeof(R) + 4 + 4);   // root partial, exponent, weight
-        for (int p = tid; p < P; p += BS) {
-            const int ex = re[p];
-            if (ex == GAPT) continue;
-            const V4<R> a = ld4<R>(rp + p);
-            const double L = p0 * (double)a.x + p1 * (double)a.y + p2 * (double)a.z + p3 * (double)a.w;
-            acc += (double)wts[p] * (log(L) + (double)ex * 0.69314718055994530942);
+    // whole waves of 64 patterns; wave w takes blocks w, w + BS / 64, ...
+    for (int pb = uni(tid & ~63); pb < P; pb += BS) {
+        const uint32_t lane = tid & 63, p = (uint32_t)pb + lane;
+        GBL char *blk = parts + (int64_t)(pb >> 6) * blkB;
+        ChildIn<R> o;
+        if (A.n > 0) o = prune_pattern<R>(A, blk, blkB, p);
+        if (!in_regs) o = slot_load<R>(make_buf(blk, blkB), rb * A.I + r - uni(c->S), lane, A.I);
+        // log sum_j pi_j L_j + exponent * ln 2; all-gap columns contribute 0
+        if (o.x != GAPT && (int)p < P) {
+            const double L = p0 * (double)o.v.x + p1 * (double)o.v.y + p2 * (double)o.v.z + p3 * (double)o.v.w;
+            acc += (double)wts[p] * (log(L) + (double)o.x * 0.69314718055994530942);
         }
     }
     return block_sum(acc, c->red);
 }
 
 // ------------------------------------------------------ ancestral sampling
+
+// A slot's partial and exponent at pattern l of a block (each lane its own block).
+template <typename R>
+__device__ __forceinline__ ChildIn<R> site_load(const GBL char *blk, uint32_t slot, uint32_t l, int I)
+{
+    ChildIn<R> in;
+    in.v = ld4<R>((const GBL V4<R> *)(blk + part_off<R>(slot)) + l);
+    in.x = ((const GBL int32_t *)(blk + exp_off<R>(slot, I)))[l];
+    return in;
+}
 
 // BPP_C::Update_Tg(tosample=true) (src/PhyloAcc-ST/bpp_c.cpp:672-733) for every
 // site, plus the per-branch transition counts that getEmission
@@ -528,14 +694,14 @@ template <typename R, int BS, int SH>
 __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c3)
 {
     const int tid = threadIdx.x, S = uni(c->S), n_int = uni(c->n_int), GG = uni(c->GG), Ppad = uni(c->Ppad);
-    const size_t bufI = (size_t)uni(c->I) * Ppad;
+    const int I = uni(c->I);
+    const int blkB = block_bytes(I, sizeof(R));
     const int r = uni(c->root);
     const uint32_t k0 = M->key0, k1 = M->key1;
     const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
     // the context's array pointers, read once: stores and atomics into LDS
     // arrays would otherwise make every use reload them
-    const GBL V4<R> *parts = uni_ptr(c->parts);
-    const GBL int32_t *exps = uni_ptr(c->exps);
+    const GBL char *parts = uni_ptr(c->parts);
     const GBL uint8_t *codes = uni_ptr(c->codes);
     const GBL int32_t *site = uni_ptr(c->site);
     GBL uint32_t *amb = uni_ptr(c->amb);
@@ -561,17 +727,18 @@ __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c
     }
     for (int g = tid; g < GG; g += BS) {
         const int p = site[g];
-        U4 blk = philox(0, (uint32_t)g, c2, c3, k0, k1);
+        const GBL char *blk = parts + (int64_t)(p >> 6) * blkB;
+        U4 rnd = philox(0, (uint32_t)g, c2, c3, k0, k1);
         {
-            const size_t off = cur[r] * bufI + (size_t)(r - S) * Ppad + p;
+            const ChildIn<R> in = site_load<R>(blk, cur[r] * I + r - S, p & 63, I);
             double pr[4];
-            if (exps[off] == GAPT) {
+            if (in.x == GAPT) {
                 pr[0] = p0; pr[1] = p1; pr[2] = p2; pr[3] = p3;
             } else {
-                const V4<R> a = ld4<R>(parts + off);
+                const V4<R> a = in.v;
                 pr[0] = p0 * (double)a.x; pr[1] = p1 * (double)a.y; pr[2] = p2 * (double)a.z; pr[3] = p3 * (double)a.w;
             }
-            tgs[(r - S) * BS + tid] = (uint8_t)categorical<4>(pr, u01(blk.x));
+            tgs[(r - S) * BS + tid] = (uint8_t)categorical<4>(pr, u01(rnd.x));
         }
         // internal nodes in reverse post-order, K at a time: a chunk's partial
         // loads do not depend on its draws, so they are all issued first.  A
@@ -603,16 +770,16 @@ __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c
                         if (!(f & NF_MISSING))
                             ex[j] = codes[(size_t)(kids & 0xffff) * Ppad + p] | (codes[(size_t)((uint32_t)kids >> 16) * Ppad + p] << 8);
                     } else if (!(f & NF_MISSING)) {
-                        const size_t off = uni(cur[s]) * bufI + (size_t)(s - S) * Ppad + p;
-                        ex[j] = exps[off];
-                        av[j] = ld4<R>(parts + off);
+                        const ChildIn<R> in = site_load<R>(blk, uni(cur[s]) * I + s - S, p & 63, I);
+                        ex[j] = in.x;
+                        av[j] = in.v;
                     }
                 }
             }
 #pragma unroll
             for (int j = 0; j < K; j++, t++) {
                 if (kb - j < 0) break;
-                if ((t & 3) == 0) blk = philox((uint32_t)(t >> 2), (uint32_t)g, c2, c3, k0, k1);
+                if ((t & 3) == 0) rnd = philox((uint32_t)(t >> 2), (uint32_t)g, c2, c3, k0, k1);
                 const int s = sn[j];
                 if (fl[j] & NF_MISSING) continue;
                 if ((fl[j] & NF_CHERRY) && ex[j] != GAPT) {
@@ -628,7 +795,7 @@ __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c
                 const LDS R *PT = PTc + 16 * s;
                 double pr[4] = {(double)PT[0 * 4 + tp] * (double)a.x, (double)PT[1 * 4 + tp] * (double)a.y,
                                 (double)PT[2 * 4 + tp] * (double)a.z, (double)PT[3 * 4 + tp] * (double)a.w};
-                const int ts = categorical<4>(pr, u01(pick(blk, t & 3)));
+                const int ts = categorical<4>(pr, u01(pick(rnd, t & 3)));
                 tgs[(s - S) * BS + tid] = (uint8_t)ts;
                 lds_add(&hist[s * 16 + tp * 4 + ts], 1u);
             }
@@ -1075,6 +1242,42 @@ __device__ __noinline__ void node_desc(LDS uint32_t *d, const int32_t *tab, int 
     d[3] = bits;
 }
 
+// Pruning order: post-order, the child with the larger subtree (in internal
+// nodes) first, child 0 on ties.  Subtree sizes go up the tree level by level
+// and subtree starts come down it; both live in the storage of the messages.
+template <typename R, int BS>
+__device__ __noinline__ void pruning_order(CP<R> c, const int32_t *tab, int N)
+{
+    const int tid = threadIdx.x, S = c->S, n_up = c->n_up, n_down = c->n_down, root = c->root;
+    const int32_t *ch0 = tab + tab_ch0(N), *ch1 = tab + tab_ch1(N);
+    LDS int32_t *size = (LDS int32_t *)c->E, *start = size + N;
+    for (int i = tid; i < N; i += BS) size[i] = 0;
+    __syncthreads();
+    for (int h = 0; h < n_up; h++) {
+        for (int q = (h == 0 ? 0 : c->upoff[h - 1]) + tid; q < c->upoff[h]; q += BS) {
+            const int s = c->up[q];
+            size[s] = 1 + size[ch0[s]] + size[ch1[s]];
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        start[root] = 0;
+        c->porder[size[root] - 1] = (int16_t)root;
+    }
+    __syncthreads();
+    for (int d = 0; d < n_down; d++) {
+        for (int q = (d == 0 ? 0 : c->downoff[d - 1]) + tid; q < c->downoff[d]; q += BS) {
+            const int s = c->down[q], p = c->par[s];
+            if (s < S) continue;
+            const int a = ch0[p], b = ch1[p], first = size[a] >= size[b] ? a : b;
+            const int st = start[p] + (s == first ? 0 : size[first]);
+            start[s] = st;
+            c->porder[st + size[s] - 1] = (int16_t)s;
+        }
+        __syncthreads();
+    }
+}
+
 template <typename R, int BS, int SH>
 __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int work)
 {
@@ -1090,8 +1293,7 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
         char *base = A->scratch + (size_t)blockIdx.x * A->slot_bytes;
         const int64_t bo = A->big_off ? A->big_off[work] : -1;
         char *pbase = bo >= 0 ? A->big + bo : base + A->off_parts;
-        c->parts = (GBL V4<R> *)pbase;
-        c->exps = (GBL int32_t *)(pbase + chain_exps_off(N, M->S, E.Ppad, sizeof(R)));
+        c->parts = (GBL char *)pbase;
         c->plin = (GBL double *)(base + A->off_plin);
         c->logt = (GBL double *)(base + A->off_logt);
         c->amb = (GBL uint32_t *)(base + A->off_amb);
@@ -1125,6 +1327,7 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
         const int s = c->inodes[q];
         if (is_cherry(tab, N, M->S, E.root, s)) c->flags[s] |= NF_CHERRY;
     }
+    pruning_order<R, BS>(c, tab, N);
     // null-rate tables (rate 1), fixed for the element
     for (int q = tid; q < c->n_nodes - 1; q += BS) class_table<R>(M, c, 0, c->nodes[q], 1.0, 0);
     __syncthreads();

@@ -56,6 +56,7 @@ struct Ctx {
     LDS int16_t *par, *nodes, *inodes, *porder, *up, *upoff, *down, *downoff, *tz;
     LDS uint32_t *desc;    // [I][4] static pruning descriptor of each internal node (node_desc)
     LDS uint32_t *steps;   // [I][4] the steps of a pass (build_steps)
+    LDS uint32_t *srec;    // [I][2] the steps of the sampler (sample_steps)
     LDS uint8_t *flags, *fixZ, *dirty, *cur, *changed;
     LDS int8_t *Z, *maxZ;
     LDS double *E, *beta;
@@ -67,7 +68,7 @@ struct Ctx {
     double TMf[9], TMn[9];  // log_TM_Int for fixZ / free nodes, [i*3+j] = log P(child i | parent j)
     double red[16];
     unsigned long long bytes;   // algorithmic HBM bytes of this element's passes (see prune / sample_sites)
-    int accept_n, accept_c, max_m, skip, accept, fail, work, nch, n_steps, last_step;   // fail: PA_F_* bits
+    int accept_n, accept_c, max_m, skip, accept, fail, work, nch, n_steps, last_step, n_stored, n_cherry, n_leaf;   // fail: PA_F_* bits
 };
 
 template <typename R>
@@ -121,6 +122,7 @@ __host__ __device__ size_t smem_arrays(int N, int S, int BS, LDS char *base, CP<
     o = al(o, 16);      // descriptors are read as 16-byte vectors
     if constexpr (BIND) c->desc = (LDS uint32_t *)(base + o);
     o += (size_t)16 * (I > 0 ? I : 1);
+    PA_TAKE(srec, uint32_t, 2 * (I > 0 ? I : 1));
     PA_TAKE(par, int16_t, N);
     PA_TAKE(nodes, int16_t, N);
     PA_TAKE(inodes, int16_t, N);
@@ -189,6 +191,18 @@ __device__ __forceinline__ Buf make_buf(T *base, int bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc((void *)(T *)base, 0, bytes, 0x00027000);
 }
+__device__ __forceinline__ int code_bytes(int S, int Ppad)
+{
+    const uint64_t n = (uint64_t)S * (uint32_t)Ppad;
+    return (int)(uint32_t)(n < 0xffffffffu ? n : 0xffffffffu);
+}
+
+template <int... J, typename F>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, J...>, F &&f) { (f(std::integral_constant<int, J>()), ...); }
+// f(0) ... f(n - 1) with constant arguments: what it indexes stays in registers
+template <int n, typename F>
+__device__ __forceinline__ void each(F &&f) { each_of(std::make_integer_sequence<int, n>(), f); }
+
 template <typename R>
 __device__ __forceinline__ V4<R> buf_ld4(Buf b, uint32_t lane_off, uint32_t off)
 {
@@ -648,7 +662,7 @@ __device__ __noinline__ double prune(MP M, CP<R> c, int mode, int cls)
     A.amb = uni(c->has_amb);
     A.steps = uni_ptr(c->steps);
     A.PT = uni_ptr(c->PTc);
-    A.codes = make_buf(uni_ptr(c->codes), (int)std::min<int64_t>((int64_t)uni(c->S) * uni(c->Ppad), INT32_MAX));
+    A.codes = make_buf(uni_ptr(c->codes), code_bytes(uni(c->S), uni(c->Ppad)));
     GBL char *parts = uni_ptr(c->parts);
     const int blkB = block_bytes(A.I, sizeof(R));
     const int r = uni(c->root);
@@ -676,151 +690,177 @@ __device__ __noinline__ double prune(MP M, CP<R> c, int mode, int cls)
 
 // ------------------------------------------------------ ancestral sampling
 
-// A slot's partial and exponent at pattern l of a block (each lane its own block).
-template <typename R>
-__device__ __forceinline__ ChildIn<R> site_load(const GBL char *blk, uint32_t slot, uint32_t l, int I)
-{
-    ChildIn<R> in;
-    in.v = ld4<R>((const GBL V4<R> *)(blk + part_off<R>(slot)) + l);
-    in.x = ((const GBL int32_t *)(blk + exp_off<R>(slot, I)))[l];
-    return in;
-}
+// One step of the sampler: an internal node, in reverse post-order (step 0
+// the root).  Two words, built when the element is bound (sample_steps):
+//   r0: node | parent << 10 | SR_* bits
+//   r1: the node's leaf children A | B << 10 (0: none)
+enum { SR_ID = 0x3ff, SR_PAR_SHIFT = 10, SR_MISS = 1 << 20, SR_CHERRY = 1 << 21,
+       SR_PREV = 1 << 22,                          // the parent is the step before
+       SR_LEAF_A = 1 << 23, SR_LEAF_B = 1 << 24,   // leaf children that are counted
+       SR_MISS_A = 1 << 25, SR_MISS_B = 1 << 26,   // a cherry's missing leaves
+       SR_CUR = 1 << 27 };                         // the buffer holding the node's partial (follows cur)
 
 // BPP_C::Update_Tg(tosample=true) (src/PhyloAcc-ST/bpp_c.cpp:672-733) for every
 // site, plus the per-branch transition counts that getEmission
 // (bpp_c2.cpp:355-390) sums over.  Uniform for site g, sampling position t
 // (0 = root, then internal nodes in reverse post-order): ANC stream, c1 = g.
+//
+// One thread per site, whole waves.  As in a pass, what bounds it is the time
+// of one step: the steps' words are read ahead, the loads of the next K steps
+// are in flight (the same four loads every step, so that their waits are
+// counted), the parent's base is in a register when the parent was the step
+// before and otherwise read a step early, and a node counts its own leaf
+// children, whose parent's base it has just drawn.
 template <typename R, int BS, int SH>
 __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c3)
 {
-    const int tid = threadIdx.x, S = uni(c->S), n_int = uni(c->n_int), GG = uni(c->GG), Ppad = uni(c->Ppad);
-    const int I = uni(c->I);
-    const int blkB = block_bytes(I, sizeof(R));
-    const int r = uni(c->root);
-    const uint32_t k0 = M->key0, k1 = M->key1;
+    constexpr int K = Shape<R, SH>::K, UN = K < 4 ? 4 : K;     // steps unrolled: whole blocks of four draws
+    const int tid = threadIdx.x, S = uni(c->S), I = uni(c->I), n_int = uni(c->n_int), GG = uni(c->GG), Ppad = uni(c->Ppad);
+    const int blkB = block_bytes(I, sizeof(R)), amb_on = uni(c->has_amb);
+    const uint32_t k0 = (uint32_t)uni((int)M->key0), k1 = (uint32_t)uni((int)M->key1);
     const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
-    // the context's array pointers, read once: stores and atomics into LDS
-    // arrays would otherwise make every use reload them
     const GBL char *parts = uni_ptr(c->parts);
-    const GBL uint8_t *codes = uni_ptr(c->codes);
+    const Buf codes = make_buf(uni_ptr(c->codes), code_bytes(S, Ppad));
     const GBL int32_t *site = uni_ptr(c->site);
     GBL uint32_t *amb = uni_ptr(c->amb);
-    LDS uint8_t *tgs = uni_ptr(c->tgs);
+    LDS uint8_t *tgs = uni_ptr(c->tgs) + tid;
     LDS uint32_t *hist = uni_ptr(c->hist);
-    const LDS int16_t *inodes = uni_ptr(c->inodes), *par = uni_ptr(c->par);
-    const LDS uint8_t *flags = uni_ptr(c->flags), *cur = uni_ptr(c->cur);
-    const LDS uint32_t *desc = uni_ptr(c->desc);
+    const LDS uint32_t *srec = uni_ptr(c->srec);
     const LDS R *PTc = uni_ptr(c->PTc);
     for (int i = tid; i < 16 * c->N; i += BS) hist[i] = 0;   // shares storage with the proposal matrices
     __syncthreads();
     if (tid == 0) {
         // per site: pattern index, root partial, each non-missing internal node's partial
         // (a cherry's two leaf codes), each leaf code
+        c->bytes += (unsigned long long)GG * (4 + (4 * sizeof(R) + 4) * c->n_stored + 2 * c->n_cherry + c->n_leaf);
+    }
+    const uint32_t r_slot = (srec[0] & SR_ID) - S;
+    for (int gb = uni(tid & ~63); gb < GG; gb += BS) {
+        const int g = gb + (tid & 63);
+        const bool on = g < GG;
+        const int p = site[on ? g : GG - 1];
+        // this pattern's entries of slot 0
+        const GBL char *pp = parts + (int64_t)(p >> 6) * blkB + (p & 63) * sizeof(V4<R>);
+        const GBL char *pe = parts + (int64_t)(p >> 6) * blkB + exp_off<R>(0, I) + (p & 63) * 4;
+        uint32_t r0[K], r1[K], nr0 = srec[0], nr1 = srec[1];
+        ChildIn<R> in[K];
+        int cdA[K], cdB[K];
+        auto fetch = [&](auto J, int t) __attribute__((always_inline)) {
+            constexpr int j = decltype(J)::value;
+            r0[j] = (uint32_t)uni((int)nr0);
+            r1[j] = (uint32_t)uni((int)nr1);
+            const LDS uint32_t *nx = srec + 2 * (t + 1 < n_int ? t + 1 : t);
+            nr0 = nx[0];
+            nr1 = nx[1];
+            // a cherry has no stored partial: the load goes where the root's went
+            uint32_t slot = (r0[j] & (SR_CHERRY | SR_MISS)) ? r_slot : (r0[j] & SR_ID) - S;
+            slot += ((r0[j] & SR_CUR) && !(r0[j] & (SR_CHERRY | SR_MISS))) ? I : 0;
+            in[j].v = ld4<R>((const GBL V4<R> *)(pp + (uint64_t)part_off<R>(slot)));
+            in[j].x = *(const GBL int32_t *)(pe + (uint64_t)(slot * 256));
+            cdA[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, (r1[j] & SR_ID) * Ppad, 0);
+            cdB[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, ((r1[j] >> 10) & SR_ID) * Ppad, 0);
+        };
+        U4 rnd{0, 0, 0, 0};
+        int ts = 0, tp = 0;
+        auto count_leaf = [&](int y, int code) __attribute__((always_inline)) {
+            if (on && code < 4) lds_add(&hist[y * 16 + ts * 4 + code], 1u);
+            if (amb_on && on && code > PA_OTHER_CODE)
+                __hip_atomic_fetch_add(&amb[y * 24 + ts * 6 + (code - 6)], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        auto step = [&](auto JJ, int t) __attribute__((always_inline)) {
+            constexpr int jj = decltype(JJ)::value, j = jj % K;
+            if ((jj & 3) == 0) rnd = philox((uint32_t)(t >> 2), (uint32_t)g, c2, c3, k0, k1);
+            const double u = u01(pick(rnd, jj & 3));
+            const uint32_t w0 = r0[j], w1 = r1[j];
+            const int s = w0 & SR_ID;
+            const int tp_read = tp & 3;
+            // the next step's parent, unless it is this node
+            if (t + 1 < n_int) tp = tgs[(((r0[(j + 1) % K] >> SR_PAR_SHIFT) & SR_ID) - S) * BS];
+            if (!(w0 & SR_MISS)) {
+                ChildIn<R> a;
+                if (w0 & SR_CHERRY) {
+                    // the partial a pass would have stored: the leaves' messages combined
+                    V4<R> ma, mb;
+                    int e = 0;
+                    bool ga, gb2;
+                    message<R, SK_LEAF>(PTc + 16 * (w1 & SR_ID), amb_on, cdA[j], in[j], ma, e, ga);
+                    message<R, SK_LEAF>(PTc + 16 * ((w1 >> 10) & SR_ID), amb_on, cdB[j], in[j], mb, e, gb2);
+                    if (w0 & SR_MISS_A) ma.x = ma.y = ma.z = ma.w = (R)1;
+                    if (w0 & SR_MISS_B) mb.x = mb.y = mb.z = mb.w = (R)1;
+                    a = combine<R>(ma, mb, 0, ga && gb2);
+                } else {
+                    a.v = in[j].v;
+                    a.x = in[j].x;
+                }
+                const bool has = a.x != GAPT;       // else no base below it at this site: not drawn
+                double pr[4];
+                int from = 0;
+                if (t == 0) {
+                    pr[0] = has ? p0 * (double)a.v.x : p0; pr[1] = has ? p1 * (double)a.v.y : p1;
+                    pr[2] = has ? p2 * (double)a.v.z : p2; pr[3] = has ? p3 * (double)a.v.w : p3;
+                } else {
+                    from = (w0 & SR_PREV) ? ts : tp_read;
+                    const LDS R *PT = PTc + 16 * s + from;
+                    pr[0] = (double)PT[0] * (double)a.v.x; pr[1] = (double)PT[4] * (double)a.v.y;
+                    pr[2] = (double)PT[8] * (double)a.v.z; pr[3] = (double)PT[12] * (double)a.v.w;
+                }
+                ts = categorical<4>(pr, u);
+                tgs[(s - S) * BS] = (uint8_t)ts;
+                if (t != 0 && on && has) lds_add(&hist[s * 16 + from * 4 + ts], 1u);
+                if (w0 & SR_LEAF_A) count_leaf(w1 & SR_ID, cdA[j]);
+                if (w0 & SR_LEAF_B) count_leaf((w1 >> 10) & SR_ID, cdB[j]);
+            }
+            if (t + K < n_int) fetch(std::integral_constant<int, j>(), t + K);
+        };
+        each<K>([&](auto J) __attribute__((always_inline)) { if (decltype(J)::value < n_int) fetch(J, decltype(J)::value); });
+        for (int t0 = 0; t0 < n_int; t0 += UN)
+            each<UN>([&](auto J) __attribute__((always_inline)) { if (t0 + decltype(J)::value < n_int) step(J, t0 + decltype(J)::value); });
+    }
+}
+
+// The sampler's step words (layout at SR_*) and the node counts its bytes
+// are counted from.
+template <typename R, int BS>
+__device__ __noinline__ void sample_steps(CP<R> c)
+{
+    const int S = c->S, n_int = c->n_int;
+    for (int t = threadIdx.x; t < n_int; t += BS) {
+        const int s = c->inodes[n_int - 1 - t];
+        const LDS uint32_t *dd = c->desc + 4 * (s - S);
+        const int x0 = dd[0] & 0xffff, x1 = dd[0] >> 16;
+        const int f = c->flags[s], f0 = c->flags[x0], f1 = c->flags[x1];
+        uint32_t w0 = (uint32_t)s | ((f & NF_MISSING) ? SR_MISS : 0) | ((f & NF_CHERRY) ? SR_CHERRY : 0), w1 = 0;
+        if (t > 0) {
+            const int par = c->par[s];
+            w0 |= (uint32_t)par << SR_PAR_SHIFT;
+            if (par == c->inodes[n_int - t]) w0 |= SR_PREV;
+        } else {
+            w0 |= (uint32_t)s << SR_PAR_SHIFT;      // not read
+        }
+        if (x0 < S) {
+            w1 |= (uint32_t)x0;
+            if (f0 & NF_MISSING) w0 |= SR_MISS_A;
+            else if (f0 & NF_IN_TREE) w0 |= SR_LEAF_A;
+        }
+        if (x1 < S) {
+            w1 |= (uint32_t)x1 << 10;
+            if (f1 & NF_MISSING) w0 |= SR_MISS_B;
+            else if (f1 & NF_IN_TREE) w0 |= SR_LEAF_B;
+        }
+        c->srec[2 * t] = w0;
+        c->srec[2 * t + 1] = w1;
+    }
+    if (threadIdx.x == 0) {
         int nint = 0, nch = 0, nleaf = 0;
         for (int k = 0; k < n_int; k++) {
-            const uint8_t f = flags[inodes[k]];
+            const uint8_t f = c->flags[c->inodes[k]];
             if (f & NF_MISSING) continue;
             if (f & NF_CHERRY) nch++; else nint++;
         }
-        for (int q = 0; q < S; q++) nleaf += (flags[q] & NF_IN_TREE) && !(flags[q] & NF_MISSING);
-        c->bytes += (unsigned long long)GG * (4 + (4 * sizeof(R) + 4) * nint + 2 * nch + nleaf);
-    }
-    for (int g = tid; g < GG; g += BS) {
-        const int p = site[g];
-        const GBL char *blk = parts + (int64_t)(p >> 6) * blkB;
-        U4 rnd = philox(0, (uint32_t)g, c2, c3, k0, k1);
-        {
-            const ChildIn<R> in = site_load<R>(blk, cur[r] * I + r - S, p & 63, I);
-            double pr[4];
-            if (in.x == GAPT) {
-                pr[0] = p0; pr[1] = p1; pr[2] = p2; pr[3] = p3;
-            } else {
-                const V4<R> a = in.v;
-                pr[0] = p0 * (double)a.x; pr[1] = p1 * (double)a.y; pr[2] = p2 * (double)a.z; pr[3] = p3 * (double)a.w;
-            }
-            tgs[(r - S) * BS + tid] = (uint8_t)categorical<4>(pr, u01(rnd.x));
-        }
-        // internal nodes in reverse post-order, K at a time: a chunk's partial
-        // loads do not depend on its draws, so they are all issued first.  A
-        // cherry's slot holds its two leaf codes (low and second byte) until
-        // its partial is recomputed.
-        constexpr int K = Shape<R, SH>::K;
-        int t = 1;
-        for (int kb = n_int - 2; kb >= 0; kb -= K) {
-            // node ids, flags, buffers and cherry leaves are the same on every
-            // lane: they live in scalar registers
-            int ex[K], sn[K], fl[K], kid[K];
-            V4<R> av[K];
-#pragma unroll
-            for (int j = 0; j < K; j++) {
-                const int k = kb - j;
-                ex[j] = GAPT;
-                sn[j] = 0;
-                fl[j] = NF_MISSING;
-                kid[j] = 0;
-                av[j].x = av[j].y = av[j].z = av[j].w = (R)0;
-                if (k >= 0) {
-                    const int s = uni(inodes[k]);
-                    const int f = uni(flags[s]);
-                    sn[j] = s;
-                    fl[j] = f;
-                    if (f & NF_CHERRY) {
-                        const int kids = uni((int)desc[4 * (s - S)]);
-                        kid[j] = kids;
-                        if (!(f & NF_MISSING))
-                            ex[j] = codes[(size_t)(kids & 0xffff) * Ppad + p] | (codes[(size_t)((uint32_t)kids >> 16) * Ppad + p] << 8);
-                    } else if (!(f & NF_MISSING)) {
-                        const ChildIn<R> in = site_load<R>(blk, uni(cur[s]) * I + s - S, p & 63, I);
-                        ex[j] = in.x;
-                        av[j] = in.v;
-                    }
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < K; j++, t++) {
-                if (kb - j < 0) break;
-                if ((t & 3) == 0) rnd = philox((uint32_t)(t >> 2), (uint32_t)g, c2, c3, k0, k1);
-                const int s = sn[j];
-                if (fl[j] & NF_MISSING) continue;
-                if ((fl[j] & NF_CHERRY) && ex[j] != GAPT) {
-                    const int yA = kid[j] & 0xffff, yB = (int)((uint32_t)kid[j] >> 16);
-                    const ChildIn<R> in = cherry_in<R>(PTc + 16 * yA, PTc + 16 * yB, uni(flags[yA]) & NF_MISSING,
-                                                       uni(flags[yB]) & NF_MISSING, false, ex[j] & 255, ex[j] >> 8);
-                    ex[j] = in.x;
-                    av[j] = in.v;
-                }
-                if (ex[j] == GAPT) continue;     // missing node, or an all-gap subtree at this site
-                const int tp = tgs[(uni(par[s]) - S) * BS + tid];
-                const V4<R> a = av[j];
-                const LDS R *PT = PTc + 16 * s;
-                double pr[4] = {(double)PT[0 * 4 + tp] * (double)a.x, (double)PT[1 * 4 + tp] * (double)a.y,
-                                (double)PT[2 * 4 + tp] * (double)a.z, (double)PT[3 * 4 + tp] * (double)a.w};
-                const int ts = categorical<4>(pr, u01(pick(rnd, t & 3)));
-                tgs[(s - S) * BS + tid] = (uint8_t)ts;
-                lds_add(&hist[s * 16 + tp * 4 + ts], 1u);
-            }
-        }
-        // leaves, 8 codes loaded at a time
-        for (int sb = 0; sb < S; sb += 8) {
-            int cd[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int s = sb + j;
-                cd[j] = PA_GAP_CODE;
-                if (s < S) {
-                    const int f = uni(flags[s]);
-                    if ((f & NF_IN_TREE) && !(f & NF_MISSING)) cd[j] = codes[(size_t)s * Ppad + p];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int s = sb + j, code = cd[j];
-                if (code == PA_GAP_CODE || code == PA_OTHER_CODE) continue;
-                const int tp = tgs[(uni(par[s]) - S) * BS + tid];
-                if (code < 4) lds_add(&hist[s * 16 + tp * 4 + code], 1u);
-                else __hip_atomic_fetch_add(&amb[s * 24 + tp * 6 + (code - 6)], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
-        }
+        for (int q = 0; q < S; q++) nleaf += (c->flags[q] & NF_IN_TREE) && !(c->flags[q] & NF_MISSING);
+        c->n_stored = nint;
+        c->n_cherry = nch;
+        c->n_leaf = nleaf;
     }
 }
 
@@ -1128,7 +1168,10 @@ __device__ __forceinline__ void sample_rate(MP M, CP<R> c, int ms, int m, int re
         if (c->accept) {
             for (int q = tid; q < c->n_int; q += BS) {
                 const int s = c->inodes[q];
-                if (c->dirty[s] && !(c->flags[s] & NF_MISSING)) c->cur[s] ^= 1;
+                if (c->dirty[s] && !(c->flags[s] & NF_MISSING)) {
+                    c->cur[s] ^= 1;
+                    c->srec[2 * (c->n_int - 1 - q)] ^= SR_CUR;
+                }
             }
         }
     }
@@ -1328,6 +1371,8 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
         if (is_cherry(tab, N, M->S, E.root, s)) c->flags[s] |= NF_CHERRY;
     }
     pruning_order<R, BS>(c, tab, N);
+    __syncthreads();
+    sample_steps<R, BS>(c);
     // null-rate tables (rate 1), fixed for the element
     for (int q = tid; q < c->n_nodes - 1; q += BS) class_table<R>(M, c, 0, c->nodes[q], 1.0, 0);
     __syncthreads();
@@ -1356,6 +1401,7 @@ __device__ __noinline__ void init_model(MP M, CP<R> c, int resZ)
         c->fixZ[s] = (uint8_t)fz;
         c->cur[s] = 0;
     }
+    for (int t = tid; t < c->n_int; t += BS) c->srec[2 * t] &= ~(uint32_t)SR_CUR;
     if (tid == 0) {
         c->prop_c = 1.2;
         c->prop_n = (double)1 / c->GG * 10;

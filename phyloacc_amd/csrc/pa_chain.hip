@@ -53,13 +53,14 @@ struct Ctx {
     GBL uint32_t *amb;     // [S][24]
     const GBL double *dist2;   // [N] branch lengths (element node table)
     // LDS arrays
-    LDS int16_t *par, *nodes, *inodes, *porder, *up, *upoff, *down, *downoff, *tz;
+    LDS int16_t *par, *nodes, *inodes, *porder, *upoff;
+    LDS uint32_t *urec;    // [I] internal nodes by level: node | child 0 << 10 | child 1 << 20
     LDS uint32_t *desc;    // [I][4] static pruning descriptor of each internal node (node_desc)
     LDS uint32_t *steps;   // [I][4] the steps of a pass (build_steps)
     LDS uint32_t *srec;    // [I][2] the steps of the sampler (sample_steps)
     LDS uint8_t *flags, *fixZ, *dirty, *cur, *changed;
     LDS int8_t *Z, *maxZ;
-    LDS double *E, *beta;
+    LDS double *E, *msg;   // [N][3] emissions, then Z messages at a node; messages to its parent
     LDS R *PTc, *PTp;      // [N][16], PT[i*4+j] = P_{j->i}
     LDS uint32_t *hist, *cnt9;
     LDS uint8_t *tgs;
@@ -112,7 +113,7 @@ __host__ __device__ size_t smem_arrays(int N, int S, int BS, LDS char *base, CP<
         o += al(szB, 32);
         if constexpr (BIND) {
             c->E = (LDS double *)(base + o);
-            c->beta = (LDS double *)(base + o) + 3 * N;
+            c->msg = (LDS double *)(base + o) + 3 * N;
             c->tgs = (LDS uint8_t *)(base + o);
             c->cnt9 = (LDS uint32_t *)(base + o);
             c->steps = (LDS uint32_t *)(base + o);
@@ -123,15 +124,12 @@ __host__ __device__ size_t smem_arrays(int N, int S, int BS, LDS char *base, CP<
     if constexpr (BIND) c->desc = (LDS uint32_t *)(base + o);
     o += (size_t)16 * (I > 0 ? I : 1);
     PA_TAKE(srec, uint32_t, 2 * (I > 0 ? I : 1));
+    PA_TAKE(urec, uint32_t, I > 0 ? I : 1);
     PA_TAKE(par, int16_t, N);
     PA_TAKE(nodes, int16_t, N);
     PA_TAKE(inodes, int16_t, N);
     PA_TAKE(porder, int16_t, I > 0 ? I : 1);
-    PA_TAKE(up, int16_t, N);
-    PA_TAKE(upoff, int16_t, N + 1);
-    PA_TAKE(down, int16_t, N);
-    PA_TAKE(downoff, int16_t, N + 1);
-    PA_TAKE(tz, int16_t, N);
+    PA_TAKE(upoff, int16_t, I + 1);
     PA_TAKE(flags, uint8_t, N);
     PA_TAKE(fixZ, uint8_t, N);
     PA_TAKE(dirty, uint8_t, N);
@@ -728,6 +726,8 @@ __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c
     const LDS uint32_t *srec = uni_ptr(c->srec);
     const LDS R *PTc = uni_ptr(c->PTc);
     for (int i = tid; i < 16 * c->N; i += BS) hist[i] = 0;   // shares storage with the proposal matrices
+    if (amb_on)
+        for (int i = tid; i < 24 * S; i += BS) amb[i] = 0;
     __syncthreads();
     if (tid == 0) {
         // per site: pattern index, root partial, each non-missing internal node's partial
@@ -864,51 +864,65 @@ __device__ __noinline__ void sample_steps(CP<R> c)
     }
 }
 
-// getEmission (src/PhyloAcc-ST/bpp_c2.cpp:355-390): E[s][k] from the counts.
+// getEmission (src/PhyloAcc-ST/bpp_c2.cpp:355-390): E[s][k] from the counts,
+// one thread per (branch, class), its sixteen log entries loaded together.
 template <typename R, int BS, int SH>
 __device__ __noinline__ void emissions(CP<R> c)
 {
-    const int N = c->N;
-    for (int q = threadIdx.x; q < c->n_nodes - 1; q += BS) {
-        const int s = c->nodes[q];
-        if (c->flags[s] & NF_MISSING) continue;
-        LDS uint32_t *h = c->hist + s * 16;
+    const int N = uni(c->N), n_item = 3 * (uni(c->n_nodes) - 1);
+    const LDS int16_t *nodes = uni_ptr(c->nodes);
+    const LDS uint8_t *flags = uni_ptr(c->flags);
+    for (int it = threadIdx.x; it < n_item; it += BS) {
+        const int q = it / 3, k = it - 3 * q, s = nodes[q];
+        if (flags[s] & NF_MISSING) continue;
+        const GBL double *L = c->logt + ((size_t)k * N + s) * 16;
+        const LDS uint32_t *h = c->hist + s * 16;
+        double l[16];
         uint32_t n[16];
 #pragma unroll
-        for (int i = 0; i < 16; i++) { n[i] = h[i]; h[i] = 0; }
-#pragma unroll 1
-        for (int k = 0; k < 3; k++) {
-            const GBL double *L = c->logt + ((size_t)k * N + s) * 16;
-            double e = 0;
+        for (int i = 0; i < 16; i++) l[i] = L[i];
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+        for (int i = 0; i < 16; i++) n[i] = h[i];
+        double e = 0;
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (n[j * 4 + i]) e += (double)n[j * 4 + i] * L[i * 4 + j];
-            c->E[s * 3 + k] = e;
-        }
-        if (c->has_amb && s < c->S) {
-            GBL uint32_t *a = c->amb + s * 24;
-            for (int k = 0; k < 3; k++) {
-                const GBL double *P = c->plin + ((size_t)k * N + s) * 16;
-                double e = 0;
-                for (int j = 0; j < 4; j++)
-                    for (int x = 0; x < 6; x++) {
-                        const uint32_t cnt = a[j * 6 + x];
-                        if (!cnt) continue;
-                        const int code = 6 + x;
-                        const int b1 = (code == 6 || code == 9 || code == 11) ? 0 : (code == 7 || code == 10) ? 1 : 2;
-                        const int b2 = (code == 6 || code == 10) ? 2 : (code == 9) ? 1 : 3;
-                        e += (double)cnt * log(P[j * 4 + b1] + P[j * 4 + b2]);
-                    }
-                c->E[s * 3 + k] += e;
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const double t = e + (double)n[j * 4 + i] * l[i * 4 + j];
+                e = n[j * 4 + i] ? t : e;
             }
-            for (int i = 0; i < 24; i++) a[i] = 0;
+        if (c->has_amb && s < c->S) {
+            const GBL uint32_t *a = c->amb + s * 24;
+            const GBL double *P = c->plin + ((size_t)k * N + s) * 16;
+            double ea = 0;
+            for (int j = 0; j < 4; j++)
+                for (int x = 0; x < 6; x++) {
+                    const uint32_t cnt = a[j * 6 + x];
+                    if (!cnt) continue;
+                    const int code = 6 + x;
+                    const int b1 = (code == 6 || code == 9 || code == 11) ? 0 : (code == 7 || code == 10) ? 1 : 2;
+                    const int b2 = (code == 6 || code == 10) ? 2 : (code == 9) ? 1 : 3;
+                    ea += (double)cnt * log(P[j * 4 + b1] + P[j * 4 + b2]);
+                }
+            e += ea;
         }
+        c->E[s * 3 + k] = e;
     }
 }
 
 // ----------------------------------------------------------------- Z update
+
+// exp(a - m), exp(b - m), exp(d - m) for m the largest of the three: the
+// largest one's is 1 (NaN when m is infinite), so two exponentials do.
+__device__ __forceinline__ void exp3(double a, double b, double d, double m, double &ea, double &eb, double &ed)
+{
+    const double one = 1.0 + (m - m);
+    const bool am = a == m, bm = !am && b == m;
+    const double x = exp((am ? b : a) - m), y = exp((am || bm ? d : b) - m);
+    ea = am ? one : x;
+    eb = am ? x : (bm ? one : y);
+    ed = am || bm ? y : one;
+}
 
 // log sum_i exp(T[i*3+j] + y[i]) for parent class j, with the column's own
 // maximum taken out first (log_multi2, src/PhyloAcc-ST/bpp.hpp:447-460);
@@ -918,84 +932,125 @@ __device__ __forceinline__ double log_col(const LDS double *T, int j, double y0,
     const double a = T[j] + y0, b = T[3 + j] + y1, d = T[6 + j] + y2;
     const double mx = fmax(a, fmax(b, d));
     if (mx == -INFINITY) return -INFINITY;
-    return mx + log(exp(a - mx) + exp(b - mx) + exp(d - mx));
+    double ea, eb, ed;
+    exp3(a, b, d, mx, ea, eb, ed);
+    return mx + log(ea + eb + ed);
 }
 
-// BPP_C::Update_Z_subtree (src/PhyloAcc-ST/bpp_c.cpp:1182-1293) in log space,
-// one tree level per step: upward messages by height, then top-down draws by
-// depth.  The draw for node s uses Z-stream slot tz[s].  Log space matters:
-// over thousands of sites the classes' emissions differ by thousands of
-// nats, and products of linear messages would underflow to zero.
+// BPP_C::Update_Z_subtree (src/PhyloAcc-ST/bpp_c.cpp:1182-1293) in log space:
+// messages up the tree, then draws down it; the draw for node s uses Z-stream
+// slot tz[s], its place in the reverse post-order.  Log space matters: over
+// thousands of sites the classes' emissions differ by thousands of nats, and
+// products of linear messages would underflow to zero.
+//
+// The phase is a chain of dependent logarithms and exponentials, so only what
+// depends on the level below is left in the chain: the leaves' messages are
+// computed by all threads at once; one wave then takes the internal levels, a
+// lane per (node, parent class), without barriers; and the draws are tabled
+// for every node and every class its parent could take, all at once, so that
+// going down the tree is following each node's ancestors through those
+// tables.
 template <typename R, int BS, int SH>
 __device__ __noinline__ void update_Z(MP M, CP<R> c, uint32_t c2, uint32_t c3)
 {
     const int tid = threadIdx.x;
     const Key key{M->key0, M->key1};
-    for (int q = tid; q < c->n_nodes; q += BS) {
-        const int s = c->nodes[q];
-        double e0, e1, e2;
-        if (s == c->root) { e0 = e1 = e2 = 0; }
-        else if (c->flags[s] & NF_MISSING) { e0 = log(M->nconstomis); e1 = log(M->constomis); e2 = log(M->nconstomis); }
-        else { e0 = c->E[s * 3]; e1 = c->E[s * 3 + 1]; e2 = c->E[s * 3 + 2]; }
-        c->beta[s * 3 + 0] = e0;
-        c->beta[s * 3 + 1] = e1;
-        c->beta[s * 3 + 2] = c->fixZ[s] ? -INFINITY : e2;
+    const int n_nodes = uni(c->n_nodes), S = uni(c->S), N = uni(c->N), root = uni(c->root), n_up = uni(c->n_up);
+    const LDS int16_t *nodes = uni_ptr(c->nodes), *par = uni_ptr(c->par), *upoff = uni_ptr(c->upoff);
+    const LDS uint32_t *urec = uni_ptr(c->urec);
+    const LDS uint8_t *flags = uni_ptr(c->flags), *fixZ = uni_ptr(c->fixZ);
+    const LDS double *TMf = uni_ptr(c->TMf), *TMn = uni_ptr(c->TMn);
+    LDS double *beta = uni_ptr(c->E), *msg = uni_ptr(c->msg);      // beta starts as the emissions
+    for (int q = tid; q < n_nodes; q += BS) {
+        const int s = nodes[q];
+        if (s == root) {
+            beta[s * 3] = beta[s * 3 + 1] = beta[s * 3 + 2] = 0;
+        } else if (flags[s] & NF_MISSING) {
+            beta[s * 3] = beta[s * 3 + 2] = log(M->nconstomis);
+            beta[s * 3 + 1] = log(M->constomis);
+        }
+        if (fixZ[s]) beta[s * 3 + 2] = -INFINITY;
         c->changed[s] = 0;
         c->dirty[s] = 0;
     }
     if (tid == 0) c->nch = 0;
     __syncthreads();
-    const int n_up = c->n_up, n_down = c->n_down;
-    for (int h = 0; h < n_up; h++) {
-        // one lane per (node, parent class): the classes' messages are independent
-        const int a = h == 0 ? 0 : c->upoff[h - 1], b = c->upoff[h];
-        for (int q = 3 * a + tid; q < 3 * b; q += BS) {
-            const int p = c->up[q / 3], j = q - 3 * (q / 3);
-            double bj = c->beta[p * 3 + j];
-            const uint32_t kids = c->desc[4 * (p - c->S)];
-            for (int w = 0; w < 2; w++) {
-                const int x = w ? (int)(kids >> 16) : (int)(kids & 0xffff);
-                const LDS double *T = c->fixZ[x] ? c->TMf : c->TMn;
-                bj += log_col(T, j, c->beta[x * 3], c->beta[x * 3 + 1], c->beta[x * 3 + 2]);
-            }
-            c->beta[p * 3 + j] = bj;
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        // root prior (1/2, 1/2, 0)
-        const int r = c->root;
-        const double l0 = c->beta[r * 3] + log(0.5), l1 = c->beta[r * 3 + 1] + log(0.5);
-        const double mx = fmax(l0, l1);
-        double pr[3] = {exp(l0 - mx), exp(l1 - mx), 0.0};
-        const int z = categorical<3>(pr, slot_uniform(key, 0, c2, c3, 0));
-        if (c->Z[r] != z) c->changed[r] = 1;
-        c->Z[r] = (int8_t)z;
+    for (int i = tid; i < 3 * S; i += BS) {
+        const int s = i / 3, j = i - 3 * s;
+        if (!(flags[s] & NF_IN_TREE)) continue;
+        msg[i] = log_col(fixZ[s] ? TMf : TMn, j, beta[s * 3], beta[s * 3 + 1], beta[s * 3 + 2]);
     }
     __syncthreads();
-    for (int d = 0; d < n_down; d++) {
-        const int a = d == 0 ? 0 : c->downoff[d - 1], b = c->downoff[d];
-        for (int q = a + tid; q < b; q += BS) {
-            const int s = c->down[q];
-            const int zp = c->Z[c->par[s]];
-            const LDS double *T = c->fixZ[s] ? c->TMf : c->TMn;
-            const double y0 = T[0 * 3 + zp] + c->beta[s * 3], y1 = T[1 * 3 + zp] + c->beta[s * 3 + 1],
-                         y2 = T[2 * 3 + zp] + c->beta[s * 3 + 2];
-            const double mx = fmax(y0, fmax(y1, y2));
-            double pr[3] = {exp(y0 - mx), exp(y1 - mx), exp(y2 - mx)};
-            const int z = categorical<3>(pr, slot_uniform(key, 0, c2, c3, (uint32_t)c->tz[s]));
-            if (c->Z[s] != z) c->changed[s] = 1;
-            c->Z[s] = (int8_t)z;
+    if (tid < 64) {
+        // 21 nodes at a time, three lanes each: a node's lanes read its beta
+        // together before they write it
+        const int r = tid / 3, j = tid - 3 * r;
+        int a = 0, b = uni(upoff[0]);
+        uint32_t rec = r < b ? urec[r] : 0;
+        for (int h = 0; h < n_up; h++) {
+            const int b2 = h + 1 < n_up ? uni(upoff[h + 1]) : b;
+            for (int q0 = a; q0 < b; q0 += 21) {
+                const bool on = tid < 63 && q0 + r < b;
+                const uint32_t w = rec;
+                // the next group's record
+                const int qn = (q0 + 21 < b ? q0 + 21 : b) + r;
+                rec = qn < b2 ? urec[qn] : 0;
+                if (on) {
+                    const int p = w & 0x3ff, x0 = (w >> 10) & 0x3ff, x1 = w >> 20;
+                    const LDS double *T = fixZ[p] ? TMf : TMn;
+                    const double b0 = beta[p * 3] + msg[x0 * 3] + msg[x1 * 3], b1 = beta[p * 3 + 1] + msg[x0 * 3 + 1] + msg[x1 * 3 + 1],
+                                 bb = beta[p * 3 + 2] + msg[x0 * 3 + 2] + msg[x1 * 3 + 2];
+                    __builtin_amdgcn_wave_barrier();
+                    beta[p * 3 + j] = j == 0 ? b0 : (j == 1 ? b1 : bb);
+                    msg[p * 3 + j] = log_col(T, j, b0, b1, bb);
+                }
+                // the lanes of a wave see each other's LDS writes in program order
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+            a = b;
+            b = b2;
         }
-        __syncthreads();
     }
-    // dirty = strict ancestors of changed nodes (getUpdateNode, bpp_c.cpp:620-642)
-    const int N = c->N;
-    for (int q = tid; q < c->n_nodes; q += BS) {
-        const int s = c->nodes[q];
-        if (!c->changed[s]) continue;
+    __syncthreads();
+    // every node's draw for each class of its parent; the root's has the prior (1/2, 1/2, 0) and no parent
+    LDS uint8_t *zn = (LDS uint8_t *)msg;
+    const int n_item = 3 * (n_nodes - 1) + 1;
+    for (int i = tid; i < n_item; i += BS) {
+        const int q = i / 3, zp = i - 3 * q, s = nodes[q];
+        const LDS double *T = fixZ[s] ? TMf : TMn;
+        const bool rt = q == n_nodes - 1;
+        const double y0 = (rt ? log(0.5) : T[0 * 3 + zp]) + beta[s * 3], y1 = (rt ? log(0.5) : T[1 * 3 + zp]) + beta[s * 3 + 1],
+                     y2 = (rt ? -INFINITY : T[2 * 3 + zp]) + beta[s * 3 + 2];
+        const double mx = fmax(y0, fmax(y1, y2));
+        double pr[3];
+        exp3(y0, y1, y2, mx, pr[0], pr[1], pr[2]);
+        zn[s * 4 + zp] = (uint8_t)categorical<3>(pr, slot_uniform(key, 0, c2, c3, (uint32_t)(n_nodes - 1 - q)));
+    }
+    __syncthreads();
+    const LDS uint32_t *znw = (const LDS uint32_t *)msg;
+    const int z_root = uni((int)zn[root * 4]);
+    for (int q = tid; q < n_nodes; q += BS) {
+        const int s = nodes[q];
+        int z = z_root;
+        if (s != root) {
+            // w: the node's class for each class of the ancestor reached so far
+            uint32_t w = znw[s];
+            int a = par[s];
+            while (a != root) {
+                const uint32_t f = znw[a];
+                const int up = par[a];
+                w = ((w >> (8 * (f & 3))) & 3) | ((w >> (8 * ((f >> 8) & 3)) & 3) << 8) | ((w >> (8 * ((f >> 16) & 3)) & 3) << 16);
+                a = up;
+            }
+            z = (w >> (8 * z_root)) & 3;
+        }
+        if (c->Z[s] == z) continue;
+        c->Z[s] = (int8_t)z;
+        c->changed[s] = 1;
         c->nch = 1;     // every writer stores the same value
-        for (int j = c->par[s]; j != N; j = c->par[j]) c->dirty[j] = 1;
+        // dirty = strict ancestors of changed nodes (getUpdateNode, bpp_c.cpp:620-642)
+        for (int a = par[s]; a != N; a = par[a]) c->dirty[a] = 1;
     }
     __syncthreads();
 }
@@ -1293,12 +1348,13 @@ __device__ __noinline__ void pruning_order(CP<R> c, const int32_t *tab, int N)
 {
     const int tid = threadIdx.x, S = c->S, n_up = c->n_up, n_down = c->n_down, root = c->root;
     const int32_t *ch0 = tab + tab_ch0(N), *ch1 = tab + tab_ch1(N);
+    const int32_t *down = tab + tab_down(N), *downoff = tab + tab_downoff(N);
     LDS int32_t *size = (LDS int32_t *)c->E, *start = size + N;
     for (int i = tid; i < N; i += BS) size[i] = 0;
     __syncthreads();
     for (int h = 0; h < n_up; h++) {
         for (int q = (h == 0 ? 0 : c->upoff[h - 1]) + tid; q < c->upoff[h]; q += BS) {
-            const int s = c->up[q];
+            const int s = c->urec[q] & 0x3ff;
             size[s] = 1 + size[ch0[s]] + size[ch1[s]];
         }
         __syncthreads();
@@ -1309,8 +1365,8 @@ __device__ __noinline__ void pruning_order(CP<R> c, const int32_t *tab, int N)
     }
     __syncthreads();
     for (int d = 0; d < n_down; d++) {
-        for (int q = (d == 0 ? 0 : c->downoff[d - 1]) + tid; q < c->downoff[d]; q += BS) {
-            const int s = c->down[q], p = c->par[s];
+        for (int q = (d == 0 ? 0 : downoff[d - 1]) + tid; q < downoff[d]; q += BS) {
+            const int s = down[q], p = c->par[s];
             if (s < S) continue;
             const int a = ch0[p], b = ch1[p], first = size[a] >= size[b] ? a : b;
             const int st = start[p] + (s == first ? 0 : size[first]);
@@ -1351,20 +1407,16 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
         c->flags[i] = (uint8_t)tab[tab_flags(N) + i];
         c->nodes[i] = (int16_t)tab[tab_nodes(N) + i];
         c->inodes[i] = (int16_t)tab[tab_int(N) + i];
-        c->up[i] = (int16_t)tab[tab_up(N) + i];
-        c->down[i] = (int16_t)tab[tab_down(N) + i];
-        c->tz[i] = (int16_t)tab[tab_tz(N) + i];
-        for (int k = 0; k < 16; k++) c->hist[16 * i + k] = 0;
         c->cur[i] = 0;
         c->dirty[i] = 0;
     }
-    for (int i = tid; i <= N; i += BS) {
-        c->upoff[i] = (int16_t)tab[tab_upoff(N) + i];
-        c->downoff[i] = (int16_t)tab[tab_downoff(N) + i];
+    for (int i = tid; i < E.n_up; i += BS) c->upoff[i] = (int16_t)tab[tab_upoff(N) + i];
+    for (int q = tid; q < E.n_int; q += BS) {
+        const int v = tab[tab_up(N) + q];
+        c->urec[q] = (uint32_t)v | ((uint32_t)tab[tab_ch0(N) + v] << 10) | ((uint32_t)tab[tab_ch1(N) + v] << 20);
     }
     for (int s = M->S + tid; s < N; s += BS) node_desc(c->desc + 4 * (s - M->S), tab, N, M->S, E.root, s);
     __syncthreads();
-    for (int i = tid; i < M->S * 24; i += BS) c->amb[i] = 0;
     // cherries (both children leaves; never the root) are recomputed where read
     for (int q = tid; q < c->n_int; q += BS) {
         const int s = c->inodes[q];

@@ -65,9 +65,10 @@ struct Ctx {
     LDS uint32_t *hist, *cnt9;
     LDS uint8_t *tgs;
     // chain scalars
-    double loglik, nrate, crate, g, l, l2, prop_n, prop_c, proposal, r, max_loglik;
+    double loglik, nrate, crate, g, l, l2, prop_n, prop_c, proposal, old_rate, r, max_loglik;
     double TMf[9], TMn[9];  // log_TM_Int for fixZ / free nodes, [i*3+j] = log P(child i | parent j)
-    double red[16];
+    double red[4], gam[8], mh[5];   // block sums; a sweep's gamma variates; Metropolis terms
+    int has_cls[2];                 // any branch in class 1 (conserved), 2 (accelerated)
     unsigned long long bytes;   // algorithmic HBM bytes of this element's passes (see prune / sample_sites)
     int accept_n, accept_c, max_m, skip, accept, fail, work, nch, n_steps, last_step, n_stored, n_cherry, n_leaf;   // fail: PA_F_* bits
 };
@@ -230,53 +231,81 @@ __device__ __forceinline__ void lds_add(LDS uint32_t *p, uint32_t v)
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// P(t) = V diag(exp(lam t)) Vi, clamped at 0; out[j*4+i] = P_{j->i}
-template <typename OutPtr>
-__device__ __forceinline__ void ptrans(MP M, double t, OutPtr out)
+// Row j of P(t) = V diag(exp(lam t)) Vi, clamped at 0: out[i] = P_{j->i}.
+// Called by whole quads of lanes, lane j of a quad for row j of one matrix:
+// each lane takes one of the four exponentials and reads the others from its
+// quad.
+__device__ __forceinline__ double quad_lane(double v, int k)
 {
-    double e[4];
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    int lo = (int)(uint32_t)u, hi = (int)(uint32_t)(u >> 32);
+#define PA_QUAD(K) { lo = __builtin_amdgcn_mov_dpp(lo, K * 0x55, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, K * 0x55, 0xf, 0xf, true); }
+    if (k == 0) PA_QUAD(0) else if (k == 1) PA_QUAD(1) else if (k == 2) PA_QUAD(2) else PA_QUAD(3)
+#undef PA_QUAD
+    return __builtin_bit_cast(double, (unsigned long long)(uint32_t)lo | ((unsigned long long)(uint32_t)hi << 32));
+}
+
+__device__ __forceinline__ void ptrans_row(MP M, double t, int j, double (&out)[4])
+{
+    const double ej = exp(M->lam[j] * t);
+    const double e[4] = {quad_lane(ej, 0), quad_lane(ej, 1), quad_lane(ej, 2), quad_lane(ej, 3)};
 #pragma unroll
-    for (int k = 0; k < 4; k++) e[k] = exp(M->lam[k] * t);
-#pragma unroll 1
-    for (int j = 0; j < 4; j++)
+    for (int i = 0; i < 4; i++) {
+        double s = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) s += M->V[j * 4 + k] * e[k] * M->Vi[k * 4 + i];
+        out[i] = s < 0 ? 0.0 : s;
+    }
+}
+
+// Class tables of every branch for class k (0 null, 1 conserved, 2 accelerated)
+// at rate r, a lane per matrix row.
+// mode 0: model start (dist2 > 1e-10 -> P(dist2*r), else identity; bpp_c.cpp:187-228)
+// mode 1: refresh after a rate change (dist2 < 1e-10 keeps the old table;
+//         bpp_c.cpp:1115-1131), with the current matrices of the class's branches
+template <typename R, int BS>
+__device__ __noinline__ void class_tables(MP M, CP<R> c, int k, double r, int mode)
+{
+    const int N = uni(c->N), n_item = 4 * (uni(c->n_nodes) - 1);
+    const LDS int16_t *nodes = uni_ptr(c->nodes);
+    const GBL double *dist2 = uni_ptr(c->dist2);
+    for (int it = threadIdx.x; it < n_item; it += BS) {
+        const int s = nodes[it >> 2], j = it & 3;
+        const double d = dist2[s];
+        GBL double *P = c->plin + ((size_t)k * N + s) * 16;
+        GBL double *L = c->logt + ((size_t)k * N + s) * 16;
+        if (mode == 1 && d < 1e-10) continue;       // a whole quad
+        double row[4];
+        ptrans_row(M, d * r, j, row);
+        if (mode == 0 && !(d > 1e-10)) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) row[i] = i == j ? 1.0 : 0.0;
+        }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            double s = 0;
-#pragma unroll
-            for (int k = 0; k < 4; k++) s += M->V[j * 4 + k] * e[k] * M->Vi[k * 4 + i];
-            out[j * 4 + i] = s < 0 ? 0.0 : s;
+            P[j * 4 + i] = row[i];
+            L[i * 4 + j] = log(row[i]);
         }
+        if (mode == 1) {
+            const int z = c->Z[s];
+            if (z == k) {
+                LDS R *dst = c->PTc + 16 * s;
+#pragma unroll
+                for (int i = 0; i < 4; i++) dst[i * 4 + j] = (R)row[i];
+            }
+        }
+    }
 }
 
-// class tables for branch s, class k (0 null, 1 conserved, 2 accelerated) at rate r.
-// mode 0: model start (dist2 > 1e-10 -> P(dist2*r), else identity; bpp_c.cpp:187-228)
-// mode 1: refresh after a rate change (dist2 < 1e-10 keeps the old table; bpp_c.cpp:1115-1131)
-template <typename R>
-__device__ __noinline__ void class_table(MP M, CP<R> c, int k, int s, double r, int mode)
-{
-    const double d = c->dist2[s];
-    GBL double *P = c->plin + ((size_t)k * c->N + s) * 16;
-    GBL double *L = c->logt + ((size_t)k * c->N + s) * 16;
-    if (mode == 1 && d < 1e-10) return;
-    if (d > 1e-10 || mode == 1) ptrans(M, d * r, P);
-    else
-        for (int i = 0; i < 16; i++) P[i] = (i % 5 == 0) ? 1.0 : 0.0;
-#pragma unroll 1
-    for (int q = 0; q < 16; q++) L[q] = log(P[(q & 3) * 4 + (q >> 2)]);
-}
-
-// PT of the current class of every branch: all branches (only_cls = -1),
-// those with Z == only_cls, or (REFRESH_CHANGED) those whose Z the last Z
-// update changed
-constexpr int REFRESH_CHANGED = -2;
+// PT of the current class of every branch, or (changed_only) of those whose Z
+// the last Z update changed
 template <typename R, int BS, int SH>
-__device__ __noinline__ void refresh_PTc(CP<R> c, int only_cls)
+__device__ __noinline__ void refresh_PTc(CP<R> c, bool changed_only)
 {
     for (int q = threadIdx.x; q < c->n_nodes - 1; q += BS) {
         const int s = c->nodes[q];
         const int z = c->Z[s];
-        if (only_cls >= 0 && z != only_cls) continue;
-        if (only_cls == REFRESH_CHANGED && !c->changed[s]) continue;
+        if (changed_only && !c->changed[s]) continue;
         const int k = z == 2 ? 2 : (z == 0 ? 0 : 1);
         const GBL double *P = c->plin + ((size_t)k * c->N + s) * 16;
         LDS R *dst = c->PTc + 16 * s;
@@ -443,18 +472,18 @@ struct PassArgs {
     const LDS uint32_t *steps;
     const LDS R *PT;             // [2N][16]: the current matrices, then the proposal's
     Buf codes;
-    int n, I, amb;
+    int n, I;
 };
 
 // One child's message at one pattern, or ones where it holds no base; adds
 // its exponent and reports the gap.
-template <typename R, int K>
-__device__ __forceinline__ void message(const LDS R *PT, int amb, int code, const ChildIn<R> &in, V4<R> &o, int &e, bool &gap)
+template <typename R, int K, bool AMB>
+__device__ __forceinline__ void message(const LDS R *PT, int code, const ChildIn<R> &in, V4<R> &o, int &e, bool &gap)
 {
     if constexpr (K == SK_LEAF) {
         gap = code == PA_GAP_CODE || code == PA_OTHER_CODE;
         o = ld4<R>((const LDS V4<R> *)(PT + 4 * (code & 3)));
-        if (amb && code > PA_OTHER_CODE) {
+        if (AMB && code > PA_OTHER_CODE) {
             o.x = o.y = o.z = o.w = (R)1;
             leaf_mul<R>(PT, code, o.x, o.y, o.z, o.w);
         }
@@ -518,7 +547,7 @@ __device__ __forceinline__ ChildIn<R> slot_load(Buf blk, uint32_t slot, uint32_t
 // a child that is no leaf loads row 0's code, and a cherry, which is kept in
 // registers only, stores through a buffer of no bytes (the hardware drops
 // accesses outside a buffer).
-template <typename R>
+template <typename R, bool AMB>
 __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL char *base, int blk_bytes, uint32_t p)
 {
     const int n = A.n;
@@ -560,28 +589,28 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
         V4<R> a, b;
         ChildIn<R> out;
         if (type == ST_PL) {
-            message<R, SK_PREV>(PA, 0, 0, res[j ^ 1], a, e, ga);
-            message<R, SK_LEAF>(PB, A.amb, cdB[j], inB[j], b, e, gb);
+            message<R, SK_PREV, AMB>(PA, 0, res[j ^ 1], a, e, ga);
+            message<R, SK_LEAF, AMB>(PB, cdB[j], inB[j], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else if (type == ST_LL) {
-            message<R, SK_LEAF>(PA, A.amb, cdA[j], inA[j], a, e, ga);
-            message<R, SK_LEAF>(PB, A.amb, cdB[j], inB[j], b, e, gb);
+            message<R, SK_LEAF, AMB>(PA, cdA[j], inA[j], a, e, ga);
+            message<R, SK_LEAF, AMB>(PB, cdB[j], inB[j], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else if (type == ST_PP2) {
-            message<R, SK_PREV>(PA, 0, 0, res[j ^ 1], a, e, ga);
-            message<R, SK_PREV2>(PB, 0, 0, res[j], b, e, gb);
+            message<R, SK_PREV, AMB>(PA, 0, res[j ^ 1], a, e, ga);
+            message<R, SK_PREV2, AMB>(PB, 0, res[j], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else if (type == ST_SP) {
-            message<R, SK_STORED>(PA, 0, 0, inA[j], a, e, ga);
-            message<R, SK_PREV>(PB, 0, 0, res[j ^ 1], b, e, gb);
+            message<R, SK_STORED, AMB>(PA, 0, inA[j], a, e, ga);
+            message<R, SK_PREV, AMB>(PB, 0, res[j ^ 1], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else if (type == ST_SL) {
-            message<R, SK_STORED>(PA, 0, 0, inA[j], a, e, ga);
-            message<R, SK_LEAF>(PB, A.amb, cdB[j], inB[j], b, e, gb);
+            message<R, SK_STORED, AMB>(PA, 0, inA[j], a, e, ga);
+            message<R, SK_LEAF, AMB>(PB, cdB[j], inB[j], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else if (type == ST_SS) {
-            message<R, SK_STORED>(PA, 0, 0, inA[j], a, e, ga);
-            message<R, SK_STORED>(PB, 0, 0, inB[j], b, e, gb);
+            message<R, SK_STORED, AMB>(PA, 0, inA[j], a, e, ga);
+            message<R, SK_STORED, AMB>(PB, 0, inB[j], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else {
             // any sources, missing nodes: a missing child contributes nothing, but its gap state still
@@ -626,6 +655,43 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
     return r;
 }
 
+// The pattern loop of a pass: this thread's part of the root's log sum.
+template <typename R, int BS, bool AMB>
+__device__ __forceinline__ double prune_patterns(MP M, CP<R> c, int mode)
+{
+    const int tid = threadIdx.x;
+    const int P = uni(c->P);
+    PassArgs<R> A;
+    A.n = uni(c->n_steps);
+    A.I = uni(c->I);
+    A.steps = uni_ptr(c->steps);
+    A.PT = uni_ptr(c->PTc);
+    A.codes = make_buf(uni_ptr(c->codes), code_bytes(uni(c->S), uni(c->Ppad)));
+    GBL char *parts = uni_ptr(c->parts);
+    const int blkB = block_bytes(A.I, sizeof(R));
+    const int r = uni(c->root);
+    const GBL int32_t *wts = uni_ptr(c->wts);
+    const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
+    // the root is the last step of every pass that visits it
+    const bool in_regs = A.n > 0 && uni(c->last_step) == r && !(uni(c->flags[r]) & NF_MISSING);
+    const int rc = uni(c->cur[r]), rb = (mode == PR_PROP && uni(c->dirty[r])) ? 1 - rc : rc;
+    double acc = 0;
+    // whole waves of 64 patterns; wave w takes blocks w, w + BS / 64, ...
+    for (int pb = uni(tid & ~63); pb < P; pb += BS) {
+        const uint32_t lane = tid & 63, p = (uint32_t)pb + lane;
+        GBL char *blk = parts + (int64_t)(pb >> 6) * blkB;
+        ChildIn<R> o;
+        if (A.n > 0) o = prune_pattern<R, AMB>(A, blk, blkB, p);
+        if (!in_regs) o = slot_load<R>(make_buf(blk, blkB), rb * A.I + r - uni(c->S), lane, A.I);
+        // log sum_j pi_j L_j + exponent * ln 2; all-gap columns contribute 0
+        if (o.x != GAPT && (int)p < P) {
+            const double L = p0 * (double)o.v.x + p1 * (double)o.v.y + p2 * (double)o.v.z + p3 * (double)o.v.w;
+            acc += (double)wts[p] * (log(L) + (double)o.x * 0.69314718055994530942);
+        }
+    }
+    return acc;
+}
+
 // One pruning pass (BPP_C::Update_Tg(tosample=false), src/PhyloAcc-ST/bpp_c.cpp:644-671,
 // and log_f_Xz, bpp_c.cpp:860-928).  FULL: every internal node of the tree
 // (missing nodes only record their GAPT flag) into the current buffer.
@@ -650,39 +716,9 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
 template <typename R, int BS, int SH>
 __device__ __noinline__ double prune(MP M, CP<R> c, int mode, int cls)
 {
-    const int tid = threadIdx.x;
-    const int P = uni(c->P);
-    if (tid < 64) build_steps<R>(c, mode, cls);
+    if (threadIdx.x < 64) build_steps<R>(c, mode, cls);
     __syncthreads();
-    PassArgs<R> A;
-    A.n = uni(c->n_steps);
-    A.I = uni(c->I);
-    A.amb = uni(c->has_amb);
-    A.steps = uni_ptr(c->steps);
-    A.PT = uni_ptr(c->PTc);
-    A.codes = make_buf(uni_ptr(c->codes), code_bytes(uni(c->S), uni(c->Ppad)));
-    GBL char *parts = uni_ptr(c->parts);
-    const int blkB = block_bytes(A.I, sizeof(R));
-    const int r = uni(c->root);
-    const GBL int32_t *wts = uni_ptr(c->wts);
-    const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
-    // the root is the last step of every pass that visits it
-    const bool in_regs = A.n > 0 && uni(c->last_step) == r && !(uni(c->flags[r]) & NF_MISSING);
-    const int rc = uni(c->cur[r]), rb = (mode == PR_PROP && uni(c->dirty[r])) ? 1 - rc : rc;
-    double acc = 0;
-    // whole waves of 64 patterns; wave w takes blocks w, w + BS / 64, ...
-    for (int pb = uni(tid & ~63); pb < P; pb += BS) {
-        const uint32_t lane = tid & 63, p = (uint32_t)pb + lane;
-        GBL char *blk = parts + (int64_t)(pb >> 6) * blkB;
-        ChildIn<R> o;
-        if (A.n > 0) o = prune_pattern<R>(A, blk, blkB, p);
-        if (!in_regs) o = slot_load<R>(make_buf(blk, blkB), rb * A.I + r - uni(c->S), lane, A.I);
-        // log sum_j pi_j L_j + exponent * ln 2; all-gap columns contribute 0
-        if (o.x != GAPT && (int)p < P) {
-            const double L = p0 * (double)o.v.x + p1 * (double)o.v.y + p2 * (double)o.v.z + p3 * (double)o.v.w;
-            acc += (double)wts[p] * (log(L) + (double)o.x * 0.69314718055994530942);
-        }
-    }
+    const double acc = uni(c->has_amb) ? prune_patterns<R, BS, true>(M, c, mode) : prune_patterns<R, BS, false>(M, c, mode);
     return block_sum(acc, c->red);
 }
 
@@ -691,12 +727,13 @@ __device__ __noinline__ double prune(MP M, CP<R> c, int mode, int cls)
 // One step of the sampler: an internal node, in reverse post-order (step 0
 // the root).  Two words, built when the element is bound (sample_steps):
 //   r0: node | parent << 10 | SR_* bits
-//   r1: the node's leaf children A | B << 10 (0: none)
+//   r1: the node's leaf children A | B << 10 (0: none) | the slot of its partial << 22 (follows cur; a cherry has
+//       none stored, and its load goes where the root's does)
 enum { SR_ID = 0x3ff, SR_PAR_SHIFT = 10, SR_MISS = 1 << 20, SR_CHERRY = 1 << 21,
        SR_PREV = 1 << 22,                          // the parent is the step before
        SR_LEAF_A = 1 << 23, SR_LEAF_B = 1 << 24,   // leaf children that are counted
        SR_MISS_A = 1 << 25, SR_MISS_B = 1 << 26,   // a cherry's missing leaves
-       SR_CUR = 1 << 27 };                         // the buffer holding the node's partial (follows cur)
+       SR_SLOT_SHIFT = 22 };
 
 // BPP_C::Update_Tg(tosample=true) (src/PhyloAcc-ST/bpp_c.cpp:672-733) for every
 // site, plus the per-branch transition counts that getEmission
@@ -709,32 +746,22 @@ enum { SR_ID = 0x3ff, SR_PAR_SHIFT = 10, SR_MISS = 1 << 20, SR_CHERRY = 1 << 21,
 // counted), the parent's base is in a register when the parent was the step
 // before and otherwise read a step early, and a node counts its own leaf
 // children, whose parent's base it has just drawn.
-template <typename R, int BS, int SH>
-__device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c3)
+template <typename R, int BS, int SH, bool AMB>
+__device__ __forceinline__ void draw_sites(MP M, CP<R> c, uint32_t c2, uint32_t c3)
 {
     constexpr int K = Shape<R, SH>::K, UN = K < 4 ? 4 : K;     // steps unrolled: whole blocks of four draws
     const int tid = threadIdx.x, S = uni(c->S), I = uni(c->I), n_int = uni(c->n_int), GG = uni(c->GG), Ppad = uni(c->Ppad);
-    const int blkB = block_bytes(I, sizeof(R)), amb_on = uni(c->has_amb);
+    const int blkB = block_bytes(I, sizeof(R));
     const uint32_t k0 = (uint32_t)uni((int)M->key0), k1 = (uint32_t)uni((int)M->key1);
     const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
     const GBL char *parts = uni_ptr(c->parts);
     const Buf codes = make_buf(uni_ptr(c->codes), code_bytes(S, Ppad));
     const GBL int32_t *site = uni_ptr(c->site);
     GBL uint32_t *amb = uni_ptr(c->amb);
-    LDS uint8_t *tgs = uni_ptr(c->tgs) + tid;
+    LDS uint8_t *tgs = uni_ptr(c->tgs) + tid - S * BS;      // node s: [s * BS]
     LDS uint32_t *hist = uni_ptr(c->hist);
     const LDS uint32_t *srec = uni_ptr(c->srec);
     const LDS R *PTc = uni_ptr(c->PTc);
-    for (int i = tid; i < 16 * c->N; i += BS) hist[i] = 0;   // shares storage with the proposal matrices
-    if (amb_on)
-        for (int i = tid; i < 24 * S; i += BS) amb[i] = 0;
-    __syncthreads();
-    if (tid == 0) {
-        // per site: pattern index, root partial, each non-missing internal node's partial
-        // (a cherry's two leaf codes), each leaf code
-        c->bytes += (unsigned long long)GG * (4 + (4 * sizeof(R) + 4) * c->n_stored + 2 * c->n_cherry + c->n_leaf);
-    }
-    const uint32_t r_slot = (srec[0] & SR_ID) - S;
     for (int gb = uni(tid & ~63); gb < GG; gb += BS) {
         const int g = gb + (tid & 63);
         const bool on = g < GG;
@@ -752,9 +779,7 @@ __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c
             const LDS uint32_t *nx = srec + 2 * (t + 1 < n_int ? t + 1 : t);
             nr0 = nx[0];
             nr1 = nx[1];
-            // a cherry has no stored partial: the load goes where the root's went
-            uint32_t slot = (r0[j] & (SR_CHERRY | SR_MISS)) ? r_slot : (r0[j] & SR_ID) - S;
-            slot += ((r0[j] & SR_CUR) && !(r0[j] & (SR_CHERRY | SR_MISS))) ? I : 0;
+            const uint32_t slot = r1[j] >> SR_SLOT_SHIFT;
             in[j].v = ld4<R>((const GBL V4<R> *)(pp + (uint64_t)part_off<R>(slot)));
             in[j].x = *(const GBL int32_t *)(pe + (uint64_t)(slot * 256));
             cdA[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, (r1[j] & SR_ID) * Ppad, 0);
@@ -764,7 +789,7 @@ __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c
         int ts = 0, tp = 0;
         auto count_leaf = [&](int y, int code) __attribute__((always_inline)) {
             if (on && code < 4) lds_add(&hist[y * 16 + ts * 4 + code], 1u);
-            if (amb_on && on && code > PA_OTHER_CODE)
+            if (AMB && on && code > PA_OTHER_CODE)
                 __hip_atomic_fetch_add(&amb[y * 24 + ts * 6 + (code - 6)], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         };
         auto step = [&](auto JJ, int t) __attribute__((always_inline)) {
@@ -775,7 +800,7 @@ __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c
             const int s = w0 & SR_ID;
             const int tp_read = tp & 3;
             // the next step's parent, unless it is this node
-            if (t + 1 < n_int) tp = tgs[(((r0[(j + 1) % K] >> SR_PAR_SHIFT) & SR_ID) - S) * BS];
+            if (t + 1 < n_int) tp = tgs[((r0[(j + 1) % K] >> SR_PAR_SHIFT) & SR_ID) * BS];
             if (!(w0 & SR_MISS)) {
                 ChildIn<R> a;
                 if (w0 & SR_CHERRY) {
@@ -783,8 +808,8 @@ __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c
                     V4<R> ma, mb;
                     int e = 0;
                     bool ga, gb2;
-                    message<R, SK_LEAF>(PTc + 16 * (w1 & SR_ID), amb_on, cdA[j], in[j], ma, e, ga);
-                    message<R, SK_LEAF>(PTc + 16 * ((w1 >> 10) & SR_ID), amb_on, cdB[j], in[j], mb, e, gb2);
+                    message<R, SK_LEAF, AMB>(PTc + 16 * (w1 & SR_ID), cdA[j], in[j], ma, e, ga);
+                    message<R, SK_LEAF, AMB>(PTc + 16 * ((w1 >> 10) & SR_ID), cdB[j], in[j], mb, e, gb2);
                     if (w0 & SR_MISS_A) ma.x = ma.y = ma.z = ma.w = (R)1;
                     if (w0 & SR_MISS_B) mb.x = mb.y = mb.z = mb.w = (R)1;
                     a = combine<R>(ma, mb, 0, ga && gb2);
@@ -805,7 +830,7 @@ __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c
                     pr[2] = (double)PT[8] * (double)a.v.z; pr[3] = (double)PT[12] * (double)a.v.w;
                 }
                 ts = categorical<4>(pr, u);
-                tgs[(s - S) * BS] = (uint8_t)ts;
+                tgs[s * BS] = (uint8_t)ts;
                 if (t != 0 && on && has) lds_add(&hist[s * 16 + from * 4 + ts], 1u);
                 if (w0 & SR_LEAF_A) count_leaf(w1 & SR_ID, cdA[j]);
                 if (w0 & SR_LEAF_B) count_leaf((w1 >> 10) & SR_ID, cdB[j]);
@@ -816,6 +841,23 @@ __device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c
         for (int t0 = 0; t0 < n_int; t0 += UN)
             each<UN>([&](auto J) __attribute__((always_inline)) { if (t0 + decltype(J)::value < n_int) step(J, t0 + decltype(J)::value); });
     }
+}
+
+template <typename R, int BS, int SH>
+__device__ __noinline__ void sample_sites(MP M, CP<R> c, uint32_t c2, uint32_t c3)
+{
+    const int tid = threadIdx.x, amb_on = uni(c->has_amb), n_hist = 16 * uni(c->N), n_amb = 24 * uni(c->S);
+    for (int i = tid; i < n_hist; i += BS) c->hist[i] = 0;   // shares storage with the proposal matrices
+    if (amb_on)
+        for (int i = tid; i < n_amb; i += BS) c->amb[i] = 0;
+    if (tid == 0) {
+        // per site: pattern index, root partial, each non-missing internal node's partial
+        // (a cherry's two leaf codes), each leaf code
+        c->bytes += (unsigned long long)c->GG * (4 + (4 * sizeof(R) + 4) * c->n_stored + 2 * c->n_cherry + c->n_leaf);
+    }
+    __syncthreads();
+    if (amb_on) draw_sites<R, BS, SH, true>(M, c, c2, c3);
+    else draw_sites<R, BS, SH, false>(M, c, c2, c3);
 }
 
 // The sampler's step words (layout at SR_*) and the node counts its bytes
@@ -847,8 +889,9 @@ __device__ __noinline__ void sample_steps(CP<R> c)
             if (f1 & NF_MISSING) w0 |= SR_MISS_B;
             else if (f1 & NF_IN_TREE) w0 |= SR_LEAF_B;
         }
+        const int v = (f & (NF_MISSING | NF_CHERRY)) ? c->root : s;
         c->srec[2 * t] = w0;
-        c->srec[2 * t + 1] = w1;
+        c->srec[2 * t + 1] = w1 | (uint32_t)(v - S) << SR_SLOT_SHIFT;      // buffer 0
     }
     if (threadIdx.x == 0) {
         int nint = 0, nch = 0, nleaf = 0;
@@ -1057,38 +1100,99 @@ __device__ __noinline__ void update_Z(MP M, CP<R> c, uint32_t c2, uint32_t c3)
 
 // ------------------------------------------------------------- rate update
 
-__device__ __forceinline__ void set_TM(LDS double *F, LDS double *T, double g, double l, double l2)
+// log_TM_Int, [i*3+j] = log P(child i | parent j), the six logarithms a lane
+// each (lane < 64 of one wave).  fixZ nodes (bpp_c.cpp:305-316, 577-585):
+// column 2 is never set there and keeps its initial log 1 (a fixZ node's
+// parent is never accelerated, so it is unused).
+__device__ __forceinline__ void set_TM(LDS double *F, LDS double *T, double g, double l, double l2, int lane)
 {
-    // log_TM_Int, [i*3+j] = log P(child i | parent j).  fixZ nodes
-    // (bpp_c.cpp:305-316, 577-585): column 2 is never set there and keeps its
-    // initial log 1 (a fixZ node's parent is never accelerated, so it is unused).
-    const double lg = log(g), l1g = log(1 - g);
-    F[0] = l1g; F[3] = lg; F[6] = -INFINITY;
-    F[1] = -INFINITY; F[4] = 0; F[7] = -INFINITY;
-    F[2] = 0; F[5] = 0; F[8] = 0;
-    T[0] = l1g; T[3] = lg; T[6] = -INFINITY;
     const double y = 1 - l;   // the reference forms P(1 -> 2) as 1 - (1 - l)
-    T[1] = -INFINITY; T[4] = log(y); T[7] = log(1 - y);
-    T[2] = -INFINITY; T[5] = log(l2); T[8] = log(1 - l2);
+    const double x = lane == 0 ? 1 - g : lane == 1 ? g : lane == 2 ? y : lane == 3 ? 1 - y : lane == 4 ? l2 : 1 - l2;
+    const double v = log(x);
+    if (lane == 0) { F[0] = v; T[0] = v; F[6] = F[1] = F[7] = T[6] = T[1] = T[2] = -INFINITY; }
+    else if (lane == 1) { F[3] = v; T[3] = v; F[4] = F[2] = F[5] = F[8] = 0; }
+    else if (lane == 2) T[4] = v;
+    else if (lane == 3) T[7] = v;
+    else if (lane == 4) T[5] = v;
+    else if (lane == 5) T[8] = v;
 }
 
-// Scalar head of BPP_C::sample_rate (src/PhyloAcc-ST/bpp_c.cpp:930-1041): prior draw
-// when no branch carries the class, else the proposal and its range checks.
+// The gamma variates of one sweep, drawn together by one wave (a draw is a
+// long chain of FP64 functions, so its time is the same for one lane or
+// eight): lanes 0-5 those of the three transition Beta draws
+// (BPP_C::sample_transition, src/PhyloAcc-ST/bpp_c.cpp:522-613;
+// Beta(a, b) = X / (X + Y), X ~ Gamma(a) on sub-stream 2k, Y ~ Gamma(b) on
+// sub-stream 2k + 1, the l2 pair not drawn when its prior is off), lane 6 the
+// accelerated rate's proposal (bpp_c.cpp:1000-1010) or, when no branch
+// carries the class, its prior draw, lane 7 the conserved rate's prior draw.
+// Each variate has its own stream, so drawing early changes none.  The counts
+// cnt9 and has_cls are those of the Z the rates are drawn under.
+enum { GV_R2 = 6, GV_R1 = 7, GV_N = 8 };
+
 template <typename R>
-__device__ __noinline__ void rate_propose(MP M, CP<R> c, int ms, int m, int resZ, bool neut, double old)
+__device__ __noinline__ void draw_gammas(MP M, CP<R> c, int ms, int m, int resZ)
 {
+    const int j = threadIdx.x;
+    const Key key{M->key0, M->key1};
+    double n[9], nf[9];
+    for (int i = 0; i < 9; i++) { n[i] = c->cnt9[i]; nf[i] = n[i] - c->cnt9[9 + i]; }
+    double shape, scale = 1.0;
+    uint32_t sub = (uint32_t)j, c3 = tagword(ms, TAG_TRANS);
+    bool on = true;
+    switch (j) {
+    case 0: shape = M->ha_g + n[1 * 3 + 0] + n[2 * 3 + 0]; break;
+    case 1: shape = M->hb_g + n[0]; break;
+    case 2: shape = M->ha_l + nf[2 * 3 + 1]; break;
+    case 3: shape = M->hb_l + nf[1 * 3 + 1]; break;
+    case 4: shape = M->ha_l2 + nf[1 * 3 + 2]; on = M->ha_l2 != 0; break;
+    case 5: shape = M->hb_l2 + nf[2 * 3 + 2]; on = M->ha_l2 != 0; break;
+    case GV_R2:
+        c3 = tagword(ms, TAG_R2);
+        if (c->has_cls[1]) {
+            shape = c->nrate / c->prop_n;
+            scale = c->prop_n;
+            sub = 1;
+        } else {
+            shape = M->nprior_a;
+            scale = M->nprior_b;
+            sub = 2;
+            on = resZ != 0;
+        }
+        break;
+    default:
+        c3 = tagword(ms, TAG_R1);
+        shape = M->cprior_a;
+        scale = M->cprior_b;
+        sub = 2;
+        on = !c->has_cls[0] && resZ != 0;
+        break;
+    }
+    double x = 0.0;
+    int capped = 0;
+    if (on) {
+        Stream st{key, sub, (uint32_t)m, c3, 0};
+        x = gamma_draw(st, shape, scale, &capped);
+    }
+    if (capped) __hip_atomic_fetch_or(&c->fail, PA_F_SAMPLER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    c->gam[j] = x;
+}
+
+// Scalar head of BPP_C::sample_rate (src/PhyloAcc-ST/bpp_c.cpp:930-1041), one
+// lane: the prior draw when no branch carries the class, else the proposal
+// and its range checks.
+template <typename R>
+__device__ __forceinline__ void rate_propose(MP M, CP<R> c, int ms, int m, int resZ, bool neut)
+{
+    const double old = neut ? c->nrate : c->crate;
+    c->old_rate = old;
     const Key key{M->key0, M->key1};
     const uint32_t c3 = tagword(ms, neut ? TAG_R2 : TAG_R1), c2 = (uint32_t)m;
-    const double pa = neut ? M->nprior_a : M->cprior_a, pb = neut ? M->nprior_b : M->cprior_b;
     double cur = old;
     c->skip = 1;
     c->accept = 0;
-    if (!c->dirty[c->root]) {
+    if (!c->has_cls[neut ? 1 : 0]) {
         if (resZ != 0) {
-            Stream sp{key, 2, c2, c3, 0};
-            int capped = 0;
-            cur = gamma_draw(sp, pa, pb, &capped);
-            if (capped) c->fail |= PA_F_SAMPLER;
+            cur = c->gam[neut ? GV_R2 : GV_R1];
             if (neut) {
                 if (M->ropt == 1 && cur < M->nlb) cur = old;
                 else if (M->ropt == 2 && cur < c->crate) cur = old;
@@ -1102,10 +1206,7 @@ __device__ __noinline__ void rate_propose(MP M, CP<R> c, int ms, int m, int resZ
         double prop;
         int skip = 0;
         if (neut) {
-            Stream sg{key, 1, c2, c3, 0};
-            int capped = 0;
-            prop = gamma_draw(sg, cur / c->prop_n, c->prop_n, &capped);
-            if (capped) c->fail |= PA_F_SAMPLER;
+            prop = c->gam[GV_R2];
             if (M->ropt == 1 && prop < M->nlb) skip = 1;
             else if (M->ropt == 2 && prop < c->crate) skip = 1;
         } else {
@@ -1126,22 +1227,34 @@ __device__ __noinline__ void rate_propose(MP M, CP<R> c, int ms, int m, int resZ
     if (neut) c->nrate = cur; else c->crate = cur;
 }
 
+// The terms of the Metropolis ratio (bpp_c.cpp:1046-1094) that do not need
+// the proposal's likelihood, a lane each, FP64: the prior densities of the
+// proposal and the old rate, the proposal densities (r2) or the logarithms
+// (r1) of the two, and the log of the acceptance uniform.
+template <typename R>
+__device__ __noinline__ void rate_terms(MP M, CP<R> c, bool neut, double old, int lane)
+{
+    if (lane >= 5) return;
+    const double prop = c->proposal, x = (lane == 1 || lane == 2) ? old : prop;
+    double a = neut ? M->nprior_a : M->cprior_a, b = neut ? M->nprior_b : M->cprior_b;
+    if (lane == 2) { a = prop / c->prop_n; b = c->prop_n; }
+    else if (lane == 3) { a = old / c->prop_n; b = c->prop_n; }
+    double t;
+    if (lane == 4) t = log(c->r);
+    else if (!neut && lane >= 2) t = log(x);
+    else t = log_gamma_pdf(x, a, b);
+    c->mh[lane] = t;
+}
+
 // Metropolis decision (bpp_c.cpp:1046-1094), FP64.
 template <typename R>
-__device__ __noinline__ void rate_decide(MP M, CP<R> c, bool neut, double old, double lnew)
+__device__ __forceinline__ void rate_decide(CP<R> c, bool neut, double lnew)
 {
-    const double pa = neut ? M->nprior_a : M->cprior_a, pb = neut ? M->nprior_b : M->cprior_b;
-    const double prop = c->proposal;
-    double MH;
-    if (neut)
-        MH = lnew - c->loglik + log_gamma_pdf(prop, pa, pb) - log_gamma_pdf(old, pa, pb) +
-             log_gamma_pdf(old, prop / c->prop_n, c->prop_n) - log_gamma_pdf(prop, old / c->prop_n, c->prop_n);
-    else
-        MH = lnew - c->loglik + log_gamma_pdf(prop, pa, pb) - log_gamma_pdf(old, pa, pb) + log(old) - log(prop);
-    if (log(c->r) < MH) {
+    const double MH = lnew - c->loglik + c->mh[0] - c->mh[1] + c->mh[2] - c->mh[3];
+    if (c->mh[4] < MH) {
         c->accept = 1;
         c->loglik = lnew;
-        if (neut) c->nrate = prop; else c->crate = prop;
+        if (neut) c->nrate = c->proposal; else c->crate = c->proposal;
     }
 }
 
@@ -1170,36 +1283,31 @@ __device__ __noinline__ void rate_adapt(MP M, CP<R> c, int m, bool neut)
 template <typename R, int BS, int SH>
 __device__ __noinline__ void build_prop_tables(MP M, CP<R> c, int cls, double prop)
 {
-    for (int q = threadIdx.x; q < c->n_nodes - 1; q += BS) {
-        const int s = c->nodes[q];
-        if (c->Z[s] != cls || (c->flags[s] & NF_MISSING)) continue;
-        const double t = c->dist2[s] * prop;
-        double e[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) e[k] = exp(M->lam[k] * t);
+    const int n_item = 4 * (uni(c->n_nodes) - 1);
+    const LDS int16_t *nodes = uni_ptr(c->nodes);
+    const GBL double *dist2 = uni_ptr(c->dist2);
+    for (int it = threadIdx.x; it < n_item; it += BS) {
+        const int s = nodes[it >> 2], j = it & 3;
+        if (c->Z[s] != cls || (c->flags[s] & NF_MISSING)) continue;     // a whole quad
+        double row[4];
+        ptrans_row(M, dist2[s] * prop, j, row);
         LDS R *dst = c->PTp + 16 * s;
-#pragma unroll 1
-        for (int j = 0; j < 4; j++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                double v = 0;
-#pragma unroll
-                for (int k = 0; k < 4; k++) v += M->V[j * 4 + k] * e[k] * M->Vi[k * 4 + i];
-                dst[i * 4 + j] = (R)(v < 0 ? 0.0 : v);
-            }
+        for (int i = 0; i < 4; i++) dst[i * 4 + j] = (R)row[i];
     }
 }
 
+// dirty (cleared before) = ancestors of the branches of a class
 template <typename R, int BS, int SH>
 __device__ __noinline__ void mark_class(CP<R> c, int cls)
 {
-    const int tid = threadIdx.x, N = c->N;
-    for (int q = tid; q < c->n_nodes; q += BS) c->dirty[c->nodes[q]] = 0;
-    __syncthreads();
-    for (int q = tid; q < c->n_nodes; q += BS) {
-        const int s = c->nodes[q];
+    const int N = uni(c->N), n_nodes = uni(c->n_nodes);
+    const LDS int16_t *nodes = uni_ptr(c->nodes), *par = uni_ptr(c->par);
+    LDS uint8_t *dirty = uni_ptr(c->dirty);
+    for (int q = threadIdx.x; q < n_nodes; q += BS) {
+        const int s = nodes[q];
         if ((c->flags[s] & NF_MISSING) || c->Z[s] != cls) continue;
-        for (int j = c->par[s]; j != N; j = c->par[j]) c->dirty[j] = 1;
+        for (int j = par[s]; j != N; j = par[j]) dirty[j] = 1;
     }
 }
 
@@ -1209,34 +1317,33 @@ __device__ __forceinline__ void sample_rate(MP M, CP<R> c, int ms, int m, int re
 {
     const int tid = threadIdx.x;
     const int cls = neut ? 2 : 1;
-    const double old = neut ? c->nrate : c->crate;
-    mark_class<R, BS, SH>(c, cls);
+    if (c->has_cls[neut ? 1 : 0])
+        for (int q = tid; q < c->n_nodes; q += BS) c->dirty[c->nodes[q]] = 0;
+    if (tid == 0) rate_propose<R>(M, c, ms, m, resZ, neut);
     __syncthreads();
-    if (tid == 0) rate_propose<R>(M, c, ms, m, resZ, neut, old);
-    __syncthreads();
+    const double old = c->old_rate;
     if (!c->skip) {
+        mark_class<R, BS, SH>(c, cls);
         build_prop_tables<R, BS, SH>(M, c, cls, c->proposal);
+        if (tid >= BS - 64) rate_terms<R>(M, c, neut, old, tid - (BS - 64));
         __syncthreads();
         const double lnew = prune<R, BS, SH>(M, c, PR_PROP, cls);
-        if (tid == 0) rate_decide<R>(M, c, neut, old, lnew);
+        if (tid == 0) rate_decide<R>(c, neut, lnew);
         __syncthreads();
         if (c->accept) {
             for (int q = tid; q < c->n_int; q += BS) {
                 const int s = c->inodes[q];
                 if (c->dirty[s] && !(c->flags[s] & NF_MISSING)) {
-                    c->cur[s] ^= 1;
-                    c->srec[2 * (c->n_int - 1 - q)] ^= SR_CUR;
+                    const int cu = c->cur[s] ^ 1;
+                    c->cur[s] = (uint8_t)cu;
+                    LDS uint32_t *r1 = c->srec + 2 * (c->n_int - 1 - q) + 1;
+                    if (!(c->flags[s] & NF_CHERRY)) *r1 = (*r1 & ((1u << SR_SLOT_SHIFT) - 1)) | (uint32_t)(cu * c->I + s - c->S) << SR_SLOT_SHIFT;
                 }
             }
         }
     }
     const double now = neut ? c->nrate : c->crate;
-    if (now != old) {
-        for (int q = tid; q < c->n_nodes - 1; q += BS) class_table<R>(M, c, cls, c->nodes[q], now, 1);
-        __syncthreads();
-        refresh_PTc<R, BS, SH>(c, cls);
-    }
-    __syncthreads();
+    if (now != old) class_tables<R, BS>(M, c, cls, now, 1);
     if (tid == 0) {
         if (now != old) { if (neut) c->accept_n += 1; else c->accept_c += 1; }
         rate_adapt<R>(M, c, m, neut);
@@ -1244,58 +1351,33 @@ __device__ __forceinline__ void sample_rate(MP M, CP<R> c, int ms, int m, int re
     __syncthreads();
 }
 
-// The three Beta draws of BPP_C::sample_transition (src/PhyloAcc-ST/bpp_c.cpp:522-613),
-// Beta(a, b) = X / (X + Y) with X ~ Gamma(a) on sub-stream 2k and Y ~ Gamma(b) on
-// sub-stream 2k + 1 (beta_draw).  The six gamma variates are independent, so lane j < 6
-// draws the one of sub-stream j into red[j]; the l2 pair is not drawn when its prior is off.
-template <typename R>
-__device__ __noinline__ void transition_gamma(MP M, CP<R> c, int ms, int m, int j)
-{
-    const Key key{M->key0, M->key1};
-    const uint32_t c3 = tagword(ms, TAG_TRANS), c2 = (uint32_t)m;
-    double n[9], nf[9];
-    for (int i = 0; i < 9; i++) { n[i] = c->cnt9[i]; nf[i] = n[i] - c->cnt9[9 + i]; }
-    double shape;
-    switch (j) {
-    case 0: shape = M->ha_g + n[1 * 3 + 0] + n[2 * 3 + 0]; break;
-    case 1: shape = M->hb_g + n[0]; break;
-    case 2: shape = M->ha_l + nf[2 * 3 + 1]; break;
-    case 3: shape = M->hb_l + nf[1 * 3 + 1]; break;
-    case 4: shape = M->ha_l2 + nf[1 * 3 + 2]; break;
-    default: shape = M->hb_l2 + nf[2 * 3 + 2]; break;
-    }
-    double x = 0.0;
-    if (j < 4 || M->ha_l2 != 0) {
-        Stream st{key, (uint32_t)j, c2, c3, 0};
-        int capped = 0;
-        x = gamma_draw(st, shape, 1.0, &capped);
-        if (capped)   // up to six lanes draw at once
-            __hip_atomic_fetch_or(&c->fail, PA_F_SAMPLER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    c->red[j] = x;
-}
-
+// The Z-transition counts and which rate classes any branch carries, then the
+// sweep's gamma variates and the transition probabilities they give
+// (BPP_C::sample_transition, src/PhyloAcc-ST/bpp_c.cpp:522-613).  Both depend
+// on Z alone, so they follow the Z update.
 template <typename R, int BS, int SH>
-__device__ __forceinline__ void sample_transition(MP M, CP<R> c, int ms, int m)
+__device__ __forceinline__ void sample_transition(MP M, CP<R> c, int ms, int m, int resZ)
 {
     const int tid = threadIdx.x;
     if (tid < 18) c->cnt9[tid] = 0;
+    if (tid < 2) c->has_cls[tid] = 0;
     __syncthreads();
     for (int q = tid; q < c->n_nodes - 1; q += BS) {
         const int s = c->nodes[q];
         const int zi = c->Z[s], zp = c->Z[c->par[s]];
         lds_add(&c->cnt9[zi * 3 + zp], 1u);
         if (c->fixZ[s]) lds_add(&c->cnt9[9 + zi * 3 + zp], 1u);
+        if (zi > 0 && !(c->flags[s] & NF_MISSING)) c->has_cls[zi - 1] = 1;     // every writer stores the same value
     }
     __syncthreads();
-    if (tid < 6) transition_gamma<R>(M, c, ms, m, tid);
+    if (tid < GV_N) draw_gammas<R>(M, c, ms, m, resZ);
     __syncthreads();
-    if (tid == 0) {
-        const double g = c->red[0] / (c->red[0] + c->red[1]);
-        const double l = c->red[2] / (c->red[2] + c->red[3]);
-        const double l2 = M->ha_l2 == 0 ? 0.0 : c->red[4] / (c->red[4] + c->red[5]);
-        c->g = g; c->l = l; c->l2 = l2;
-        set_TM(c->TMf, c->TMn, g, l, l2);
+    if (tid < 64) {
+        const double g = c->gam[0] / (c->gam[0] + c->gam[1]);
+        const double l = c->gam[2] / (c->gam[2] + c->gam[3]);
+        const double l2 = M->ha_l2 == 0 ? 0.0 : c->gam[4] / (c->gam[4] + c->gam[5]);
+        if (tid == 0) { c->g = g; c->l = l; c->l2 = l2; }
+        set_TM(c->TMf, c->TMn, g, l, l2, tid);
     }
     __syncthreads();
 }
@@ -1426,7 +1508,7 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
     __syncthreads();
     sample_steps<R, BS>(c);
     // null-rate tables (rate 1), fixed for the element
-    for (int q = tid; q < c->n_nodes - 1; q += BS) class_table<R>(M, c, 0, c->nodes[q], 1.0, 0);
+    class_tables<R, BS>(M, c, 0, 1.0, 0);
     __syncthreads();
 }
 
@@ -1453,7 +1535,12 @@ __device__ __noinline__ void init_model(MP M, CP<R> c, int resZ)
         c->fixZ[s] = (uint8_t)fz;
         c->cur[s] = 0;
     }
-    for (int t = tid; t < c->n_int; t += BS) c->srec[2 * t] &= ~(uint32_t)SR_CUR;
+    for (int t = tid; t < c->n_int; t += BS) {
+        // every node's partial in buffer 0
+        const int s = c->inodes[c->n_int - 1 - t], v = (c->flags[s] & (NF_MISSING | NF_CHERRY)) ? root : s;
+        LDS uint32_t *r1 = c->srec + 2 * t + 1;
+        *r1 = (*r1 & ((1u << SR_SLOT_SHIFT) - 1)) | (uint32_t)(v - c->S) << SR_SLOT_SHIFT;
+    }
     if (tid == 0) {
         c->prop_c = 1.2;
         c->prop_n = (double)1 / c->GG * 10;
@@ -1462,38 +1549,44 @@ __device__ __noinline__ void init_model(MP M, CP<R> c, int resZ)
         c->nrate = M->init_nrate;
         c->crate = M->init_crate;
         c->g = M->init_grate; c->l = M->init_lrate; c->l2 = M->ha_l2 == 0 ? 0.0 : M->init_lrate2;
-        set_TM(c->TMf, c->TMn, c->g, c->l, c->l2);
         c->fail = 0;
     }
+    if (tid < 64) set_TM(c->TMf, c->TMn, M->init_grate, M->init_lrate, M->ha_l2 == 0 ? 0.0 : M->init_lrate2, tid);
     __syncthreads();
     const double cr = c->crate, nr = c->nrate;
-    for (int q = tid; q < c->n_nodes - 1; q += BS) {
-        const int s = c->nodes[q];
-        class_table<R>(M, c, 1, s, cr, 0);
-        class_table<R>(M, c, 2, s, nr, 0);
-    }
+    class_tables<R, BS>(M, c, 1, cr, 0);
+    class_tables<R, BS>(M, c, 2, nr, 0);
     __syncthreads();
-    refresh_PTc<R, BS, SH>(c, -1);
+    refresh_PTc<R, BS, SH>(c, false);
     __syncthreads();
 }
 
-// BPP_C::MonitorChain (src/PhyloAcc-ST/bpp_c.cpp:741-834), thread 0
+// BPP_C::MonitorChain (src/PhyloAcc-ST/bpp_c.cpp:741-834), one wave: the two
+// prior densities a lane each
 template <typename R>
-__device__ __noinline__ void monitor(MP M, CP<R> c, int m, int resZ, double *trd, int T)
+__device__ __noinline__ void monitor(MP M, CP<R> c, int m, int resZ, double *trd, int T, int lane)
 {
-    double full = c->loglik + log_gamma_pdf(c->crate, M->cprior_a, M->cprior_b);
-    if (resZ != 0) full += log_gamma_pdf(c->nrate, M->nprior_a, M->nprior_b);
-    if (trd) {
-        trd[0 * T + m] = c->loglik; trd[1 * T + m] = full; trd[2 * T + m] = c->nrate;
-        trd[3 * T + m] = c->crate; trd[4 * T + m] = c->g; trd[5 * T + m] = c->l; trd[6 * T + m] = c->l2;
+    const double loglik = c->loglik, nrate = c->nrate, crate = c->crate;
+    const bool neut = lane & 1;
+    const double d = log_gamma_pdf(neut ? nrate : crate, neut ? M->nprior_a : M->cprior_a, neut ? M->nprior_b : M->cprior_b);
+    double full = loglik + __shfl(d, 0, 64);
+    const double dn = __shfl(d, 1, 64);
+    if (resZ != 0) full += dn;
+    if (trd && lane == 0) {
+        trd[0 * T + m] = loglik; trd[1 * T + m] = full; trd[2 * T + m] = nrate;
+        trd[3 * T + m] = crate; trd[4 * T + m] = c->g; trd[5 * T + m] = c->l; trd[6 * T + m] = c->l2;
     }
     if (m >= M->burnin && full > c->max_loglik) {
-        c->max_loglik = full;
-        c->max_m = m;
-        for (int i = 0; i < M->N; i++) c->maxZ[i] = c->Z[i];
+        for (int i = lane; i < M->N; i += 64) c->maxZ[i] = c->Z[i];
+        if (lane == 0) {
+            c->max_loglik = full;
+            c->max_m = m;
+        }
     }
-    if (isnan(c->loglik)) c->fail |= PA_F_NAN;
-    else if (isinf(c->loglik)) c->fail |= c->loglik > 0 ? PA_F_POS_INF : PA_F_NEG_INF;
+    if (lane == 0) {
+        if (isnan(loglik)) c->fail |= PA_F_NAN;
+        else if (isinf(loglik)) c->fail |= loglik > 0 ? PA_F_POS_INF : PA_F_NEG_INF;
+    }
 }
 
 template <typename R, int BS, int SH>
@@ -1529,23 +1622,24 @@ __device__ __forceinline__ void run_model(MP M, CP<R> c, const ChainArgs *A, int
     for (int m = 0; m < T; m++) {
         if (trz)
             for (int i = tid; i < N; i += BS) trz[(size_t)m * N + i] = c->Z[i];
-        if (tid == 0) monitor<R>(M, c, m, resZ, trd, T);
+        // the last wave, which has the fewest sites to draw
+        if (tid >= BS - 64) monitor<R>(M, c, m, resZ, trd, T, tid - (BS - 64));
         if (m == T - 1) break;
         sample_sites<R, BS, SH>(M, c, (uint32_t)m, tagword(ms, TAG_ANC));
         __syncthreads();
         emissions<R, BS, SH>(c);
         __syncthreads();
         update_Z<R, BS, SH>(M, c, (uint32_t)m, tagword(ms, TAG_Z));
-        refresh_PTc<R, BS, SH>(c, REFRESH_CHANGED);
+        refresh_PTc<R, BS, SH>(c, true);
         __syncthreads();
         if (c->nch) {
             const double l = prune<R, BS, SH>(M, c, PR_DIRTY, 0);
             if (tid == 0) c->loglik = l;
             __syncthreads();
         }
+        sample_transition<R, BS, SH>(M, c, ms, m, resZ);
         sample_rate<R, BS, SH>(M, c, ms, m, resZ, true);
         sample_rate<R, BS, SH>(M, c, ms, m, resZ, false);
-        sample_transition<R, BS, SH>(M, c, ms, m);
     }
     __syncthreads();
     write_results<R, BS, SH>(M, c, A, ms, work);

@@ -56,8 +56,8 @@ struct Ctx {
     LDS int16_t *par, *nodes, *inodes, *porder, *upoff;
     LDS uint32_t *urec;    // [I] internal nodes by level: node | child 0 << 10 | child 1 << 20
     LDS uint32_t *desc;    // [I][4] static pruning descriptor of each internal node (node_desc)
-    LDS uint32_t *steps;   // [I][4] the steps of a pass (build_steps)
-    LDS uint32_t *srec;    // [I][2] the steps of the sampler (sample_steps)
+    LDS uint32_t *steps;   // [I + 1][4] the steps of a pass (build_steps)
+    LDS uint32_t *srec;    // [I + 1][2] the steps of the sampler (sample_steps)
     LDS uint8_t *flags, *fixZ, *dirty, *cur, *changed;
     LDS int8_t *Z, *maxZ;
     LDS double *E, *msg;   // [N][3] emissions, then Z messages at a node; messages to its parent
@@ -104,7 +104,7 @@ __host__ __device__ size_t smem_arrays(int N, int S, int BS, LDS char *base, CP<
     //      proposal matrices (rate updates).  sample_sites clears the
     //      counters before it counts.
     {
-        const size_t szA = std::max({(size_t)(I > 0 ? I : 1) * BS, (size_t)6 * N * sizeof(double), (size_t)20 * 4});
+        const size_t szA = std::max({(size_t)(I > 0 ? I : 1) * BS, (size_t)6 * N * sizeof(double), (size_t)20 * 4, (size_t)16 * (I + 1)});
         const size_t szB = std::max((size_t)16 * N * sizeof(uint32_t), (size_t)16 * N * sizeof(R));
         o = al(o, 32);
         if constexpr (BIND) {
@@ -124,7 +124,8 @@ __host__ __device__ size_t smem_arrays(int N, int S, int BS, LDS char *base, CP<
     o = al(o, 16);      // descriptors are read as 16-byte vectors
     if constexpr (BIND) c->desc = (LDS uint32_t *)(base + o);
     o += (size_t)16 * (I > 0 ? I : 1);
-    PA_TAKE(srec, uint32_t, 2 * (I > 0 ? I : 1));
+    o = al(o, 8);       // sampler steps as 8-byte vectors
+    PA_TAKE(srec, uint32_t, 2 * (I + 1));
     PA_TAKE(urec, uint32_t, I > 0 ? I : 1);
     PA_TAKE(par, int16_t, N);
     PA_TAKE(nodes, int16_t, N);
@@ -183,6 +184,7 @@ size_t slot_scratch_bytes(int N, int S, int Pcap, int fp64, size_t *off)
 // offset and a scalar one, and an access outside the region is dropped (a
 // load gives 0).
 typedef __amdgpu_buffer_rsrc_t Buf;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <typename T>
@@ -456,6 +458,7 @@ __device__ __forceinline__ void build_steps(CP<R> c, int mode, int cls)
         n_leaf += __popcll(nodes & __ballot(leaves & 1)) + __popcll(nodes & __ballot(leaves & 2));
         n_cherry += __popcll(nodes & __ballot(cherries & 1)) + __popcll(nodes & __ballot(cherries & 2));
     }
+    if (lane < 4) steps[4 * base + lane] = 0;       // the step read ahead of the end
     if (lane == 0) {
         c->n_steps = base;
         c->last_step = last1;
@@ -469,7 +472,7 @@ __device__ __forceinline__ void build_steps(CP<R> c, int mode, int cls)
 // The scalar arguments of a pass's pattern loop.
 template <typename R>
 struct PassArgs {
-    const LDS uint32_t *steps;
+    const LDS u32x4 *steps;
     const LDS R *PT;             // [2N][16]: the current matrices, then the proposal's
     Buf codes;
     int n, I;
@@ -544,9 +547,9 @@ __device__ __forceinline__ ChildIn<R> slot_load(Buf blk, uint32_t slot, uint32_t
 // steps.  All lanes run (patterns are padded to whole waves).  Every step
 // issues the same code loads and stores, whether it needs them or not, since
 // a step's wait for its loads counts the memory operations issued after them:
-// a child that is no leaf loads row 0's code, and a cherry, which is kept in
-// registers only, stores through a buffer of no bytes (the hardware drops
-// accesses outside a buffer).
+// a child that is no leaf loads row 0's code, the steps past the last are an
+// empty one, and a cherry, which is kept in registers only, stores through a
+// buffer of no bytes (the hardware drops accesses outside a buffer).
 template <typename R, bool AMB>
 __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL char *base, int blk_bytes, uint32_t p)
 {
@@ -555,7 +558,7 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
     const Buf blk = make_buf(base, blk_bytes);
     ChildIn<R> inA[2], inB[2], res[2];
     int cdA[2], cdB[2];
-    uint32_t w[2][4], nw[4];
+    uint32_t w[2][4];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         res[j].x = GAPT;
@@ -563,16 +566,13 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
         inA[j] = inB[j] = res[j];
         cdA[j] = cdB[j] = 0;
     }
-#pragma unroll
-    for (int i = 0; i < 4; i++) nw[i] = A.steps[i];
+    u32x4 nw = A.steps[0];
     // words and inputs of step k into set j
     auto fetch = [&](auto J, int k) __attribute__((always_inline)) {
         constexpr int j = decltype(J)::value;
 #pragma unroll
         for (int i = 0; i < 4; i++) w[j][i] = (uint32_t)uni((int)nw[i]);
-        const LDS uint32_t *nx = A.steps + 4 * (k + 1 < n ? k + 1 : k);
-#pragma unroll
-        for (int i = 0; i < 4; i++) nw[i] = nx[i];
+        nw = A.steps[k + 1 < n ? k + 1 : n];
         const uint32_t w0 = w[j][0];
         if (w0 & SB_STORED_A) inA[j] = slot_load<R>(blk, (w0 >> SB_SLOT_A_SHIFT) & 511, lane, A.I);
         if (w0 & SB_STORED_B) inB[j] = slot_load<R>(blk, w[j][3] >> SB_SLOT_B_SHIFT, lane, A.I);
@@ -632,7 +632,7 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
             out = combine<R>(a, b, e, ga && gb);
             if ((w0 & SB_MISS) && !(ga && gb)) out.x = 0;
         }
-        if (k + 2 < n) fetch(J, k + 2);
+        fetch(J, k + 2);
         res[j] = out;
         const uint32_t d = w0 >> SB_SLOT_SHIFT;
         const Buf to = make_buf(base, (w0 & SB_CHERRY) ? 0 : blk_bytes);
@@ -640,10 +640,12 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
         __builtin_amdgcn_raw_buffer_store_b32((uint32_t)out.x, to, lane * 4, exp_off<R>(d, A.I), 0);
     };
     fetch(std::integral_constant<int, 0>(), 0);
-    if (n > 1) fetch(std::integral_constant<int, 1>(), 1);
-    for (int k = 0; k < n; k += 2) {
+    fetch(std::integral_constant<int, 1>(), 1);
+    for (int k = 0;; k += 2) {
         step(std::integral_constant<int, 0>(), k);
-        if (k + 1 < n) step(std::integral_constant<int, 1>(), k + 1);
+        if (k + 1 >= n) break;
+        step(std::integral_constant<int, 1>(), k + 1);
+        if (k + 2 >= n) break;
     }
     const bool odd = (n - 1) & 1;
     ChildIn<R> r;
@@ -664,7 +666,7 @@ __device__ __forceinline__ double prune_patterns(MP M, CP<R> c, int mode)
     PassArgs<R> A;
     A.n = uni(c->n_steps);
     A.I = uni(c->I);
-    A.steps = uni_ptr(c->steps);
+    A.steps = (const LDS u32x4 *)uni_ptr(c->steps);
     A.PT = uni_ptr(c->PTc);
     A.codes = make_buf(uni_ptr(c->codes), code_bytes(uni(c->S), uni(c->Ppad)));
     GBL char *parts = uni_ptr(c->parts);
@@ -760,7 +762,7 @@ __device__ __forceinline__ void draw_sites(MP M, CP<R> c, uint32_t c2, uint32_t 
     GBL uint32_t *amb = uni_ptr(c->amb);
     LDS uint8_t *tgs = uni_ptr(c->tgs) + tid - S * BS;      // node s: [s * BS]
     LDS uint32_t *hist = uni_ptr(c->hist);
-    const LDS uint32_t *srec = uni_ptr(c->srec);
+    const LDS u32x2 *srec = (const LDS u32x2 *)uni_ptr(c->srec);
     const LDS R *PTc = uni_ptr(c->PTc);
     for (int gb = uni(tid & ~63); gb < GG; gb += BS) {
         const int g = gb + (tid & 63);
@@ -769,16 +771,15 @@ __device__ __forceinline__ void draw_sites(MP M, CP<R> c, uint32_t c2, uint32_t 
         // this pattern's entries of slot 0
         const GBL char *pp = parts + (int64_t)(p >> 6) * blkB + (p & 63) * sizeof(V4<R>);
         const GBL char *pe = parts + (int64_t)(p >> 6) * blkB + exp_off<R>(0, I) + (p & 63) * 4;
-        uint32_t r0[K], r1[K], nr0 = srec[0], nr1 = srec[1];
+        uint32_t r0[K], r1[K];
+        u32x2 nr = srec[0];
         ChildIn<R> in[K];
         int cdA[K], cdB[K];
         auto fetch = [&](auto J, int t) __attribute__((always_inline)) {
             constexpr int j = decltype(J)::value;
-            r0[j] = (uint32_t)uni((int)nr0);
-            r1[j] = (uint32_t)uni((int)nr1);
-            const LDS uint32_t *nx = srec + 2 * (t + 1 < n_int ? t + 1 : t);
-            nr0 = nx[0];
-            nr1 = nx[1];
+            r0[j] = (uint32_t)uni((int)nr.x);
+            r1[j] = (uint32_t)uni((int)nr.y);
+            nr = srec[t + 1 < n_int ? t + 1 : n_int];
             const uint32_t slot = r1[j] >> SR_SLOT_SHIFT;
             in[j].v = ld4<R>((const GBL V4<R> *)(pp + (uint64_t)part_off<R>(slot)));
             in[j].x = *(const GBL int32_t *)(pe + (uint64_t)(slot * 256));
@@ -800,7 +801,7 @@ __device__ __forceinline__ void draw_sites(MP M, CP<R> c, uint32_t c2, uint32_t 
             const int s = w0 & SR_ID;
             const int tp_read = tp & 3;
             // the next step's parent, unless it is this node
-            if (t + 1 < n_int) tp = tgs[((r0[(j + 1) % K] >> SR_PAR_SHIFT) & SR_ID) * BS];
+            tp = tgs[((r0[(j + 1) % K] >> SR_PAR_SHIFT) & SR_ID) * BS];
             if (!(w0 & SR_MISS)) {
                 ChildIn<R> a;
                 if (w0 & SR_CHERRY) {
@@ -835,11 +836,12 @@ __device__ __forceinline__ void draw_sites(MP M, CP<R> c, uint32_t c2, uint32_t 
                 if (w0 & SR_LEAF_A) count_leaf(w1 & SR_ID, cdA[j]);
                 if (w0 & SR_LEAF_B) count_leaf((w1 >> 10) & SR_ID, cdB[j]);
             }
-            if (t + K < n_int) fetch(std::integral_constant<int, j>(), t + K);
+            fetch(std::integral_constant<int, j>(), t + K);
         };
-        each<K>([&](auto J) __attribute__((always_inline)) { if (decltype(J)::value < n_int) fetch(J, decltype(J)::value); });
+        each<K>([&](auto J) __attribute__((always_inline)) { fetch(J, decltype(J)::value); });
+        // whole groups of UN steps: those past the last node are missing nodes
         for (int t0 = 0; t0 < n_int; t0 += UN)
-            each<UN>([&](auto J) __attribute__((always_inline)) { if (t0 + decltype(J)::value < n_int) step(J, t0 + decltype(J)::value); });
+            each<UN>([&](auto J) __attribute__((always_inline)) { step(J, t0 + decltype(J)::value); });
     }
 }
 
@@ -894,6 +896,9 @@ __device__ __noinline__ void sample_steps(CP<R> c)
         c->srec[2 * t + 1] = w1 | (uint32_t)(v - S) << SR_SLOT_SHIFT;      // buffer 0
     }
     if (threadIdx.x == 0) {
+        // the steps past the last
+        c->srec[2 * n_int] = (uint32_t)c->root | (uint32_t)c->root << SR_PAR_SHIFT | SR_MISS;
+        c->srec[2 * n_int + 1] = (uint32_t)(c->root - S) << SR_SLOT_SHIFT;
         int nint = 0, nch = 0, nleaf = 0;
         for (int k = 0; k < n_int; k++) {
             const uint8_t f = c->flags[c->inodes[k]];

@@ -36,6 +36,7 @@
 #include "pa_rng.h"
 #include "pa_chain.h"
 #include "pa_device.h"
+#include "pa_prune.h"
 
 namespace pa {
 namespace chain {
@@ -156,14 +157,11 @@ size_t chain_smem_bytes(int N, int S, int BS, int fp64)
 }
 
 // Partials of an element, by block of 64 patterns: two buffers of I node
-// slots of 64 4-vectors of R, then as many slots of 64 exponents (slot =
-// buffer * I + node - S).  A wave's block is one contiguous region, so every
-// address in a pass is a scalar base and a small offset.
-__host__ __device__ inline int block_bytes(int I, int rs) { return 2 * I * 64 * (4 * rs + 4); }
-
+// slots (slot = buffer * I + node - S).  A wave's block is one contiguous
+// region, so every address in a pass is a scalar base and a small offset.
 size_t chain_part_bytes(int N, int S, int Ppad, int fp64)
 {
-    return al((size_t)(Ppad / 64) * (size_t)block_bytes(N - S, fp64 ? 8 : 4), 256);
+    return al((size_t)(Ppad / 64) * (size_t)block_bytes(2 * (N - S), fp64 ? 8 : 4), 256);
 }
 
 // Per-workgroup HBM scratch layout (bytes), shared with the host: the rate
@@ -179,54 +177,6 @@ size_t slot_scratch_bytes(int N, int S, int Pcap, int fp64, size_t *off)
 }
 
 // ------------------------------------------------------------------ helpers
-
-// A region of memory as a raw buffer: loads and stores take a lane's byte
-// offset and a scalar one, and an access outside the region is dropped (a
-// load gives 0).
-typedef __amdgpu_buffer_rsrc_t Buf;
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-__device__ __forceinline__ Buf make_buf(T *base, int bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc((void *)(T *)base, 0, bytes, 0x00027000);
-}
-__device__ __forceinline__ int code_bytes(int S, int Ppad)
-{
-    const uint64_t n = (uint64_t)S * (uint32_t)Ppad;
-    return (int)(uint32_t)(n < 0xffffffffu ? n : 0xffffffffu);
-}
-
-template <int... J, typename F>
-__device__ __forceinline__ void each_of(std::integer_sequence<int, J...>, F &&f) { (f(std::integral_constant<int, J>()), ...); }
-// f(0) ... f(n - 1) with constant arguments: what it indexes stays in registers
-template <int n, typename F>
-__device__ __forceinline__ void each(F &&f) { each_of(std::make_integer_sequence<int, n>(), f); }
-
-template <typename R>
-__device__ __forceinline__ V4<R> buf_ld4(Buf b, uint32_t lane_off, uint32_t off)
-{
-    if constexpr (sizeof(R) == 4) {
-        return __builtin_bit_cast(V4<R>, __builtin_amdgcn_raw_buffer_load_b128(b, lane_off, off, 0));
-    } else {
-        struct { u32x4 lo, hi; } v = {__builtin_amdgcn_raw_buffer_load_b128(b, lane_off, off, 0),
-                                      __builtin_amdgcn_raw_buffer_load_b128(b, lane_off + 16, off, 0)};
-        return __builtin_bit_cast(V4<R>, v);
-    }
-}
-template <typename R>
-__device__ __forceinline__ void buf_st4(Buf b, const V4<R> &v, uint32_t lane_off, uint32_t off)
-{
-    if constexpr (sizeof(R) == 4) {
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), b, lane_off, off, 0);
-    } else {
-        struct P { u32x4 lo, hi; };
-        const P p = __builtin_bit_cast(P, v);
-        __builtin_amdgcn_raw_buffer_store_b128(p.lo, b, lane_off, off, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(p.hi, b, lane_off + 16, off, 0);
-    }
-}
 
 __device__ __forceinline__ void lds_add(LDS uint32_t *p, uint32_t v)
 {
@@ -333,24 +283,6 @@ enum { KD_LEAF = 0, KD_STORED = 1, KD_CHERRY = 2 };
 enum { DB_KIND1_SHIFT = 2, DB_MISS0 = 1 << 4, DB_MISS1 = 1 << 5, DB_MISS_A0 = 1 << 6, DB_MISS_B0 = 1 << 7,
        DB_MISS_A1 = 1 << 8, DB_MISS_B1 = 1 << 9, DB_MISS = 1 << 10 };
 
-// One step of a pass: an internal node the pass visits, or a cherry whose
-// parent it visits.  Four words:
-//   w0: type | SB_* bits | child A's slot << 14 | the node's slot, in the buffer it is written to, << 23
-//   w1, w2: the code row offsets of children A and B (row 0 for a child that is no leaf)
-//   w3: the children's matrices A | B << 10 (the node's id, + N for a proposal matrix) | child B's slot << 20
-// A child comes from its leaf code (L), its stored partial (S), or the result
-// of the step just before (P) or the one before that (P2), which the thread
-// still holds in registers.  The types are the combinations that occur when
-// nothing is missing, so each is straight code; ST_GEN takes any sources and
-// missing nodes.  The two children's order does not matter: their messages
-// are multiplied.
-enum { SK_LEAF = 0, SK_STORED = 1, SK_PREV = 2, SK_PREV2 = 3 };
-enum { ST_LL = 0, ST_PL = 1, ST_PP2 = 2, ST_SL = 3, ST_SP = 4, ST_SS = 5, ST_GEN = 6 };
-enum { SB_TYPE = 7, SB_STORED_A = 1 << 3, SB_STORED_B = 1 << 4, SB_CHERRY = 1 << 5, SB_MISS = 1 << 6, SB_MISS_A = 1 << 7,
-       SB_MISS_B = 1 << 8, SB_KIND_A_SHIFT = 9, SB_KIND_B_SHIFT = 11, SB_SLOT_A_SHIFT = 14, SB_SLOT_SHIFT = 23,
-       SB_MAT_MASK = 0x3ff, SB_MAT_B_SHIFT = 10, SB_SLOT_B_SHIFT = 20 };
-static_assert(MAXN <= 512, "slots (below 2 I <= N) in nine bits, matrices (below 2 N) in ten");
-
 // Pattern-loop shapes the autotuner picks among.  U: patterns a thread takes
 // through a pass together (they share each step's matrices); K: internal
 // nodes whose partials one sampling chunk loads before drawing.  Shape 0 is
@@ -420,28 +352,14 @@ __device__ __forceinline__ void build_steps(CP<R> c, int mode, int cls)
                 leaves |= (k == KD_LEAF) << j;
                 cherries |= (k == KD_CHERRY) << j;
             }
-            // child A: a stored node before the previous result, that before the one before it, a leaf last
-            const int rank = 0x2103;      // a nibble per kind
-            const int a = ((rank >> (4 * kind[1])) & 15) < ((rank >> (4 * kind[0])) & 15) ? 1 : 0;
-            const int ka = a ? kind[1] : kind[0], kb = a ? kind[0] : kind[1];
-            const int ma = a ? miss[1] : miss[0], mb = a ? miss[0] : miss[1];
-            int type = ST_GEN;
-            if (!(d3 & DB_MISS) && !ma && !mb) {
-                if (ka == SK_LEAF) type = ST_LL;
-                else if (ka == SK_PREV) type = kb == SK_LEAF ? ST_PL : (kb == SK_PREV2 ? ST_PP2 : ST_GEN);
-                else if (ka == SK_STORED) type = kb == SK_LEAF ? ST_SL : (kb == SK_PREV ? ST_SP : (kb == SK_STORED ? ST_SS : ST_GEN));
-            }
             const int cs = cur[s];
-            const int dst = (prop ? 1 - cs : cs) * I + s - S;
-            LDS uint32_t *w = steps + 4 * (base + __popcll(below));
-            w[0] = (uint32_t)type | (ka == SK_STORED ? SB_STORED_A : 0) | (kb == SK_STORED ? SB_STORED_B : 0) |
-                   ((f & NF_CHERRY) ? SB_CHERRY : 0) | ((d3 & DB_MISS) ? SB_MISS : 0) | (ma ? SB_MISS_A : 0) |
-                   (mb ? SB_MISS_B : 0) | ((uint32_t)ka << SB_KIND_A_SHIFT) | ((uint32_t)kb << SB_KIND_B_SHIFT) |
-                   ((uint32_t)(a ? slot[1] : slot[0]) << SB_SLOT_A_SHIFT) | ((uint32_t)dst << SB_SLOT_SHIFT);
-            w[1] = (uint32_t)(a ? row[1] : row[0]);
-            w[2] = (uint32_t)(a ? row[0] : row[1]);
-            w[3] = (uint32_t)(a ? m[1] : m[0]) | ((uint32_t)(a ? m[0] : m[1]) << SB_MAT_B_SHIFT) |
-                   ((uint32_t)(a ? slot[0] : slot[1]) << SB_SLOT_B_SHIFT);
+            StepDef d;
+            d.miss = (d3 & DB_MISS) != 0;
+            d.nostore = (f & NF_CHERRY) != 0;
+            d.slot_to = (prop ? 1 - cs : cs) * I + s - S;
+#pragma unroll
+            for (int j = 0; j < 2; j++) { d.kind[j] = kind[j]; d.miss_kid[j] = miss[j]; d.mat[j] = m[j]; d.row[j] = row[j]; d.slot[j] = slot[j]; }
+            encode_step(steps + 4 * (base + __popcll(below)), d);
         }
         const int cnt = __popcll(bal);
         if (cnt) {
@@ -469,194 +387,6 @@ __device__ __forceinline__ void build_steps(CP<R> c, int mode, int cls)
     }
 }
 
-// The scalar arguments of a pass's pattern loop.
-template <typename R>
-struct PassArgs {
-    const LDS u32x4 *steps;
-    const LDS R *PT;             // [2N][16]: the current matrices, then the proposal's
-    Buf codes;
-    int n, I;
-};
-
-// One child's message at one pattern, or ones where it holds no base; adds
-// its exponent and reports the gap.
-template <typename R, int K, bool AMB>
-__device__ __forceinline__ void message(const LDS R *PT, int code, const ChildIn<R> &in, V4<R> &o, int &e, bool &gap)
-{
-    if constexpr (K == SK_LEAF) {
-        gap = code == PA_GAP_CODE || code == PA_OTHER_CODE;
-        o = ld4<R>((const LDS V4<R> *)(PT + 4 * (code & 3)));
-        if (AMB && code > PA_OTHER_CODE) {
-            o.x = o.y = o.z = o.w = (R)1;
-            leaf_mul<R>(PT, code, o.x, o.y, o.z, o.w);
-        }
-        o.x = gap ? (R)1 : o.x; o.y = gap ? (R)1 : o.y; o.z = gap ? (R)1 : o.z; o.w = gap ? (R)1 : o.w;
-    } else {
-        gap = in.x == GAPT;
-        int x = in.x;
-        const V4<R> v = in.v;
-        const V4<R> m0 = ld4<R>((const LDS V4<R> *)(PT + 0)), m1 = ld4<R>((const LDS V4<R> *)(PT + 4));
-        const V4<R> m2 = ld4<R>((const LDS V4<R> *)(PT + 8)), m3 = ld4<R>((const LDS V4<R> *)(PT + 12));
-        o.x = m0.x * v.x + m1.x * v.y + m2.x * v.z + m3.x * v.w;
-        o.y = m0.y * v.x + m1.y * v.y + m2.y * v.z + m3.y * v.w;
-        o.z = m0.z * v.x + m1.z * v.y + m2.z * v.z + m3.z * v.w;
-        o.w = m0.w * v.x + m1.w * v.y + m2.w * v.z + m3.w * v.w;
-        if (__ballot(gap)) {
-            // rare: some lane's subtree holds only gaps
-            o.x = gap ? (R)1 : o.x; o.y = gap ? (R)1 : o.y; o.z = gap ? (R)1 : o.z; o.w = gap ? (R)1 : o.w;
-            x = gap ? 0 : x;
-        }
-        e += x;
-    }
-}
-
-// A node from its children's messages: their product, rescaled by a power of two.
-template <typename R>
-__device__ __forceinline__ ChildIn<R> combine(const V4<R> &a, const V4<R> &b, int e, bool gap)
-{
-    const R x = a.x * b.x, y = a.y * b.y, z = a.z * b.z, w = a.w * b.w;
-    const R mx = fmax(fmax(x, y), fmax(z, w));
-    int kx = 0;
-    frexp(mx, &kx);
-    ChildIn<R> r;
-    r.v.x = ldexp(x, -kx); r.v.y = ldexp(y, -kx); r.v.z = ldexp(z, -kx); r.v.w = ldexp(w, -kx);
-    r.x = gap ? GAPT : e + kx;
-    return r;
-}
-
-// Byte offsets of a slot's partials and exponents within a pattern block.
-template <typename R>
-__device__ __forceinline__ uint32_t part_off(uint32_t slot) { return slot * (64 * (uint32_t)sizeof(V4<R>)); }
-template <typename R>
-__device__ __forceinline__ uint32_t exp_off(uint32_t slot, int I) { return (uint32_t)(2 * I) * (64 * (uint32_t)sizeof(V4<R>)) + slot * 256; }
-
-// Slot's partial and exponent of this lane's pattern, from the block's buffer.
-template <typename R>
-__device__ __forceinline__ ChildIn<R> slot_load(Buf blk, uint32_t slot, uint32_t lane, int I)
-{
-    ChildIn<R> in;
-    in.v = buf_ld4<R>(blk, lane * (uint32_t)sizeof(V4<R>), part_off<R>(slot));
-    in.x = (int)__builtin_amdgcn_raw_buffer_load_b32(blk, lane * 4, exp_off<R>(slot, I), 0);
-    return in;
-}
-
-// Takes one pattern a lane (pattern p, of the block at base) through every
-// step and returns the last step's partial and exponent.  The inputs of step
-// k + 2 are loaded while step k is computed and its words are read a step
-// before that, so neither a memory nor an LDS round trip stands between two
-// steps.  All lanes run (patterns are padded to whole waves).  Every step
-// issues the same code loads and stores, whether it needs them or not, since
-// a step's wait for its loads counts the memory operations issued after them:
-// a child that is no leaf loads row 0's code, the steps past the last are an
-// empty one, and a cherry, which is kept in registers only, stores through a
-// buffer of no bytes (the hardware drops accesses outside a buffer).
-template <typename R, bool AMB>
-__device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL char *base, int blk_bytes, uint32_t p)
-{
-    const int n = A.n;
-    const uint32_t lane = threadIdx.x & 63;
-    const Buf blk = make_buf(base, blk_bytes);
-    ChildIn<R> inA[2], inB[2], res[2];
-    int cdA[2], cdB[2];
-    uint32_t w[2][4];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        res[j].x = GAPT;
-        res[j].v.x = res[j].v.y = res[j].v.z = res[j].v.w = (R)0;
-        inA[j] = inB[j] = res[j];
-        cdA[j] = cdB[j] = 0;
-    }
-    u32x4 nw = A.steps[0];
-    // words and inputs of step k into set j
-    auto fetch = [&](auto J, int k) __attribute__((always_inline)) {
-        constexpr int j = decltype(J)::value;
-#pragma unroll
-        for (int i = 0; i < 4; i++) w[j][i] = (uint32_t)uni((int)nw[i]);
-        nw = A.steps[k + 1 < n ? k + 1 : n];
-        const uint32_t w0 = w[j][0];
-        if (w0 & SB_STORED_A) inA[j] = slot_load<R>(blk, (w0 >> SB_SLOT_A_SHIFT) & 511, lane, A.I);
-        if (w0 & SB_STORED_B) inB[j] = slot_load<R>(blk, w[j][3] >> SB_SLOT_B_SHIFT, lane, A.I);
-        cdA[j] = __builtin_amdgcn_raw_buffer_load_b8(A.codes, p, w[j][1], 0);
-        cdB[j] = __builtin_amdgcn_raw_buffer_load_b8(A.codes, p, w[j][2], 0);
-    };
-    auto step = [&](auto J, int k) __attribute__((always_inline)) {
-        constexpr int j = decltype(J)::value;
-        const uint32_t w0 = w[j][0];
-        const int type = w0 & SB_TYPE;
-        const LDS R *PA = A.PT + 16 * (w[j][3] & SB_MAT_MASK), *PB = A.PT + 16 * ((w[j][3] >> SB_MAT_B_SHIFT) & SB_MAT_MASK);
-        int e = 0;
-        bool ga, gb;
-        V4<R> a, b;
-        ChildIn<R> out;
-        if (type == ST_PL) {
-            message<R, SK_PREV, AMB>(PA, 0, res[j ^ 1], a, e, ga);
-            message<R, SK_LEAF, AMB>(PB, cdB[j], inB[j], b, e, gb);
-            out = combine<R>(a, b, e, ga && gb);
-        } else if (type == ST_LL) {
-            message<R, SK_LEAF, AMB>(PA, cdA[j], inA[j], a, e, ga);
-            message<R, SK_LEAF, AMB>(PB, cdB[j], inB[j], b, e, gb);
-            out = combine<R>(a, b, e, ga && gb);
-        } else if (type == ST_PP2) {
-            message<R, SK_PREV, AMB>(PA, 0, res[j ^ 1], a, e, ga);
-            message<R, SK_PREV2, AMB>(PB, 0, res[j], b, e, gb);
-            out = combine<R>(a, b, e, ga && gb);
-        } else if (type == ST_SP) {
-            message<R, SK_STORED, AMB>(PA, 0, inA[j], a, e, ga);
-            message<R, SK_PREV, AMB>(PB, 0, res[j ^ 1], b, e, gb);
-            out = combine<R>(a, b, e, ga && gb);
-        } else if (type == ST_SL) {
-            message<R, SK_STORED, AMB>(PA, 0, inA[j], a, e, ga);
-            message<R, SK_LEAF, AMB>(PB, cdB[j], inB[j], b, e, gb);
-            out = combine<R>(a, b, e, ga && gb);
-        } else if (type == ST_SS) {
-            message<R, SK_STORED, AMB>(PA, 0, inA[j], a, e, ga);
-            message<R, SK_STORED, AMB>(PB, 0, inB[j], b, e, gb);
-            out = combine<R>(a, b, e, ga && gb);
-        } else {
-            // any sources, missing nodes: a missing child contributes nothing, but its gap state still
-            // decides whether the parent is all-gap at this pattern
-            const int ka = (w0 >> SB_KIND_A_SHIFT) & 3, kb = (w0 >> SB_KIND_B_SHIFT) & 3;
-            auto source = [&](int kind, const ChildIn<R> &ld, int code) __attribute__((always_inline)) {
-                const ChildIn<R> r1 = res[j ^ 1], r2 = res[j];
-                ChildIn<R> ci;
-                ci.x = kind == SK_PREV ? r1.x : (kind == SK_PREV2 ? r2.x : (kind == SK_LEAF ? code : ld.x));
-                ci.v.x = kind == SK_PREV ? r1.v.x : (kind == SK_PREV2 ? r2.v.x : ld.v.x);
-                ci.v.y = kind == SK_PREV ? r1.v.y : (kind == SK_PREV2 ? r2.v.y : ld.v.y);
-                ci.v.z = kind == SK_PREV ? r1.v.z : (kind == SK_PREV2 ? r2.v.z : ld.v.z);
-                ci.v.w = kind == SK_PREV ? r1.v.w : (kind == SK_PREV2 ? r2.v.w : ld.v.w);
-                return ci;
-            };
-            a.x = a.y = a.z = a.w = b.x = b.y = b.z = b.w = (R)1;
-            child_apply<R>(ka == SK_LEAF, w0 & SB_MISS_A, PA, source(ka, inA[j], cdA[j]), a.x, a.y, a.z, a.w, e, ga);
-            child_apply<R>(kb == SK_LEAF, w0 & SB_MISS_B, PB, source(kb, inB[j], cdB[j]), b.x, b.y, b.z, b.w, e, gb);
-            out = combine<R>(a, b, e, ga && gb);
-            if ((w0 & SB_MISS) && !(ga && gb)) out.x = 0;
-        }
-        fetch(J, k + 2);
-        res[j] = out;
-        const uint32_t d = w0 >> SB_SLOT_SHIFT;
-        const Buf to = make_buf(base, (w0 & SB_CHERRY) ? 0 : blk_bytes);
-        buf_st4<R>(to, out.v, lane * (uint32_t)sizeof(V4<R>), part_off<R>(d));
-        __builtin_amdgcn_raw_buffer_store_b32((uint32_t)out.x, to, lane * 4, exp_off<R>(d, A.I), 0);
-    };
-    fetch(std::integral_constant<int, 0>(), 0);
-    fetch(std::integral_constant<int, 1>(), 1);
-    for (int k = 0;; k += 2) {
-        step(std::integral_constant<int, 0>(), k);
-        if (k + 1 >= n) break;
-        step(std::integral_constant<int, 1>(), k + 1);
-        if (k + 2 >= n) break;
-    }
-    const bool odd = (n - 1) & 1;
-    ChildIn<R> r;
-    r.x = odd ? res[1].x : res[0].x;
-    r.v.x = odd ? res[1].v.x : res[0].v.x;
-    r.v.y = odd ? res[1].v.y : res[0].v.y;
-    r.v.z = odd ? res[1].v.z : res[0].v.z;
-    r.v.w = odd ? res[1].v.w : res[0].v.w;
-    return r;
-}
-
 // The pattern loop of a pass: this thread's part of the root's log sum.
 template <typename R, int BS, bool AMB>
 __device__ __forceinline__ double prune_patterns(MP M, CP<R> c, int mode)
@@ -665,12 +395,12 @@ __device__ __forceinline__ double prune_patterns(MP M, CP<R> c, int mode)
     const int P = uni(c->P);
     PassArgs<R> A;
     A.n = uni(c->n_steps);
-    A.I = uni(c->I);
+    A.slots = 2 * uni(c->I);
     A.steps = (const LDS u32x4 *)uni_ptr(c->steps);
     A.PT = uni_ptr(c->PTc);
     A.codes = make_buf(uni_ptr(c->codes), code_bytes(uni(c->S), uni(c->Ppad)));
     GBL char *parts = uni_ptr(c->parts);
-    const int blkB = block_bytes(A.I, sizeof(R));
+    const int I = uni(c->I), blkB = block_bytes(2 * I, sizeof(R));
     const int r = uni(c->root);
     const GBL int32_t *wts = uni_ptr(c->wts);
     const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
@@ -683,8 +413,8 @@ __device__ __forceinline__ double prune_patterns(MP M, CP<R> c, int mode)
         const uint32_t lane = tid & 63, p = (uint32_t)pb + lane;
         GBL char *blk = parts + (int64_t)(pb >> 6) * blkB;
         ChildIn<R> o;
-        if (A.n > 0) o = prune_pattern<R, AMB>(A, blk, blkB, p);
-        if (!in_regs) o = slot_load<R>(make_buf(blk, blkB), rb * A.I + r - uni(c->S), lane, A.I);
+        if (A.n > 0) o = prune_pattern<R, AMB, 2, true>(A, blk, blkB, p);
+        if (!in_regs) o = slot_load<R>(make_buf(blk, blkB), rb * I + r - uni(c->S), lane, 2 * I);
         // log sum_j pi_j L_j + exponent * ln 2; all-gap columns contribute 0
         if (o.x != GAPT && (int)p < P) {
             const double L = p0 * (double)o.v.x + p1 * (double)o.v.y + p2 * (double)o.v.z + p3 * (double)o.v.w;
@@ -753,7 +483,7 @@ __device__ __forceinline__ void draw_sites(MP M, CP<R> c, uint32_t c2, uint32_t 
 {
     constexpr int K = Shape<R, SH>::K, UN = K < 4 ? 4 : K;     // steps unrolled: whole blocks of four draws
     const int tid = threadIdx.x, S = uni(c->S), I = uni(c->I), n_int = uni(c->n_int), GG = uni(c->GG), Ppad = uni(c->Ppad);
-    const int blkB = block_bytes(I, sizeof(R));
+    const int blkB = block_bytes(2 * I, sizeof(R));
     const uint32_t k0 = (uint32_t)uni((int)M->key0), k1 = (uint32_t)uni((int)M->key1);
     const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
     const GBL char *parts = uni_ptr(c->parts);
@@ -770,7 +500,7 @@ __device__ __forceinline__ void draw_sites(MP M, CP<R> c, uint32_t c2, uint32_t 
         const int p = site[on ? g : GG - 1];
         // this pattern's entries of slot 0
         const GBL char *pp = parts + (int64_t)(p >> 6) * blkB + (p & 63) * sizeof(V4<R>);
-        const GBL char *pe = parts + (int64_t)(p >> 6) * blkB + exp_off<R>(0, I) + (p & 63) * 4;
+        const GBL char *pe = parts + (int64_t)(p >> 6) * blkB + exp_off<R>(0, 2 * I) + (p & 63) * 4;
         uint32_t r0[K], r1[K];
         u32x2 nr = srec[0];
         ChildIn<R> in[K];
@@ -1427,43 +1157,6 @@ __device__ __noinline__ void node_desc(LDS uint32_t *d, const int32_t *tab, int 
     d[3] = bits;
 }
 
-// Pruning order: post-order, the child with the larger subtree (in internal
-// nodes) first, child 0 on ties.  Subtree sizes go up the tree level by level
-// and subtree starts come down it; both live in the storage of the messages.
-template <typename R, int BS>
-__device__ __noinline__ void pruning_order(CP<R> c, const int32_t *tab, int N)
-{
-    const int tid = threadIdx.x, S = c->S, n_up = c->n_up, n_down = c->n_down, root = c->root;
-    const int32_t *ch0 = tab + tab_ch0(N), *ch1 = tab + tab_ch1(N);
-    const int32_t *down = tab + tab_down(N), *downoff = tab + tab_downoff(N);
-    LDS int32_t *size = (LDS int32_t *)c->E, *start = size + N;
-    for (int i = tid; i < N; i += BS) size[i] = 0;
-    __syncthreads();
-    for (int h = 0; h < n_up; h++) {
-        for (int q = (h == 0 ? 0 : c->upoff[h - 1]) + tid; q < c->upoff[h]; q += BS) {
-            const int s = c->urec[q] & 0x3ff;
-            size[s] = 1 + size[ch0[s]] + size[ch1[s]];
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        start[root] = 0;
-        c->porder[size[root] - 1] = (int16_t)root;
-    }
-    __syncthreads();
-    for (int d = 0; d < n_down; d++) {
-        for (int q = (d == 0 ? 0 : downoff[d - 1]) + tid; q < downoff[d]; q += BS) {
-            const int s = down[q], p = c->par[s];
-            if (s < S) continue;
-            const int a = ch0[p], b = ch1[p], first = size[a] >= size[b] ? a : b;
-            const int st = start[p] + (s == first ? 0 : size[first]);
-            start[s] = st;
-            c->porder[st + size[s] - 1] = (int16_t)s;
-        }
-        __syncthreads();
-    }
-}
-
 template <typename R, int BS, int SH>
 __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int work)
 {
@@ -1497,6 +1190,7 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
         c->cur[i] = 0;
         c->dirty[i] = 0;
     }
+    for (int i = tid; i < E.n_int; i += BS) c->porder[i] = (int16_t)((uint32_t)tab[tab_porder(N) + i] & PO_NODE);
     for (int i = tid; i < E.n_up; i += BS) c->upoff[i] = (int16_t)tab[tab_upoff(N) + i];
     for (int q = tid; q < E.n_int; q += BS) {
         const int v = tab[tab_up(N) + q];
@@ -1509,8 +1203,6 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
         const int s = c->inodes[q];
         if (is_cherry(tab, N, M->S, E.root, s)) c->flags[s] |= NF_CHERRY;
     }
-    pruning_order<R, BS>(c, tab, N);
-    __syncthreads();
     sample_steps<R, BS>(c);
     // null-rate tables (rate 1), fixed for the element
     class_tables<R, BS>(M, c, 0, 1.0, 0);

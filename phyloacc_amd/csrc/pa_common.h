@@ -52,10 +52,12 @@ struct ElemDev {
 
 // Node table layout (int32 words, per element; N = model N).
 //   ch0[N] ch1[N] par[N] flags[N] nodes[N] internal[N]
-//   up[N] up_off[N+1] down[N] down_off[N+1] tz[N] dist2 (double, 2N words)
+//   up[N] up_off[N+1] down[N] down_off[N+1] tz[N] dist2 (double, 2N words) porder[N/2+1]
 //   up: internal nodes of the element's tree by height (1, 2, ...);
 //       level h occupies up[up_off[h-1] .. up_off[h]).
 //   down: non-root nodes by depth (1, 2, ...), same convention.
+//   porder: the internal nodes in pruning order (post-order, the child with the
+//       larger subtree first, child 0 on ties), PO_* words.
 //   tz[s]: position of node s in the reverse post-order (root = 0), the Z-update draw slot.
 PA_TAB int tab_ch0(int N) { return 0; }
 PA_TAB int tab_ch1(int N) { return N; }
@@ -69,6 +71,14 @@ PA_TAB int tab_down(int N) { return 8 * N + 1; }
 PA_TAB int tab_downoff(int N) { return 9 * N + 1; }
 PA_TAB int tab_tz(int N) { return 10 * N + 2; }
 PA_TAB int tab_dist(int N) { return (11 * N + 3) & ~1; }       // even -> 8-byte aligned doubles
-PA_TAB int tab_words(int N) { return tab_dist(N) + 2 * N + 2; }  // even, so every table stays aligned
+PA_TAB int tab_porder(int N) { return tab_dist(N) + 2 * N; }
+PA_TAB int tab_words(int N) { return (tab_porder(N) + N / 2 + 2) & ~1; }  // even, so every table stays aligned
+
+// A word of porder: the node; how many earlier nodes' partials are waiting
+// for their parent when it is reached (its stack depth); and, when its parent
+// comes more than two nodes later, that its partial waits in the slot given.
+// A waiting partial's subtree is at least as large as the rest of its parent's
+// (two internal nodes or more), so the depth stays below log2 of the nodes.
+enum : uint32_t { PO_NODE = 0x3ffu, PO_DEPTH_SHIFT = 10, PO_DEPTH = 31u, PO_WAITS = 1u << 15, PO_SLOT_SHIFT = 16 };
 
 }  // namespace pa

@@ -26,6 +26,7 @@
 #include "pa_common.h"
 #include "pa_kernels.h"
 #include "pa_device.h"
+#include "pa_prune.h"
 #include "pa_eig.h"
 #include "pa_rng.h"
 
@@ -153,7 +154,7 @@ __device__ __forceinline__ size_t node_slot(int x, int f, int S, int N)
 // P(t) = V diag(exp(lam t)) Vi, clamped at 0, built in FP64, from the
 // model's eigensystem or a gBGC class's (lam, V, Vi in LDS or global memory).
 template <typename R, typename PE>
-__device__ void branch_matrix_from(PE lam, PE V, PE Vi, CP<R> c, int s, double d, double rate)
+__device__ void branch_matrix_from(PE lam, PE V, PE Vi, LDS R *PT, int s, double d, double rate)
 {
     double P[16];
     if (!(d <= 1e-10)) {          // a NaN length gives a NaN matrix, not the identity
@@ -174,17 +175,44 @@ __device__ void branch_matrix_from(PE lam, PE V, PE Vi, CP<R> c, int s, double d
 #pragma unroll
         for (int q = 0; q < 16; q++) P[q] = (q % 5 == 0) ? 1.0 : 0.0;
     }
-    LDS R *dst = c->PT + 16 * s;
+    LDS R *dst = PT + 16 * s;
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) dst[i * 4 + j] = (R)P[j * 4 + i];
 }
 
-template <typename R>
-__device__ void branch_matrix(MP M, CP<R> c, int s, double d, double rate)
+// The matrices of every branch of work position w, whose node table is tab.
+// A branch takes the rate of its class: Z = 0 (neutral) rate 1, Z = 2
+// (accelerated) r2, any other Z (1, conserved) r1; an own-tree element takes
+// its lengths from len_in.
+template <typename R, int BS>
+__device__ __forceinline__ void branch_matrices(MP M, AP A, LDS R *PT, const int32_t *tab, int n_nodes, int w, int row)
 {
-    branch_matrix_from<R>(M->lam, M->V, M->Vi, c, s, d, rate);
+    const int N = M->N;
+    const bool own = A->len_in != nullptr, gb = A->gb_eig != nullptr;
+    const double r1 = own || gb ? 1.0 : A->rates_in[2 * w], r2 = own || gb ? 1.0 : A->rates_in[2 * w + 1];
+    const double *dist = (const double *)(tab + tab_dist(N));
+    for (int q = threadIdx.x; q < n_nodes - 1; q += BS) {
+        const int s = tab[tab_nodes(N) + q];
+        if (own) {
+            const double len = A->len_in[(size_t)row * N + s];
+            if (A->el_eig) {
+                const double *E = A->el_eig + (size_t)w * GB_EIG_WORDS;
+                branch_matrix_from<R>(E, E + 4, E + 20, PT, s, len, 1.0);
+            } else {
+                branch_matrix_from<R>(M->lam, M->V, M->Vi, PT, s, len, 1.0);
+            }
+        } else if (gb) {
+            const int z = A->Zin[(size_t)w * N + s];
+            const int k = (z == 2 ? 2 : (z == 0 ? 0 : 1)) + (A->Bin[(size_t)w * N + s] != 0 ? 3 : 0);
+            const double *E = A->gb_eig + ((size_t)w * GB_CLASSES + k) * GB_EIG_WORDS;
+            branch_matrix_from<R>(E, E + 4, E + 20, PT, s, dist[s], 1.0);
+        } else {
+            const int z = A->Zin[(size_t)w * N + s];
+            branch_matrix_from<R>(M->lam, M->V, M->Vi, PT, s, dist[s], z == 2 ? r2 : (z == 0 ? 1.0 : r1));
+        }
+    }
 }
 
 // gBGC classes (BPP_C::init_cache_TM, src/PhyloAcc-ST-GBGC/SRC/bpp_c.cpp:
@@ -632,7 +660,7 @@ __device__ inline int leaf_base(int code)
 template <typename R, int BS>
 __device__ __noinline__ void gt_history(MP M, CP<R> c, AP A, int row)
 {
-    const int N = c->N, S = c->S, Ppad = c->Ppad, root = c->root, n_nodes = c->n_nodes;
+    const int S = c->S, Ppad = c->Ppad, root = c->root, n_nodes = c->n_nodes;
     const int len = A->hist_len[row], stride = A->hist_ns[row];
     GBL int8_t *out = (GBL int8_t *)A->hist + A->hist_off[row];
     const GBL int32_t *site = c->site;
@@ -759,9 +787,7 @@ __device__ __noinline__ void gt_candidates(MP M, CP<R> c, AP A, int w, int row)
 // ---------------------------------------------------------- element setup
 
 // Binds work position w: the element's node table into LDS, its slot, and
-// the transition matrix of every branch.  A branch takes the rate of its
-// class: Z = 0 (neutral) rate 1, Z = 2 (accelerated) r2, any other Z (1,
-// conserved) r1; an own-tree element takes its lengths from len_in.
+// the transition matrix of every branch.
 template <typename R, int BS>
 __device__ __noinline__ void bind_element(MP M, CP<R> c, AP A, int w)
 {
@@ -827,29 +853,7 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, AP A, int w)
             c->path = 1;
         }
     }
-    const bool own = A->len_in != nullptr, gb = A->gb_eig != nullptr;
-    const double r1 = own || gb ? 1.0 : A->rates_in[2 * w], r2 = own || gb ? 1.0 : A->rates_in[2 * w + 1];
-    const double *dist = (const double *)(tab + tab_dist(N));
-    for (int q = tid; q < c->n_nodes - 1; q += BS) {
-        const int s = c->nodes[q];
-        if (own) {
-            const double len = A->len_in[(size_t)(A->len_row ? A->len_row[w] : w) * N + s];
-            if (A->el_eig) {
-                const double *E = A->el_eig + (size_t)w * GB_EIG_WORDS;
-                branch_matrix_from<R>(E, E + 4, E + 20, c, s, len, 1.0);
-            } else {
-                branch_matrix<R>(M, c, s, len, 1.0);
-            }
-        } else if (gb) {
-            const int z = A->Zin[(size_t)w * N + s];
-            const int k = (z == 2 ? 2 : (z == 0 ? 0 : 1)) + (A->Bin[(size_t)w * N + s] != 0 ? 3 : 0);
-            const double *E = A->gb_eig + ((size_t)w * GB_CLASSES + k) * GB_EIG_WORDS;
-            branch_matrix_from<R>(E, E + 4, E + 20, c, s, dist[s], 1.0);
-        } else {
-            const int z = A->Zin[(size_t)w * N + s];
-            branch_matrix<R>(M, c, s, dist[s], z == 2 ? r2 : (z == 0 ? 1.0 : r1));
-        }
-    }
+    branch_matrices<R, BS>(M, A, c->PT, tab, c->n_nodes, w, row);
     __syncthreads();
 }
 
@@ -921,12 +925,201 @@ __global__ void __launch_bounds__(BS, 3) loglik_kernel(ModelDev Mk, LoglikArgs A
     }
 }
 
+// ------------------------------------------------------------- scores only
+//
+// A launch that wants nothing but log-likelihoods (no histories, candidate
+// scores or resident partials) keeps no partials: a pass over the element's
+// nodes in pruning order holds the one or two it needs next in registers,
+// and a node whose parent comes later waits in a stack of a few slots per
+// wave.  What is left is bound by the instructions of a step (about 100 a
+// node and 64 patterns), no longer by storing and reloading every node.
+
+constexpr int SCORE_DEPTH = 4;      // steps a leaf code is loaded ahead
+
+// Stack slots of a wave for trees of I internal nodes (the depth of a waiting
+// partial is below log2 of the nodes, see PO_WAITS).
+__host__ __device__ inline int score_slots(int I)
+{
+    int d = 1;
+    while ((1 << d) <= I) d++;
+    return d;
+}
+
+template <typename R>
+__host__ __device__ inline size_t score_smem(int N)
+{
+    // matrices, then one step per internal node and the empty one behind them
+    return (size_t)16 * N * sizeof(R) + (size_t)16 * (N / 2 + 2);
+}
+
+size_t score_smem_bytes(int N, int fp64)
+{
+    return (fp64 ? score_smem<double>(N) : score_smem<float>(N)) + sizeof(ModelDev) + sizeof(LoglikArgs) + 256;
+}
+
+// The steps of the pass over every internal node, one node a thread, and the
+// bytes a pass that stores every node but the cherries would move per
+// pattern (the counted bytes of a call).
+template <typename R, int BS>
+__device__ __forceinline__ void score_steps(MP M, LDS uint32_t *steps, LDS uint32_t *per, const int32_t *tab, int n_int, int root, int Ppad)
+{
+    const int N = M->N, S = M->S;
+    const int32_t *po = tab + tab_porder(N), *ch0 = tab + tab_ch0(N), *ch1 = tab + tab_ch1(N), *fl = tab + tab_flags(N);
+    constexpr uint32_t W = 4 * sizeof(R) + 4;
+    for (int t = threadIdx.x; t <= n_int; t += BS) {
+        LDS uint32_t *o = steps + 4 * t;
+        if (t == n_int) {
+            o[0] = o[1] = o[2] = o[3] = 0;
+            continue;
+        }
+        const uint32_t word = (uint32_t)po[t];
+        const int s = word & PO_NODE;
+        const int p1 = t > 0 ? (int)((uint32_t)po[t - 1] & PO_NODE) : -1, p2 = t > 1 ? (int)((uint32_t)po[t - 2] & PO_NODE) : -1;
+        const int x[2] = {ch0[s], ch1[s]};
+        StepDef d;
+        d.miss = fl[s] & NF_MISSING;
+        d.nostore = !(word & PO_WAITS);
+        d.slot_to = (word >> PO_SLOT_SHIFT) & 31;
+        uint32_t b = W;
+        for (int j = 0; j < 2; j++) {
+            const bool leaf = x[j] < S;
+            d.kind[j] = leaf ? SK_LEAF : (x[j] == p1 ? SK_PREV : (x[j] == p2 ? SK_PREV2 : SK_STORED));
+            d.miss_kid[j] = (fl[x[j]] & NF_MISSING) ? 1 : 0;
+            d.mat[j] = x[j];
+            d.row[j] = leaf ? x[j] * Ppad : 0;
+            d.slot[j] = d.kind[j] == SK_STORED ? (int)((word >> PO_DEPTH_SHIFT) & PO_DEPTH) : 0;
+            b += leaf ? 1 : (ch0[x[j]] < S && ch1[x[j]] < S ? 2 : W);
+        }
+        encode_step(o, d);
+        const bool cherry = s != root && x[0] < S && x[1] < S;
+        if (!cherry) __hip_atomic_fetch_add(per, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+}
+
+// The sums of a pass (log_f_Xz, src/PhyloAcc-ST/bpp_c2.cpp:392-425): log
+// sum_j pi_j L_j + exponent * ln 2 over the patterns, or over the sites of
+// the two prefixes by way of a table of the patterns' terms.  FP64; all-gap
+// columns contribute 0.
+template <typename R, int BS, bool AMB>
+__device__ __forceinline__ void score_patterns(MP M, AP A, const PassArgs<R> &a, const ElemDev &E, const double (&pi)[4], char *scratch,
+                                               int row, LDS double *red, double &s0, double &s1)
+{
+    const int tid = threadIdx.x, P = E.P;
+    const GBL int32_t *wts = (const GBL int32_t *)(A->wts + E.off_w);
+    GBL double *term = (GBL double *)scratch;
+    const size_t term_bytes = ((size_t)E.Ppad * 8 + 255) & ~(size_t)255;
+    const int blkB = block_bytes(a.slots, sizeof(R));
+    GBL char *stack = (GBL char *)scratch + term_bytes + (size_t)uni(tid >> 6) * blkB;
+    const bool pre = A->pre_len != nullptr;
+    double acc = 0, acc1 = 0;
+    for (int pb = uni(tid & ~63); pb < P; pb += BS) {
+        const int p = pb + (tid & 63);
+        const ChildIn<R> o = prune_pattern<R, AMB, SCORE_DEPTH, false>(a, stack, blkB, (uint32_t)p);
+        double t = 0;
+        if (o.x != GAPT) {
+            const double L = pi[0] * (double)o.v.x + pi[1] * (double)o.v.y + pi[2] * (double)o.v.z + pi[3] * (double)o.v.w;
+            t = log(L) + (double)o.x * 0.69314718055994530942;
+        }
+        if (pre) term[p] = t;
+        else if (p < P && o.x != GAPT) acc += (double)wts[p] * t;
+    }
+    if (pre) {
+        __syncthreads();
+        const GBL int32_t *site = (const GBL int32_t *)(A->site + E.off_site);
+        const int n0 = A->pre_len[2 * row], n1 = A->pre_len[2 * row + 1];
+        for (int g = tid; g < n0; g += BS) {
+            const double t = term[site[g]];
+            acc += t;
+            if (g < n1) acc1 += t;
+        }
+        s1 = block_sum(acc1, red);
+    }
+    s0 = block_sum(acc, red);
+}
+
+template <typename R, int BS>
+__global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak)
+{
+    extern __shared__ __align__(32) char smem_raw[];
+    __shared__ ModelDev Ms;
+    __shared__ LoglikArgs As;
+    __shared__ double red[4];
+    __shared__ int work_sh;
+    __shared__ uint32_t per_sh;
+    MP M = to_lds(Mk, (LDS ModelDev *)&Ms);
+    AP A = to_lds(Ak, (LDS LoglikArgs *)&As);
+    __syncthreads();
+    const int N = uni(M->N), S = uni(M->S), tid = threadIdx.x;
+    LDS R *PT = (LDS R *)(LDS char *)smem_raw;
+    LDS uint32_t *steps = (LDS uint32_t *)(PT + 16 * N);
+    for (;;) {
+        if (tid == 0) {
+            work_sh = atomicAdd(A->queue, 1);
+            per_sh = 0;
+        }
+        __syncthreads();
+        const int w = uni(work_sh);
+        if (w >= uni(A->n_work)) break;
+        // an id outside the arenas, or a filtered element (no patterns), scores NaN
+        const int id = uni(A->work[w]);
+        if (id < 0 || id >= uni(A->n_elems) || A->elems[id].P <= 0) {
+            if (tid == 0) A->ll_out[w] = __builtin_nan("");
+            __syncthreads();
+            continue;
+        }
+        const ElemDev E = A->elems[id];
+        const int row = A->len_row ? uni(A->len_row[w]) : w;
+        const int32_t *hdr = A->hdr_call ? A->hdr_call + (size_t)row * 4 : nullptr;
+        const int32_t *tab = A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab;
+        const int root = uni(hdr ? hdr[0] : E.root), n_nodes = uni(hdr ? hdr[1] : E.n_nodes), n_int = (n_nodes - 1) / 2;
+        score_steps<R, BS>(M, steps, (LDS uint32_t *)&per_sh, tab, n_int, root, E.Ppad);
+        branch_matrices<R, BS>(M, A, PT, tab, n_nodes, w, row);
+        const double *pw = A->el_pi ? A->el_pi + (size_t)w * 4 : nullptr;
+        double pi[4];
+        for (int j = 0; j < 4; j++) pi[j] = pw ? pw[j] : M->pi[j];
+        const int64_t bo = A->big_off ? A->big_off[w] : -1;
+        char *scratch = bo >= 0 ? A->big + bo : A->scratch + (int64_t)blockIdx.x * A->slot_bytes;
+        __syncthreads();
+        PassArgs<R> a;
+        a.steps = (const LDS u32x4 *)steps;
+        a.PT = PT;
+        a.codes = make_buf((GBL uint8_t *)(A->codes + E.off_codes), code_bytes(S, E.Ppad));
+        a.n = n_int;
+        a.slots = score_slots(N - S);
+        double s0 = 0, s1 = 0;
+        if (E.has_amb) score_patterns<R, BS, true>(M, A, a, E, pi, scratch, row, (LDS double *)red, s0, s1);
+        else score_patterns<R, BS, false>(M, A, a, E, pi, scratch, row, (LDS double *)red, s0, s1);
+        if (tid == 0) {
+            A->ll_out[w] = s0;
+            if (A->pre_len) A->ll_out2[w] = s1;
+            if (A->row_out0) {
+                A->row_out0[row] = s0;
+                if (A->pre_len) A->row_out1[row] = s1;
+            }
+            // and the root's partial, exponent and pattern weight
+            if (A->counters) atomicAdd(A->counters, (unsigned long long)E.P * (per_sh + 4 * sizeof(R) + 8));
+        }
+        __syncthreads();
+    }
+}
+
 __global__ void reset_queue(int *q) { *q = 0; }
+
+static bool scores_only(const LoglikArgs &A) { return !A.hist_draw && !A.cand_score && !A.alt; }
 
 template <typename R, int BS>
 static hipError_t launch_t(const ModelDev &M, const LoglikArgs &A, int grid, hipStream_t st)
 {
     // dynamic LDS above 64 KB needs the per-kernel limit raised (large trees only)
+    if (scores_only(A)) {
+        const size_t sm = score_smem<R>(M.N);
+        if (sm > 65536) {
+            const hipError_t err = hipFuncSetAttribute((const void *)score_kernel<R, BS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
+            if (err != hipSuccess) return err;
+        }
+        hipLaunchKernelGGL((score_kernel<R, BS>), dim3(grid), dim3(BS), sm, st, M, A);
+        return hipGetLastError();
+    }
     const size_t sm = smem_arrays<R, false>(M.N, nullptr, nullptr);
     if (sm > 65536) {
         const hipError_t err = hipFuncSetAttribute((const void *)loglik_kernel<R, BS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
@@ -943,27 +1136,26 @@ hipError_t launch_reset(int *q, hipStream_t st)
 }
 
 template <typename R, int BS>
-static int blocks_t(int N)
+static int blocks_t(int N, bool scores)
 {
-    const size_t sm = smem_arrays<R, false>(N, nullptr, nullptr);
-    if (sm > 65536 &&
-        hipFuncSetAttribute((const void *)loglik_kernel<R, BS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm) != hipSuccess)
-        return 0;
+    const void *k = scores ? (const void *)score_kernel<R, BS> : (const void *)loglik_kernel<R, BS>;
+    const size_t sm = scores ? score_smem<R>(N) : smem_arrays<R, false>(N, nullptr, nullptr);
+    if (sm > 65536 && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm) != hipSuccess) return 0;
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, loglik_kernel<R, BS>, BS, sm) != hipSuccess) return 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k, BS, sm) != hipSuccess) return 0;
     return nb;
 }
 
-int loglik_blocks_per_cu(int fp64, int BS, int N)
+int loglik_blocks_per_cu(int fp64, int BS, int N, bool scores)
 {
     if (fp64) {
-        if (BS == 64) return blocks_t<double, 64>(N);
-        if (BS == 128) return blocks_t<double, 128>(N);
-        if (BS == 256) return blocks_t<double, 256>(N);
+        if (BS == 64) return blocks_t<double, 64>(N, scores);
+        if (BS == 128) return blocks_t<double, 128>(N, scores);
+        if (BS == 256) return blocks_t<double, 256>(N, scores);
     } else {
-        if (BS == 64) return blocks_t<float, 64>(N);
-        if (BS == 128) return blocks_t<float, 128>(N);
-        if (BS == 256) return blocks_t<float, 256>(N);
+        if (BS == 64) return blocks_t<float, 64>(N, scores);
+        if (BS == 128) return blocks_t<float, 128>(N, scores);
+        if (BS == 256) return blocks_t<float, 256>(N, scores);
     }
     return 0;
 }

@@ -371,6 +371,28 @@ static void fill_table(const TreeModel &tm, const std::vector<int> &ch2, const s
     }
     double *D = (double *)(T + tab_dist(N));
     for (int i = 0; i < N; i++) D[i] = dist2[i];
+    // pruning order: subtree sizes (internal nodes) upwards, then each node's
+    // first place and depth downwards (a parent comes after its children here)
+    {
+        thread_local std::vector<int> size, start, deep;
+        size.assign(N, 0);
+        start.assign(N, 0);
+        deep.assign(N, 0);
+        thread_local std::vector<uint32_t> waits;
+        waits.assign(N, 0);
+        for (int v : internal) size[v] = 1 + size[ch2[2 * v]] + size[ch2[2 * v + 1]];
+        for (int k = (int)internal.size() - 1; k >= 0; k--) {
+            const int v = internal[k], a = ch2[2 * v], b = ch2[2 * v + 1];
+            const int f = size[a] >= size[b] ? a : b, g = f == a ? b : a;
+            T[tab_porder(N) + start[v] + size[v] - 1] = (int32_t)((uint32_t)v | ((uint32_t)deep[v] << PO_DEPTH_SHIFT) | waits[v]);
+            const bool wait = size[g] >= 2;
+            start[f] = start[v];
+            start[g] = start[v] + size[f];
+            deep[f] = deep[v];
+            deep[g] = deep[v] + (wait ? 1 : 0);
+            if (wait) waits[f] = PO_WAITS | ((uint32_t)deep[v] << PO_SLOT_SHIFT);
+        }
+    }
     n_up = hmax;
     n_down = dmax;
     *nodes_out = &nodes;
@@ -938,10 +960,11 @@ static int chain_grid_max(pa_engine *e, int fp64, int BS, int shape)
     const int N = e->tm.N, S = e->tm.S;
     return e->n_cu * fit_per_cu(e, chain::chain_smem_bytes(N, S, BS, fp64), BS, chain::chain_blocks_per_cu(fp64, BS, N, S, shape));
 }
-static int loglik_grid_max(pa_engine *e, int fp64, int BS)
+static int loglik_grid_max(pa_engine *e, int fp64, int BS, bool scores)
 {
     const int N = e->tm.N;
-    return e->n_cu * fit_per_cu(e, loglik_smem_bytes(N, fp64), BS, loglik_blocks_per_cu(fp64, BS, N));
+    return e->n_cu * fit_per_cu(e, scores ? score_smem_bytes(N, fp64) : loglik_smem_bytes(N, fp64), BS,
+                                loglik_blocks_per_cu(fp64, BS, N, scores));
 }
 
 // Scratch of one persistent launch of `grid` workgroups over elements of
@@ -1055,7 +1078,7 @@ static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp6
     const int BS = loglik_block(e, ids, n, fp64);
     const size_t smem = loglik_smem_bytes(N, fp64);
     if (smem > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
-    const int grid = std::min(n, loglik_grid_max(e, fp64, BS));
+    const int grid = std::min(n, loglik_grid_max(e, fp64, BS, !A.hist_draw && !A.cand_score && !A.alt));
     // resident partials come with their own arena and offsets
     const bool resident = A.alt != nullptr;
     std::vector<int> ppad(resident ? 0 : n);
@@ -1722,7 +1745,7 @@ pa_status gt_plan_build(pa_engine *e, const int32_t *ids, int32_t n, const doubl
     }
     p->BS = loglik_block(e, sorted.data(), n, fp64);
     if (loglik_smem_bytes(N, fp64) > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
-    p->grid = std::min(n, loglik_grid_max(e, fp64, p->BS));
+    p->grid = std::min(n, loglik_grid_max(e, fp64, p->BS, false));
     HIPCHK(e, hipMalloc(&p->work.p, (size_t)n * 4));
     HIPCHK(e, hipMalloc(&p->row.p, (size_t)n * 4));
     HIPCHK(e, hipMalloc(&p->bo.p, (size_t)n * 8));
@@ -2026,7 +2049,7 @@ extern "C" pa_status pa_loglik_noalloc(pa_engine *e, const int32_t *d_ids, int32
         return fail(e, PA_E_INPUT, "the longest element (" + std::to_string(e->max_ppad) + " padded patterns) needs " +
                                        std::to_string(slot) + " B of scratch, over the " + std::to_string(usable) +
                                        " B of the allocation-free entry point");
-    const int grid = (int)std::min<size_t>({(size_t)n, (size_t)loglik_grid_max(e, fp64, BS), usable / slot});
+    const int grid = (int)std::min<size_t>({(size_t)n, (size_t)loglik_grid_max(e, fp64, BS, true), usable / slot});
     LoglikArgs A;
     memset(&A, 0, sizeof A);
     A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab;
@@ -2864,7 +2887,7 @@ static pa_status lane_launch(pa_server *s, Lane &L, bool others_busy)
     pa_engine *e = s->e;
     const int N = e->tm.N, S = e->tm.S;
     const int gmax_c = chain_grid_max(e, s->fp64, s->BS, s->shape);
-    const int gmax_l = loglik_grid_max(e, s->fp64, s->BS);
+    const int gmax_l = loglik_grid_max(e, s->fp64, s->BS, true);
     const size_t room = s->pool.largest();
     const double now = pa_serve_clock();
     // chain requests: slots for min(k, grid) workgroups plus the long elements' own regions

@@ -130,8 +130,12 @@ size_t loglik_slot_bytes(int N, int S, int Pcap, int fp64);
 size_t loglik_resident_bytes(int N, int S, int Ppad, int fp64);
 // Dynamic LDS bytes of one workgroup (the launch's dynamic allocation).
 size_t loglik_dyn_smem_bytes(int N, int fp64);
-// Workgroups of the likelihood kernel resident on one CU (registers, LDS, launch bound).
-int loglik_blocks_per_cu(int fp64, int BS, int N);
+// LDS bytes of one workgroup of a launch that only scores (no histories,
+// candidate scores or resident partials).
+size_t score_smem_bytes(int N, int fp64);
+// Workgroups of the likelihood kernel (or of the one that only scores)
+// resident on one CU (registers, LDS, launch bound).
+int loglik_blocks_per_cu(int fp64, int BS, int N, bool scores);
 hipError_t launch_loglik(const ModelDev &M, const LoglikArgs &A, int fp64, int BS, int grid, hipStream_t st);
 
 // Size of the device scratch array of the allocation-free likelihood entry

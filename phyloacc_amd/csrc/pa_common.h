@@ -52,7 +52,7 @@ struct ElemDev {
 
 // Node table layout (int32 words, per element; N = model N).
 //   ch0[N] ch1[N] par[N] flags[N] nodes[N] internal[N]
-//   up[N] up_off[N+1] down[N] down_off[N+1] tz[N] dist2 (double, 2N words) porder[N/2+1]
+//   up[N] up_off[N+1] down[N] down_off[N+1] tz[N] porder[N/2+1] dist2 (double, 2N words)
 //   up: internal nodes of the element's tree by height (1, 2, ...);
 //       level h occupies up[up_off[h-1] .. up_off[h]).
 //   down: non-root nodes by depth (1, 2, ...), same convention.
@@ -70,9 +70,11 @@ PA_TAB int tab_upoff(int N) { return 7 * N; }
 PA_TAB int tab_down(int N) { return 8 * N + 1; }
 PA_TAB int tab_downoff(int N) { return 9 * N + 1; }
 PA_TAB int tab_tz(int N) { return 10 * N + 2; }
-PA_TAB int tab_dist(int N) { return (11 * N + 3) & ~1; }       // even -> 8-byte aligned doubles
-PA_TAB int tab_porder(int N) { return tab_dist(N) + 2 * N; }
-PA_TAB int tab_words(int N) { return (tab_porder(N) + N / 2 + 2) & ~1; }  // even, so every table stays aligned
+PA_TAB int tab_porder(int N) { return 11 * N + 2; }
+// behind everything the tree's shape decides, so that a new tree's table can
+// replace what lies before the lengths
+PA_TAB int tab_dist(int N) { return (tab_porder(N) + N / 2 + 2) & ~1; }   // even -> 8-byte aligned doubles
+PA_TAB int tab_words(int N) { return tab_dist(N) + 2 * N + 2; }           // even, so every table stays aligned
 
 // A word of porder: the node; how many earlier nodes' partials are waiting
 // for their parent when it is reached (its stack depth); and, when its parent

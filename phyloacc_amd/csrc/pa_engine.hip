@@ -957,6 +957,11 @@ size_t score_smem_bytes(int N, int fp64)
     return (fp64 ? score_smem<double>(N) : score_smem<float>(N)) + sizeof(ModelDev) + sizeof(LoglikArgs) + 256;
 }
 
+size_t score_slot_bytes(int N, int S, int BS, int Pcap, int fp64)
+{
+    return al((size_t)Pcap * 8, 256) + (size_t)(BS / 64) * block_bytes(score_slots(N - S), fp64 ? 8 : 4);
+}
+
 // The steps of the pass over every internal node, one node a thread, and the
 // bytes a pass that stores every node but the cherries would move per
 // pattern (the counted bytes of a call).
@@ -996,25 +1001,38 @@ __device__ __forceinline__ void score_steps(MP M, LDS uint32_t *steps, LDS uint3
     }
 }
 
+// Brings the codes of one block of 64 patterns (a cache line of every leaf's
+// row) near, a row a lane; the value only keeps the loads.  The rows are read
+// once a call, mostly from HBM, whose latency is longer than the steps a code
+// is loaded ahead.
+__device__ __forceinline__ uint32_t touch_codes(Buf codes, int S, int Ppad, int pb)
+{
+    uint32_t x = 0;
+    for (int r = threadIdx.x & 63; r < S; r += 64) x |= __builtin_amdgcn_raw_buffer_load_b32(codes, r * Ppad + pb, 0, 0);
+    return x;
+}
+
 // The sums of a pass (log_f_Xz, src/PhyloAcc-ST/bpp_c2.cpp:392-425): log
 // sum_j pi_j L_j + exponent * ln 2 over the patterns, or over the sites of
 // the two prefixes by way of a table of the patterns' terms.  FP64; all-gap
 // columns contribute 0.
 template <typename R, int BS, bool AMB>
 __device__ __forceinline__ void score_patterns(MP M, AP A, const PassArgs<R> &a, const ElemDev &E, const double (&pi)[4], char *scratch,
-                                               int row, LDS double *red, double &s0, double &s1)
+                                               int row, int first, int P, LDS double *red, double &s0, double &s1)
 {
-    const int tid = threadIdx.x, P = E.P;
+    const int tid = threadIdx.x;
     const GBL int32_t *wts = (const GBL int32_t *)(A->wts + E.off_w);
     GBL double *term = (GBL double *)scratch;
-    const size_t term_bytes = ((size_t)E.Ppad * 8 + 255) & ~(size_t)255;
+    const size_t term_bytes = A->pre_len ? al((size_t)E.Ppad * 8, 256) : 0;
     const int blkB = block_bytes(a.slots, sizeof(R));
     GBL char *stack = (GBL char *)scratch + term_bytes + (size_t)uni(tid >> 6) * blkB;
     const bool pre = A->pre_len != nullptr;
     double acc = 0, acc1 = 0;
-    for (int pb = uni(tid & ~63); pb < P; pb += BS) {
+    for (int pb = first + uni(tid & ~63); pb < P; pb += BS) {
         const int p = pb + (tid & 63);
+        const uint32_t ahead = pb + BS < P ? touch_codes(a.codes, uni(M->S), E.Ppad, pb + BS) : 0;
         const ChildIn<R> o = prune_pattern<R, AMB, SCORE_DEPTH, false>(a, stack, blkB, (uint32_t)p);
+        asm volatile("" ::"v"(ahead));
         double t = 0;
         if (o.x != GAPT) {
             const double L = pi[0] * (double)o.v.x + pi[1] * (double)o.v.y + pi[2] * (double)o.v.z + pi[3] * (double)o.v.w;
@@ -1058,8 +1076,11 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
             per_sh = 0;
         }
         __syncthreads();
-        const int w = uni(work_sh);
-        if (w >= uni(A->n_work)) break;
+        const int it = uni(work_sh);
+        if (it >= uni(A->items ? A->n_items : A->n_work)) break;
+        ScoreItem item{it, 0, 0, -1};
+        if (A->items) item = A->items[it];
+        const int w = uni(item.w), part = uni(item.part);
         // an id outside the arenas, or a filtered element (no patterns), scores NaN
         const int id = uni(A->work[w]);
         if (id < 0 || id >= uni(A->n_elems) || A->elems[id].P <= 0) {
@@ -1072,6 +1093,10 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
         const int32_t *hdr = A->hdr_call ? A->hdr_call + (size_t)row * 4 : nullptr;
         const int32_t *tab = A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab;
         const int root = uni(hdr ? hdr[0] : E.root), n_nodes = uni(hdr ? hdr[1] : E.n_nodes), n_int = (n_nodes - 1) / 2;
+        const int first = uni(item.p0), P = part < 0 ? E.P : uni(item.p1);
+        PassArgs<R> a;
+        a.codes = make_buf((GBL uint8_t *)(A->codes + E.off_codes), code_bytes(S, E.Ppad));
+        const uint32_t ahead = first + (tid & ~63) < P ? touch_codes(a.codes, S, E.Ppad, first + (tid & ~63)) : 0;
         score_steps<R, BS>(M, steps, (LDS uint32_t *)&per_sh, tab, n_int, root, E.Ppad);
         branch_matrices<R, BS>(M, A, PT, tab, n_nodes, w, row);
         const double *pw = A->el_pi ? A->el_pi + (size_t)w * 4 : nullptr;
@@ -1079,31 +1104,52 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
         for (int j = 0; j < 4; j++) pi[j] = pw ? pw[j] : M->pi[j];
         const int64_t bo = A->big_off ? A->big_off[w] : -1;
         char *scratch = bo >= 0 ? A->big + bo : A->scratch + (int64_t)blockIdx.x * A->slot_bytes;
+        asm volatile("" ::"v"(ahead));
         __syncthreads();
-        PassArgs<R> a;
         a.steps = (const LDS u32x4 *)steps;
         a.PT = PT;
-        a.codes = make_buf((GBL uint8_t *)(A->codes + E.off_codes), code_bytes(S, E.Ppad));
         a.n = n_int;
         a.slots = score_slots(N - S);
         double s0 = 0, s1 = 0;
-        if (E.has_amb) score_patterns<R, BS, true>(M, A, a, E, pi, scratch, row, (LDS double *)red, s0, s1);
-        else score_patterns<R, BS, false>(M, A, a, E, pi, scratch, row, (LDS double *)red, s0, s1);
+        if (E.has_amb) score_patterns<R, BS, true>(M, A, a, E, pi, scratch, row, first, P, (LDS double *)red, s0, s1);
+        else score_patterns<R, BS, false>(M, A, a, E, pi, scratch, row, first, P, (LDS double *)red, s0, s1);
         if (tid == 0) {
-            A->ll_out[w] = s0;
-            if (A->pre_len) A->ll_out2[w] = s1;
-            if (A->row_out0) {
-                A->row_out0[row] = s0;
-                if (A->pre_len) A->row_out1[row] = s1;
+            if (part >= 0) {
+                A->part_sum[part] = s0;
+            } else {
+                A->ll_out[w] = s0;
+                if (A->pre_len) A->ll_out2[w] = s1;
+                if (A->row_out0) {
+                    A->row_out0[row] = s0;
+                    if (A->pre_len) A->row_out1[row] = s1;
+                }
             }
             // and the root's partial, exponent and pattern weight
-            if (A->counters) atomicAdd(A->counters, (unsigned long long)E.P * (per_sh + 4 * sizeof(R) + 8));
+            if (A->counters) atomicAdd(A->counters, (unsigned long long)(P - first) * (per_sh + 4 * sizeof(R) + 8));
         }
         __syncthreads();
     }
 }
 
 __global__ void reset_queue(int *q) { *q = 0; }
+
+__global__ void score_sum_kernel(LoglikArgs A, const ScoreSplit *splits, int n)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const ScoreSplit s = splits[i];
+    double t = 0;
+    for (int k = 0; k < s.n; k++) t += A.part_sum[s.part0 + k];
+    A.ll_out[s.w] = t;
+    if (A.row_out0) A.row_out0[A.len_row ? A.len_row[s.w] : s.w] = t;
+}
+
+hipError_t launch_score_sum(const LoglikArgs &A, const ScoreSplit *splits, int n, hipStream_t st)
+{
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(score_sum_kernel, dim3((n + 63) / 64), dim3(64), 0, st, A, splits, n);
+    return hipGetLastError();
+}
 
 static bool scores_only(const LoglikArgs &A) { return !A.hist_draw && !A.cand_score && !A.alt; }
 

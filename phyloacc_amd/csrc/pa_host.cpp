@@ -949,9 +949,9 @@ static int pick_block(pa_engine *e, const int32_t *work, int32_t n)
 // Workgroups resident on one CU at once, from the runtime's occupancy query
 // of the kernel itself (registers under its launch bound, LDS, waves); the
 // LDS and wave count alone bound it when the query fails.
-static int fit_per_cu(pa_engine *e, size_t smem, int BS, int queried)
+static int fit_per_cu(pa_engine *e, size_t smem, int BS, int queried, int most = 8)
 {
-    const int per_cu = (int)std::min<size_t>(8, e->lds_per_cu / smem);
+    const int per_cu = (int)std::min<size_t>(most, e->lds_per_cu / smem);
     const int bound = std::max(1, std::min(per_cu, 2048 / BS));
     return queried > 0 ? std::min(queried, bound) : bound;
 }
@@ -960,11 +960,11 @@ static int chain_grid_max(pa_engine *e, int fp64, int BS, int shape)
     const int N = e->tm.N, S = e->tm.S;
     return e->n_cu * fit_per_cu(e, chain::chain_smem_bytes(N, S, BS, fp64), BS, chain::chain_blocks_per_cu(fp64, BS, N, S, shape));
 }
-static int loglik_grid_max(pa_engine *e, int fp64, int BS, bool scores)
+static int loglik_grid_max(pa_engine *e, int fp64, int BS, bool scores, int most = 8)
 {
     const int N = e->tm.N;
     return e->n_cu * fit_per_cu(e, scores ? score_smem_bytes(N, fp64) : loglik_smem_bytes(N, fp64), BS,
-                                loglik_blocks_per_cu(fp64, BS, N, scores));
+                                loglik_blocks_per_cu(fp64, BS, N, scores), most);
 }
 
 // Scratch of one persistent launch of `grid` workgroups over elements of
@@ -1072,19 +1072,68 @@ static int loglik_block(pa_engine *e, const int32_t *work, int32_t n, int fp64)
     return meanP <= 600 ? 128 : 256;
 }
 
+// The work items of a scoring launch: an element of more than `most` patterns
+// in parts of that many.  A part costs its workgroup the element's set-up
+// (steps and matrices, about as long as one pass of BS patterns), so a part
+// holds at least that many patterns, as many as give every CU four, and at
+// most eight passes: 20,000 elements of 43 species with one of 7,000 patterns
+// took 1.57 ms unsplit, which was that element's own time in one workgroup,
+// and 0.64 ms split; one element of 10,000 sites 0.79 and 0.04 ms.  Returns
+// the number of parts (0: no element is split, and there are no items).
+static int split_elements(pa_engine *e, const int32_t *ids, int n, int BS, std::vector<ScoreItem> &items,
+                          std::vector<ScoreSplit> &splits)
+{
+    int64_t total = 0;
+    int longest = 0;
+    for (int i = 0; i < n; i++) {
+        total += e->elems[ids[i]].P;
+        longest = std::max(longest, e->elems[ids[i]].P);
+    }
+    const int64_t even = (total / std::max(1, 4 * e->n_cu) + BS - 1) / BS * BS;
+    const int most = (int)std::min<int64_t>(8 * BS, std::max<int64_t>(BS, even));
+    if (longest <= most) return 0;
+    int parts = 0;
+    std::vector<ScoreItem> whole;
+    for (int i = 0; i < n; i++) {
+        const int P = e->elems[ids[i]].P;
+        if (P <= most) { whole.push_back({i, 0, P, -1}); continue; }
+        const ScoreSplit s{i, parts, (P + most - 1) / most};
+        splits.push_back(s);
+        for (int k = 0; k < s.n; k++) items.push_back({i, k * most, std::min(P, (k + 1) * most), parts++});
+    }
+    items.insert(items.end(), whole.begin(), whole.end());
+    return parts;
+}
+
 static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp64, LoglikArgs &A, DevBuf *bufs)
 {
     const int S = e->tm.S, N = e->tm.N;
     const int BS = loglik_block(e, ids, n, fp64);
     const size_t smem = loglik_smem_bytes(N, fp64);
     if (smem > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
-    const int grid = std::min(n, loglik_grid_max(e, fp64, BS, !A.hist_draw && !A.cand_score && !A.alt));
+    const bool scores = !A.hist_draw && !A.cand_score && !A.alt;
+    // a scoring workgroup's slot is small, so as many run as registers and LDS
+    // allow (16 of 64 threads a CU)
+    const int grid_max = loglik_grid_max(e, fp64, BS, scores, scores ? 16 : 8);
+    // long elements are scored in parts, so that one does not outlast the rest
+    std::vector<ScoreItem> items;
+    std::vector<ScoreSplit> splits;
+    const int parts = scores && !A.pre_len ? split_elements(e, ids, n, BS, items, splits) : 0;
+    const int grid = std::min(parts ? (int)items.size() : n, grid_max);
     // resident partials come with their own arena and offsets
     const bool resident = A.alt != nullptr;
-    std::vector<int> ppad(resident ? 0 : n);
-    for (int i = 0; i < (int)ppad.size(); i++) ppad[i] = e->elems[ids[i]].Ppad;
-    const ScratchPlan pl = resident ? ScratchPlan()
-                                    : plan_scratch(ppad, grid, 0, [&](int p) { return loglik_slot_bytes(N, S, p, fp64); });
+    ScratchPlan pl;
+    if (scores) {
+        int most = 0;
+        if (A.pre_len)
+            for (int i = 0; i < n; i++) most = std::max(most, e->elems[ids[i]].Ppad);
+        pl.slot = score_slot_bytes(N, S, BS, most, fp64);
+        pl.slots = pl.total = pl.slot * (size_t)grid;
+    } else if (!resident) {
+        std::vector<int> ppad(n);
+        for (int i = 0; i < n; i++) ppad[i] = e->elems[ids[i]].Ppad;
+        pl = plan_scratch(ppad, grid, 0, [&](int p) { return loglik_slot_bytes(N, S, p, fp64); });
+    }
     // the previous call synchronised its stream, so its scratch is free to reuse
     if (!resident && pl.total > e->ll_scratch_bytes) {
         (void)hipFree(e->d_ll_scratch);
@@ -1097,7 +1146,7 @@ static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp6
     int64_t *d_bo = (int64_t *)((char *)bufs[1].p + ((sizeof(int32_t) * n + 15) & ~(size_t)15));
     unsigned long long *d_cnt = (unsigned long long *)(d_bo + n);
     HIPCHK(e, hipMemcpyAsync(bufs[1].p, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, e->stream));
-    if (!resident) HIPCHK(e, hipMemcpyAsync(d_bo, pl.big_off.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice, e->stream));
+    if (pl.big) HIPCHK(e, hipMemcpyAsync(d_bo, pl.big_off.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice, e->stream));
     HIPCHK(e, hipMemsetAsync(d_cnt, 0, 8, e->stream));
     A.counters = d_cnt;
     A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab;
@@ -1111,9 +1160,22 @@ static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp6
         A.big = (char *)e->d_ll_scratch + pl.slots;
         A.big_off = pl.big ? d_bo : nullptr;
     }
+    DevBuf ib;
+    ScoreSplit *d_splits = nullptr;
+    if (parts) {
+        const size_t pb = (size_t)parts * 8, ab = items.size() * sizeof(ScoreItem), sb = splits.size() * sizeof(ScoreSplit);
+        HIPCHK(e, hipMalloc(&ib.p, pb + ab + sb));
+        A.part_sum = (double *)ib.p;
+        A.items = (const ScoreItem *)((char *)ib.p + pb);
+        A.n_items = (int)items.size();
+        d_splits = (ScoreSplit *)((char *)ib.p + pb + ab);
+        HIPCHK(e, hipMemcpyAsync((char *)ib.p + pb, items.data(), ab, hipMemcpyHostToDevice, e->stream));
+        HIPCHK(e, hipMemcpyAsync(d_splits, splits.data(), sb, hipMemcpyHostToDevice, e->stream));
+    }
     HIPCHK(e, launch_reset(A.queue, e->stream));
     HIPCHK(e, hipEventRecord(e->ll_t0, e->stream));
     HIPCHK(e, launch_loglik(e->M, A, fp64, BS, grid, e->stream));
+    HIPCHK(e, launch_score_sum(A, d_splits, (int)splits.size(), e->stream));
     HIPCHK(e, hipEventRecord(e->ll_t1, e->stream));
     HIPCHK(e, hipStreamSynchronize(e->stream));
     e->ll_last_plan_bytes = pl.total;

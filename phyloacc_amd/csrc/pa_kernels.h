@@ -18,6 +18,11 @@
 
 namespace pa {
 
+// Patterns [p0, p1) of work position w (p0 a multiple of 64); part: see LoglikArgs.
+struct ScoreItem { int w, p0, p1, part; };
+// A split element's parts: work position w, parts [part0, part0 + n).
+struct ScoreSplit { int w, part0, n; };
+
 // Arguments of the log-likelihood launch.  Work position w evaluates element
 // work[w] either at ancestral states Zin[w] and rates rates_in[w] over the
 // element's stored branch lengths, or, when len_in is set, at the per-call
@@ -65,6 +70,13 @@ struct LoglikArgs {
     // (gt_eig_kernel).
     const double *el_eig;     // [n_work][GB_EIG_WORDS]
     const double *el_pi;      // [n_work][4]
+    // Work items of a launch that only scores, or null (item i = work position
+    // i, all its patterns): n_items ranges of patterns.  An item with part >=
+    // 0 covers part of its element and leaves its sum in part_sum[part]; the
+    // sums of a split element are then added in order (launch_score_sum).
+    const struct ScoreItem *items;
+    int n_items;
+    double *part_sum;
     // Two site prefixes per caller row, or null: instead of the pattern sum,
     // the root sums run over the element's sites, g < pre_len[r][0] into
     // ll_out and g < pre_len[r][1] into ll_out2 (r = len_row[w], or w; the
@@ -130,6 +142,11 @@ size_t loglik_slot_bytes(int N, int S, int Pcap, int fp64);
 size_t loglik_resident_bytes(int N, int S, int Ppad, int fp64);
 // Dynamic LDS bytes of one workgroup (the launch's dynamic allocation).
 size_t loglik_dyn_smem_bytes(int N, int fp64);
+// Bytes of one workgroup's HBM slot in a launch that only scores: the stacks
+// of its waves, and with site prefixes the terms of Pcap (padded) patterns
+// (Pcap 0: none).  Never more than loglik_slot_bytes of the element's own
+// padded patterns, so a launch with such slots can score too.
+size_t score_slot_bytes(int N, int S, int BS, int Pcap, int fp64);
 // LDS bytes of one workgroup of a launch that only scores (no histories,
 // candidate scores or resident partials).
 size_t score_smem_bytes(int N, int fp64);
@@ -144,5 +161,7 @@ hipError_t launch_loglik(const ModelDev &M, const LoglikArgs &A, int fp64, int B
 constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)256 << 20;
 hipError_t noalloc_scratch(int device, char **ptr);
 hipError_t launch_reset(int *q, hipStream_t st);
+// The split elements' log-likelihoods from their parts' sums.
+hipError_t launch_score_sum(const LoglikArgs &A, const ScoreSplit *splits, int n, hipStream_t st);
 
 }  // namespace pa

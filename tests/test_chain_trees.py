@@ -78,3 +78,28 @@ def test_chains_match_the_oracle_on_any_tree(require_gpu, shape, S, ambiguous):
     f = eng.run_chains(ids, precision=E.PA_FP32, traces=True)
     # the state before the first draw: the same (Z, r), so the difference is the FP32 partials'
     np.testing.assert_allclose(f["loglik"][:, :, 0], r["loglik"][:, :, 0], rtol=1e-6)
+
+
+@pytest.mark.gpu
+def test_split_elements_score_like_whole_ones(require_gpu):
+    """A scoring launch takes long elements in parts, each at least a pass of
+    the workgroup's 256 patterns: elements just below, at and above one and
+    two parts, alone and in a batch, against the oracle (FP64 sums in another
+    order: the bound of the other likelihood tests)."""
+    w = _workload("random", 40, 3)
+    sizes = np.array([255, 256, 257, 511, 513, 1030])
+    rng = np.random.default_rng(5)
+    w.align = synth.simulate(w.tree, w.pi, w.Q, sizes, np.full((len(sizes), w.tree.N), 0.7), 0.05, rng)
+    starts = np.concatenate([[0], np.cumsum(sizes)[:-1]]).astype(np.int64)
+    eng = E.Engine.from_workload(w, E.default_options(compress_patterns=0))
+    ids, st = eng.add_elements(w.align, starts, sizes)
+    assert (st == E.PA_ELEM_OK).all()
+    Z = np.where(rng.random((len(ids), eng.N)) < 0.2, 2, 1).astype(np.int32)
+    Z[:, eng.N - 1] = 0
+    rates = np.tile([0.4, 2.0], (len(ids), 1))
+    m, oo = O.model_from_workload(w), O.default_options()
+    ref = np.array([O.Element(m, oo, w.align, starts[k], sizes[k]).loglik(Z[k], 0.4, 2.0) for k in range(len(ids))])
+    np.testing.assert_allclose(eng.loglik(ids, Z, rates, E.PA_FP64), ref, rtol=1e-9)
+    np.testing.assert_allclose(eng.loglik(ids, Z, rates, E.PA_FP32), ref, rtol=1e-6)
+    one = [eng.loglik(ids[k:k + 1], Z[k:k + 1], rates[k:k + 1], E.PA_FP64)[0] for k in range(len(ids))]
+    np.testing.assert_allclose(one, ref, rtol=1e-9)

@@ -191,7 +191,7 @@ __device__ __forceinline__ void branch_matrices(MP M, AP A, LDS R *PT, const int
 {
     const int N = M->N;
     const bool own = A->len_in != nullptr, gb = A->gb_eig != nullptr;
-    const double r1 = own || gb ? 1.0 : A->rates_in[2 * w], r2 = own || gb ? 1.0 : A->rates_in[2 * w + 1];
+    const double r1 = own || gb ? 1.0 : A->rates_in[2 * row], r2 = own || gb ? 1.0 : A->rates_in[2 * row + 1];
     const double *dist = (const double *)(tab + tab_dist(N));
     for (int q = threadIdx.x; q < n_nodes - 1; q += BS) {
         const int s = tab[tab_nodes(N) + q];
@@ -204,12 +204,12 @@ __device__ __forceinline__ void branch_matrices(MP M, AP A, LDS R *PT, const int
                 branch_matrix_from<R>(M->lam, M->V, M->Vi, PT, s, len, 1.0);
             }
         } else if (gb) {
-            const int z = A->Zin[(size_t)w * N + s];
-            const int k = (z == 2 ? 2 : (z == 0 ? 0 : 1)) + (A->Bin[(size_t)w * N + s] != 0 ? 3 : 0);
-            const double *E = A->gb_eig + ((size_t)w * GB_CLASSES + k) * GB_EIG_WORDS;
+            const int z = A->Zin[(size_t)row * N + s];
+            const int k = (z == 2 ? 2 : (z == 0 ? 0 : 1)) + (A->Bin[(size_t)row * N + s] != 0 ? 3 : 0);
+            const double *E = A->gb_eig + ((size_t)row * GB_CLASSES + k) * GB_EIG_WORDS;
             branch_matrix_from<R>(E, E + 4, E + 20, PT, s, dist[s], 1.0);
         } else {
-            const int z = A->Zin[(size_t)w * N + s];
+            const int z = A->Zin[(size_t)row * N + s];
             branch_matrix_from<R>(M->lam, M->V, M->Vi, PT, s, dist[s], z == 2 ? r2 : (z == 0 ? 1.0 : r1));
         }
     }

@@ -529,6 +529,7 @@ struct pa_engine {
     std::mutex sched_mu;
     std::vector<int32_t> sched_ids, sched_order;
     std::vector<HostElem> elems;
+    std::vector<int32_t> n_pat;     // patterns per element (-1: filtered): the per-call loops read these alone
     bool dev_dirty = true;
     std::vector<struct pa_batch *> batches;   // prepared batches, freed with the engine
     hipEvent_t ll_t0 = nullptr, ll_t1 = nullptr;   // around the last log-likelihood launch
@@ -545,10 +546,13 @@ struct pa_engine {
     uint64_t arena_gen = 0;                  // bumped whenever the device arenas move (prepared batches check it)
     // log-likelihood calls: scratch slots and per-call branch lengths, kept
     // between calls and grown when a call needs more (freed with the engine)
-    void *d_ll_scratch = nullptr, *d_ll_len = nullptr;
-    size_t ll_scratch_bytes = 0, ll_len_bytes = 0;
-    void *h_ll_len = nullptr;       // pinned staging of the per-call lengths
-    size_t h_ll_len_bytes = 0;
+    void *d_ll_scratch = nullptr;
+    size_t ll_scratch_bytes = 0;
+    // a call's inputs and results: a pinned block and a device block of the
+    // same layout (CallBlock)
+    char *h_io = nullptr, *d_io = nullptr;
+    size_t io_bytes = 0;
+    bool io_busy = false;           // a call has started copies and not waited for them
     void *h_tab_stage = nullptr;    // pinned staging of accepted gene trees' node tables
     size_t h_tab_stage_bytes = 0;
     size_t ll_last_plan_bytes = 0;           // scratch the last likelihood launch used
@@ -710,8 +714,8 @@ extern "C" void pa_engine_destroy(pa_engine *e)
         free_arenas(e);
         (void)hipFree(e->d_queue);
         (void)hipFree(e->d_ll_scratch);
-        (void)hipFree(e->d_ll_len);
-        (void)hipHostFree(e->h_ll_len);
+        (void)hipFree(e->d_io);
+        (void)hipHostFree(e->h_io);
         (void)hipHostFree(e->h_tab_stage);
         (void)hipFree(e->hist.d);
         if (e->ll_t0) (void)hipEventDestroy(e->ll_t0);
@@ -735,6 +739,8 @@ extern "C" pa_status pa_elements_add(pa_engine *e, const char *const *rows, cons
             for (int i = (int)t; i < n; i += (int)nt) encode_element(e->tm, e->opt, rows, starts[i], lengths[i], e->elems[base + i]);
         });
     for (auto &x : th) x.join();
+    e->n_pat.resize(base + n);
+    for (int i = 0; i < n; i++) e->n_pat[base + i] = e->elems[base + i].filtered ? -1 : e->elems[base + i].P;
     for (int i = 0; i < n; i++) {
         if (ids) ids[i] = (int32_t)(base + i);
         if (status) status[i] = e->elems[base + i].filtered ? PA_ELEM_FILTERED : PA_ELEM_OK;
@@ -770,6 +776,8 @@ extern "C" pa_status pa_elements_add_trees(pa_engine *e, const char *const *rows
                 encode_element(e->tm, e->opt, rows, starts[i], lengths[i], e->elems[base + i], children + (size_t)i * 2 * N);
         });
     for (auto &x : th) x.join();
+    e->n_pat.resize(base + n);
+    for (int i = 0; i < n; i++) e->n_pat[base + i] = e->elems[base + i].filtered ? -1 : e->elems[base + i].P;
     for (int i = 0; i < n; i++) {
         if (ids) ids[i] = (int32_t)(base + i);
         if (status) status[i] = e->elems[base + i].filtered ? PA_ELEM_FILTERED : PA_ELEM_OK;
@@ -1015,43 +1023,83 @@ static const size_t PA_RETAIN_MAX = (size_t)8 << 30;
 static void release_ll_buffers(pa_engine *e)
 {
     (void)hipFree(e->d_ll_scratch);
-    (void)hipFree(e->d_ll_len);
-    (void)hipHostFree(e->h_ll_len);
+    (void)hipFree(e->d_io);
+    (void)hipHostFree(e->h_io);
     (void)hipHostFree(e->h_tab_stage);
-    e->d_ll_scratch = e->d_ll_len = nullptr;
-    e->h_ll_len = e->h_tab_stage = nullptr;
-    e->ll_scratch_bytes = e->ll_len_bytes = e->h_ll_len_bytes = e->h_tab_stage_bytes = 0;
+    e->d_ll_scratch = e->h_tab_stage = nullptr;
+    e->d_io = e->h_io = nullptr;
+    e->ll_scratch_bytes = e->io_bytes = e->h_tab_stage_bytes = 0;
 }
 
-// Per-call lengths to the device: copied into a retained pinned buffer by up
-// to 16 threads, then one asynchronous copy on the engine stream (the
-// launch that reads them follows on that stream and the call waits for it).
-static pa_status upload_lengths(pa_engine *e, const double *lengths, size_t bytes)
-{
-    // no copy of an earlier call may still read the staging buffer
-    HIPCHK(e, hipStreamSynchronize(e->stream));
-    if (bytes > e->h_ll_len_bytes) {
-        (void)hipHostFree(e->h_ll_len);
-        e->h_ll_len = nullptr;
-        e->h_ll_len_bytes = 0;
-        HIPCHK(e, hipHostMalloc(&e->h_ll_len, bytes));
-        e->h_ll_len_bytes = bytes;
+// A likelihood call's inputs and results in the engine's retained blocks:
+// the inputs are laid out one after another in pinned memory and go up in one
+// copy, the results come down in one.  Calls that grow the blocks, like all
+// calls on one engine, do not overlap.
+namespace {
+struct CallBlock {
+    pa_engine *e;
+    size_t off = 0;
+    explicit CallBlock(pa_engine *eng) : e(eng) {}
+    static size_t up(size_t b) { return (b + 255) & ~(size_t)255; }
+    pa_status reserve(size_t bytes)
+    {
+        // a call that failed half way may have left copies in flight
+        if (e->io_busy) HIPCHK(e, hipStreamSynchronize(e->stream));
+        e->io_busy = true;
+        if (bytes <= e->io_bytes) return PA_OK;
+        (void)hipFree(e->d_io);
+        (void)hipHostFree(e->h_io);
+        e->d_io = e->h_io = nullptr;
+        e->io_bytes = 0;
+        bytes = up(bytes + bytes / 4);
+        HIPCHK(e, hipMalloc(&e->d_io, bytes));
+        HIPCHK(e, hipHostMalloc(&e->h_io, bytes));
+        e->io_bytes = bytes;
+        return PA_OK;
     }
-    const size_t chunk = (size_t)4 << 20;
-    const int parts = (int)std::min<size_t>(16, (bytes + chunk - 1) / chunk);
-    if (parts <= 1) {
-        memcpy(e->h_ll_len, lengths, bytes);
-    } else {
+    // the next `bytes` of the layout (within what was reserved): host and device addresses
+    char *take(size_t bytes, char **dev)
+    {
+        char *h = e->h_io + off;
+        *dev = e->d_io + off;
+        off += up(bytes);
+        return h;
+    }
+    template <typename T>
+    T *put(const T *src, size_t n)
+    {
+        char *d;
+        char *h = take(n * sizeof(T), &d);
+        copy(h, src, n * sizeof(T));
+        return (T *)d;
+    }
+    // large inputs by up to 16 threads
+    static void copy(char *dst, const void *src, size_t bytes)
+    {
+        const size_t chunk = (size_t)2 << 20;
+        const int parts = (int)std::min<size_t>(16, bytes / chunk);
+        if (parts <= 1) {
+            memcpy(dst, src, bytes);
+            return;
+        }
         const size_t per = (bytes / parts + 63) & ~(size_t)63;
         std::vector<std::thread> th;
-        for (int t = 0; t < parts; t++) {
-            const size_t a = std::min(bytes, per * t), b = std::min(bytes, per * (t + 1));
-            if (b > a) th.emplace_back([=]() { memcpy((char *)e->h_ll_len + a, (const char *)lengths + a, b - a); });
+        for (int t = 1; t < parts; t++) {
+            const size_t a = std::min(bytes, per * t), b = t == parts - 1 ? bytes : std::min(bytes, per * (t + 1));
+            if (b > a) th.emplace_back([=]() { memcpy(dst + a, (const char *)src + a, b - a); });
         }
+        memcpy(dst, src, std::min(bytes, per));
         for (auto &x : th) x.join();
     }
-    HIPCHK(e, hipMemcpyAsync(e->d_ll_len, e->h_ll_len, bytes, hipMemcpyHostToDevice, e->stream));
-    return PA_OK;
+};
+}  // namespace
+
+// Room of the layout that run_kernel and its results take for n rows.
+static size_t call_room(pa_engine *e, const int32_t *ids, int n)
+{
+    size_t parts = 0;
+    for (int i = 0; i < n; i++) parts += (size_t)(e->n_pat[ids[i]] / 64 + 1);
+    return (size_t)n * (4 + 8 + sizeof(ScoreItem) + sizeof(ScoreSplit) + 4 * 8) + parts * (sizeof(ScoreItem) + 8) + 4096;
 }
 
 // Fixed-(Z, r) log-likelihood launch: one persistent launch over ids (in
@@ -1065,7 +1113,7 @@ static int loglik_block(pa_engine *e, const int32_t *work, int32_t n, int fp64)
 {
     if (e->n_cu > 0 && n < 4 * e->n_cu) return 256;
     double meanP = 0;
-    for (int i = 0; i < n; i++) meanP += e->elems[work[i]].P;
+    for (int i = 0; i < n; i++) meanP += e->n_pat[work[i]];
     meanP /= std::max(1, n);
     if (meanP <= 96) return 64;
     if (fp64) return meanP <= 200 ? 128 : 256;
@@ -1086,8 +1134,8 @@ static int split_elements(pa_engine *e, const int32_t *ids, int n, int BS, std::
     int64_t total = 0;
     int longest = 0;
     for (int i = 0; i < n; i++) {
-        total += e->elems[ids[i]].P;
-        longest = std::max(longest, e->elems[ids[i]].P);
+        total += e->n_pat[ids[i]];
+        longest = std::max(longest, (int)e->n_pat[ids[i]]);
     }
     const int64_t even = (total / std::max(1, 4 * e->n_cu) + BS - 1) / BS * BS;
     const int most = (int)std::min<int64_t>(8 * BS, std::max<int64_t>(BS, even));
@@ -1095,7 +1143,7 @@ static int split_elements(pa_engine *e, const int32_t *ids, int n, int BS, std::
     int parts = 0;
     std::vector<ScoreItem> whole;
     for (int i = 0; i < n; i++) {
-        const int P = e->elems[ids[i]].P;
+        const int P = e->n_pat[ids[i]];
         if (P <= most) { whole.push_back({i, 0, P, -1}); continue; }
         const ScoreSplit s{i, parts, (P + most - 1) / most};
         splits.push_back(s);
@@ -1105,7 +1153,9 @@ static int split_elements(pa_engine *e, const int32_t *ids, int n, int BS, std::
     return parts;
 }
 
-static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp64, LoglikArgs &A, DevBuf *bufs)
+// The call's other inputs are in B already; the results by caller row (A.len_row) come back in res0 and, with site
+// prefixes, res1.
+static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp64, LoglikArgs &A, CallBlock &B, double *res0, double *res1)
 {
     const int S = e->tm.S, N = e->tm.N;
     const int BS = loglik_block(e, ids, n, fp64);
@@ -1126,7 +1176,7 @@ static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp6
     if (scores) {
         int most = 0;
         if (A.pre_len)
-            for (int i = 0; i < n; i++) most = std::max(most, e->elems[ids[i]].Ppad);
+            for (int i = 0; i < n; i++) most = std::max(most, (e->n_pat[ids[i]] + 63) & ~63);
         pl.slot = score_slot_bytes(N, S, BS, most, fp64);
         pl.slots = pl.total = pl.slot * (size_t)grid;
     } else if (!resident) {
@@ -1142,16 +1192,35 @@ static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp6
         HIPCHK(e, hipMalloc(&e->d_ll_scratch, pl.total));
         e->ll_scratch_bytes = pl.total;
     }
-    HIPCHK(e, hipMalloc(&bufs[1].p, sizeof(int32_t) * n + sizeof(int64_t) * n + 32));
-    int64_t *d_bo = (int64_t *)((char *)bufs[1].p + ((sizeof(int32_t) * n + 15) & ~(size_t)15));
-    unsigned long long *d_cnt = (unsigned long long *)(d_bo + n);
-    HIPCHK(e, hipMemcpyAsync(bufs[1].p, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, e->stream));
-    if (pl.big) HIPCHK(e, hipMemcpyAsync(d_bo, pl.big_off.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice, e->stream));
-    HIPCHK(e, hipMemsetAsync(d_cnt, 0, 8, e->stream));
-    A.counters = d_cnt;
+    A.work = B.put(ids, n);
+    const int64_t *d_bo = pl.big ? B.put(pl.big_off.data(), n) : nullptr;
+    const ScoreSplit *d_splits = nullptr;
+    if (parts) {
+        A.items = B.put(items.data(), items.size());
+        A.n_items = (int)items.size();
+        d_splits = B.put(splits.data(), splits.size());
+    }
+    // the byte counter, cleared with the inputs, and the results behind it
+    char *d_cnt, *d_out, *d_part;
+    char *h_cnt = B.take(8, &d_cnt);
+    memset(h_cnt, 0, 8);
+    const size_t in_bytes = B.off;
+    char *h_out = B.take((size_t)n * 16, &d_out);
+    B.take((size_t)n * 16, &d_part);          // by work position, not read back
+    A.ll_out = (double *)d_part;
+    A.ll_out2 = (double *)d_part + n;
+    if (!A.row_out0) {
+        A.row_out0 = (double *)d_out;
+        A.row_out1 = (double *)d_out + n;
+    }
+    const bool rows_here = A.row_out0 == (double *)d_out;
+    B.take((size_t)parts * 8, &d_part);
+    A.part_sum = (double *)d_part;
+    if (B.off > e->io_bytes) return fail(e, PA_E_STATE, "call block too small");
+    HIPCHK(e, hipMemcpyAsync(e->d_io, e->h_io, in_bytes, hipMemcpyHostToDevice, e->stream));
+    A.counters = (unsigned long long *)d_cnt;
     A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab;
     A.n_elems = (int)e->elems.size();
-    A.work = (const int32_t *)bufs[1].p;
     A.n_work = n;
     A.queue = e->d_queue;
     if (!resident) {
@@ -1160,29 +1229,27 @@ static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp6
         A.big = (char *)e->d_ll_scratch + pl.slots;
         A.big_off = pl.big ? d_bo : nullptr;
     }
-    DevBuf ib;
-    ScoreSplit *d_splits = nullptr;
-    if (parts) {
-        const size_t pb = (size_t)parts * 8, ab = items.size() * sizeof(ScoreItem), sb = splits.size() * sizeof(ScoreSplit);
-        HIPCHK(e, hipMalloc(&ib.p, pb + ab + sb));
-        A.part_sum = (double *)ib.p;
-        A.items = (const ScoreItem *)((char *)ib.p + pb);
-        A.n_items = (int)items.size();
-        d_splits = (ScoreSplit *)((char *)ib.p + pb + ab);
-        HIPCHK(e, hipMemcpyAsync((char *)ib.p + pb, items.data(), ab, hipMemcpyHostToDevice, e->stream));
-        HIPCHK(e, hipMemcpyAsync(d_splits, splits.data(), sb, hipMemcpyHostToDevice, e->stream));
-    }
     HIPCHK(e, launch_reset(A.queue, e->stream));
     HIPCHK(e, hipEventRecord(e->ll_t0, e->stream));
     HIPCHK(e, launch_loglik(e->M, A, fp64, BS, grid, e->stream));
     HIPCHK(e, launch_score_sum(A, d_splits, (int)splits.size(), e->stream));
     HIPCHK(e, hipEventRecord(e->ll_t1, e->stream));
+    const size_t back = (size_t)(h_out - h_cnt) + (rows_here ? (size_t)n * (A.pre_len ? 16 : 8) : 0);
+    HIPCHK(e, hipMemcpyAsync(h_cnt, d_cnt, back, hipMemcpyDeviceToHost, e->stream));
     HIPCHK(e, hipStreamSynchronize(e->stream));
     e->ll_last_plan_bytes = pl.total;
     float ms = 0;
     unsigned long long cnt = 0;
     HIPCHK(e, hipEventElapsedTime(&ms, e->ll_t0, e->ll_t1));
-    HIPCHK(e, hipMemcpy(&cnt, d_cnt, sizeof cnt, hipMemcpyDeviceToHost));
+    memcpy(&cnt, h_cnt, sizeof cnt);
+    e->io_busy = false;
+    if (!rows_here) {
+        HIPCHK(e, hipMemcpy(res0, A.row_out0, (size_t)n * 8, hipMemcpyDeviceToHost));
+        if (A.pre_len) HIPCHK(e, hipMemcpy(res1, A.row_out1, (size_t)n * 8, hipMemcpyDeviceToHost));
+    } else {
+        memcpy(res0, h_out, (size_t)n * 8);
+        if (A.pre_len) memcpy(res1, h_out + (size_t)n * 8, (size_t)n * 8);
+    }
     e->ll_stats.elapsed_ms = ms;
     e->ll_stats.algorithmic_bytes = (double)cnt;
     e->ll_stats.grid = grid;
@@ -1278,7 +1345,7 @@ static pa_status check_ids(pa_engine *e, const int32_t *ids, int32_t n)
 {
     for (int i = 0; i < n; i++) {
         if (ids[i] < 0 || ids[i] >= (int)e->elems.size()) return fail(e, PA_E_INPUT, "element id out of range");
-        if (e->elems[ids[i]].filtered) return fail(e, PA_E_INPUT, "element " + std::to_string(ids[i]) + " is filtered");
+        if (e->n_pat[ids[i]] < 0) return fail(e, PA_E_INPUT, "element " + std::to_string(ids[i]) + " is filtered");
     }
     return PA_OK;
 }
@@ -1321,33 +1388,19 @@ extern "C" pa_status pa_loglik(pa_engine *e, const int32_t *ids, int32_t n, cons
     if ((st = upload(e)) != PA_OK) return st;
     HIPCHK(e, hipSetDevice(e->device));
     const int N = e->tm.N;
-    std::vector<int32_t> order = schedule(e, ids, n, PA_RUN_BATCHED);
-    std::vector<int32_t> Zw((size_t)n * N);
-    std::vector<double> rw((size_t)n * 2);
-    for (int i = 0; i < n; i++) {
-        memcpy(&Zw[(size_t)i * N], Z + (size_t)order[i] * N, sizeof(int32_t) * N);
-        rw[2 * i] = rates[2 * order[i]];
-        rw[2 * i + 1] = rates[2 * order[i] + 1];
-    }
-    DevBuf bufs[6];
-    HIPCHK(e, hipMalloc(&bufs[3].p, Zw.size() * 4));
-    HIPCHK(e, hipMalloc(&bufs[4].p, rw.size() * 8));
-    HIPCHK(e, hipMalloc(&bufs[5].p, (size_t)n * 8));
-    HIPCHK(e, hipMemcpy(bufs[3].p, Zw.data(), Zw.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(e, hipMemcpy(bufs[4].p, rw.data(), rw.size() * 8, hipMemcpyHostToDevice));
+    const std::vector<int32_t> order = schedule(e, ids, n, PA_RUN_BATCHED);
+    CallBlock B(e);
+    if ((st = B.reserve(call_room(e, ids, n) + (size_t)n * (4 * N + 16 + 4) + 1024)) != PA_OK) return st;
     LoglikArgs A;
     memset(&A, 0, sizeof A);
-    A.Zin = (const int32_t *)bufs[3].p;
-    A.rates_in = (const double *)bufs[4].p;
-    A.ll_out = (double *)bufs[5].p;
+    A.len_row = B.put(order.data(), n);
+    A.Zin = B.put(Z, (size_t)n * N);
+    A.rates_in = B.put(rates, (size_t)n * 2);
     std::vector<int32_t> sorted(n);
     for (int i = 0; i < n; i++) sorted[i] = ids[order[i]];
-    st = run_kernel(e, sorted.data(), n, precision == PA_FP64, A, bufs);
+    st = run_kernel(e, sorted.data(), n, precision == PA_FP64, A, B, out, nullptr);
     if (st != PA_OK) return st;
-    std::vector<double> ll(n);
-    HIPCHK(e, hipMemcpy(ll.data(), bufs[5].p, (size_t)n * 8, hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; i++) out[order[i]] = ll[i];
-    if (e->ll_scratch_bytes + e->ll_len_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
+    if (e->ll_scratch_bytes + e->io_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
     return PA_OK;
 }
 
@@ -1369,38 +1422,26 @@ extern "C" pa_status pa_loglik_gbgc(pa_engine *e, const int32_t *ids, int32_t n,
     if ((st = upload(e)) != PA_OK) return st;
     HIPCHK(e, hipSetDevice(e->device));
     const int N = e->tm.N;
-    std::vector<int32_t> order = schedule(e, ids, n, PA_RUN_BATCHED);
-    std::vector<int32_t> Zw((size_t)n * N), Bw((size_t)n * N);
-    std::vector<double> sw((size_t)n * 3);
-    for (int i = 0; i < n; i++) {
-        memcpy(&Zw[(size_t)i * N], Z + (size_t)order[i] * N, sizeof(int32_t) * N);
-        memcpy(&Bw[(size_t)i * N], B + (size_t)order[i] * N, sizeof(int32_t) * N);
-        memcpy(&sw[(size_t)i * 3], sel + (size_t)order[i] * 3, sizeof(double) * 3);
-    }
-    DevBuf bufs[8];
-    HIPCHK(e, hipMalloc(&bufs[3].p, Zw.size() * 4));
-    HIPCHK(e, hipMalloc(&bufs[4].p, sw.size() * 8));
-    HIPCHK(e, hipMalloc(&bufs[5].p, (size_t)n * 8));
-    HIPCHK(e, hipMalloc(&bufs[6].p, Bw.size() * 4));
-    HIPCHK(e, hipMalloc(&bufs[7].p, (size_t)n * GB_CLASSES * GB_EIG_WORDS * 8));
-    HIPCHK(e, hipMemcpy(bufs[3].p, Zw.data(), Zw.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(e, hipMemcpy(bufs[4].p, sw.data(), sw.size() * 8, hipMemcpyHostToDevice));
-    HIPCHK(e, hipMemcpy(bufs[6].p, Bw.data(), Bw.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(e, launch_gbgc_eig(e->Q0, (const double *)bufs[4].p, n, (double *)bufs[7].p, e->stream));
+    const std::vector<int32_t> order = schedule(e, ids, n, PA_RUN_BATCHED);
+    const size_t eig_bytes = (size_t)n * GB_CLASSES * GB_EIG_WORDS * 8;
+    CallBlock K(e);
+    if ((st = K.reserve(call_room(e, ids, n) + (size_t)n * (8 * N + 24 + 4) + eig_bytes + 2048)) != PA_OK) return st;
     LoglikArgs A;
     memset(&A, 0, sizeof A);
-    A.Zin = (const int32_t *)bufs[3].p;
-    A.Bin = (const int32_t *)bufs[6].p;
-    A.gb_eig = (const double *)bufs[7].p;
-    A.ll_out = (double *)bufs[5].p;
+    // the selections first, so that the eigensystems are built while the rest is laid out
+    const double *d_sel = K.put(sel, (size_t)n * 3);
+    HIPCHK(e, hipMemcpyAsync(e->d_io, e->h_io, K.off, hipMemcpyHostToDevice, e->stream));
+    char *d_eig = e->d_io + e->io_bytes - CallBlock::up(eig_bytes);     // device only, behind the layout
+    HIPCHK(e, launch_gbgc_eig(e->Q0, d_sel, n, (double *)d_eig, e->stream));
+    A.gb_eig = (const double *)d_eig;
+    A.len_row = K.put(order.data(), n);
+    A.Zin = K.put(Z, (size_t)n * N);
+    A.Bin = K.put(B, (size_t)n * N);
     std::vector<int32_t> sorted(n);
     for (int i = 0; i < n; i++) sorted[i] = ids[order[i]];
-    st = run_kernel(e, sorted.data(), n, precision == PA_FP64, A, bufs);
+    st = run_kernel(e, sorted.data(), n, precision == PA_FP64, A, K, out, nullptr);
     if (st != PA_OK) return st;
-    std::vector<double> ll(n);
-    HIPCHK(e, hipMemcpy(ll.data(), bufs[5].p, (size_t)n * 8, hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; i++) out[order[i]] = ll[i];
-    if (e->ll_scratch_bytes + e->ll_len_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
+    if (e->ll_scratch_bytes + e->io_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
     return PA_OK;
 }
 
@@ -1445,52 +1486,37 @@ static pa_status loglik_lengths_impl(pa_engine *e, const int32_t *ids, int32_t n
     if (st != PA_OK) return st;
     if ((st = upload(e)) != PA_OK) return st;
     const int N = e->tm.N;
-    std::vector<int32_t> order = schedule(e, ids, n, PA_RUN_BATCHED);
+    const std::vector<int32_t> order = schedule(e, ids, n, PA_RUN_BATCHED);
     // the lengths go up in the caller's row order; work position w reads row order[w]
-    const size_t lbytes = (size_t)n * N * 8;
-    DevBuf bufs[10];
-    HIPCHK(e, hipMalloc(&bufs[5].p, (size_t)n * 8));
-    HIPCHK(e, hipMalloc(&bufs[6].p, (size_t)n * 4));
-    if (!dev_len && lbytes > e->ll_len_bytes) {
-        (void)hipFree(e->d_ll_len);
-        e->d_ll_len = nullptr;
-        e->ll_len_bytes = 0;
-        HIPCHK(e, hipMalloc(&e->d_ll_len, lbytes));
-        e->ll_len_bytes = lbytes;
-    }
-    if (!dev_len && (st = upload_lengths(e, lengths, lbytes)) != PA_OK) return st;
-    HIPCHK(e, hipMemcpy(bufs[6].p, order.data(), (size_t)n * 4, hipMemcpyHostToDevice));
+    const size_t lbytes = dev_len ? 0 : (size_t)n * N * 8, eig_bytes = piA ? (size_t)n * (GB_EIG_WORDS + 4) * 8 : 0;
+    CallBlock B(e);
+    if ((st = B.reserve(call_room(e, ids, n) + lbytes + eig_bytes + (size_t)n * (4 + 8 + 8) + 4096)) != PA_OK) return st;
     LoglikArgs A;
     memset(&A, 0, sizeof A);
-    A.ll_out = (double *)bufs[5].p;
-    A.len_in = dev_len ? gx->d_len : (const double *)e->d_ll_len;
-    if (gx) { A.row_out0 = gx->d_row0; A.row_out1 = gx->d_row1; }
-    A.len_row = (const int32_t *)bufs[6].p;
     if (piA) {
+        // the base frequencies first, so that the eigensystems are built while the rest is laid out
         double inst[6];
         gt_exchangeabilities(e, inst);
-        std::vector<double> pw(n);
+        char *d;
+        double *pw = (double *)B.take((size_t)n * 8, &d);
         for (int i = 0; i < n; i++) pw[i] = piA[order[i]];
-        HIPCHK(e, hipMalloc(&bufs[7].p, (size_t)n * 8));
-        HIPCHK(e, hipMalloc(&bufs[8].p, (size_t)n * GB_EIG_WORDS * 8));
-        HIPCHK(e, hipMalloc(&bufs[9].p, (size_t)n * 4 * 8));
-        HIPCHK(e, hipMemcpy(bufs[7].p, pw.data(), (size_t)n * 8, hipMemcpyHostToDevice));
-        HIPCHK(e, launch_gt_eig(inst, (const double *)bufs[7].p, n, (double *)bufs[8].p, (double *)bufs[9].p, e->stream));
-        A.el_eig = (const double *)bufs[8].p;
-        A.el_pi = (const double *)bufs[9].p;
+        HIPCHK(e, hipMemcpyAsync(e->d_io, e->h_io, B.off, hipMemcpyHostToDevice, e->stream));
+        double *d_eig = (double *)(e->d_io + e->io_bytes - CallBlock::up(eig_bytes));    // device only, behind the layout
+        HIPCHK(e, launch_gt_eig(inst, (const double *)d, n, d_eig, d_eig + (size_t)n * GB_EIG_WORDS, e->stream));
+        A.el_eig = d_eig;
+        A.el_pi = d_eig + (size_t)n * GB_EIG_WORDS;
     }
+    A.len_row = B.put(order.data(), n);
+    A.len_in = dev_len ? gx->d_len : B.put(lengths, (size_t)n * N);
+    if (gx) { A.row_out0 = gx->d_row0; A.row_out1 = gx->d_row1; }
     std::vector<int32_t> sorted(n);
     for (int i = 0; i < n; i++) sorted[i] = ids[order[i]];
-    DevBuf pre[2];
     if (lens0) {
         // the two site prefixes per caller row; the root sums walk the sites
-        std::vector<int32_t> pl((size_t)n * 2);
+        char *d;
+        int32_t *pl = (int32_t *)B.take((size_t)n * 8, &d);
         for (int i = 0; i < n; i++) { pl[2 * i] = lens0[i]; pl[2 * i + 1] = lens1[i]; }
-        HIPCHK(e, hipMalloc(&pre[0].p, pl.size() * 4));
-        HIPCHK(e, hipMalloc(&pre[1].p, (size_t)n * 8));
-        HIPCHK(e, hipMemcpy(pre[0].p, pl.data(), pl.size() * 4, hipMemcpyHostToDevice));
-        A.pre_len = (const int32_t *)pre[0].p;
-        A.ll_out2 = (double *)pre[1].p;
+        A.pre_len = (const int32_t *)d;
         A.site = e->d_site;
     }
     // resident partials: every work position's region in the caller's arena
@@ -1553,18 +1579,11 @@ static pa_status loglik_lengths_impl(pa_engine *e, const int32_t *ids, int32_t n
             A.cand_score = (double *)gb[11].p;
         }
     }
-    st = run_kernel(e, sorted.data(), n, precision == PA_FP64, A, bufs);
+    st = run_kernel(e, sorted.data(), n, precision == PA_FP64, A, B, out, out1);
     if (st != PA_OK) return st;
-    std::vector<double> ll(n);
-    HIPCHK(e, hipMemcpy(ll.data(), bufs[5].p, (size_t)n * 8, hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; i++) out[order[i]] = ll[i];
-    if (lens0) {
-        HIPCHK(e, hipMemcpy(ll.data(), pre[1].p, (size_t)n * 8, hipMemcpyDeviceToHost));
-        for (int i = 0; i < n; i++) out1[order[i]] = ll[i];
-    }
     if (gx && gx->cand_score)
         HIPCHK(e, hipMemcpy(gx->cand_score, gb[11].p, (size_t)n * gx->cand_max * 8, hipMemcpyDeviceToHost));
-    if (e->ll_scratch_bytes + e->ll_len_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
+    if (e->ll_scratch_bytes + e->io_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
     return PA_OK;
 }
 

@@ -24,10 +24,10 @@ struct ScoreItem { int w, p0, p1, part; };
 struct ScoreSplit { int w, part0, n; };
 
 // Arguments of the log-likelihood launch.  Work position w evaluates element
-// work[w] either at ancestral states Zin[w] and rates rates_in[w] over the
-// element's stored branch lengths, or, when len_in is set, at the per-call
-// lengths (row len_row[w], or w, of len_in) with every branch at rate 1 (Zin,
-// rates_in unused).
+// work[w] with row r = len_row[w] (or w) of the call's arrays: either at
+// ancestral states Zin[r] and rates rates_in[r] over the element's stored
+// branch lengths, or, when len_in is set, at the lengths len_in[r] with every
+// branch at rate 1 (Zin, rates_in unused).
 struct LoglikArgs {
     const ElemDev *elems;
     const int32_t *work;      // element ids in schedule order
@@ -52,17 +52,17 @@ struct LoglikArgs {
     // and reads every other node's partial where it is.
     const uint8_t *alt;
     const int32_t *path_node;
-    const int32_t *Zin;       // [n_work][N] (when len_in is null)
-    const double *rates_in;   // [n_work][2] (r1, r2) (when len_in is null)
+    const int32_t *Zin;       // [rows][N] (when len_in is null)
+    const double *rates_in;   // [rows][2] (r1, r2) (when len_in is null)
     const double *len_in;     // [rows][N] per-call branch lengths, or null
-    const int32_t *len_row;   // [n_work] row of len_in for each work position, or null (row w)
+    const int32_t *len_row;   // [n_work] the call's row of each work position, or null (row w)
     double *ll_out;           // [n_work]
-    // gBGC substitution model, or null: branch s of work position w takes
-    // P(dist) of class k = c(Z) + 3 * (Bin[w][s] != 0), c(0) = 0 (background),
-    // c(2) = 2 (accelerated), else 1 (conserved), whose eigensystem is
-    // gb_eig[w][k] = {lam[4], V[16], Vi[16]} (gbgc_eig_kernel).
-    const double *gb_eig;     // [n_work][6][GB_EIG_WORDS]
-    const int32_t *Bin;       // [n_work][N]
+    // gBGC substitution model, or null: branch s of row r takes P(dist) of
+    // class k = c(Z) + 3 * (Bin[r][s] != 0), c(0) = 0 (background), c(2) = 2
+    // (accelerated), else 1 (conserved), whose eigensystem is gb_eig[r][k] =
+    // {lam[4], V[16], Vi[16]} (gbgc_eig_kernel).
+    const double *gb_eig;     // [rows][6][GB_EIG_WORDS]
+    const int32_t *Bin;       // [rows][N]
     unsigned long long *counters;   // [0] += algorithmic HBM bytes of the launch, or null
     // Per-element substitution model for the own-tree path, or null: work
     // position w prunes with the eigensystem el_eig[w] = {lam[4], V[16],

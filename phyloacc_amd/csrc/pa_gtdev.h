@@ -47,10 +47,10 @@ struct GtDecideArgs {
     const int32_t *gnode, *indicator;
     double *h, *loglik, *logpz, *prior;   // the chain state, updated on acceptance
     int32_t *where;
-    // resident partials: on acceptance the nodes from gnode to the root
-    // switch slots (the launch wrote their new partials into the other one)
+    // resident partials: on acceptance the stored partials of the nodes from
+    // gnode to the root are stale (the proposal's pass stored none of them)
     const int32_t *par, *root;
-    uint8_t *alt;                // [n][N]
+    uint8_t *stale;              // [n][N]
     int32_t *accepted;
 };
 

@@ -195,11 +195,11 @@ __global__ void gt_hdecide_kernel(GtDecideArgs a)
     a.accepted[i] = 1;
     a.h[(size_t)i * a.N + a.gnode[i]] = a.prop[i];
     a.where[(size_t)i * a.N + a.gnode[i]] = a.wnew[i];
-    if (a.alt) {
+    if (a.stale) {
         const int32_t *par = a.par + (size_t)i * a.N;
-        uint8_t *alt = a.alt + (size_t)i * a.N;
+        uint8_t *stale = a.stale + (size_t)i * a.N;
         for (int x = a.gnode[i], k = 0; x >= 0 && x < a.N && k < a.N; x = par[x], k++) {
-            alt[x] ^= 1;
+            stale[x] = 1;
             if (x == a.root[i]) break;
         }
     }

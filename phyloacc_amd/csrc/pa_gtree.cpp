@@ -833,7 +833,7 @@ struct pa_gt_session {
     // resident partials of the current trees, at one precision
     int res_prec = -1;
     char *big = nullptr;
-    uint8_t *alt = nullptr;
+    uint8_t *stale = nullptr;
     std::vector<int64_t> big_off;
     GtPlan *plan = nullptr;
     std::vector<int32_t> h_gnode, h_ind, h_acc, l0, l1;   // staged for the asynchronous copies
@@ -879,8 +879,8 @@ static void session_prop_args(pa_gt_session *s, GtPropArgs &a)
 }
 
 // The partials of every element's current tree, kept in HBM at this
-// precision (two slots per internal node, all in their first): the current
-// trees' lengths, then one full pass that stores every node's partial.
+// precision: the current trees' lengths, then one full pass that stores every
+// node's partial (no node stale).
 static pa_status session_resident(pa_gt_session *s, int32_t precision)
 {
     pa_engine *e = s->e;
@@ -906,8 +906,8 @@ static pa_status session_resident(pa_gt_session *s, int32_t precision)
     if (hipMalloc(&s->big, std::max<size_t>(total, 256)) != hipSuccess)
         return engine_fail(e, PA_E_OOM, "gene-tree session: no device memory for the resident partials (" +
                                          std::to_string(total >> 20) + " MiB)");
-    if (!s->alt && s->get(&s->alt, (size_t)n * N) != hipSuccess) return engine_fail(e, PA_E_OOM, "session slot bits");
-    if (hipMemsetAsync(s->alt, 0, (size_t)n * N, stream) != hipSuccess) return engine_fail(e, PA_E_DEVICE, "session slot bits");
+    if (!s->stale && s->get(&s->stale, (size_t)n * N) != hipSuccess) return engine_fail(e, PA_E_OOM, "session stale marks");
+    if (hipMemsetAsync(s->stale, 0, (size_t)n * N, stream) != hipSuccess) return engine_fail(e, PA_E_DEVICE, "session stale marks");
     GtPropArgs a;
     session_prop_args(s, a);
     a.lengths_only = 1;
@@ -918,7 +918,7 @@ static pa_status session_resident(pa_gt_session *s, int32_t precision)
     x.d_row1 = s->out1;
     x.d_big = s->big;
     x.row_big_off = s->big_off.data();
-    x.d_alt = s->alt;
+    x.d_stale = s->stale;
     if ((st = gt_plan_build(e, s->ids.data(), n, s->piA.empty() ? nullptr : s->piA.data(), precision, x, &s->plan)) !=
         PA_OK)
         return st;
@@ -1051,13 +1051,13 @@ extern "C" pa_status pa_gt_session_branch_len(pa_gt_session *s, const int32_t *g
     a.key0 = ev.key0; a.key1 = ev.key1; a.m = m; a.slot = slot;
     if (launch_gt_hprop(a, stream) != hipSuccess) return engine_fail(e, PA_E_DEVICE, "height proposal launch failed");
     // the proposals' likelihoods: each element's path from the moved node to
-    // the root, into the slots its current partials do not use
+    // the root
     if ((st = gt_plan_run(e, s->plan, s->l0.data(), s->l1.data(), s->gnode)) != PA_OK) return st;
     GtDecideArgs d;
     d.n = n; d.N = N;
     d.win = s->win; d.prop = s->prop; d.rdraw = s->rdraw; d.prior_new = s->prior_new; d.lz_new = s->lz_new;
     d.wnew = s->wnew; d.where = s->where;
-    d.par = s->par; d.root = s->root; d.alt = s->alt;
+    d.par = s->par; d.root = s->root; d.stale = s->stale;
     d.lnew0 = s->out0; d.lnew1 = s->out1; d.gnode = s->gnode; d.indicator = s->ind;
     d.h = s->h; d.loglik = s->ll; d.logpz = s->lz; d.prior = s->prior; d.accepted = s->acc;
     if (launch_gt_hdecide(d, stream) != hipSuccess) return engine_fail(e, PA_E_DEVICE, "height decision launch failed");
@@ -1137,7 +1137,7 @@ extern "C" pa_status pa_gt_session_sweep(pa_gt_session *s, const int32_t *gnodes
         d.n = n; d.N = N;
         d.win = s->win; d.prop = s->prop; d.rdraw = s->rdraw; d.prior_new = s->prior_new; d.lz_new = s->lz_new;
         d.wnew = s->wnew; d.where = s->where;
-        d.par = s->par; d.root = s->root; d.alt = s->alt;
+        d.par = s->par; d.root = s->root; d.stale = s->stale;
         d.lnew0 = s->out0; d.lnew1 = s->out1; d.gnode = gn; d.indicator = s->ind;
         d.h = s->h; d.loglik = s->ll; d.logpz = s->lz; d.prior = s->prior; d.accepted = s->sw_acc + (size_t)j * n;
         if (launch_gt_hdecide(d, stream) != hipSuccess) return engine_fail(e, PA_E_DEVICE, "height decision launch failed");

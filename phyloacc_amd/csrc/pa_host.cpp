@@ -968,11 +968,11 @@ static int chain_grid_max(pa_engine *e, int fp64, int BS, int shape)
     const int N = e->tm.N, S = e->tm.S;
     return e->n_cu * fit_per_cu(e, chain::chain_smem_bytes(N, S, BS, fp64), BS, chain::chain_blocks_per_cu(fp64, BS, N, S, shape));
 }
-static int loglik_grid_max(pa_engine *e, int fp64, int BS, bool scores, int most = 8)
+static int loglik_grid_max(pa_engine *e, int fp64, int BS, LoglikUse use, int most = 8)
 {
     const int N = e->tm.N;
-    return e->n_cu * fit_per_cu(e, scores ? score_smem_bytes(N, fp64) : loglik_smem_bytes(N, fp64), BS,
-                                loglik_blocks_per_cu(fp64, BS, N, scores), most);
+    return e->n_cu * fit_per_cu(e, use == LoglikUse::Score ? score_smem_bytes(N, fp64) : loglik_smem_bytes(N, fp64), BS,
+                                loglik_blocks_per_cu(fp64, BS, N, use), most);
 }
 
 // Scratch of one persistent launch of `grid` workgroups over elements of
@@ -1161,17 +1161,18 @@ static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp6
     const int BS = loglik_block(e, ids, n, fp64);
     const size_t smem = loglik_smem_bytes(N, fp64);
     if (smem > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
-    const bool scores = !A.hist_draw && !A.cand_score && !A.alt;
+    const LoglikUse use = loglik_use(A);
+    const bool scores = use == LoglikUse::Score;
     // a scoring workgroup's slot is small, so as many run as registers and LDS
     // allow (16 of 64 threads a CU)
-    const int grid_max = loglik_grid_max(e, fp64, BS, scores, scores ? 16 : 8);
+    const int grid_max = loglik_grid_max(e, fp64, BS, use, scores ? 16 : 8);
     // long elements are scored in parts, so that one does not outlast the rest
     std::vector<ScoreItem> items;
     std::vector<ScoreSplit> splits;
     const int parts = scores && !A.pre_len ? split_elements(e, ids, n, BS, items, splits) : 0;
     const int grid = std::min(parts ? (int)items.size() : n, grid_max);
     // resident partials come with their own arena and offsets
-    const bool resident = A.alt != nullptr;
+    const bool resident = A.stale != nullptr;
     ScratchPlan pl;
     if (scores) {
         int most = 0;
@@ -1182,7 +1183,7 @@ static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp6
     } else if (!resident) {
         std::vector<int> ppad(n);
         for (int i = 0; i < n; i++) ppad[i] = e->elems[ids[i]].Ppad;
-        pl = plan_scratch(ppad, grid, 0, [&](int p) { return loglik_slot_bytes(N, S, p, fp64); });
+        pl = plan_scratch(ppad, grid, 0, [&](int p) { return loglik_resident_bytes(N, S, p, fp64); });
     }
     // the previous call synchronised its stream, so its scratch is free to reuse
     if (!resident && pl.total > e->ll_scratch_bytes) {
@@ -1522,14 +1523,14 @@ static pa_status loglik_lengths_impl(pa_engine *e, const int32_t *ids, int32_t n
     // resident partials: every work position's region in the caller's arena
     DevBuf rb;
     if (gx && gx->d_big) {
-        if (!gx->d_alt || !gx->row_big_off) return fail(e, PA_E_INPUT, "resident partials need slot bits and offsets");
+        if (!gx->d_stale || !gx->row_big_off) return fail(e, PA_E_INPUT, "resident partials need stale marks and offsets");
         std::vector<int64_t> bo(n);
         for (int i = 0; i < n; i++) bo[i] = gx->row_big_off[order[i]];
         HIPCHK(e, hipMalloc(&rb.p, (size_t)n * 8));
         HIPCHK(e, hipMemcpy(rb.p, bo.data(), (size_t)n * 8, hipMemcpyHostToDevice));
         A.big = gx->d_big;
         A.big_off = (const int64_t *)rb.p;
-        A.alt = gx->d_alt;
+        A.stale = gx->d_stale;
         A.path_node = gx->d_path;
     }
     // gene-tree moves: per-row trees, history draws, candidate scores (rows in the caller's order)
@@ -1807,7 +1808,7 @@ pa_status gt_plan_build(pa_engine *e, const int32_t *ids, int32_t n, const doubl
                         const GtExtra &x, GtPlan **out)
 {
     *out = nullptr;
-    if (n <= 0 || !x.d_len || !x.d_big || !x.row_big_off || !x.d_alt) return fail(e, PA_E_INPUT, "incomplete plan");
+    if (n <= 0 || !x.d_len || !x.d_big || !x.row_big_off || !x.d_stale) return fail(e, PA_E_INPUT, "incomplete plan");
     pa_status st = check_ids(e, ids, n);
     if (st != PA_OK) return st;
     if ((st = upload(e)) != PA_OK) return st;
@@ -1826,7 +1827,7 @@ pa_status gt_plan_build(pa_engine *e, const int32_t *ids, int32_t n, const doubl
     }
     p->BS = loglik_block(e, sorted.data(), n, fp64);
     if (loglik_smem_bytes(N, fp64) > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
-    p->grid = std::min(n, loglik_grid_max(e, fp64, p->BS, false));
+    p->grid = std::min(n, loglik_grid_max(e, fp64, p->BS, LoglikUse::Keep));
     HIPCHK(e, hipMalloc(&p->work.p, (size_t)n * 4));
     HIPCHK(e, hipMalloc(&p->row.p, (size_t)n * 4));
     HIPCHK(e, hipMalloc(&p->bo.p, (size_t)n * 8));
@@ -1861,7 +1862,7 @@ pa_status gt_plan_build(pa_engine *e, const int32_t *ids, int32_t n, const doubl
     A.row_out1 = x.d_row1;
     A.big = x.d_big;
     A.big_off = (const int64_t *)p->bo.p;
-    A.alt = x.d_alt;
+    A.stale = x.d_stale;
     A.work = (const int32_t *)p->work.p;
     A.n_work = n;
     A.counters = (unsigned long long *)p->cnt.p;
@@ -2130,7 +2131,7 @@ extern "C" pa_status pa_loglik_noalloc(pa_engine *e, const int32_t *d_ids, int32
         return fail(e, PA_E_INPUT, "the longest element (" + std::to_string(e->max_ppad) + " padded patterns) needs " +
                                        std::to_string(slot) + " B of scratch, over the " + std::to_string(usable) +
                                        " B of the allocation-free entry point");
-    const int grid = (int)std::min<size_t>({(size_t)n, (size_t)loglik_grid_max(e, fp64, BS, true), usable / slot});
+    const int grid = (int)std::min<size_t>({(size_t)n, (size_t)loglik_grid_max(e, fp64, BS, LoglikUse::Score), usable / slot});
     LoglikArgs A;
     memset(&A, 0, sizeof A);
     A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab;
@@ -2968,7 +2969,7 @@ static pa_status lane_launch(pa_server *s, Lane &L, bool others_busy)
     pa_engine *e = s->e;
     const int N = e->tm.N, S = e->tm.S;
     const int gmax_c = chain_grid_max(e, s->fp64, s->BS, s->shape);
-    const int gmax_l = loglik_grid_max(e, s->fp64, s->BS, true);
+    const int gmax_l = loglik_grid_max(e, s->fp64, s->BS, LoglikUse::Score);
     const size_t room = s->pool.largest();
     const double now = pa_serve_clock();
     // chain requests: slots for min(k, grid) workgroups plus the long elements' own regions

@@ -39,11 +39,12 @@ struct GtExtra {
     int cand_max = 0;
     double *cand_score = nullptr;                     // out: [n][cand_max]
     // resident partials: row r's at d_big + row_big_off[r] (loglik_resident_bytes),
-    // node slots chosen by d_alt [n][N]; rows with d_path[r] >= 0 prune that
-    // node's path to the root only (device arrays, rows in the caller's order)
+    // d_stale [n][N] marking the nodes whose stored partial is not the current
+    // tree's; rows with d_path[r] >= 0 score that node's path to the root only
+    // (device arrays, rows in the caller's order)
     char *d_big = nullptr;
     const int64_t *row_big_off = nullptr;             // host
-    const uint8_t *d_alt = nullptr;
+    uint8_t *d_stale = nullptr;
     const int32_t *d_path = nullptr;
 };
 // The engine's gene-node histories: the device arena of the last
@@ -57,7 +58,7 @@ struct GtHistory {
 };
 GtHistory &engine_history(pa_engine *e);
 // A resident-partials likelihood launch prepared once for a fixed batch
-// (x: d_len, d_big, row_big_off, d_alt; d_row0/1 optional); each run uploads
+// (x: d_len, d_big, row_big_off, d_stale; d_row0/1 optional); each run uploads
 // the prefix lengths (lens0 null: the pattern sum, no prefixes) and launches
 // on the engine stream without waiting; gt_plan_stats waits and records the
 // launch's time and counted bytes.

@@ -40,17 +40,18 @@ struct LoglikArgs {
     char *scratch;            // one slot per workgroup
     int64_t slot_bytes;
     // Elements too long for a slot: work position w keeps its partials at
-    // big + big_off[w] (loglik_slot_bytes of its own Ppad); big_off[w] < 0,
+    // big + big_off[w] (loglik_resident_bytes of its Ppad); big_off[w] < 0,
     // or big_off null, means the workgroup's slot.
     char *big;
     const int64_t *big_off;
     // Resident partials (gene-tree height moves), or null: every work
     // position's partials stay at big + big_off[w] (loglik_resident_bytes of
-    // its Ppad: two slots per internal node), node x of row r in its second
-    // slot when alt[r][x] != 0.  A row with path_node[r] >= 0 prunes only the
-    // path from that node to the root, into the slots alt does not select,
-    // and reads every other node's partial where it is.
-    const uint8_t *alt;
+    // its Ppad), node x's in slot x - S; stale[r][x] != 0 says that row r's
+    // stored partial of x is not its current tree's.  A row with path_node[r]
+    // >= 0 scores the path from that node to the root and stores none of it;
+    // the stale nodes off the path that it needs are stored first, and marked
+    // current.
+    uint8_t *stale;
     const int32_t *path_node;
     const int32_t *Zin;       // [rows][N] (when len_in is null)
     const double *rates_in;   // [rows][2] (r1, r2) (when len_in is null)
@@ -135,13 +136,10 @@ hipError_t launch_gt_eig(const double *inst /*[6], host*/, const double *piA /*[
 // LDS bytes of one workgroup (dynamic arrays + context + argument blocks).
 size_t loglik_smem_bytes(int N, int fp64);
 // Bytes of one workgroup's HBM slot for elements of up to Pcap (padded)
-// patterns: the partials [I][Pcap] (4 values each) and their exponents.
+// patterns: the partials (4 values each) and exponents of every internal node.
 size_t loglik_slot_bytes(int N, int S, int Pcap, int fp64);
-// Bytes of one element's resident partials at Ppad patterns (two slots per
-// internal node and their exponents).
+// Bytes of one element's resident partials at Ppad patterns, and its root terms.
 size_t loglik_resident_bytes(int N, int S, int Ppad, int fp64);
-// Dynamic LDS bytes of one workgroup (the launch's dynamic allocation).
-size_t loglik_dyn_smem_bytes(int N, int fp64);
 // Bytes of one workgroup's HBM slot in a launch that only scores: the stacks
 // of its waves, and with site prefixes the terms of Pcap (padded) patterns
 // (Pcap 0: none).  Never more than loglik_slot_bytes of the element's own
@@ -150,9 +148,15 @@ size_t score_slot_bytes(int N, int S, int BS, int Pcap, int fp64);
 // LDS bytes of one workgroup of a launch that only scores (no histories,
 // candidate scores or resident partials).
 size_t score_smem_bytes(int N, int fp64);
-// Workgroups of the likelihood kernel (or of the one that only scores)
-// resident on one CU (registers, LDS, launch bound).
-int loglik_blocks_per_cu(int fp64, int BS, int N, bool scores);
+// What a launch is for: log-likelihoods alone; resident partials; candidate
+// scores; a history draw.
+enum class LoglikUse { Score, Keep, Candidates, History };
+inline LoglikUse loglik_use(const LoglikArgs &A)
+{
+    return A.hist_draw ? LoglikUse::History : A.cand_score ? LoglikUse::Candidates : A.stale ? LoglikUse::Keep : LoglikUse::Score;
+}
+// Workgroups resident on one CU (registers, LDS, launch bound).
+int loglik_blocks_per_cu(int fp64, int BS, int N, LoglikUse use);
 hipError_t launch_loglik(const ModelDev &M, const LoglikArgs &A, int fp64, int BS, int grid, hipStream_t st);
 
 // Size of the device scratch array of the allocation-free likelihood entry

@@ -183,33 +183,6 @@ __device__ __forceinline__ void lds_add(LDS uint32_t *p, uint32_t v)
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Row j of P(t) = V diag(exp(lam t)) Vi, clamped at 0: out[i] = P_{j->i}.
-// Called by whole quads of lanes, lane j of a quad for row j of one matrix:
-// each lane takes one of the four exponentials and reads the others from its
-// quad.
-__device__ __forceinline__ double quad_lane(double v, int k)
-{
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    int lo = (int)(uint32_t)u, hi = (int)(uint32_t)(u >> 32);
-#define PA_QUAD(K) { lo = __builtin_amdgcn_mov_dpp(lo, K * 0x55, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, K * 0x55, 0xf, 0xf, true); }
-    if (k == 0) PA_QUAD(0) else if (k == 1) PA_QUAD(1) else if (k == 2) PA_QUAD(2) else PA_QUAD(3)
-#undef PA_QUAD
-    return __builtin_bit_cast(double, (unsigned long long)(uint32_t)lo | ((unsigned long long)(uint32_t)hi << 32));
-}
-
-__device__ __forceinline__ void ptrans_row(MP M, double t, int j, double (&out)[4])
-{
-    const double ej = exp(M->lam[j] * t);
-    const double e[4] = {quad_lane(ej, 0), quad_lane(ej, 1), quad_lane(ej, 2), quad_lane(ej, 3)};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        double s = 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++) s += M->V[j * 4 + k] * e[k] * M->Vi[k * 4 + i];
-        out[i] = s < 0 ? 0.0 : s;
-    }
-}
-
 // Class tables of every branch for class k (0 null, 1 conserved, 2 accelerated)
 // at rate r, a lane per matrix row.
 // mode 0: model start (dist2 > 1e-10 -> P(dist2*r), else identity; bpp_c.cpp:187-228)
@@ -228,7 +201,7 @@ __device__ __noinline__ void class_tables(MP M, CP<R> c, int k, double r, int mo
         GBL double *L = c->logt + ((size_t)k * N + s) * 16;
         if (mode == 1 && d < 1e-10) continue;       // a whole quad
         double row[4];
-        ptrans_row(M, d * r, j, row);
+        ptrans_row(&M->lam[0], d * r, j, row);
         if (mode == 0 && !(d > 1e-10)) {
 #pragma unroll
             for (int i = 0; i < 4; i++) row[i] = i == j ? 1.0 : 0.0;
@@ -1025,7 +998,7 @@ __device__ __noinline__ void build_prop_tables(MP M, CP<R> c, int cls, double pr
         const int s = nodes[it >> 2], j = it & 3;
         if (c->Z[s] != cls || (c->flags[s] & NF_MISSING)) continue;     // a whole quad
         double row[4];
-        ptrans_row(M, dist2[s] * prop, j, row);
+        ptrans_row(&M->lam[0], dist2[s] * prop, j, row);
         LDS R *dst = c->PTp + 16 * s;
 #pragma unroll
         for (int i = 0; i < 4; i++) dst[i * 4 + j] = (R)row[i];

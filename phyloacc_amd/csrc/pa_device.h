@@ -69,6 +69,33 @@ __device__ __forceinline__ double block_sum(double v, LDS double *red)
 // the node is a cherry (a non-root internal node whose children are both
 // leaves), whose partial is recomputed where it is read.
 constexpr uint8_t NF_CHERRY = 0x80;
+// Row j of P(t) = V diag(exp(lam t)) Vi, clamped at 0: out[i] = P_{j->i}.
+// Called by whole quads of lanes, lane j of a quad for row j of one matrix:
+// each lane takes one of the four exponentials and reads the others from its
+// quad.  E: lam[4], V[16], Vi[16].
+__device__ __forceinline__ double quad_lane(double v, int k)
+{
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    int lo = (int)(uint32_t)u, hi = (int)(uint32_t)(u >> 32);
+#define PA_QUAD(K) { lo = __builtin_amdgcn_mov_dpp(lo, K * 0x55, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, K * 0x55, 0xf, 0xf, true); }
+    if (k == 0) PA_QUAD(0) else if (k == 1) PA_QUAD(1) else if (k == 2) PA_QUAD(2) else PA_QUAD(3)
+#undef PA_QUAD
+    return __builtin_bit_cast(double, (unsigned long long)(uint32_t)lo | ((unsigned long long)(uint32_t)hi << 32));
+}
+
+__device__ __forceinline__ void ptrans_row(const LDS double *E, double t, int j, double (&out)[4])
+{
+    const double ej = exp(E[j] * t);
+    const double e[4] = {quad_lane(ej, 0), quad_lane(ej, 1), quad_lane(ej, 2), quad_lane(ej, 3)};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        double s = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) s += E[4 + j * 4 + k] * e[k] * E[20 + k * 4 + i];
+        out[i] = s < 0 ? 0.0 : s;
+    }
+}
+
 template <typename R>
 __device__ __forceinline__ void leaf_mul(const LDS R *PT, int code, R &a0, R &a1, R &a2, R &a3)
 {

@@ -78,71 +78,54 @@ size_t loglik_resident_bytes(int N, int S, int Ppad, int fp64)
 
 // ------------------------------------------------------------------ helpers
 
-// Transition matrix of branch s into PT: P(d * rate) for length d > 1e-10,
-// else the identity (BPP_C::initMats, src/PhyloAcc-ST/bpp_c.cpp:187-228).
-// P(t) = V diag(exp(lam t)) Vi, clamped at 0, built in FP64, from the
-// model's eigensystem or a gBGC class's (lam, V, Vi in LDS or global memory).
-template <typename R, typename PE>
-__device__ void branch_matrix_from(PE lam, PE V, PE Vi, LDS R *PT, int s, double d, double rate)
+// A work position's own eigensystems (the gBGC classes of its row, or its
+// element's base frequencies) are kept in LDS behind the rest.
+size_t loglik_eig_bytes(const LoglikArgs &A) { return A.gb_eig ? GB_CLASSES * GB_EIG_WORDS * 8 : A.el_eig ? GB_EIG_WORDS * 8 : 0; }
+
+__device__ __forceinline__ void fetch_eig(AP A, LDS double *eig, int w, int row)
 {
-    double P[16];
-    if (!(d <= 1e-10)) {          // a NaN length gives a NaN matrix, not the identity
-        const double t = d * rate;
-        double e[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) e[k] = exp(lam[k] * t);
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                double v = 0;
-#pragma unroll
-                for (int k = 0; k < 4; k++) v += V[j * 4 + k] * e[k] * Vi[k * 4 + i];
-                P[j * 4 + i] = v < 0 ? 0.0 : v;
-            }
-    } else {
-#pragma unroll
-        for (int q = 0; q < 16; q++) P[q] = (q % 5 == 0) ? 1.0 : 0.0;
-    }
-    LDS R *dst = PT + 16 * s;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) dst[i * 4 + j] = (R)P[j * 4 + i];
+    const double *src = A->gb_eig ? A->gb_eig + (size_t)row * GB_CLASSES * GB_EIG_WORDS : A->el_eig ? A->el_eig + (size_t)w * GB_EIG_WORDS : nullptr;
+    const int words = A->gb_eig ? GB_CLASSES * GB_EIG_WORDS : A->el_eig ? GB_EIG_WORDS : 0;
+    for (int i = threadIdx.x; i < words; i += blockDim.x) eig[i] = src[i];
 }
 
-// The matrix of branch s of work position w (row `row` of the call), whose
-// node table is tab.  A branch takes the rate of its class: Z = 0 (neutral)
-// rate 1, Z = 2 (accelerated) r2, any other Z (1, conserved) r1; an own-tree
+// Row j of the matrix of branch s into PT (PT[16 s + 4 i + j] = P_{j->i}), by
+// lane j of a quad (ptrans_row): P(d * rate) in FP64 for length d > 1e-10,
+// else the identity (BPP_C::initMats, src/PhyloAcc-ST/bpp_c.cpp:187-228).  A
+// thread a matrix took its 16 entries and four exponentials in turn (about
+// 1,200 instructions, and registers for an eigensystem), with most of a
+// workgroup idle.  A branch takes the rate of its class: Z = 0 (neutral) rate
+// 1, Z = 2 (accelerated) r2, any other Z (1, conserved) r1; an own-tree
 // element takes its lengths from len_in.
 template <typename R>
-__device__ __forceinline__ void work_matrix(MP M, AP A, LDS R *PT, const int32_t *tab, int s, int w, int row)
+__device__ __forceinline__ void work_matrix_row(MP M, AP A, const LDS double *eig, LDS R *PT, const int32_t *tab, int s, int j, int row)
 {
     const int N = M->N;
     const double *dist = (const double *)(tab + tab_dist(N));
+    const LDS double *E = &M->lam[0];
+    double d, rate = 1.0;
     if (A->len_in) {
-        const double len = A->len_in[(size_t)row * N + s];
-        if (A->el_eig) {
-            const double *E = A->el_eig + (size_t)w * GB_EIG_WORDS;
-            branch_matrix_from<R>(E, E + 4, E + 20, PT, s, len, 1.0);
-        } else {
-            branch_matrix_from<R>(M->lam, M->V, M->Vi, PT, s, len, 1.0);
-        }
-    } else if (A->gb_eig) {
-        const int z = A->Zin[(size_t)row * N + s];
-        const int k = (z == 2 ? 2 : (z == 0 ? 0 : 1)) + (A->Bin[(size_t)row * N + s] != 0 ? 3 : 0);
-        const double *E = A->gb_eig + ((size_t)row * GB_CLASSES + k) * GB_EIG_WORDS;
-        branch_matrix_from<R>(E, E + 4, E + 20, PT, s, dist[s], 1.0);
+        d = A->len_in[(size_t)row * N + s];
+        if (A->el_eig) E = eig;
     } else {
         const int z = A->Zin[(size_t)row * N + s];
-        branch_matrix_from<R>(M->lam, M->V, M->Vi, PT, s, dist[s], z == 2 ? A->rates_in[2 * row + 1] : (z == 0 ? 1.0 : A->rates_in[2 * row]));
+        d = dist[s];
+        if (A->gb_eig) E = eig + ((z == 2 ? 2 : (z == 0 ? 0 : 1)) + (A->Bin[(size_t)row * N + s] != 0 ? 3 : 0)) * GB_EIG_WORDS;
+        else rate = z == 2 ? A->rates_in[2 * row + 1] : (z == 0 ? 1.0 : A->rates_in[2 * row]);
     }
+    double r[4];
+    ptrans_row(E, d * rate, j, r);
+    LDS R *dst = PT + 16 * s + j;
+#pragma unroll
+    for (int i = 0; i < 4; i++) dst[4 * i] = (R)(d <= 1e-10 ? (i == j ? 1.0 : 0.0) : r[i]);      // a NaN length gives a NaN matrix
 }
 
+// The matrices of every branch of work position w, whose node table is tab.
 template <typename R, int BS>
-__device__ __forceinline__ void branch_matrices(MP M, AP A, LDS R *PT, const int32_t *tab, int n_nodes, int w, int row)
+__device__ __forceinline__ void branch_matrices(MP M, AP A, const LDS double *eig, LDS R *PT, const int32_t *tab, int n_nodes, int row)
 {
-    for (int q = threadIdx.x; q < n_nodes - 1; q += BS) work_matrix<R>(M, A, PT, tab, tab[tab_nodes(M->N) + q], w, row);
+    const int32_t *nodes = tab + tab_nodes(M->N);
+    for (int it = threadIdx.x; it < 4 * (n_nodes - 1); it += BS) work_matrix_row<R>(M, A, eig, PT, tab, nodes[it >> 2], it & 3, row);
 }
 
 // gBGC classes (BPP_C::init_cache_TM, src/PhyloAcc-ST-GBGC/SRC/bpp_c.cpp:
@@ -382,6 +365,7 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
     const int N = uni(M->N), S = uni(M->S), tid = threadIdx.x;
     LDS R *PT = (LDS R *)(LDS char *)smem_raw;
     LDS uint32_t *steps = (LDS uint32_t *)(PT + 16 * N);
+    LDS double *eig = (LDS double *)((LDS char *)smem_raw + score_smem<R>(N));
     for (;;) {
         if (tid == 0) {
             work_sh = atomicAdd(A->queue, 1);
@@ -410,7 +394,9 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
         a.codes = make_buf((GBL uint8_t *)(A->codes + E.off_codes), code_bytes(S, E.Ppad));
         const uint32_t ahead = first + (tid & ~63) < P ? touch_codes(a.codes, S, E.Ppad, first + (tid & ~63)) : 0;
         score_steps<R, BS>(M, steps, (LDS uint32_t *)&per_sh, tab, n_int, root, E.Ppad);
-        branch_matrices<R, BS>(M, A, PT, tab, n_nodes, w, row);
+        fetch_eig(A, eig, w, row);
+        __syncthreads();
+        branch_matrices<R, BS>(M, A, eig, PT, tab, n_nodes, row);
         const double *pw = A->el_pi ? A->el_pi + (size_t)w * 4 : nullptr;
         double pi[4];
         for (int j = 0; j < 4; j++) pi[j] = pw ? pw[j] : M->pi[j];
@@ -473,7 +459,7 @@ __host__ __device__ inline size_t keep_smem(int N, int BS, bool history)
 size_t loglik_smem_bytes(int N, int fp64)
 {
     return (fp64 ? keep_smem<double>(N, 256, false) : keep_smem<float>(N, 256, false)) + sizeof(ModelDev) + sizeof(LoglikArgs) +
-           CAND_CHUNK * (16 + 4 + 4) * 8 + 512;
+           CAND_CHUNK * (16 + 4) * 8 + 256;
 }
 
 // Waves per SIMD the kernel is declared for.
@@ -881,6 +867,7 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
     __syncthreads();
     const int N = uni(M->N), S = uni(M->S), I = N - S, tid = threadIdx.x;
     const KeepLds<R> k = keep_lds<R>((LDS char *)smem_raw, N);
+    LDS double *eig = (LDS double *)((LDS char *)smem_raw + keep_smem<R>(N, BS, USE == LoglikUse::History));
     for (;;) {
         if (tid == 0) work_sh = atomicAdd(A->queue, 1);
         __syncthreads();
@@ -909,6 +896,7 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
             k.mark[i] = (uint8_t)(((f & NF_MISSING) ? MK_MISS : 0) | (stale && stale[i] ? MK_STALE : 0) |
                                   (i >= S && i != root && a >= 0 && a < S && b >= 0 && b < S ? MK_CHERRY : 0));
         }
+        fetch_eig(A, eig, w, row);
         __syncthreads();
         if (path && tid == 0)
             for (int x = moved, q = 0; x >= 0 && x < N && q < N; x = k.par[x], q++) {
@@ -928,9 +916,9 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
         __syncthreads();
         const int n = uni(n_sh);
         // the matrices of the steps' children
-        for (int i = tid; i < 2 * n; i += BS) {
-            const uint32_t m = k.steps[4 * (i >> 1) + 3];
-            work_matrix<R>(M, A, k.PT, tab, (i & 1) ? (m >> SB_MAT_B_SHIFT) & SB_MAT_MASK : m & SB_MAT_MASK, w, row);
+        for (int i = tid; i < 8 * n; i += BS) {
+            const uint32_t m = k.steps[4 * (i >> 3) + 3];
+            work_matrix_row<R>(M, A, eig, k.PT, tab, (i & 4) ? (m >> SB_MAT_B_SHIFT) & SB_MAT_MASK : m & SB_MAT_MASK, i & 3, row);
         }
         const double *pw = A->el_pi ? A->el_pi + (size_t)w * 4 : nullptr;
         double pi[4];
@@ -996,7 +984,7 @@ static hipError_t launch_t(const ModelDev &M, const LoglikArgs &A, int grid, hip
 {
     // dynamic LDS above 64 KB needs the per-kernel limit raised (large trees only)
     if (loglik_use(A) == LoglikUse::Score) {
-        const size_t sm = score_smem<R>(M.N);
+        const size_t sm = score_smem<R>(M.N) + loglik_eig_bytes(A);
         if (sm > 65536) {
             const hipError_t err = hipFuncSetAttribute((const void *)score_kernel<R, BS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
             if (err != hipSuccess) return err;
@@ -1006,7 +994,7 @@ static hipError_t launch_t(const ModelDev &M, const LoglikArgs &A, int grid, hip
     }
     auto keep = [&](auto U) {
         constexpr LoglikUse use = decltype(U)::value;
-        const size_t sm = keep_smem<R>(M.N, BS, use == LoglikUse::History);
+        const size_t sm = keep_smem<R>(M.N, BS, use == LoglikUse::History) + loglik_eig_bytes(A);
         if (sm > 65536) {
             const hipError_t err = hipFuncSetAttribute((const void *)keep_kernel<R, BS, use>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
             if (err != hipSuccess) return err;

@@ -968,10 +968,10 @@ static int chain_grid_max(pa_engine *e, int fp64, int BS, int shape)
     const int N = e->tm.N, S = e->tm.S;
     return e->n_cu * fit_per_cu(e, chain::chain_smem_bytes(N, S, BS, fp64), BS, chain::chain_blocks_per_cu(fp64, BS, N, S, shape));
 }
-static int loglik_grid_max(pa_engine *e, int fp64, int BS, LoglikUse use, int most = 8)
+static int loglik_grid_max(pa_engine *e, int fp64, int BS, LoglikUse use, int most = 8, size_t eig = 0)
 {
     const int N = e->tm.N;
-    return e->n_cu * fit_per_cu(e, use == LoglikUse::Score ? score_smem_bytes(N, fp64) : loglik_smem_bytes(N, fp64), BS,
+    return e->n_cu * fit_per_cu(e, (use == LoglikUse::Score ? score_smem_bytes(N, fp64) : loglik_smem_bytes(N, fp64)) + eig, BS,
                                 loglik_blocks_per_cu(fp64, BS, N, use), most);
 }
 
@@ -1165,7 +1165,7 @@ static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp6
     const bool scores = use == LoglikUse::Score;
     // a scoring workgroup's slot is small, so as many run as registers and LDS
     // allow (16 of 64 threads a CU)
-    const int grid_max = loglik_grid_max(e, fp64, BS, use, scores ? 16 : 8);
+    const int grid_max = loglik_grid_max(e, fp64, BS, use, scores ? 16 : 8, loglik_eig_bytes(A));
     // long elements are scored in parts, so that one does not outlast the rest
     std::vector<ScoreItem> items;
     std::vector<ScoreSplit> splits;

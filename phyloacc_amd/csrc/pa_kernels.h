@@ -148,6 +148,8 @@ size_t score_slot_bytes(int N, int S, int BS, int Pcap, int fp64);
 // LDS bytes of one workgroup of a launch that only scores (no histories,
 // candidate scores or resident partials).
 size_t score_smem_bytes(int N, int fp64);
+// And the LDS of a launch whose work positions have eigensystems of their own.
+size_t loglik_eig_bytes(const LoglikArgs &A);
 // What a launch is for: log-likelihoods alone; resident partials; candidate
 // scores; a history draw.
 enum class LoglikUse { Score, Keep, Candidates, History };

@@ -78,6 +78,21 @@ size_t loglik_resident_bytes(int N, int S, int Ppad, int fp64)
 
 // ------------------------------------------------------------------ helpers
 
+// An element's record in scalar registers.  What is read through a pointer
+// held in LDS is not known to be the same in every lane, and a buffer made
+// from it would be used lane group by lane group, in a loop around every load.
+__device__ __forceinline__ ElemDev uni_elem(const ElemDev *e)
+{
+    ElemDev E;
+    const uint32_t *src = (const uint32_t *)e;
+    uint32_t w[sizeof(ElemDev) / 4];
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(ElemDev) / 4); i++) w[i] = (uint32_t)uni((int)src[i]);
+    __builtin_memcpy(&E, w, sizeof E);
+    return E;
+}
+
+
 // A work position's own eigensystems (the gBGC classes of its row, or its
 // element's base frequencies) are kept in LDS behind the rest.
 size_t loglik_eig_bytes(const LoglikArgs &A) { return A.gb_eig ? GB_CLASSES * GB_EIG_WORDS * 8 : A.el_eig ? GB_EIG_WORDS * 8 : 0; }
@@ -384,14 +399,14 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
             __syncthreads();
             continue;
         }
-        const ElemDev E = A->elems[id];
+        const ElemDev E = uni_elem(A->elems + id);
         const int row = A->len_row ? uni(A->len_row[w]) : w;
         const int32_t *hdr = A->hdr_call ? A->hdr_call + (size_t)row * 4 : nullptr;
-        const int32_t *tab = A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab;
+        const int32_t *tab = uni_ptr(A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab);
         const int root = uni(hdr ? hdr[0] : E.root), n_nodes = uni(hdr ? hdr[1] : E.n_nodes), n_int = (n_nodes - 1) / 2;
         const int first = uni(item.p0), P = part < 0 ? E.P : uni(item.p1);
         PassArgs<R> a;
-        a.codes = make_buf((GBL uint8_t *)(A->codes + E.off_codes), code_bytes(S, E.Ppad));
+        a.codes = make_buf(uni_ptr((GBL uint8_t *)(A->codes + E.off_codes)), code_bytes(S, E.Ppad));
         const uint32_t ahead = first + (tid & ~63) < P ? touch_codes(a.codes, S, E.Ppad, first + (tid & ~63)) : 0;
         score_steps<R, BS>(M, steps, (LDS uint32_t *)&per_sh, tab, n_int, root, E.Ppad);
         fetch_eig(A, eig, w, row);
@@ -401,7 +416,7 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
         double pi[4];
         for (int j = 0; j < 4; j++) pi[j] = pw ? pw[j] : M->pi[j];
         const int64_t bo = A->big_off ? A->big_off[w] : -1;
-        char *scratch = bo >= 0 ? A->big + bo : A->scratch + (int64_t)blockIdx.x * A->slot_bytes;
+        char *scratch = uni_ptr(bo >= 0 ? A->big + bo : A->scratch + (int64_t)blockIdx.x * A->slot_bytes);
         asm volatile("" ::"v"(ahead));
         __syncthreads();
         a.steps = (const LDS u32x4 *)steps;
@@ -611,7 +626,7 @@ __device__ __forceinline__ ChildIn<R> kept_node(const KeepLds<R> &k, const GBL c
 {
     ChildIn<R> in;
     if (k.mark[v] & MK_CHERRY) {
-        const int yA = k.ch0[v], yB = k.ch1[v];
+        const int yA = uni(k.ch0[v]), yB = uni(k.ch1[v]);
         return cherry_in<R>(k.PT + 16 * yA, k.PT + 16 * yB, k.mark[yA] & MK_MISS, k.mark[yB] & MK_MISS, k.mark[v] & MK_MISS,
                             __builtin_amdgcn_raw_buffer_load_b8(codes, p, yA * Ppad, 0), __builtin_amdgcn_raw_buffer_load_b8(codes, p, yB * Ppad, 0));
     }
@@ -669,7 +684,7 @@ __device__ __forceinline__ void draw_history(MP M, AP A, const KeepLds<R> &k, co
                                              const GBL int32_t *site, int row, int n_int, int S, int I, int Ppad)
 {
     constexpr int K = 4;
-    const int tid = threadIdx.x, len = A->hist_len[row], stride = A->hist_ns[row];
+    const int tid = threadIdx.x, len = uni(A->hist_len[row]), stride = uni(A->hist_ns[row]);
     GBL int8_t *out = (GBL int8_t *)A->hist + A->hist_off[row];
     const Key key{M->key0, M->key1};
     const uint32_t c2 = (uint32_t)A->hist_sweep, c3 = tagword(0, TAG_GT_HIST);
@@ -691,8 +706,8 @@ __device__ __forceinline__ void draw_history(MP M, AP A, const KeepLds<R> &k, co
             const uint32_t slot = w[j].y >> 20, a = w[j].y & 0x3ff, b = (w[j].y >> 10) & 0x3ff;
             in[j].v = ld4<R>((const GBL V4<R> *)(pp + (uint64_t)part_off<R>(slot)));
             in[j].x = *(const GBL int32_t *)(pe + (uint64_t)(slot * 256));
-            cdA[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, (a ? a - 1 : 0) * Ppad, 0);
-            cdB[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, (b ? b - 1 : 0) * Ppad, 0);
+            cdA[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, uni((a ? a - 1 : 0) * Ppad), 0);
+            cdB[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, uni((b ? b - 1 : 0) * Ppad), 0);
         };
         int res = 4, tp = 4;
         auto step = [&](auto J, int t) __attribute__((always_inline)) {
@@ -770,13 +785,17 @@ __device__ inline void full_transition(PE lam, PE V, PE Vi, double d, LDS double
 // matrices of CAND_CHUNK candidates are built at once, a thread each, and
 // their sums meet once.
 template <typename R, int BS>
-__device__ __noinline__ void gt_candidates(MP M, AP A, const KeepLds<R> k, const GBL char *blocks, Buf codes, const GBL int32_t *site,
-                                           LDS double *Pc, LDS double *red, int w, int row, int S, int I, int Ppad,
-                                           double pi0, double pi1, double pi2, double pi3)
+__device__ __noinline__ void gt_candidates(MP M, AP A, const KeepLds<R> k, const GBL char *blocks_, const GBL uint8_t *codes_,
+                                           const GBL int32_t *site, LDS double *Pc, LDS double *red, int w, int row_, int S_, int I_,
+                                           int Ppad_, double pi0, double pi1, double pi2, double pi3)
 {
+    // arguments of a call come in vector registers
+    const int row = uni(row_), S = uni(S_), I = uni(I_), Ppad = uni(Ppad_);
+    const GBL char *blocks = uni_ptr(blocks_);
+    const Buf codes = make_buf(uni_ptr(codes_), code_bytes(S, Ppad));
     const int tid = threadIdx.x, stride = A->hist_ns[row], cm = A->cand_max;
     const GBL int8_t *tg = (const GBL int8_t *)A->hist + A->hist_off[row];
-    const int b = A->cand_branch[row], nc = A->cand_n[row], len = A->cand_sites[row];
+    const int b = uni(A->cand_branch[row]), nc = uni(A->cand_n[row]), len = uni(A->cand_sites[row]);
     const double *E = A->el_eig ? A->el_eig + (size_t)w * GB_EIG_WORDS : nullptr;
     const double pi[4] = {pi0, pi1, pi2, pi3}, lp[4] = {log(pi0), log(pi1), log(pi2), log(pi3)};
     for (int q0 = 0; q0 < nc; q0 += CAND_CHUNK) {
@@ -879,14 +898,14 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
             __syncthreads();
             continue;
         }
-        const ElemDev E = A->elems[id];
+        const ElemDev E = uni_elem(A->elems + id);
         const int row = A->len_row ? uni(A->len_row[w]) : w;
         const int32_t *hdr = A->hdr_call ? A->hdr_call + (size_t)row * 4 : nullptr;
-        const int32_t *tab = A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab;
+        const int32_t *tab = uni_ptr(A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab);
         const int root = uni(hdr ? hdr[0] : E.root), n_nodes = uni(hdr ? hdr[1] : E.n_nodes), n_int = (n_nodes - 1) / 2;
         const int moved = A->path_node ? uni(A->path_node[row]) : -1;
         const bool path = moved >= S && moved < N;
-        const Buf codes = make_buf((GBL uint8_t *)(A->codes + E.off_codes), code_bytes(S, E.Ppad));
+        const Buf codes = make_buf(uni_ptr((GBL uint8_t *)(A->codes + E.off_codes)), code_bytes(S, E.Ppad));
         GBL uint8_t *stale = A->stale ? (GBL uint8_t *)(A->stale + (size_t)row * N) : nullptr;
         for (int i = tid; i < N; i += BS) {
             const int a = tab[tab_ch0(N) + i], b = tab[tab_ch1(N) + i], f = tab[tab_flags(N) + i];
@@ -924,7 +943,7 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
         double pi[4];
         for (int j = 0; j < 4; j++) pi[j] = pw ? pw[j] : M->pi[j];
         const int64_t bo = A->big_off ? A->big_off[w] : -1;
-        GBL char *blocks = (GBL char *)(bo >= 0 ? A->big + bo : A->scratch + (int64_t)blockIdx.x * A->slot_bytes);
+        GBL char *blocks = uni_ptr((GBL char *)(bo >= 0 ? A->big + bo : A->scratch + (int64_t)blockIdx.x * A->slot_bytes));
         __syncthreads();
         PassArgs<R> a;
         a.steps = (const LDS u32x4 *)k.steps;
@@ -943,7 +962,7 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
             else draw_history<R, BS, false>(M, A, k, blocks, codes, pi, site, row, n_int, S, I, E.Ppad);
         }
         if constexpr (USE == LoglikUse::Candidates)
-            gt_candidates<R, BS>(M, A, k, blocks, codes, site, (LDS double *)Pc, (LDS double *)red, w, row, S, I, E.Ppad, pi[0], pi[1], pi[2], pi[3]);
+            gt_candidates<R, BS>(M, A, k, blocks, (const GBL uint8_t *)(A->codes + E.off_codes), site, (LDS double *)Pc, (LDS double *)red, w, row, S, I, E.Ppad, pi[0], pi[1], pi[2], pi[3]);
         if (tid == 0) {
             A->ll_out[w] = s0;
             if (A->pre_len) A->ll_out2[w] = s1;

@@ -104,8 +104,8 @@ __device__ __forceinline__ void fetch_eig(AP A, LDS double *eig, int w, int row)
     for (int i = threadIdx.x; i < words; i += blockDim.x) eig[i] = src[i];
 }
 
-// Row j of the matrix of branch s into PT (PT[16 s + 4 i + j] = P_{j->i}), by
-// lane j of a quad (ptrans_row): P(d * rate) in FP64 for length d > 1e-10,
+// Row j of the matrix of branch s, of length d, into PT (PT[16 s + 4 i + j] =
+// P_{j->i}), by lane j of a quad (ptrans_row): P(d * rate) in FP64 for length d > 1e-10,
 // else the identity (BPP_C::initMats, src/PhyloAcc-ST/bpp_c.cpp:187-228).  A
 // thread a matrix took its 16 entries and four exponentials in turn (about
 // 1,200 instructions, and registers for an eigensystem), with most of a
@@ -113,19 +113,15 @@ __device__ __forceinline__ void fetch_eig(AP A, LDS double *eig, int w, int row)
 // 1, Z = 2 (accelerated) r2, any other Z (1, conserved) r1; an own-tree
 // element takes its lengths from len_in.
 template <typename R>
-__device__ __forceinline__ void work_matrix_row(MP M, AP A, const LDS double *eig, LDS R *PT, const int32_t *tab, int s, int j, int row)
+__device__ __forceinline__ void work_matrix_row(MP M, AP A, const LDS double *eig, LDS R *PT, double d, int cls, int s, int j, int row)
 {
-    const int N = M->N;
-    const double *dist = (const double *)(tab + tab_dist(N));
     const LDS double *E = &M->lam[0];
-    double d, rate = 1.0;
+    double rate = 1.0;
     if (A->len_in) {
-        d = A->len_in[(size_t)row * N + s];
         if (A->el_eig) E = eig;
     } else {
-        const int z = A->Zin[(size_t)row * N + s];
-        d = dist[s];
-        if (A->gb_eig) E = eig + ((z == 2 ? 2 : (z == 0 ? 0 : 1)) + (A->Bin[(size_t)row * N + s] != 0 ? 3 : 0)) * GB_EIG_WORDS;
+        const int z = cls & 3;
+        if (A->gb_eig) E = eig + (z + (cls & 4 ? 3 : 0)) * GB_EIG_WORDS;
         else rate = z == 2 ? A->rates_in[2 * row + 1] : (z == 0 ? 1.0 : A->rates_in[2 * row]);
     }
     double r[4];
@@ -135,13 +131,17 @@ __device__ __forceinline__ void work_matrix_row(MP M, AP A, const LDS double *ei
     for (int i = 0; i < 4; i++) dst[4 * i] = (R)(d <= 1e-10 ? (i == j ? 1.0 : 0.0) : r[i]);      // a NaN length gives a NaN matrix
 }
 
-// The matrices of every branch of work position w, whose node table is tab.
-template <typename R, int BS>
-__device__ __forceinline__ void branch_matrices(MP M, AP A, const LDS double *eig, LDS R *PT, const int32_t *tab, int n_nodes, int row)
-{
-    const int32_t *nodes = tab + tab_nodes(M->N);
-    for (int it = threadIdx.x; it < 4 * (n_nodes - 1); it += BS) work_matrix_row<R>(M, A, eig, PT, tab, nodes[it >> 2], it & 3, row);
-}
+// What a pass needs of node i, where its matrix will be: the length (double)
+// and the class (0 neutral, 2 accelerated, 1 any other Z; + 4 with gBGC) of its
+// branch.  Staged with every load in flight: a matrix read them one behind the
+// other from memory, through the node list, in each of its workgroup's rounds
+// (45 us of 270 an element of 120 leaves).
+template <typename R>
+__device__ __forceinline__ LDS double *node_len(LDS R *PT, int i) { return (LDS double *)(PT + 16 * i); }
+template <typename R>
+__device__ __forceinline__ LDS int32_t *node_int(LDS R *PT, int i) { return (LDS int32_t *)(PT + 16 * i) + 2; }
+
+__device__ __forceinline__ int branch_class(AP A, int z, int b) { return A->len_in ? 0 : (z == 2 ? 2 : (z == 0 ? 0 : 1)) + (A->gb_eig && b != 0 ? 4 : 0); }
 
 // gBGC classes (BPP_C::init_cache_TM, src/PhyloAcc-ST-GBGC/SRC/bpp_c.cpp:
 // 1563-1621, with the rate matrices of Gibbs, bpp_c.cpp:191-197): one thread
@@ -272,14 +272,41 @@ size_t score_slot_bytes(int N, int S, int BS, int Pcap, int fp64)
     return al((size_t)Pcap * 8, 256) + (size_t)(BS / 64) * block_bytes(score_slots(N - S), fp64 ? 8 : 4);
 }
 
-// The steps of the pass over every internal node, one node a thread, and the
+// The nodes' words of a scoring pass, where their matrices will be (node_len).
+// Then its steps, every internal node, one node a thread, and the
 // bytes a pass that stores every node but the cherries would move per
 // pattern (the counted bytes of a call).
 template <typename R, int BS>
-__device__ __forceinline__ void score_steps(MP M, LDS uint32_t *steps, LDS uint32_t *per, const int32_t *tab, int n_int, int root, int Ppad)
+__device__ __forceinline__ void score_stage(MP M, AP A, LDS R *PT, const int32_t *tab, int n_int, int row)
 {
-    const int N = M->N, S = M->S;
+    const int N = uni(M->N);
     const int32_t *po = tab + tab_porder(N), *ch0 = tab + tab_ch0(N), *ch1 = tab + tab_ch1(N), *fl = tab + tab_flags(N);
+    const double *len = A->len_in ? A->len_in + (size_t)row * N : (const double *)(tab + tab_dist(N));
+    const int32_t *zin = A->len_in ? tab : A->Zin + (size_t)row * N;      // (unused with lengths of its own)
+    const int32_t *bin = A->gb_eig ? A->Bin + (size_t)row * N : tab;      // (unused without gBGC)
+    // two nodes a thread, past the end the last one again
+    for (int i0 = threadIdx.x; i0 < N; i0 += 2 * BS) {
+        const int i1 = i0 + BS < N ? i0 + BS : i0;
+        const double l0 = len[i0], l1 = len[i1];
+        const int z0 = zin[i0], z1 = zin[i1], g0 = bin[i0], g1 = bin[i1];
+        const int a0 = ch0[i0], a1 = ch0[i1], b0 = ch1[i0], b1 = ch1[i1], f0 = fl[i0], f1 = fl[i1];
+        const int o0 = po[i0 < n_int ? i0 : 0], o1 = po[i1 < n_int ? i1 : 0];
+        auto put = [&](int i, double l, int z, int g, int a, int b, int f, int o) __attribute__((always_inline)) {
+            LDS int32_t *w = node_int(PT, i);
+            *node_len(PT, i) = l;
+            w[0] = branch_class(A, z, g);
+            w[1] = (a & 0x3ff) | (b & 0x3ff) << 10 | ((f & NF_MISSING) ? 1 << 20 : 0);
+            w[2] = o;        // the i-th node of the pruning order
+        };
+        put(i0, l0, z0, g0, a0, b0, f0, o0);
+        put(i1, l1, z1, g1, a1, b1, f1, o1);
+    }
+}
+
+template <typename R, int BS>
+__device__ __forceinline__ void score_steps(MP M, LDS R *PT, LDS uint32_t *steps, LDS uint32_t *per, int n_int, int root, int Ppad)
+{
+    const int S = uni(M->S);
     constexpr uint32_t W = 4 * sizeof(R) + 4;
     for (int t = threadIdx.x; t <= n_int; t += BS) {
         LDS uint32_t *o = steps + 4 * t;
@@ -287,23 +314,24 @@ __device__ __forceinline__ void score_steps(MP M, LDS uint32_t *steps, LDS uint3
             o[0] = o[1] = o[2] = o[3] = 0;
             continue;
         }
-        const uint32_t word = (uint32_t)po[t];
-        const int s = word & PO_NODE;
-        const int p1 = t > 0 ? (int)((uint32_t)po[t - 1] & PO_NODE) : -1, p2 = t > 1 ? (int)((uint32_t)po[t - 2] & PO_NODE) : -1;
-        const int x[2] = {ch0[s], ch1[s]};
+        const uint32_t word = (uint32_t)node_int(PT, t)[2];
+        const int s = word & PO_NODE, mine = node_int(PT, s)[1];
+        const int p1 = t > 0 ? (int)((uint32_t)node_int(PT, t - 1)[2] & PO_NODE) : -1, p2 = t > 1 ? (int)((uint32_t)node_int(PT, t - 2)[2] & PO_NODE) : -1;
+        const int x[2] = {mine & 0x3ff, (mine >> 10) & 0x3ff};
         StepDef d;
-        d.miss = fl[s] & NF_MISSING;
+        d.miss = mine >> 20 & 1;
         d.nostore = !(word & PO_WAITS);
         d.slot_to = (word >> PO_SLOT_SHIFT) & 31;
         uint32_t b = W;
         for (int j = 0; j < 2; j++) {
             const bool leaf = x[j] < S;
+            const int kid = node_int(PT, x[j])[1];
             d.kind[j] = leaf ? SK_LEAF : (x[j] == p1 ? SK_PREV : (x[j] == p2 ? SK_PREV2 : SK_STORED));
-            d.miss_kid[j] = (fl[x[j]] & NF_MISSING) ? 1 : 0;
+            d.miss_kid[j] = kid >> 20 & 1;
             d.mat[j] = x[j];
             d.row[j] = leaf ? x[j] * Ppad : 0;
             d.slot[j] = d.kind[j] == SK_STORED ? (int)((word >> PO_DEPTH_SHIFT) & PO_DEPTH) : 0;
-            b += leaf ? 1 : (ch0[x[j]] < S && ch1[x[j]] < S ? 2 : W);
+            b += leaf ? 1 : ((kid & 0x3ff) < S && (kid >> 10 & 0x3ff) < S ? 2 : W);
         }
         encode_step(o, d);
         const bool cherry = s != root && x[0] < S && x[1] < S;
@@ -381,9 +409,9 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
     LDS R *PT = (LDS R *)(LDS char *)smem_raw;
     LDS uint32_t *steps = (LDS uint32_t *)(PT + 16 * N);
     LDS double *eig = (LDS double *)((LDS char *)smem_raw + score_smem<R>(N));
-    for (;;) {
+    for (bool first_work = true;; first_work = false) {
         if (tid == 0) {
-            work_sh = atomicAdd(A->queue, 1);
+            work_sh = first_work ? (int)blockIdx.x : (int)gridDim.x + atomicAdd(A->queue, 1);
             per_sh = 0;
         }
         __syncthreads();
@@ -399,23 +427,26 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
             __syncthreads();
             continue;
         }
-        const ElemDev E = uni_elem(A->elems + id);
         const int row = A->len_row ? uni(A->len_row[w]) : w;
-        const int32_t *hdr = A->hdr_call ? A->hdr_call + (size_t)row * 4 : nullptr;
-        const int32_t *tab = uni_ptr(A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab);
-        const int root = uni(hdr ? hdr[0] : E.root), n_nodes = uni(hdr ? hdr[1] : E.n_nodes), n_int = (n_nodes - 1) / 2;
-        const int first = uni(item.p0), P = part < 0 ? E.P : uni(item.p1);
-        PassArgs<R> a;
-        a.codes = make_buf(uni_ptr((GBL uint8_t *)(A->codes + E.off_codes)), code_bytes(S, E.Ppad));
-        const uint32_t ahead = first + (tid & ~63) < P ? touch_codes(a.codes, S, E.Ppad, first + (tid & ~63)) : 0;
-        score_steps<R, BS>(M, steps, (LDS uint32_t *)&per_sh, tab, n_int, root, E.Ppad);
-        fetch_eig(A, eig, w, row);
-        __syncthreads();
-        branch_matrices<R, BS>(M, A, eig, PT, tab, n_nodes, row);
         const double *pw = A->el_pi ? A->el_pi + (size_t)w * 4 : nullptr;
         double pi[4];
         for (int j = 0; j < 4; j++) pi[j] = pw ? pw[j] : M->pi[j];
         const int64_t bo = A->big_off ? A->big_off[w] : -1;
+        const ElemDev E = uni_elem(A->elems + id);
+        const int32_t *hdr = A->hdr_call ? A->hdr_call + (size_t)row * 4 : nullptr;
+        const int32_t *tab = uni_ptr(A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab);
+        const int root = uni(hdr ? hdr[0] : E.root), n_int = (uni(hdr ? hdr[1] : E.n_nodes) - 1) / 2;
+        const int first = uni(item.p0), P = part < 0 ? E.P : uni(item.p1);
+        PassArgs<R> a;
+        a.codes = make_buf(uni_ptr((GBL uint8_t *)(A->codes + E.off_codes)), code_bytes(S, E.Ppad));
+        const uint32_t ahead = first + (tid & ~63) < P ? touch_codes(a.codes, S, E.Ppad, first + (tid & ~63)) : 0;
+        score_stage<R, BS>(M, A, PT, tab, n_int, row);
+        fetch_eig(A, eig, w, row);
+        __syncthreads();
+        score_steps<R, BS>(M, PT, steps, (LDS uint32_t *)&per_sh, n_int, root, E.Ppad);
+        __syncthreads();
+        // every node's matrix (the root's and absent nodes' are never read)
+        for (int i = tid; i < 4 * N; i += BS) work_matrix_row<R>(M, A, eig, PT, *node_len(PT, i >> 2), *node_int(PT, i >> 2), i >> 2, i & 3, row);
         char *scratch = uni_ptr(bo >= 0 ? A->big + bo : A->scratch + (int64_t)blockIdx.x * A->slot_bytes);
         asm volatile("" ::"v"(ahead));
         __syncthreads();
@@ -466,15 +497,16 @@ constexpr int CAND_CHUNK = 16;      // candidates whose matrices are built toget
 template <typename R>
 __host__ __device__ inline size_t keep_smem(int N, int BS, bool history)
 {
-    // matrices, steps, children and parents, marks; the sampler's steps and the threads' bases
+    // matrices, steps, the internal nodes' children and pruning order, parents, marks; the sampler's steps and the
+    // threads' bases
     const size_t I = N / 2 + 1;
-    return (size_t)16 * N * sizeof(R) + 16 * (I + 1) + al((size_t)7 * N, 16) + (history ? 8 * (I + 2) + I * BS : 0);
+    return (size_t)16 * N * sizeof(R) + 16 * (I + 1) + al(3 * (size_t)N + 6 * I, 16) + (history ? 8 * (I + 2) + I * BS : 0);
 }
 
-size_t loglik_smem_bytes(int N, int fp64)
+size_t loglik_smem_bytes(int N, int fp64, LoglikUse use)
 {
     return (fp64 ? keep_smem<double>(N, 256, false) : keep_smem<float>(N, 256, false)) + sizeof(ModelDev) + sizeof(LoglikArgs) +
-           CAND_CHUNK * (16 + 4) * 8 + 256;
+           (use == LoglikUse::Keep ? 0 : CAND_CHUNK * (16 + 4) * 8) + 256;
 }
 
 // Waves per SIMD the kernel is declared for.
@@ -484,14 +516,15 @@ template <typename R>
 struct KeepLds {
     LDS R *PT;
     LDS uint32_t *steps;         // [I + 1][4]
-    LDS int16_t *ch0, *ch1, *par;
+    LDS int16_t *ch0, *ch1;      // indexed by node, internal nodes only
+    LDS int16_t *par, *order;    // [N]; [I] the nodes in pruning order
     LDS uint8_t *mark;
     LDS u32x2 *hrec;             // [I + 2] the history's steps
     LDS uint8_t *tgs;            // [I][BS] the threads' drawn bases
 };
 
 template <typename R>
-__device__ __forceinline__ KeepLds<R> keep_lds(LDS char *base, int N)
+__device__ __forceinline__ KeepLds<R> keep_lds(LDS char *base, int N, int S)
 {
     KeepLds<R> k;
     const size_t I = N / 2 + 1;
@@ -499,89 +532,102 @@ __device__ __forceinline__ KeepLds<R> keep_lds(LDS char *base, int N)
     LDS char *o = base + (size_t)16 * N * sizeof(R);
     k.steps = (LDS uint32_t *)o;
     o += 16 * (I + 1);
-    k.ch0 = (LDS int16_t *)o;
-    k.ch1 = k.ch0 + N;
-    k.par = k.ch1 + N;
+    k.ch0 = (LDS int16_t *)o - S;
+    k.ch1 = k.ch0 + I;
+    k.order = k.ch1 + S + I;
+    k.par = k.order + I;
     k.mark = (LDS uint8_t *)(k.par + N);
-    o += al((size_t)7 * N, 16);
+    o += al(3 * (size_t)N + 6 * I, 16);
     k.hrec = (LDS u32x2 *)o;
     k.tgs = (LDS uint8_t *)(o + 8 * (I + 2));
     return k;
 }
 
-// The steps of a pass, by one wave (build_steps in pa_chain.hip): every node,
-// or (path) first the stale nodes off the path, which are stored, then the
-// path.  Returns their number; bytes: what a pass that stores the nodes it
-// scores (all, or the path's) and reads all their children would move per
-// pattern.
-template <typename R>
-__device__ __forceinline__ int keep_steps(const KeepLds<R> &k, const int32_t *po, int S, int n_int, int Ppad, bool path,
-                                          GBL uint8_t *stale, uint32_t &bytes)
+// The steps of a pass: every node, or (path) first the stale nodes off the
+// path, which are stored, then the path.  Which of 64 positions of the pruning
+// order a phase visits is a bit mask, a wave a mask (keep_visits); a position's
+// place in the list and the steps just before it follow from the masks.
+// keep_steps returns the number of steps and adds to per what a pass that
+// stores the nodes it scores (all, or the path's) and reads all their children
+// would move per pattern.
+constexpr int KEEP_CHUNKS = MAXN / 2 / 64;
+
+template <typename R, int BS>
+__device__ __forceinline__ void keep_visits(const KeepLds<R> &k, LDS unsigned long long *visit, int n_int, bool path)
+{
+    const int lane = threadIdx.x & 63;
+    for (int c = uni(threadIdx.x >> 6); c < KEEP_CHUNKS; c += BS / 64) {
+        const int q = c * 64 + lane;
+        bool a = false, b = false;
+        if (q < n_int) {
+            const int s = k.order[q], mk = k.mark[s];
+            // a cherry off the path is a step of its parent's visit
+            const int t = (mk & MK_CHERRY) && !(mk & MK_PATH) ? k.mark[k.par[s]] : mk;
+            a = path && (t & MK_STALE) && !(t & MK_PATH);
+            b = !path || (t & MK_PATH);
+        }
+        const unsigned long long va = __ballot(a), vb = __ballot(b);
+        if (lane == 0) {
+            visit[c] = va;
+            visit[KEEP_CHUNKS + c] = vb;
+        }
+    }
+}
+
+template <typename R, int BS>
+__device__ __forceinline__ int keep_steps(const KeepLds<R> &k, const LDS unsigned long long *visit, LDS uint32_t *per, int S, int n_int,
+                                          int Ppad, GBL uint8_t *stale)
 {
     constexpr int W = 4 * sizeof(R) + 4;
-    const int lane = threadIdx.x;
-    int base = 0, last1 = -1, last2 = -1;
-    uint32_t sum = 0;
-    for (int phase = path ? 0 : 1; phase < 2; phase++)
-        for (int q0 = 0; q0 < n_int; q0 += 64) {
-            const int q = q0 + lane;
-            bool v = false;
-            int s = 0, mk = 0;
-            if (q < n_int) {
-                s = (uint32_t)po[q] & PO_NODE;
-                mk = k.mark[s];
-                if (!path) {
-                    v = true;
-                } else {
-                    // a cherry off the path is a step of its parent's visit
-                    const int t = (mk & MK_CHERRY) && !(mk & MK_PATH) ? k.mark[k.par[s]] : mk;
-                    v = phase == 0 ? (t & MK_STALE) && !(t & MK_PATH) : (t & MK_PATH) != 0;
-                }
-            }
-            const unsigned long long bal = __ballot(v);
-            const unsigned long long below = bal & ((1ull << lane) - 1);
-            const int l1 = below ? 63 - __clzll(below) : -1;
-            const unsigned long long below2 = l1 >= 0 ? below ^ (1ull << l1) : 0;
-            const int l2 = below2 ? 63 - __clzll(below2) : -1;
-            const int s1 = __shfl(s, l1 < 0 ? 0 : l1, 64), s2 = __shfl(s, l2 < 0 ? 0 : l2, 64);
-            const int n1 = l1 >= 0 ? s1 : last1, n2 = l2 >= 0 ? s2 : (l1 >= 0 ? last1 : last2);
-            if (v) {
-                const int x[2] = {k.ch0[s], k.ch1[s]};
-                StepDef d;
-                d.miss = mk & MK_MISS;
-                d.nostore = (mk & MK_CHERRY) || (path && phase == 1);
-                d.slot_to = s - S;
-                uint32_t b = W;
+    const int lane = threadIdx.x & 63;
+    int total = 0;
+    for (int m = 0; m < 2 * KEEP_CHUNKS; m++) total += __popcll(visit[m]);
+    for (int c = uni(threadIdx.x >> 6); c * 64 < n_int; c += BS / 64) {
+        for (int phase = 0; phase < 2; phase++) {
+            const int m = phase * KEEP_CHUNKS + c;
+            const unsigned long long mine = visit[m];
+            if (!mine) continue;
+            if (!((mine >> lane) & 1)) continue;
+            int at = __popcll(mine & ((1ull << lane) - 1));
+            for (int x = 0; x < m; x++) at += __popcll(visit[x]);
+            // the nodes of the three steps before
+            int before[3] = {-1, -1, -1};
+            unsigned long long bits = mine & ((1ull << lane) - 1);
+            int f = m;
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const bool leaf = x[j] < S;
-                    d.kind[j] = leaf ? SK_LEAF : (x[j] == n1 ? SK_PREV : (x[j] == n2 ? SK_PREV2 : SK_STORED));
-                    d.miss_kid[j] = (k.mark[x[j]] & MK_MISS) ? 1 : 0;
-                    d.mat[j] = x[j];
-                    d.row[j] = leaf ? x[j] * Ppad : 0;
-                    d.slot[j] = leaf ? 0 : x[j] - S;
-                    b += leaf ? 1 : ((k.mark[x[j]] & MK_CHERRY) ? 2 : W);
+            for (int i = 0; i < 3; i++) {
+                while (!bits && f > 0) bits = visit[--f];
+                if (bits) {
+                    const int h = 63 - __clzll(bits);
+                    before[i] = k.order[(f % KEEP_CHUNKS) * 64 + h];
+                    bits ^= 1ull << h;
                 }
-                encode_step(k.steps + 4 * (base + __popcll(below)), d);
-                if (phase == 1 && !(mk & MK_CHERRY)) sum += b;
-                if (phase == 0 && stale && !(mk & MK_CHERRY)) stale[s] = 0;      // stored by this pass
             }
-            const int cnt = __popcll(bal);
-            if (cnt) {
-                const int h1 = 63 - __clzll(bal);
-                const unsigned long long rest = bal ^ (1ull << h1);
-                const int t1 = __shfl(s, h1, 64);
-                const int t2 = __shfl(s, rest ? 63 - __clzll(rest) : 0, 64);
-                last2 = cnt > 1 ? t2 : last1;
-                last1 = t1;
+            const int s = k.order[c * 64 + lane], mk = k.mark[s];
+            const int x[2] = {k.ch0[s], k.ch1[s]};
+            StepDef d;
+            d.miss = mk & MK_MISS;
+            d.nostore = (mk & MK_CHERRY) || (mk & MK_PATH);
+            d.slot_to = s - S;
+            uint32_t b = W;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const bool leaf = x[j] < S;
+                d.kind[j] = leaf ? SK_LEAF : (x[j] == before[0] ? SK_PREV : (x[j] == before[1] ? SK_PREV2 : SK_STORED));
+                d.late = d.late || (!leaf && x[j] == before[2]);
+                d.miss_kid[j] = (k.mark[x[j]] & MK_MISS) ? 1 : 0;
+                d.mat[j] = x[j];
+                d.row[j] = leaf ? x[j] * Ppad : 0;
+                d.slot[j] = leaf ? 0 : x[j] - S;
+                b += leaf ? 1 : ((k.mark[x[j]] & MK_CHERRY) ? 2 : W);
             }
-            base += cnt;
+            encode_step(k.steps + 4 * at, d);
+            if (phase == 1 && !(mk & MK_CHERRY)) __hip_atomic_fetch_add(per, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (phase == 0 && !(mk & MK_CHERRY)) stale[s] = 0;      // stored by this pass
         }
-    if (lane < 4) k.steps[4 * base + lane] = 0;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
-    bytes = sum;
-    return base;
+    }
+    if (threadIdx.x < 4) k.steps[4 * total + threadIdx.x] = 0;
+    return total;
 }
 
 // The pass over an element's blocks and its root sums (see score_patterns;
@@ -597,7 +643,7 @@ __device__ __forceinline__ void keep_patterns(AP A, const PassArgs<R> &a, const 
     double acc = 0, acc1 = 0;
     for (int pb = uni(tid & ~63); pb < P; pb += BS) {
         const int p = pb + (tid & 63);
-        const ChildIn<R> o = prune_pattern<R, AMB, SCORE_DEPTH, false>(a, blocks + (size_t)(pb >> 6) * blkB, blkB, (uint32_t)p);
+        const ChildIn<R> o = prune_pattern<R, AMB, SCORE_DEPTH, true, SCORE_DEPTH>(a, blocks + (size_t)(pb >> 6) * blkB, blkB, (uint32_t)p);
         double t = 0;
         if (o.x != GAPT) {
             const double L = pi[0] * (double)o.v.x + pi[1] * (double)o.v.y + pi[2] * (double)o.v.z + pi[3] * (double)o.v.w;
@@ -609,10 +655,19 @@ __device__ __forceinline__ void keep_patterns(AP A, const PassArgs<R> &a, const 
     if (pre) {
         __syncthreads();
         const int n0 = A->pre_len[2 * row], n1 = A->pre_len[2 * row + 1];
-        for (int g = tid; g < n0; g += BS) {
-            const double t = term[site[g]];
-            acc += t;
-            if (g < n1) acc1 += t;
+        // four sites' loads at a time, added in the sites' order
+        for (int g0 = tid; g0 < n0; g0 += 4 * BS) {
+            int at[4];
+            double t[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) at[i] = site[g0 + i * BS < n0 ? g0 + i * BS : g0];
+#pragma unroll
+            for (int i = 0; i < 4; i++) t[i] = term[at[i]];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if (g0 + i * BS < n0) acc += t[i];
+                if (g0 + i * BS < n1) acc1 += t[i];
+            }
         }
         s1 = block_sum(acc1, red);
     }
@@ -652,7 +707,7 @@ __device__ inline int leaf_base(int code)
 enum { HR_MISS = 1 << 20, HR_CHERRY = 1 << 21, HR_PREV = 1 << 22, HR_MISS_A = 1 << 23, HR_MISS_B = 1 << 24 };
 
 template <typename R, int BS>
-__device__ __forceinline__ void history_steps(const KeepLds<R> &k, const int32_t *po, int S, int n_int, int root)
+__device__ __forceinline__ void history_steps(const KeepLds<R> &k, int S, int n_int, int root)
 {
     for (int t = threadIdx.x; t <= n_int; t += BS) {
         u32x2 w;
@@ -661,10 +716,10 @@ __device__ __forceinline__ void history_steps(const KeepLds<R> &k, const int32_t
             w.x = (uint32_t)root | (uint32_t)root << 10 | HR_MISS;
             w.y = (uint32_t)(root - S) << 20;
         } else {
-            const int s = (uint32_t)po[n_int - 1 - t] & PO_NODE, x0 = k.ch0[s], x1 = k.ch1[s], mk = k.mark[s];
+            const int s = k.order[n_int - 1 - t], x0 = k.ch0[s], x1 = k.ch1[s], mk = k.mark[s];
             const int pa = t > 0 ? k.par[s] : s;
             w.x = (uint32_t)s | (uint32_t)pa << 10 | ((mk & MK_MISS) ? HR_MISS : 0) | ((mk & MK_CHERRY) ? HR_CHERRY : 0) |
-                  (t > 0 && (int)((uint32_t)po[n_int - t] & PO_NODE) == pa ? HR_PREV : 0) |
+                  (t > 0 && k.order[n_int - t] == pa ? HR_PREV : 0) |
                   (x0 < S && (k.mark[x0] & MK_MISS) ? HR_MISS_A : 0) | (x1 < S && (k.mark[x1] & MK_MISS) ? HR_MISS_B : 0);
             w.y = (x0 < S ? (uint32_t)x0 + 1 : 0) | (x1 < S ? (uint32_t)(x1 + 1) << 10 : 0) |
                   (uint32_t)(((mk & (MK_MISS | MK_CHERRY)) ? root : s) - S) << 20;
@@ -879,16 +934,20 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
     __shared__ ModelDev Ms;
     __shared__ LoglikArgs As;
     __shared__ double red[CAND_CHUNK * 4], Pc[CAND_CHUNK * 16];
-    __shared__ int work_sh, n_sh;
+    __shared__ unsigned long long visit[2 * KEEP_CHUNKS];
+    __shared__ int work_sh;
     __shared__ uint32_t per_sh;
     MP M = to_lds(Mk, (LDS ModelDev *)&Ms);
     AP A = to_lds(Ak, (LDS LoglikArgs *)&As);
     __syncthreads();
     const int N = uni(M->N), S = uni(M->S), I = N - S, tid = threadIdx.x;
-    const KeepLds<R> k = keep_lds<R>((LDS char *)smem_raw, N);
+    const KeepLds<R> k = keep_lds<R>((LDS char *)smem_raw, N, S);
     LDS double *eig = (LDS double *)((LDS char *)smem_raw + keep_smem<R>(N, BS, USE == LoglikUse::History));
-    for (;;) {
-        if (tid == 0) work_sh = atomicAdd(A->queue, 1);
+    for (bool first_work = true;; first_work = false) {
+        if (tid == 0) {
+            work_sh = first_work ? (int)blockIdx.x : (int)gridDim.x + atomicAdd(A->queue, 1);
+            per_sh = 0;
+        }
         __syncthreads();
         const int w = uni(work_sh);
         if (w >= uni(A->n_work)) break;
@@ -898,51 +957,68 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
             __syncthreads();
             continue;
         }
-        const ElemDev E = uni_elem(A->elems + id);
         const int row = A->len_row ? uni(A->len_row[w]) : w;
-        const int32_t *hdr = A->hdr_call ? A->hdr_call + (size_t)row * 4 : nullptr;
-        const int32_t *tab = uni_ptr(A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab);
-        const int root = uni(hdr ? hdr[0] : E.root), n_nodes = uni(hdr ? hdr[1] : E.n_nodes), n_int = (n_nodes - 1) / 2;
-        const int moved = A->path_node ? uni(A->path_node[row]) : -1;
-        const bool path = moved >= S && moved < N;
-        const Buf codes = make_buf(uni_ptr((GBL uint8_t *)(A->codes + E.off_codes)), code_bytes(S, E.Ppad));
-        GBL uint8_t *stale = A->stale ? (GBL uint8_t *)(A->stale + (size_t)row * N) : nullptr;
-        for (int i = tid; i < N; i += BS) {
-            const int a = tab[tab_ch0(N) + i], b = tab[tab_ch1(N) + i], f = tab[tab_flags(N) + i];
-            k.ch0[i] = (int16_t)a;
-            k.ch1[i] = (int16_t)b;
-            k.par[i] = (int16_t)tab[tab_par(N) + i];
-            k.mark[i] = (uint8_t)(((f & NF_MISSING) ? MK_MISS : 0) | (stale && stale[i] ? MK_STALE : 0) |
-                                  (i >= S && i != root && a >= 0 && a < S && b >= 0 && b < S ? MK_CHERRY : 0));
-        }
-        fetch_eig(A, eig, w, row);
-        __syncthreads();
-        if (path && tid == 0)
-            for (int x = moved, q = 0; x >= 0 && x < N && q < N; x = k.par[x], q++) {
-                k.mark[x] |= MK_PATH;
-                if (x == root) break;
-            }
-        __syncthreads();
-        if (tid < 64) {
-            uint32_t b = 0;
-            const int n = keep_steps<R>(k, tab + tab_porder(N), S, n_int, E.Ppad, path, stale, b);
-            if (tid == 0) {
-                n_sh = n;
-                per_sh = b;
-            }
-        }
-        if constexpr (USE == LoglikUse::History) history_steps<R, BS>(k, tab + tab_porder(N), S, n_int, root);
-        __syncthreads();
-        const int n = uni(n_sh);
-        // the matrices of the steps' children
-        for (int i = tid; i < 8 * n; i += BS) {
-            const uint32_t m = k.steps[4 * (i >> 3) + 3];
-            work_matrix_row<R>(M, A, eig, k.PT, tab, (i & 4) ? (m >> SB_MAT_B_SHIFT) & SB_MAT_MASK : m & SB_MAT_MASK, i & 3, row);
-        }
         const double *pw = A->el_pi ? A->el_pi + (size_t)w * 4 : nullptr;
         double pi[4];
         for (int j = 0; j < 4; j++) pi[j] = pw ? pw[j] : M->pi[j];
         const int64_t bo = A->big_off ? A->big_off[w] : -1;
+        const ElemDev E = uni_elem(A->elems + id);
+        const int32_t *hdr = A->hdr_call ? A->hdr_call + (size_t)row * 4 : nullptr;
+        const int32_t *tab = uni_ptr(A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab);
+        const int root = uni(hdr ? hdr[0] : E.root), n_int = (uni(hdr ? hdr[1] : E.n_nodes) - 1) / 2;
+        const int moved = A->path_node ? uni(A->path_node[row]) : -1;
+        const bool path = moved >= S && moved < N;
+        const Buf codes = make_buf(uni_ptr((GBL uint8_t *)(A->codes + E.off_codes)), code_bytes(S, E.Ppad));
+        GBL uint8_t *stale = A->stale ? (GBL uint8_t *)(A->stale + (size_t)row * N) : nullptr;
+        const int32_t *po = tab + tab_porder(N);
+        const double *len = A->len_in ? A->len_in + (size_t)row * N : (const double *)(tab + tab_dist(N));
+        const int32_t *zin = A->len_in ? tab : A->Zin + (size_t)row * N;      // (unused with lengths of its own)
+        // every load in flight at once: two nodes a thread, past the end the last one again
+        for (int i0 = tid; i0 < N; i0 += 2 * BS) {
+            const int i1 = i0 + BS < N ? i0 + BS : i0;
+            const int a0 = tab[tab_ch0(N) + i0], b0 = tab[tab_ch1(N) + i0], f0 = tab[tab_flags(N) + i0], p0 = tab[tab_par(N) + i0];
+            const int a1 = tab[tab_ch0(N) + i1], b1 = tab[tab_ch1(N) + i1], f1 = tab[tab_flags(N) + i1], p1 = tab[tab_par(N) + i1];
+            const int o0 = po[i0 < n_int ? i0 : 0], o1 = po[i1 < n_int ? i1 : 0];
+            const uint8_t *st = stale ? (const uint8_t *)stale : (const uint8_t *)tab;
+            const int s0 = st[i0], s1 = st[i1];
+            const double l0 = len[i0], l1 = len[i1];
+            const int z0 = zin[i0], z1 = zin[i1];
+            auto put = [&](int i, int a, int b, int f, int pa, int o, int st, double l, int z) __attribute__((always_inline)) {
+                if (i >= S) {
+                    k.ch0[i] = (int16_t)a;
+                    k.ch1[i] = (int16_t)b;
+                }
+                k.par[i] = (int16_t)pa;
+                if (i < n_int) k.order[i] = (int16_t)((uint32_t)o & PO_NODE);
+                k.mark[i] = (uint8_t)(((f & NF_MISSING) ? MK_MISS : 0) | (stale && st ? MK_STALE : 0) |
+                                      (i >= S && i != root && a >= 0 && a < S && b >= 0 && b < S ? MK_CHERRY : 0));
+                *node_len(k.PT, i) = l;
+                *node_int(k.PT, i) = branch_class(A, z, 0);
+            };
+            put(i0, a0, b0, f0, p0, o0, s0, l0, z0);
+            put(i1, a1, b1, f1, p1, o1, s1, l1, z1);
+        }
+        fetch_eig(A, eig, w, row);
+        __syncthreads();
+        if (path) {
+            if (tid == 0)
+                for (int x = moved, q = 0; x >= 0 && x < N && q < N; x = k.par[x], q++) {
+                    k.mark[x] |= MK_PATH;
+                    if (x == root) break;
+                }
+            __syncthreads();
+        }
+        keep_visits<R, BS>(k, (LDS unsigned long long *)visit, n_int, path);
+        __syncthreads();
+        const int n = uni(keep_steps<R, BS>(k, (LDS unsigned long long *)visit, (LDS uint32_t *)&per_sh, S, n_int, E.Ppad, stale));
+        if constexpr (USE == LoglikUse::History) history_steps<R, BS>(k, S, n_int, root);
+        __syncthreads();
+        // the matrices of the steps' children
+        for (int i = tid; i < 8 * n; i += BS) {
+            const uint32_t m = k.steps[4 * (i >> 3) + 3];
+            const int s = (i & 4) ? (m >> SB_MAT_B_SHIFT) & SB_MAT_MASK : m & SB_MAT_MASK;
+            work_matrix_row<R>(M, A, eig, k.PT, *node_len(k.PT, s), *node_int(k.PT, s), s, i & 3, row);
+        }
         GBL char *blocks = uni_ptr((GBL char *)(bo >= 0 ? A->big + bo : A->scratch + (int64_t)blockIdx.x * A->slot_bytes));
         __syncthreads();
         PassArgs<R> a;

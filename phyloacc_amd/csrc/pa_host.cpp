@@ -971,7 +971,7 @@ static int chain_grid_max(pa_engine *e, int fp64, int BS, int shape)
 static int loglik_grid_max(pa_engine *e, int fp64, int BS, LoglikUse use, int most = 8, size_t eig = 0)
 {
     const int N = e->tm.N;
-    return e->n_cu * fit_per_cu(e, (use == LoglikUse::Score ? score_smem_bytes(N, fp64) : loglik_smem_bytes(N, fp64)) + eig, BS,
+    return e->n_cu * fit_per_cu(e, (use == LoglikUse::Score ? score_smem_bytes(N, fp64) : loglik_smem_bytes(N, fp64, use)) + eig, BS,
                                 loglik_blocks_per_cu(fp64, BS, N, use), most);
 }
 

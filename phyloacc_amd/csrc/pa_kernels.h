@@ -133,8 +133,11 @@ hipError_t launch_gbgc_eig(const double *Q0 /*[16], host*/, const double *sel /*
 hipError_t launch_gt_eig(const double *inst /*[6], host*/, const double *piA /*[n], device*/, int n,
                          double *eig /*[n][36], device*/, double *pi /*[n][4], device*/, hipStream_t st);
 
+// What a launch is for: log-likelihoods alone; resident partials; candidate
+// scores; a history draw.
+enum class LoglikUse { Score, Keep, Candidates, History };
 // LDS bytes of one workgroup (dynamic arrays + context + argument blocks).
-size_t loglik_smem_bytes(int N, int fp64);
+size_t loglik_smem_bytes(int N, int fp64, LoglikUse use = LoglikUse::Candidates);
 // Bytes of one workgroup's HBM slot for elements of up to Pcap (padded)
 // patterns: the partials (4 values each) and exponents of every internal node.
 size_t loglik_slot_bytes(int N, int S, int Pcap, int fp64);
@@ -150,9 +153,6 @@ size_t score_slot_bytes(int N, int S, int BS, int Pcap, int fp64);
 size_t score_smem_bytes(int N, int fp64);
 // And the LDS of a launch whose work positions have eigensystems of their own.
 size_t loglik_eig_bytes(const LoglikArgs &A);
-// What a launch is for: log-likelihoods alone; resident partials; candidate
-// scores; a history draw.
-enum class LoglikUse { Score, Keep, Candidates, History };
 inline LoglikUse loglik_use(const LoglikArgs &A)
 {
     return A.hist_draw ? LoglikUse::History : A.cand_score ? LoglikUse::Candidates : A.stale ? LoglikUse::Keep : LoglikUse::Score;

@@ -75,7 +75,7 @@ __device__ __forceinline__ void buf_st4(Buf b, const V4<R> &v, uint32_t lane_off
 enum { SK_LEAF = 0, SK_STORED = 1, SK_PREV = 2, SK_PREV2 = 3 };
 enum { ST_LL = 0, ST_PL = 1, ST_PP2 = 2, ST_SL = 3, ST_SP = 4, ST_SS = 5, ST_GEN = 6 };
 enum { SB_TYPE = 7, SB_STORED_A = 1 << 3, SB_STORED_B = 1 << 4, SB_NOSTORE = 1 << 5, SB_MISS = 1 << 6, SB_MISS_A = 1 << 7,
-       SB_MISS_B = 1 << 8, SB_KIND_A_SHIFT = 9, SB_KIND_B_SHIFT = 11, SB_SLOT_A_SHIFT = 14, SB_SLOT_SHIFT = 23,
+       SB_MISS_B = 1 << 8, SB_KIND_A_SHIFT = 9, SB_KIND_B_SHIFT = 11, SB_LATE = 1 << 13, SB_SLOT_A_SHIFT = 14, SB_SLOT_SHIFT = 23,
        SB_MAT_MASK = 0x3ff, SB_MAT_B_SHIFT = 10, SB_SLOT_B_SHIFT = 20 };
 static_assert(MAXN <= 512, "slots (below 2 I <= N) in nine bits, matrices (below 2 N) in ten");
 
@@ -84,6 +84,7 @@ struct StepDef {
     int kind[2], miss_kid[2], mat[2], row[2], slot[2];   // SK_* source, missing, matrix, code row offset, stored slot
     int slot_to;                                         // where the node is stored
     bool miss, nostore;
+    bool late = false;                                   // a stored child is the step three before (F = 4 below)
 };
 
 __device__ __forceinline__ void encode_step(LDS uint32_t *w, const StepDef &d)
@@ -100,7 +101,7 @@ __device__ __forceinline__ void encode_step(LDS uint32_t *w, const StepDef &d)
         else if (ka == SK_STORED) type = kb == SK_LEAF ? ST_SL : (kb == SK_PREV ? ST_SP : (kb == SK_STORED ? ST_SS : ST_GEN));
     }
     w[0] = (uint32_t)type | (ka == SK_STORED ? SB_STORED_A : 0) | (kb == SK_STORED ? SB_STORED_B : 0) |
-           (d.nostore ? SB_NOSTORE : 0) | (d.miss ? SB_MISS : 0) | (ma ? SB_MISS_A : 0) | (mb ? SB_MISS_B : 0) |
+           (d.nostore ? SB_NOSTORE : 0) | (d.late ? SB_LATE : 0) | (d.miss ? SB_MISS : 0) | (ma ? SB_MISS_A : 0) | (mb ? SB_MISS_B : 0) |
            ((uint32_t)ka << SB_KIND_A_SHIFT) | ((uint32_t)kb << SB_KIND_B_SHIFT) |
            ((uint32_t)(a ? d.slot[1] : d.slot[0]) << SB_SLOT_A_SHIFT) | ((uint32_t)d.slot_to << SB_SLOT_SHIFT);
     w[1] = (uint32_t)(a ? d.row[1] : d.row[0]);
@@ -196,22 +197,26 @@ __device__ __forceinline__ ChildIn<R> slot_load(Buf blk, uint32_t slot, uint32_t
 // code, and the steps past the last are an empty one.  ALL: every step also
 // stores; a step marked SB_NOSTORE through a buffer of no bytes (the hardware
 // drops accesses outside a buffer).  Otherwise only the steps not so marked
-// store.
-template <typename R, bool AMB, int D, bool ALL>
+// store.  F = 4 (with D = 4): stored partials are loaded four steps before
+// their use, for lists whose stored partials lie in HBM; a step marked
+// SB_LATE, whose child was stored after that, loads them again.
+template <typename R, bool AMB, int D, bool ALL, int F = 2>
 __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL char *base, int blk_bytes, uint32_t p)
 {
     const int n = A.n;
     const uint32_t lane = threadIdx.x & 63;
     const Buf blk = make_buf(base, blk_bytes);
-    ChildIn<R> inA[2], inB[2], res[2];
+    static_assert(F == 2 || F == D, "stored partials are loaded two steps ahead, or with the codes");
+    ChildIn<R> inA[F], inB[F], res[2];
     int cdA[D], cdB[D];
     uint32_t w[D][4];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         res[j].x = GAPT;
         res[j].v.x = res[j].v.y = res[j].v.z = res[j].v.w = (R)0;
-        inA[j] = inB[j] = res[j];
     }
+#pragma unroll
+    for (int j = 0; j < F; j++) inA[j] = inB[j] = res[0];
     u32x4 nw = A.steps[0];
     // the words of step k into set j, its codes on their way
     auto fetch_codes = [&](auto J, int k) __attribute__((always_inline)) {
@@ -225,12 +230,17 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
     // the stored partials of the step whose words are set j
     auto fetch_stored = [&](auto J) __attribute__((always_inline)) {
         constexpr int j = decltype(J)::value;
-        if (w[j][0] & SB_STORED_A) inA[j & 1] = slot_load<R>(blk, (w[j][0] >> SB_SLOT_A_SHIFT) & 511, lane, A.slots);
-        if (w[j][0] & SB_STORED_B) inB[j & 1] = slot_load<R>(blk, w[j][3] >> SB_SLOT_B_SHIFT, lane, A.slots);
+        if (w[j][0] & SB_STORED_A) inA[j % F] = slot_load<R>(blk, (w[j][0] >> SB_SLOT_A_SHIFT) & 511, lane, A.slots);
+        if (w[j][0] & SB_STORED_B) inB[j % F] = slot_load<R>(blk, w[j][3] >> SB_SLOT_B_SHIFT, lane, A.slots);
     };
     auto step = [&](auto J, int k) __attribute__((always_inline)) {
-        constexpr int d = decltype(J)::value, j = d & 1;
+        constexpr int d = decltype(J)::value, j = d & 1, f = d % F;
         const uint32_t w0 = w[d][0];
+        if constexpr (F > 2)
+            if (w0 & SB_LATE) {
+                fetch_stored(J);
+                __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): what is in flight afterwards is as on the other path
+            }
         const int type = w0 & SB_TYPE;
         const LDS R *PA = A.PT + 16 * (w[d][3] & SB_MAT_MASK), *PB = A.PT + 16 * ((w[d][3] >> SB_MAT_B_SHIFT) & SB_MAT_MASK);
         int e = 0;
@@ -239,27 +249,27 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
         ChildIn<R> out;
         if (type == ST_PL) {
             message<R, SK_PREV, AMB>(PA, 0, res[j ^ 1], a, e, ga);
-            message<R, SK_LEAF, AMB>(PB, cdB[d], inB[j], b, e, gb);
+            message<R, SK_LEAF, AMB>(PB, cdB[d], inB[f], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else if (type == ST_LL) {
-            message<R, SK_LEAF, AMB>(PA, cdA[d], inA[j], a, e, ga);
-            message<R, SK_LEAF, AMB>(PB, cdB[d], inB[j], b, e, gb);
+            message<R, SK_LEAF, AMB>(PA, cdA[d], inA[f], a, e, ga);
+            message<R, SK_LEAF, AMB>(PB, cdB[d], inB[f], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else if (type == ST_PP2) {
             message<R, SK_PREV, AMB>(PA, 0, res[j ^ 1], a, e, ga);
             message<R, SK_PREV2, AMB>(PB, 0, res[j], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else if (type == ST_SP) {
-            message<R, SK_STORED, AMB>(PA, 0, inA[j], a, e, ga);
+            message<R, SK_STORED, AMB>(PA, 0, inA[f], a, e, ga);
             message<R, SK_PREV, AMB>(PB, 0, res[j ^ 1], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else if (type == ST_SL) {
-            message<R, SK_STORED, AMB>(PA, 0, inA[j], a, e, ga);
-            message<R, SK_LEAF, AMB>(PB, cdB[d], inB[j], b, e, gb);
+            message<R, SK_STORED, AMB>(PA, 0, inA[f], a, e, ga);
+            message<R, SK_LEAF, AMB>(PB, cdB[d], inB[f], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else if (type == ST_SS) {
-            message<R, SK_STORED, AMB>(PA, 0, inA[j], a, e, ga);
-            message<R, SK_STORED, AMB>(PB, 0, inB[j], b, e, gb);
+            message<R, SK_STORED, AMB>(PA, 0, inA[f], a, e, ga);
+            message<R, SK_STORED, AMB>(PB, 0, inB[f], b, e, gb);
             out = combine<R>(a, b, e, ga && gb);
         } else {
             // any sources, missing nodes: a missing child contributes nothing, but its gap state still
@@ -276,8 +286,8 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
                 return ci;
             };
             a.x = a.y = a.z = a.w = b.x = b.y = b.z = b.w = (R)1;
-            child_apply<R>(ka == SK_LEAF, w0 & SB_MISS_A, PA, source(ka, inA[j], cdA[d]), a.x, a.y, a.z, a.w, e, ga);
-            child_apply<R>(kb == SK_LEAF, w0 & SB_MISS_B, PB, source(kb, inB[j], cdB[d]), b.x, b.y, b.z, b.w, e, gb);
+            child_apply<R>(ka == SK_LEAF, w0 & SB_MISS_A, PA, source(ka, inA[f], cdA[d]), a.x, a.y, a.z, a.w, e, ga);
+            child_apply<R>(kb == SK_LEAF, w0 & SB_MISS_B, PB, source(kb, inB[f], cdB[d]), b.x, b.y, b.z, b.w, e, gb);
             out = combine<R>(a, b, e, ga && gb);
             if ((w0 & SB_MISS) && !(ga && gb)) out.x = 0;
         }
@@ -285,7 +295,7 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
             fetch_codes(J, k + 2);
             fetch_stored(J);
         } else {
-            fetch_stored(std::integral_constant<int, (d + 2) % D>());
+            if constexpr (F == 2) fetch_stored(std::integral_constant<int, (d + 2) % D>());
             fetch_codes(J, k + D);
         }
         res[j] = out;
@@ -295,11 +305,11 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
             buf_st4<R>(b, out.v, lane * (uint32_t)sizeof(V4<R>), part_off<R>(to));
             __builtin_amdgcn_raw_buffer_store_b32((uint32_t)out.x, b, lane * 4, exp_off<R>(to, A.slots), 0);
         }
+        if constexpr (F > 2) fetch_stored(J);
     };
     each<D>([&](auto J) __attribute__((always_inline)) { fetch_codes(J, decltype(J)::value); });
     // no step before the third has a stored child of this pass, but it may have one of an earlier pass
-    fetch_stored(std::integral_constant<int, 0>());
-    fetch_stored(std::integral_constant<int, 1>());
+    each<F>([&](auto J) __attribute__((always_inline)) { fetch_stored(J); });
     for (int k = 0; k < n; k += D)
         if (!each_while<D>([&](auto J) __attribute__((always_inline)) {
                 step(J, k + decltype(J)::value);

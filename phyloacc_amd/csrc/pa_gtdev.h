@@ -54,8 +54,7 @@ struct GtDecideArgs {
     int32_t *accepted;
 };
 
-// LDS bytes of one proposal workgroup at N species-tree nodes (the species
-// tree, the element's rows and the move's workspace)
+// Bounds the species trees that a session takes (the kernel's LDS is less)
 inline size_t gt_hprop_lds(int N) { return (size_t)129 * N + 8; }
 constexpr size_t GT_HPROP_LDS_MAX = 64 * 1024 - 64;   // and 48 bytes of static LDS
 

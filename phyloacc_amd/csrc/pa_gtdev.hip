@@ -40,26 +40,24 @@ __global__ __launch_bounds__(64) void gt_hprop_kernel(GtPropArgs a)
     __shared__ double lc[4];
     const int i = blockIdx.x, t = threadIdx.x;
     const int N = a.N, S = a.S;
-    double *H = (double *)lds, *theta = H + N, *rate = theta + N, *ldens = rate + N, *h = ldens + N;
-    double *seq = h + N, *lzseq = seq + 2 * N;
-    int32_t *up = (int32_t *)(lzseq + N), *post = up + N, *ipost = post + N, *nleaf = ipost + N, *ch = nleaf + N;
-    int32_t *par = ch + 2 * N, *Z = par + N, *where = Z + N, *end = where + N, *cnt = end + N, *below = cnt + N;
-    int32_t *soff = below + N, *fill = soff + N + 1, *blist = fill + N;
-    uint8_t *miss = (uint8_t *)(blist + 2 * N);
+    // LDS holds what is walked node by node and what the move writes; what is
+    // read once a node stays in memory.  85 N bytes let 8 waves of 120-leaf
+    // trees share a CU, where 129 N let 5: each waits on its own chain.
+    double *H = (double *)lds, *h = H + N, *seq = h + N, *lzseq = seq + 2 * N;
+    int32_t *blist = (int32_t *)lzseq;       // the born nodes' lists, done with before the terms
+    int32_t *up = (int32_t *)(lzseq + N), *ipost = up + N, *ch = ipost + N;
+    int32_t *par = ch + 2 * N, *where = par + N, *end = where + N, *cnt = end + N, *below = cnt + N;
+    int32_t *soff = below + N, *fill = soff + N + 1;
+    uint8_t *miss = (uint8_t *)(fill + N);
     const size_t r = (size_t)i * N;
+    const double *rate = a.rate, *ldens = a.ldens;
+    const int32_t *post = a.sp.post, *nleaf = a.nleaf, *Z = a.Z + r;
     for (int k = t; k < N; k += 64) {
         H[k] = a.sp.H[k];
-        theta[k] = a.sp.theta[k];
-        rate[k] = a.rate[k];
-        ldens[k] = a.ldens[k];
         up[k] = a.sp.up[k];
-        const int pk = a.sp.post[k];
-        post[k] = pk;
-        ipost[pk] = k;
-        nleaf[k] = a.nleaf[k];
+        ipost[post[k]] = k;
         h[k] = a.h[r + k];
         par[k] = a.par[r + k];
-        Z[k] = a.Z[r + k];
         where[k] = a.where[r + k];
         miss[k] = a.miss[r + k];
         cnt[k] = 0;
@@ -72,7 +70,7 @@ __global__ __launch_bounds__(64) void gt_hprop_kernel(GtPropArgs a)
     __syncthreads();
     for (int k = t; k < N; k += 64) end[k] = k == root ? N - 1 : where[par[k]];
     __syncthreads();
-    const gt::SpView sp = {S, N, up, H, theta, post, nullptr, nullptr};
+    const gt::SpView sp = {S, N, up, H, a.sp.theta, post, nullptr, nullptr};
     gt::TreeView g = {S, N, root, ch, par, nullptr, h, where, end};
     if (t == 0 && a.lengths_only) {
         status_sh = 1;
@@ -161,6 +159,7 @@ __global__ __launch_bounds__(64) void gt_hprop_kernel(GtPropArgs a)
             const int ke = nleaf[x] - below[x];
             seq[soff[ipost[x]]] = ke != 0 && ke > 1 && up[x] != N ? -gt::coal_tail(rate[x], H[up[x]], H[x], ke) : 0.0;
         }
+        __syncthreads();
         for (int q = t; q < N; q += 64) {
             double tv = 0;
             lzseq[q] = gt::logpz_term(sp, g, miss, Z, lc, a.order[r + q], &tv) ? tv : 0.0;
@@ -237,7 +236,7 @@ hipError_t launch_gt_scatter_tables(const int32_t *src, int W, const int64_t *ds
 hipError_t launch_gt_hprop(const GtPropArgs &a, hipStream_t st)
 {
     if (a.n <= 0) return hipSuccess;
-    const size_t lds = gt_hprop_lds(a.N);
+    const size_t lds = (size_t)85 * a.N + 8;
     if (lds > GT_HPROP_LDS_MAX) return hipErrorInvalidValue;
     hipLaunchKernelGGL(gt_hprop_kernel, dim3(a.n), dim3(64), lds, st, a);
     return hipGetLastError();

@@ -735,7 +735,7 @@ def gene_trees_block(E, w, steps=3, warmup=1, precision="fp32", traffic=None, or
             ks = eng.loglik_stats()     # the last timed call's kernel
             ach = ks["algorithmic_bytes"] / (ks["elapsed_ms"] / 1e3) / 1e9
             roof = {"bound": "hbm", "achieved": round(ach, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                    "frac": round(ach / HBM_PEAK_GBS, 5), "traffic": traffic, "kernel": "loglik_kernel",
+                    "frac": round(ach / HBM_PEAK_GBS, 5), "traffic": traffic, "kernel": "score_kernel",
                     "algorithmic_bytes_per_launch": ks["algorithmic_bytes"],
                     "kernel_ms": round(ks["elapsed_ms"], 3), "grid": ks["grid"], "block_threads": ks["block_threads"],
                     "lds_bytes": ks["lds_bytes"]}

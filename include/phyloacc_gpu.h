@@ -475,7 +475,8 @@ void pa_batch_destroy(pa_batch *b);
  * 256 threads, or 0 for the default chosen from the batch's mean pattern
  * count) and the pattern-loop shape 0..PA_N_SHAPES-1, a pair (U nodes
  * pruned per round, K nodes per ancestral-sampling chunk): FP32 (2, 4),
- * (1, 4), (2, 8); FP64 (1, 2), (2, 2), (1, 4).  Neither changes any result
+ * (1, 4), (2, 8); FP64 (1, 2), (2, 2), (1, 4).  A pruning pass has no rounds
+ * any more, so U is reported and changes nothing.  Neither changes any result
  * (each chain is one workgroup's, and the shapes only regroup independent
  * loads).  round_nodes / chunk_nodes report U and K of the shape at the
  * precision the autotuner ran; rate: the element-MCMC iterations/s it

@@ -7,11 +7,12 @@
 // finish; workgroups pull elements from a device work queue (persistent
 // kernel).  Within a workgroup:
 //   * threads stride over site patterns (pruning) or sites (ancestral
-//     sampling); every thread keeps the same patterns through a whole
-//     post-order pass, so no barrier is needed between tree nodes;
-//   * conditional likelihoods are pattern-major in HBM scratch, two buffers
-//     per internal node (current / proposal) so an accepted Metropolis move
-//     flips a per-node bit instead of copying partials;
+//     sampling); a pass is a list of steps in post-order (pa_prune.h), and a
+//     thread takes its patterns through the whole list, so no barrier is
+//     needed between tree nodes;
+//   * conditional likelihoods are in HBM scratch by blocks of 64 patterns, two
+//     slots per internal node (current / proposal) so an accepted Metropolis
+//     move flips a per-node bit instead of copying partials;
 //   * partials are linear-space with a power-of-two rescale per node; the
 //     cumulative exponent rides along as an int; GAPT marks all-gap subtrees
 //     (the reference's Tg >= num_base, src/PhyloAcc-ST/bpp_c.hpp:417-428);
@@ -27,7 +28,10 @@
 // address-space-3 pointers, and every sweep phase is a separate non-inlined
 // function, so each phase gets its own register allocation instead of one
 // allocation spanning the whole persistent loop.
-// No MFMA: a K=4 matvec per pattern is not a dense contraction.
+// The kernel is bound by latency and issue: a wave issues an instruction about
+// every five cycles and four share a SIMD.  Matrix instructions for the FP32
+// messages (4x4x1, bit for bit the same) took 40 % of the vector instructions
+// away and no time.
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include <algorithm>
@@ -263,12 +267,12 @@ enum { DB_KIND1_SHIFT = 2, DB_MISS0 = 1 << 4, DB_MISS1 = 1 << 5, DB_MISS_A0 = 1 
 // budget of the chain kernel.
 template <typename R, int SH>
 struct Shape;
-template <> struct Shape<float, 0> { static constexpr int U = 1, K = 4; };
-template <> struct Shape<float, 1> { static constexpr int U = 1, K = 4; };
-template <> struct Shape<float, 2> { static constexpr int U = 2, K = 8; };
-template <> struct Shape<double, 0> { static constexpr int U = 1, K = 2; };
-template <> struct Shape<double, 1> { static constexpr int U = 2, K = 2; };
-template <> struct Shape<double, 2> { static constexpr int U = 1, K = 4; };
+template <> struct Shape<float, 0> { static constexpr int K = 4; };
+template <> struct Shape<float, 1> { static constexpr int K = 4; };
+template <> struct Shape<float, 2> { static constexpr int K = 8; };
+template <> struct Shape<double, 0> { static constexpr int K = 2; };
+template <> struct Shape<double, 1> { static constexpr int K = 2; };
+template <> struct Shape<double, 2> { static constexpr int K = 4; };
 
 // The steps of a pass, written by one wave: a ballot per 64 internal nodes
 // (in pruning order) places them, and each lane encodes its own node.  A

@@ -1104,11 +1104,9 @@ static size_t call_room(pa_engine *e, const int32_t *ids, int n)
 
 // Fixed-(Z, r) log-likelihood launch: one persistent launch over ids (in
 // schedule order, largest first), one scratch slot per workgroup.
-// Block size of a likelihood launch.  The kernel keeps up to 168 VGPRs (3
-// waves per SIMD), so a wider workgroup mostly buys lanes for long elements:
-// on 20,000 120-leaf gene trees (~360 patterns) 128 threads beat 256 by 7 %
-// in FP32 (8.5 vs 9.2 ms), while FP64, with twice the partial traffic per
-// lane, is fastest at 256 (11.9 vs 13.5 ms).
+// Block size of a likelihood launch that keeps partials.  On 20,000 120-leaf
+// gene trees (~360 patterns) 128 threads beat 256 by 7 % in FP32, while FP64,
+// with twice the partial traffic per lane, is fastest at 256.
 static int loglik_block(pa_engine *e, const int32_t *work, int32_t n, int fp64)
 {
     if (e->n_cu > 0 && n < 4 * e->n_cu) return 256;
@@ -1118,6 +1116,36 @@ static int loglik_block(pa_engine *e, const int32_t *work, int32_t n, int fp64)
     if (meanP <= 96) return 64;
     if (fp64) return meanP <= 200 ? 128 : 256;
     return meanP <= 600 ? 128 : 256;
+}
+
+// Block size of a launch that only scores.  Kernel times in us at 64, 128 and
+// 256 threads:
+//   2,000 gene trees of 120 leaves, FP32            393   327   257
+//   4,500                                            761   505   531
+//   12,000                                          1847  1222  1340
+//   1,500 elements of 43 leaves (300 patterns), FP64 190   134   130
+//   9,000                                            586   502   570
+//   6,000 of 85 patterns, FP64 / FP32            252/186 214/145 272/182
+//   20,000 of 136 patterns, FP32                     410   440   610
+//   2,000 of 120 leaves, FP64                       2374  1154   643
+// So 128 threads, but: 256 where the elements are fewer than eight a CU, where
+// LDS keeps 128-thread workgroups below 16 waves a CU (the last line: five
+// workgroups), and where an element that cannot be split (site prefixes)
+// would outlast its CU's even share; 64 for short elements in more than four
+// rounds of 16 workgroups a CU.
+static int score_block(pa_engine *e, const int32_t *work, int32_t n, int fp64, bool prefixes)
+{
+    const int cu = std::max(1, e->n_cu);
+    if (n < 8 * cu) return 256;
+    int64_t total = 0;
+    int longest = 0;
+    for (int i = 0; i < n; i++) {
+        total += e->n_pat[work[i]];
+        longest = std::max(longest, (int)e->n_pat[work[i]]);
+    }
+    if (total > (int64_t)600 * n || 8 * score_smem_bytes(e->tm.N, fp64) > e->lds_per_cu) return 256;
+    if (prefixes && longest > total / (8 * cu)) return 256;
+    return total <= (int64_t)160 * n && n > 64 * cu ? 64 : 128;
 }
 
 // The work items of a scoring launch: an element of more than `most` patterns
@@ -1158,11 +1186,11 @@ static int split_elements(pa_engine *e, const int32_t *ids, int n, int BS, std::
 static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp64, LoglikArgs &A, CallBlock &B, double *res0, double *res1)
 {
     const int S = e->tm.S, N = e->tm.N;
-    const int BS = loglik_block(e, ids, n, fp64);
     const size_t smem = loglik_smem_bytes(N, fp64);
     if (smem > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
     const LoglikUse use = loglik_use(A);
     const bool scores = use == LoglikUse::Score;
+    const int BS = scores ? score_block(e, ids, n, fp64, A.pre_len != nullptr) : loglik_block(e, ids, n, fp64);
     // a scoring workgroup's slot is small, so as many run as registers and LDS
     // allow (16 of 64 threads a CU)
     const int grid_max = loglik_grid_max(e, fp64, BS, use, scores ? 16 : 8, loglik_eig_bytes(A));

@@ -243,8 +243,12 @@ __device__ __forceinline__ LDS const T *to_lds(const T &k, LDS T *dst)
 // scores or resident partials) keeps no partials: a pass over the element's
 // nodes in pruning order holds the one or two it needs next in registers,
 // and a node whose parent comes later waits in a stack of a few slots per
-// wave.  What is left is bound by the instructions of a step (about 100 a
-// node and 64 patterns), no longer by storing and reloading every node.
+// wave.  What is left is the latency of a step (about 1,500 cycles at the four
+// waves a SIMD that 128 registers allow, half of them waiting), no longer
+// storing and reloading every node: 8,000 elements of 120 leaves, FP32 3.40 ms
+// before and 0.77 now, 5,000 of 43 leaves, FP64 0.94 and 0.29.  Three waves a
+// SIMD took 0.39 ms where four took 0.36 (FP64), five 0.95 where four took 0.85
+// (FP32, spills).
 
 constexpr int SCORE_DEPTH = 4;      // steps a leaf code is loaded ahead
 
@@ -413,6 +417,8 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
     LDS double *eig = (LDS double *)((LDS char *)smem_raw + score_smem<R>(N));
     for (bool first_work = true;; first_work = false) {
         if (tid == 0) {
+            // the first position without the counter (2,048 increments at once: gene trees 819 -> 787 us);
+            // later ones when they are needed, since one taken ahead waits for this one to end
             work_sh = first_work ? (int)blockIdx.x : (int)gridDim.x + atomicAdd(A->queue, 1);
             per_sh = 0;
         }
@@ -489,8 +495,10 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
 // (gt_hdecide_kernel).  Stale nodes form a top part of the tree, and those
 // that hang off the next move's path are pruned first, into their slots.  So
 // over a sweep a node is stored about once, where storing every proposal's
-// path stored it at each move below it: the pass over 4,000 elements of 120
-// leaves took 324 us a move that way.
+// path stored it at each move below it: a move's pass over 4,000 elements of
+// 120 leaves took 324 us that way and takes 250 now, 0.57 GB moved.  What is
+// left is latency: a dozen steps for each of a wave's three blocks (half the
+// time) and the set-up of each element (a third).
 
 enum { MK_PATH = 1, MK_STALE = 2, MK_MISS = 4, MK_CHERRY = 8 };
 
@@ -511,7 +519,9 @@ size_t loglik_smem_bytes(int N, int fp64, LoglikUse use)
            (use == LoglikUse::Keep ? 0 : CAND_CHUNK * (16 + 4) * 8) + 256;
 }
 
-// Waves per SIMD the kernel is declared for.
+// Waves per SIMD the kernel is declared for: what holds its registers with few
+// or no spills (FP64 240, histories and candidates 168), and for the height
+// moves, which wait on memory, the most that LDS lets run.
 constexpr int keep_waves(int rs, LoglikUse use) { return rs == 8 ? 2 : (use == LoglikUse::Keep ? 4 : 3); }
 
 template <typename R>

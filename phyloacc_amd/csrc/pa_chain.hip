@@ -1161,7 +1161,9 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
     const int32_t *tab = A->tab + E.off_tab;
     for (int i = tid; i < N; i += BS) {
         c->par[i] = (int16_t)tab[tab_par(N) + i];
-        c->flags[i] = (uint8_t)tab[tab_flags(N) + i];
+        // the cherry bit with the rest: the step lists of other waves' threads read it behind the next barrier
+        const int f = tab[tab_flags(N) + i];
+        c->flags[i] = (uint8_t)(f | ((f & NF_IN_TREE) && is_cherry(tab, N, M->S, E.root, i) ? NF_CHERRY : 0));
         c->nodes[i] = (int16_t)tab[tab_nodes(N) + i];
         c->inodes[i] = (int16_t)tab[tab_int(N) + i];
         c->cur[i] = 0;
@@ -1175,11 +1177,6 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
     }
     for (int s = M->S + tid; s < N; s += BS) node_desc(c->desc + 4 * (s - M->S), tab, N, M->S, E.root, s);
     __syncthreads();
-    // cherries (both children leaves; never the root) are recomputed where read
-    for (int q = tid; q < c->n_int; q += BS) {
-        const int s = c->inodes[q];
-        if (is_cherry(tab, N, M->S, E.root, s)) c->flags[s] |= NF_CHERRY;
-    }
     sample_steps<R, BS>(c);
     // null-rate tables (rate 1), fixed for the element
     class_tables<R, BS>(M, c, 0, 1.0, 0);

@@ -331,7 +331,6 @@ __device__ __forceinline__ void build_steps(CP<R> c, int mode, int cls)
             }
             const int cs = cur[s];
             StepDef d;
-            d.miss = (d3 & DB_MISS) != 0;
             d.nostore = (f & NF_CHERRY) != 0;
             d.slot_to = (prop ? 1 - cs : cs) * I + s - S;
 #pragma unroll
@@ -382,7 +381,7 @@ __device__ __forceinline__ double prune_patterns(MP M, CP<R> c, int mode)
     const GBL int32_t *wts = uni_ptr(c->wts);
     const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
     // the root is the last step of every pass that visits it
-    const bool in_regs = A.n > 0 && uni(c->last_step) == r && !(uni(c->flags[r]) & NF_MISSING);
+    const bool in_regs = A.n > 0 && uni(c->last_step) == r;
     const int rc = uni(c->cur[r]), rb = (mode == PR_PROP && uni(c->dirty[r])) ? 1 - rc : rc;
     double acc = 0;
     // whole waves of 64 patterns; wave w takes blocks w, w + BS / 64, ...

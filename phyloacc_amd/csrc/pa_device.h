@@ -144,7 +144,7 @@ __device__ __forceinline__ ChildIn<R> child_load(bool leaf, bool miss, const GBL
 // would have stored.
 template <typename R>
 __device__ __forceinline__ ChildIn<R> cherry_in(const LDS R *srcA, const LDS R *srcB, bool missA, bool missB,
-                                                bool miss_x, int cA, int cB)
+                                                int cA, int cB)
 {
     ChildIn<R> in;
     in.v.x = in.v.y = in.v.z = in.v.w = (R)0;
@@ -155,8 +155,6 @@ __device__ __forceinline__ ChildIn<R> cherry_in(const LDS R *srcA, const LDS R *
     if (!missB && !gB) leaf_mul<R>(srcB, cB, a0, a1, a2, a3);
     if (gA && gB) {
         in.x = GAPT;
-    } else if (miss_x) {
-        in.x = 0;
     } else {
         const R mx = fmax(fmax(a0, a1), fmax(a2, a3));
         int kx = 0;

@@ -325,7 +325,6 @@ __device__ __forceinline__ void score_steps(MP M, LDS R *PT, LDS uint32_t *steps
         const int p1 = t > 0 ? (int)((uint32_t)node_int(PT, t - 1)[2] & PO_NODE) : -1, p2 = t > 1 ? (int)((uint32_t)node_int(PT, t - 2)[2] & PO_NODE) : -1;
         const int x[2] = {mine & 0x3ff, (mine >> 10) & 0x3ff};
         StepDef d;
-        d.miss = mine >> 20 & 1;
         d.nostore = !(word & PO_WAITS);
         d.slot_to = (word >> PO_SLOT_SHIFT) & 31;
         uint32_t b = W;
@@ -618,7 +617,6 @@ __device__ __forceinline__ int keep_steps(const KeepLds<R> &k, const LDS unsigne
             const int s = k.order[c * 64 + lane], mk = k.mark[s];
             const int x[2] = {k.ch0[s], k.ch1[s]};
             StepDef d;
-            d.miss = mk & MK_MISS;
             d.nostore = (mk & MK_CHERRY) || (mk & MK_PATH);
             d.slot_to = s - S;
             uint32_t b = W;
@@ -694,7 +692,7 @@ __device__ __forceinline__ ChildIn<R> kept_node(const KeepLds<R> &k, const GBL c
     ChildIn<R> in;
     if (k.mark[v] & MK_CHERRY) {
         const int yA = uni(k.ch0[v]), yB = uni(k.ch1[v]);
-        return cherry_in<R>(k.PT + 16 * yA, k.PT + 16 * yB, k.mark[yA] & MK_MISS, k.mark[yB] & MK_MISS, k.mark[v] & MK_MISS,
+        return cherry_in<R>(k.PT + 16 * yA, k.PT + 16 * yB, k.mark[yA] & MK_MISS, k.mark[yB] & MK_MISS,
                             __builtin_amdgcn_raw_buffer_load_b8(codes, p, yA * Ppad, 0), __builtin_amdgcn_raw_buffer_load_b8(codes, p, yB * Ppad, 0));
     }
     const GBL char *blk = blocks + (size_t)(p >> 6) * block_bytes(I, sizeof(R));

@@ -74,7 +74,7 @@ __device__ __forceinline__ void buf_st4(Buf b, const V4<R> &v, uint32_t lane_off
 // are multiplied.
 enum { SK_LEAF = 0, SK_STORED = 1, SK_PREV = 2, SK_PREV2 = 3 };
 enum { ST_LL = 0, ST_PL = 1, ST_PP2 = 2, ST_SL = 3, ST_SP = 4, ST_SS = 5, ST_GEN = 6 };
-enum { SB_TYPE = 7, SB_STORED_A = 1 << 3, SB_STORED_B = 1 << 4, SB_NOSTORE = 1 << 5, SB_MISS = 1 << 6, SB_MISS_A = 1 << 7,
+enum { SB_TYPE = 7, SB_STORED_A = 1 << 3, SB_STORED_B = 1 << 4, SB_NOSTORE = 1 << 5, SB_MISS_A = 1 << 7,
        SB_MISS_B = 1 << 8, SB_KIND_A_SHIFT = 9, SB_KIND_B_SHIFT = 11, SB_LATE = 1 << 13, SB_SLOT_A_SHIFT = 14, SB_SLOT_SHIFT = 23,
        SB_MAT_MASK = 0x3ff, SB_MAT_B_SHIFT = 10, SB_SLOT_B_SHIFT = 20 };
 static_assert(MAXN <= 512, "slots (below 2 I <= N) in nine bits, matrices (below 2 N) in ten");
@@ -83,7 +83,7 @@ static_assert(MAXN <= 512, "slots (below 2 I <= N) in nine bits, matrices (below
 struct StepDef {
     int kind[2], miss_kid[2], mat[2], row[2], slot[2];   // SK_* source, missing, matrix, code row offset, stored slot
     int slot_to;                                         // where the node is stored
-    bool miss, nostore;
+    bool nostore;
     bool late = false;                                   // a stored child is the step three before (F = 4 below)
 };
 
@@ -95,13 +95,13 @@ __device__ __forceinline__ void encode_step(LDS uint32_t *w, const StepDef &d)
     const int ka = a ? d.kind[1] : d.kind[0], kb = a ? d.kind[0] : d.kind[1];
     const int ma = a ? d.miss_kid[1] : d.miss_kid[0], mb = a ? d.miss_kid[0] : d.miss_kid[1];
     int type = ST_GEN;
-    if (!d.miss && !ma && !mb) {
+    if (!ma && !mb) {
         if (ka == SK_LEAF) type = ST_LL;
         else if (ka == SK_PREV) type = kb == SK_LEAF ? ST_PL : (kb == SK_PREV2 ? ST_PP2 : ST_GEN);
         else if (ka == SK_STORED) type = kb == SK_LEAF ? ST_SL : (kb == SK_PREV ? ST_SP : (kb == SK_STORED ? ST_SS : ST_GEN));
     }
     w[0] = (uint32_t)type | (ka == SK_STORED ? SB_STORED_A : 0) | (kb == SK_STORED ? SB_STORED_B : 0) |
-           (d.nostore ? SB_NOSTORE : 0) | (d.late ? SB_LATE : 0) | (d.miss ? SB_MISS : 0) | (ma ? SB_MISS_A : 0) | (mb ? SB_MISS_B : 0) |
+           (d.nostore ? SB_NOSTORE : 0) | (d.late ? SB_LATE : 0) | (ma ? SB_MISS_A : 0) | (mb ? SB_MISS_B : 0) |
            ((uint32_t)ka << SB_KIND_A_SHIFT) | ((uint32_t)kb << SB_KIND_B_SHIFT) |
            ((uint32_t)(a ? d.slot[1] : d.slot[0]) << SB_SLOT_A_SHIFT) | ((uint32_t)d.slot_to << SB_SLOT_SHIFT);
     w[1] = (uint32_t)(a ? d.row[1] : d.row[0]);
@@ -273,7 +273,9 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
             out = combine<R>(a, b, e, ga && gb);
         } else {
             // any sources, missing nodes: a missing child contributes nothing, but its gap state still
-            // decides whether the parent is all-gap at this pattern
+            // decides whether the parent is all-gap at this pattern.  A missing node (both children missing)
+            // so comes out as ones, its exponent that of their rescaled form like any node's: at a missing
+            // root the pattern's term is log sum_j pi_j = 0.
             const int ka = (w0 >> SB_KIND_A_SHIFT) & 3, kb = (w0 >> SB_KIND_B_SHIFT) & 3;
             auto source = [&](int kind, const ChildIn<R> &ld, int code) __attribute__((always_inline)) {
                 const ChildIn<R> r1 = res[j ^ 1], r2 = res[j];
@@ -289,7 +291,6 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
             child_apply<R>(ka == SK_LEAF, w0 & SB_MISS_A, PA, source(ka, inA[f], cdA[d]), a.x, a.y, a.z, a.w, e, ga);
             child_apply<R>(kb == SK_LEAF, w0 & SB_MISS_B, PB, source(kb, inB[f], cdB[d]), b.x, b.y, b.z, b.w, e, gb);
             out = combine<R>(a, b, e, ga && gb);
-            if ((w0 & SB_MISS) && !(ga && gb)) out.x = 0;
         }
         if constexpr (D == 2) {
             fetch_codes(J, k + 2);

@@ -442,7 +442,9 @@ typedef struct {
  * src/PhyloAcc-ST/main.cpp:466-494) of every listed element on the device.
  * Replaces the OpenMP element loop body (main.cpp:452-500: BPP_C::initMCMC +
  * BPP_C::Gibbs per model).  results: [n*3] in run order (M0, M1, M2).
- * stats may be NULL. */
+ * stats may be NULL.  Elements whose leaf codes (species x patterns, padded
+ * to 64) take 4 GiB or more give PA_E_INPUT here and in the other calls that
+ * run chains; log-likelihoods and gene-tree moves take them. */
 pa_status pa_run_chains(pa_engine *e, const int32_t *ids, int32_t n, const pa_run_config *cfg,
                         pa_chain_result *results, pa_traces *traces, pa_run_stats *stats);
 

@@ -311,7 +311,8 @@ __device__ __forceinline__ void build_steps(CP<R> c, int mode, int cls)
         if (v) {
             const LDS uint32_t *dd = desc + 4 * (s - S);
             const uint32_t d0 = dd[0], d3 = dd[3];
-            int kind[2], miss[2], m[2], row[2] = {0, 0}, slot[2] = {0, 0};
+            int kind[2], miss[2], m[2], slot[2] = {0, 0};
+            uint32_t row[2] = {0, 0};
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 const int x = j ? (int)(d0 >> 16) : (int)(d0 & 0xffff);
@@ -320,7 +321,7 @@ __device__ __forceinline__ void build_steps(CP<R> c, int mode, int cls)
                 miss[j] = (d3 & (j ? DB_MISS1 : DB_MISS0)) ? 1 : 0;
                 if (k == KD_LEAF) {
                     kind[j] = SK_LEAF;
-                    row[j] = x * Ppad;
+                    row[j] = (uint32_t)x * (uint32_t)Ppad;
                 } else {
                     const int cx = cur[x];
                     kind[j] = x == n1 ? SK_PREV : (x == n2 ? SK_PREV2 : SK_STORED);
@@ -369,12 +370,8 @@ __device__ __forceinline__ double prune_patterns(MP M, CP<R> c, int mode)
 {
     const int tid = threadIdx.x;
     const int P = uni(c->P);
-    PassArgs<R> A;
-    A.n = uni(c->n_steps);
-    A.slots = 2 * uni(c->I);
-    A.steps = (const LDS u32x4 *)uni_ptr(c->steps);
-    A.PT = uni_ptr(c->PTc);
-    A.codes = make_buf(uni_ptr(c->codes), code_bytes(uni(c->S), uni(c->Ppad)));
+    const PassArgs<R> A = {(const LDS u32x4 *)uni_ptr(c->steps), uni_ptr(c->PTc), {uni_ptr(c->codes), uni(c->S), uni(c->Ppad)}, uni(c->n_steps),
+                           2 * uni(c->I)};
     GBL char *parts = uni_ptr(c->parts);
     const int I = uni(c->I), blkB = block_bytes(2 * I, sizeof(R));
     const int r = uni(c->root);
@@ -463,7 +460,7 @@ __device__ __forceinline__ void draw_sites(MP M, CP<R> c, uint32_t c2, uint32_t 
     const uint32_t k0 = (uint32_t)uni((int)M->key0), k1 = (uint32_t)uni((int)M->key1);
     const double p0 = M->pi[0], p1 = M->pi[1], p2 = M->pi[2], p3 = M->pi[3];
     const GBL char *parts = uni_ptr(c->parts);
-    const Buf codes = make_buf(uni_ptr(c->codes), code_bytes(S, Ppad));
+    const CodeRows<false> codes(uni_ptr(c->codes), S, Ppad);
     const GBL int32_t *site = uni_ptr(c->site);
     GBL uint32_t *amb = uni_ptr(c->amb);
     LDS uint8_t *tgs = uni_ptr(c->tgs) + tid - S * BS;      // node s: [s * BS]
@@ -489,8 +486,8 @@ __device__ __forceinline__ void draw_sites(MP M, CP<R> c, uint32_t c2, uint32_t 
             const uint32_t slot = r1[j] >> SR_SLOT_SHIFT;
             in[j].v = ld4<R>((const GBL V4<R> *)(pp + (uint64_t)part_off<R>(slot)));
             in[j].x = *(const GBL int32_t *)(pe + (uint64_t)(slot * 256));
-            cdA[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, (r1[j] & SR_ID) * Ppad, 0);
-            cdB[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, ((r1[j] >> 10) & SR_ID) * Ppad, 0);
+            cdA[j] = codes.at(codes.row(r1[j] & SR_ID), p);
+            cdB[j] = codes.at(codes.row((r1[j] >> 10) & SR_ID), p);
         };
         U4 rnd{0, 0, 0, 0};
         int ts = 0, tp = 0;

@@ -309,8 +309,8 @@ __device__ __forceinline__ void score_stage(MP M, AP A, LDS R *PT, const int32_t
     }
 }
 
-template <typename R, int BS>
-__device__ __forceinline__ void score_steps(MP M, LDS R *PT, LDS uint32_t *steps, LDS uint32_t *per, int n_int, int root, int Ppad)
+template <typename R, int BS, bool WIDE>
+__device__ __forceinline__ void score_steps(MP M, LDS R *PT, LDS uint32_t *steps, LDS uint32_t *per, int n_int, int root, const CodeRows<WIDE> &codes)
 {
     const int S = uni(M->S);
     constexpr uint32_t W = 4 * sizeof(R) + 4;
@@ -334,7 +334,7 @@ __device__ __forceinline__ void score_steps(MP M, LDS R *PT, LDS uint32_t *steps
             d.kind[j] = leaf ? SK_LEAF : (x[j] == p1 ? SK_PREV : (x[j] == p2 ? SK_PREV2 : SK_STORED));
             d.miss_kid[j] = kid >> 20 & 1;
             d.mat[j] = x[j];
-            d.row[j] = leaf ? x[j] * Ppad : 0;
+            d.row[j] = leaf ? codes.row(x[j]) : 0;
             d.slot[j] = d.kind[j] == SK_STORED ? (int)((word >> PO_DEPTH_SHIFT) & PO_DEPTH) : 0;
             b += leaf ? 1 : ((kid & 0x3ff) < S && (kid >> 10 & 0x3ff) < S ? 2 : W);
         }
@@ -348,10 +348,11 @@ __device__ __forceinline__ void score_steps(MP M, LDS R *PT, LDS uint32_t *steps
 // row) near, a row a lane; the value only keeps the loads.  The rows are read
 // once a call, mostly from HBM, whose latency is longer than the steps a code
 // is loaded ahead.
-__device__ __forceinline__ uint32_t touch_codes(Buf codes, int S, int Ppad, int pb)
+template <bool WIDE>
+__device__ __forceinline__ uint32_t touch_codes(const CodeRows<WIDE> &codes, int S, int pb)
 {
     uint32_t x = 0;
-    for (int r = threadIdx.x & 63; r < S; r += 64) x |= __builtin_amdgcn_raw_buffer_load_b32(codes, r * Ppad + pb, 0, 0);
+    for (int r = threadIdx.x & 63; r < S; r += 64) x |= codes.four(r, pb);
     return x;
 }
 
@@ -359,8 +360,8 @@ __device__ __forceinline__ uint32_t touch_codes(Buf codes, int S, int Ppad, int 
 // sum_j pi_j L_j + exponent * ln 2 over the patterns, or over the sites of
 // the two prefixes by way of a table of the patterns' terms.  FP64; all-gap
 // columns contribute 0.
-template <typename R, int BS, bool AMB>
-__device__ __forceinline__ void score_patterns(MP M, AP A, const PassArgs<R> &a, const ElemDev &E, const double (&pi)[4], char *scratch,
+template <typename R, int BS, bool AMB, bool WIDE>
+__device__ __forceinline__ void score_patterns(MP M, AP A, const PassArgs<R, WIDE> &a, const ElemDev &E, const double (&pi)[4], char *scratch,
                                                int row, int first, int P, LDS double *red, double &s0, double &s1)
 {
     const int tid = threadIdx.x;
@@ -373,7 +374,7 @@ __device__ __forceinline__ void score_patterns(MP M, AP A, const PassArgs<R> &a,
     double acc = 0, acc1 = 0;
     for (int pb = first + uni(tid & ~63); pb < P; pb += BS) {
         const int p = pb + (tid & 63);
-        const uint32_t ahead = pb + BS < P ? touch_codes(a.codes, uni(M->S), E.Ppad, pb + BS) : 0;
+        const uint32_t ahead = pb + BS < P ? touch_codes(a.codes, uni(M->S), pb + BS) : 0;
         const ChildIn<R> o = prune_pattern<R, AMB, SCORE_DEPTH, false>(a, stack, blkB, (uint32_t)p);
         asm volatile("" ::"v"(ahead));
         double t = 0;
@@ -398,7 +399,7 @@ __device__ __forceinline__ void score_patterns(MP M, AP A, const PassArgs<R> &a,
     s0 = block_sum(acc, red);
 }
 
-template <typename R, int BS>
+template <typename R, int BS, bool WIDE = false>
 __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak)
 {
     extern __shared__ __align__(32) char smem_raw[];
@@ -444,23 +445,19 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
         const int32_t *tab = uni_ptr(A->tab_call ? A->tab_call + (size_t)row * tab_words(N) : A->tab + E.off_tab);
         const int root = uni(hdr ? hdr[0] : E.root), n_int = (uni(hdr ? hdr[1] : E.n_nodes) - 1) / 2;
         const int first = uni(item.p0), P = part < 0 ? E.P : uni(item.p1);
-        PassArgs<R> a;
-        a.codes = make_buf(uni_ptr((GBL uint8_t *)(A->codes + E.off_codes)), code_bytes(S, E.Ppad));
-        const uint32_t ahead = first + (tid & ~63) < P ? touch_codes(a.codes, S, E.Ppad, first + (tid & ~63)) : 0;
+        const CodeRows<WIDE> codes(uni_ptr((GBL uint8_t *)(A->codes + E.off_codes)), S, E.Ppad);
+        const uint32_t ahead = first + (tid & ~63) < P ? touch_codes(codes, S, first + (tid & ~63)) : 0;
         score_stage<R, BS>(M, A, PT, tab, n_int, row);
         fetch_eig(A, eig, w, row);
         __syncthreads();
-        score_steps<R, BS>(M, PT, steps, (LDS uint32_t *)&per_sh, n_int, root, E.Ppad);
+        score_steps<R, BS>(M, PT, steps, (LDS uint32_t *)&per_sh, n_int, root, codes);
         __syncthreads();
         // every node's matrix (the root's and absent nodes' are never read)
         for (int i = tid; i < 4 * N; i += BS) work_matrix_row<R>(M, A, eig, PT, *node_len(PT, i >> 2), *node_int(PT, i >> 2), i >> 2, i & 3, row);
         char *scratch = uni_ptr(bo >= 0 ? A->big + bo : A->scratch + (int64_t)blockIdx.x * A->slot_bytes);
         asm volatile("" ::"v"(ahead));
         __syncthreads();
-        a.steps = (const LDS u32x4 *)steps;
-        a.PT = PT;
-        a.n = n_int;
-        a.slots = score_slots(N - S);
+        const PassArgs<R, WIDE> a = {(const LDS u32x4 *)steps, PT, codes, n_int, score_slots(N - S)};
         double s0 = 0, s1 = 0;
         if (E.has_amb) score_patterns<R, BS, true>(M, A, a, E, pi, scratch, row, first, P, (LDS double *)red, s0, s1);
         else score_patterns<R, BS, false>(M, A, a, E, pi, scratch, row, first, P, (LDS double *)red, s0, s1);
@@ -585,9 +582,9 @@ __device__ __forceinline__ void keep_visits(const KeepLds<R> &k, LDS unsigned lo
     }
 }
 
-template <typename R, int BS>
+template <typename R, int BS, bool WIDE>
 __device__ __forceinline__ int keep_steps(const KeepLds<R> &k, const LDS unsigned long long *visit, LDS uint32_t *per, int S, int n_int,
-                                          int Ppad, GBL uint8_t *stale)
+                                          const CodeRows<WIDE> &codes, GBL uint8_t *stale)
 {
     constexpr int W = 4 * sizeof(R) + 4;
     const int lane = threadIdx.x & 63;
@@ -627,7 +624,7 @@ __device__ __forceinline__ int keep_steps(const KeepLds<R> &k, const LDS unsigne
                 d.late = d.late || (!leaf && x[j] == before[2]);
                 d.miss_kid[j] = (k.mark[x[j]] & MK_MISS) ? 1 : 0;
                 d.mat[j] = x[j];
-                d.row[j] = leaf ? x[j] * Ppad : 0;
+                d.row[j] = leaf ? codes.row(x[j]) : 0;
                 d.slot[j] = leaf ? 0 : x[j] - S;
                 b += leaf ? 1 : ((k.mark[x[j]] & MK_CHERRY) ? 2 : W);
             }
@@ -642,8 +639,8 @@ __device__ __forceinline__ int keep_steps(const KeepLds<R> &k, const LDS unsigne
 
 // The pass over an element's blocks and its root sums (see score_patterns;
 // with site prefixes the patterns' terms lie behind the blocks).
-template <typename R, int BS, bool AMB>
-__device__ __forceinline__ void keep_patterns(AP A, const PassArgs<R> &a, const ElemDev &E, const double (&pi)[4], GBL char *blocks,
+template <typename R, int BS, bool AMB, bool WIDE>
+__device__ __forceinline__ void keep_patterns(AP A, const PassArgs<R, WIDE> &a, const ElemDev &E, const double (&pi)[4], GBL char *blocks,
                                               const GBL int32_t *site, int row, LDS double *red, double &s0, double &s1)
 {
     const int tid = threadIdx.x, P = E.P, blkB = block_bytes(a.slots, sizeof(R));
@@ -686,14 +683,14 @@ __device__ __forceinline__ void keep_patterns(AP A, const PassArgs<R> &a, const 
 
 // A node's partial and exponent at pattern p (each lane its own block); a
 // cherry's is recomputed from its leaf codes, as a pass does.
-template <typename R>
-__device__ __forceinline__ ChildIn<R> kept_node(const KeepLds<R> &k, const GBL char *blocks, Buf codes, int S, int I, int Ppad, int v, int p)
+template <typename R, bool WIDE>
+__device__ __forceinline__ ChildIn<R> kept_node(const KeepLds<R> &k, const GBL char *blocks, const CodeRows<WIDE> &codes, int S, int I, int v, int p)
 {
     ChildIn<R> in;
     if (k.mark[v] & MK_CHERRY) {
         const int yA = uni(k.ch0[v]), yB = uni(k.ch1[v]);
         return cherry_in<R>(k.PT + 16 * yA, k.PT + 16 * yB, k.mark[yA] & MK_MISS, k.mark[yB] & MK_MISS,
-                            __builtin_amdgcn_raw_buffer_load_b8(codes, p, yA * Ppad, 0), __builtin_amdgcn_raw_buffer_load_b8(codes, p, yB * Ppad, 0));
+                            codes.at(codes.row(yA), p), codes.at(codes.row(yB), p));
     }
     const GBL char *blk = blocks + (size_t)(p >> 6) * block_bytes(I, sizeof(R));
     in.v = ld4<R>((const GBL V4<R> *)(blk + part_off<R>(v - S)) + (p & 63));
@@ -744,9 +741,9 @@ __device__ __forceinline__ void history_steps(const KeepLds<R> &k, int S, int n_
 // * L over its whole branch (the law of the reference's species-by-species
 // steps), and writes every node's base.  The steps are the chain sampler's:
 // words read ahead, the loads of the next four steps in flight.
-template <typename R, int BS, bool AMB>
-__device__ __forceinline__ void draw_history(MP M, AP A, const KeepLds<R> &k, const GBL char *blocks, Buf codes, const double (&pi)[4],
-                                             const GBL int32_t *site, int row, int n_int, int S, int I, int Ppad)
+template <typename R, int BS, bool AMB, bool WIDE>
+__device__ __forceinline__ void draw_history(MP M, AP A, const KeepLds<R> &k, const GBL char *blocks, const CodeRows<WIDE> &codes,
+                                             const double (&pi)[4], const GBL int32_t *site, int row, int n_int, int S, int I)
 {
     constexpr int K = 4;
     const int tid = threadIdx.x, len = uni(A->hist_len[row]), stride = uni(A->hist_ns[row]);
@@ -771,8 +768,8 @@ __device__ __forceinline__ void draw_history(MP M, AP A, const KeepLds<R> &k, co
             const uint32_t slot = w[j].y >> 20, a = w[j].y & 0x3ff, b = (w[j].y >> 10) & 0x3ff;
             in[j].v = ld4<R>((const GBL V4<R> *)(pp + (uint64_t)part_off<R>(slot)));
             in[j].x = *(const GBL int32_t *)(pe + (uint64_t)(slot * 256));
-            cdA[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, uni((a ? a - 1 : 0) * Ppad), 0);
-            cdB[j] = __builtin_amdgcn_raw_buffer_load_b8(codes, p, uni((b ? b - 1 : 0) * Ppad), 0);
+            cdA[j] = codes.at((uint32_t)uni((int)codes.row(a ? a - 1 : 0)), p);
+            cdB[j] = codes.at((uint32_t)uni((int)codes.row(b ? b - 1 : 0)), p);
         };
         int res = 4, tp = 4;
         auto step = [&](auto J, int t) __attribute__((always_inline)) {
@@ -849,15 +846,15 @@ __device__ inline void full_transition(PE lam, PE V, PE Vi, double d, LDS double
 // pi-average; kind 2, log sum_i pi_i P(d)_{x_b -> i} at b's own base.  The
 // matrices of CAND_CHUNK candidates are built at once, a thread each, and
 // their sums meet once.
-template <typename R, int BS>
+template <typename R, int BS, bool WIDE>
 __device__ __noinline__ void gt_candidates(MP M, AP A, const KeepLds<R> k, const GBL char *blocks_, const GBL uint8_t *codes_,
                                            const GBL int32_t *site, LDS double *Pc, LDS double *red, int w, int row_, int S_, int I_,
                                            int Ppad_, double pi0, double pi1, double pi2, double pi3)
 {
     // arguments of a call come in vector registers
-    const int row = uni(row_), S = uni(S_), I = uni(I_), Ppad = uni(Ppad_);
+    const int row = uni(row_), S = uni(S_), I = uni(I_);
     const GBL char *blocks = uni_ptr(blocks_);
-    const Buf codes = make_buf(uni_ptr(codes_), code_bytes(S, Ppad));
+    const CodeRows<WIDE> codes(uni_ptr(codes_), S, uni(Ppad_));
     const int tid = threadIdx.x, stride = A->hist_ns[row], cm = A->cand_max;
     const GBL int8_t *tg = (const GBL int8_t *)A->hist + A->hist_off[row];
     const int b = uni(A->cand_branch[row]), nc = uni(A->cand_n[row]), len = uni(A->cand_sites[row]);
@@ -891,7 +888,7 @@ __device__ __noinline__ void gt_candidates(MP M, AP A, const KeepLds<R> k, const
                 double L[4];
                 int e = 0;
                 if (b < S) {
-                    const int code = __builtin_amdgcn_raw_buffer_load_b8(codes, p, b * Ppad, 0);
+                    const int code = codes.at(codes.row(b), p);
                     for (int j = 0; j < 4; j++) L[j] = 0;
                     if (code < 4) {
                         for (int j = 0; j < 4; j++) L[j] = j == code ? 1 : 0;
@@ -901,7 +898,7 @@ __device__ __noinline__ void gt_candidates(MP M, AP A, const KeepLds<R> k, const
                         for (int j = 0; j < 4; j++) L[j] = j == b1 || j == b2 ? 1 : 0;
                     }
                 } else {
-                    const ChildIn<R> in = kept_node<R>(k, blocks, codes, S, I, Ppad, b, p);
+                    const ChildIn<R> in = kept_node<R>(k, blocks, codes, S, I, b, p);
                     L[0] = in.v.x; L[1] = in.v.y; L[2] = in.v.z; L[3] = in.v.w;
                     e = in.x;
                 }
@@ -937,7 +934,7 @@ __device__ __noinline__ void gt_candidates(MP M, AP A, const KeepLds<R> k, const
     }
 }
 
-template <typename R, int BS, LoglikUse USE>
+template <typename R, int BS, LoglikUse USE, bool WIDE = false>
 __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(ModelDev Mk, LoglikArgs Ak)
 {
     extern __shared__ __align__(32) char smem_raw[];
@@ -978,7 +975,7 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
         const int root = uni(hdr ? hdr[0] : E.root), n_int = (uni(hdr ? hdr[1] : E.n_nodes) - 1) / 2;
         const int moved = A->path_node ? uni(A->path_node[row]) : -1;
         const bool path = moved >= S && moved < N;
-        const Buf codes = make_buf(uni_ptr((GBL uint8_t *)(A->codes + E.off_codes)), code_bytes(S, E.Ppad));
+        const CodeRows<WIDE> codes(uni_ptr((GBL uint8_t *)(A->codes + E.off_codes)), S, E.Ppad);
         GBL uint8_t *stale = A->stale ? (GBL uint8_t *)(A->stale + (size_t)row * N) : nullptr;
         const int32_t *po = tab + tab_porder(N);
         const double *len = A->len_in ? A->len_in + (size_t)row * N : (const double *)(tab + tab_dist(N));
@@ -1020,7 +1017,7 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
         }
         keep_visits<R, BS>(k, (LDS unsigned long long *)visit, n_int, path);
         __syncthreads();
-        const int n = uni(keep_steps<R, BS>(k, (LDS unsigned long long *)visit, (LDS uint32_t *)&per_sh, S, n_int, E.Ppad, stale));
+        const int n = uni(keep_steps<R, BS>(k, (LDS unsigned long long *)visit, (LDS uint32_t *)&per_sh, S, n_int, codes, stale));
         if constexpr (USE == LoglikUse::History) history_steps<R, BS>(k, S, n_int, root);
         __syncthreads();
         // the matrices of the steps' children
@@ -1031,12 +1028,7 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
         }
         GBL char *blocks = uni_ptr((GBL char *)(bo >= 0 ? A->big + bo : A->scratch + (int64_t)blockIdx.x * A->slot_bytes));
         __syncthreads();
-        PassArgs<R> a;
-        a.steps = (const LDS u32x4 *)k.steps;
-        a.PT = k.PT;
-        a.codes = codes;
-        a.n = n;
-        a.slots = I;
+        const PassArgs<R, WIDE> a = {(const LDS u32x4 *)k.steps, k.PT, codes, n, I};
         const GBL int32_t *site = (const GBL int32_t *)(A->site + E.off_site);
         double s0 = 0, s1 = 0;
         if (E.has_amb) keep_patterns<R, BS, true>(A, a, E, pi, blocks, site, row, (LDS double *)red, s0, s1);
@@ -1044,11 +1036,11 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
         // every wave's partials, before sites read other waves' patterns
         __syncthreads();
         if constexpr (USE == LoglikUse::History) {
-            if (E.has_amb) draw_history<R, BS, true>(M, A, k, blocks, codes, pi, site, row, n_int, S, I, E.Ppad);
-            else draw_history<R, BS, false>(M, A, k, blocks, codes, pi, site, row, n_int, S, I, E.Ppad);
+            if (E.has_amb) draw_history<R, BS, true>(M, A, k, blocks, codes, pi, site, row, n_int, S, I);
+            else draw_history<R, BS, false>(M, A, k, blocks, codes, pi, site, row, n_int, S, I);
         }
         if constexpr (USE == LoglikUse::Candidates)
-            gt_candidates<R, BS>(M, A, k, blocks, (const GBL uint8_t *)(A->codes + E.off_codes), site, (LDS double *)Pc, (LDS double *)red, w, row, S, I, E.Ppad, pi[0], pi[1], pi[2], pi[3]);
+            gt_candidates<R, BS, WIDE>(M, A, k, blocks, (const GBL uint8_t *)(A->codes + E.off_codes), site, (LDS double *)Pc, (LDS double *)red, w, row, S, I, E.Ppad, pi[0], pi[1], pi[2], pi[3]);
         if (tid == 0) {
             A->ll_out[w] = s0;
             if (A->pre_len) A->ll_out2[w] = s1;
@@ -1084,27 +1076,27 @@ hipError_t launch_score_sum(const LoglikArgs &A, const ScoreSplit *splits, int n
 }
 
 
-template <typename R, int BS>
+template <typename R, int BS, bool WIDE = false>
 static hipError_t launch_t(const ModelDev &M, const LoglikArgs &A, int grid, hipStream_t st)
 {
     // dynamic LDS above 64 KB needs the per-kernel limit raised (large trees only)
     if (loglik_use(A) == LoglikUse::Score) {
         const size_t sm = score_smem<R>(M.N) + loglik_eig_bytes(A);
         if (sm > 65536) {
-            const hipError_t err = hipFuncSetAttribute((const void *)score_kernel<R, BS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
+            const hipError_t err = hipFuncSetAttribute((const void *)score_kernel<R, BS, WIDE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
             if (err != hipSuccess) return err;
         }
-        hipLaunchKernelGGL((score_kernel<R, BS>), dim3(grid), dim3(BS), sm, st, M, A);
+        hipLaunchKernelGGL((score_kernel<R, BS, WIDE>), dim3(grid), dim3(BS), sm, st, M, A);
         return hipGetLastError();
     }
     auto keep = [&](auto U) {
         constexpr LoglikUse use = decltype(U)::value;
         const size_t sm = keep_smem<R>(M.N, BS, use == LoglikUse::History) + loglik_eig_bytes(A);
         if (sm > 65536) {
-            const hipError_t err = hipFuncSetAttribute((const void *)keep_kernel<R, BS, use>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
+            const hipError_t err = hipFuncSetAttribute((const void *)keep_kernel<R, BS, use, WIDE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
             if (err != hipSuccess) return err;
         }
-        hipLaunchKernelGGL((keep_kernel<R, BS, use>), dim3(grid), dim3(BS), sm, st, M, A);
+        hipLaunchKernelGGL((keep_kernel<R, BS, use, WIDE>), dim3(grid), dim3(BS), sm, st, M, A);
         return hipGetLastError();
     };
     switch (loglik_use(A)) {
@@ -1151,6 +1143,7 @@ int loglik_blocks_per_cu(int fp64, int BS, int N, LoglikUse use)
 
 hipError_t launch_loglik(const ModelDev &M, const LoglikArgs &A, int fp64, int BS, int grid, hipStream_t st)
 {
+    if (A.wide) return fp64 ? launch_t<double, WIDE_BLOCK, true>(M, A, grid, st) : launch_t<float, WIDE_BLOCK, true>(M, A, grid, st);
     if (fp64) {
         if (BS == 64) return launch_t<double, 64>(M, A, grid, st);
         if (BS == 128) return launch_t<double, 128>(M, A, grid, st);

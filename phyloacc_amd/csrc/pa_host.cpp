@@ -560,6 +560,7 @@ struct pa_engine {
     // scratch array, and the arenas' longest element and mean pattern count
     char *d_noalloc = nullptr;
     int max_ppad = 0;
+    bool wide = false, wide_forced = false;  // LoglikArgs::wide of this engine's launches
     double mean_p = 0;
     std::vector<ElemDev> dev_elems;          // host copy of the uploaded descriptors (tree updates patch both)
     GtHistory hist;                          // gene-node histories of the last history draw (device)
@@ -923,6 +924,7 @@ static pa_status upload(pa_engine *e)
     for (const HostElem &E : e->elems)
         if (!E.filtered) { e->max_ppad = std::max(e->max_ppad, E.Ppad); e->mean_p += E.P; kept++; }
     if (kept) e->mean_p /= (double)kept;
+    e->wide = e->wide_forced || wide_codes(S, e->max_ppad);
     e->dev_elems = std::move(d);
     e->dev_dirty = false;
     e->arena_gen++;
@@ -1109,6 +1111,7 @@ static size_t call_room(pa_engine *e, const int32_t *ids, int n)
 // with twice the partial traffic per lane, is fastest at 256.
 static int loglik_block(pa_engine *e, const int32_t *work, int32_t n, int fp64)
 {
+    if (e->wide) return WIDE_BLOCK;
     if (e->n_cu > 0 && n < 4 * e->n_cu) return 256;
     double meanP = 0;
     for (int i = 0; i < n; i++) meanP += e->n_pat[work[i]];
@@ -1135,6 +1138,7 @@ static int loglik_block(pa_engine *e, const int32_t *work, int32_t n, int fp64)
 // rounds of 16 workgroups a CU.
 static int score_block(pa_engine *e, const int32_t *work, int32_t n, int fp64, bool prefixes)
 {
+    if (e->wide) return WIDE_BLOCK;
     const int cu = std::max(1, e->n_cu);
     if (n < 8 * cu) return 256;
     int64_t total = 0;
@@ -1248,7 +1252,7 @@ static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp6
     if (B.off > e->io_bytes) return fail(e, PA_E_STATE, "call block too small");
     HIPCHK(e, hipMemcpyAsync(e->d_io, e->h_io, in_bytes, hipMemcpyHostToDevice, e->stream));
     A.counters = (unsigned long long *)d_cnt;
-    A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab;
+    A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab; A.wide = e->wide;
     A.n_elems = (int)e->elems.size();
     A.n_work = n;
     A.queue = e->d_queue;
@@ -1376,6 +1380,18 @@ static pa_status check_ids(pa_engine *e, const int32_t *ids, int32_t n)
         if (ids[i] < 0 || ids[i] >= (int)e->elems.size()) return fail(e, PA_E_INPUT, "element id out of range");
         if (e->n_pat[ids[i]] < 0) return fail(e, PA_E_INPUT, "element " + std::to_string(ids[i]) + " is filtered");
     }
+    return PA_OK;
+}
+
+// As check_ids, for calls that run chains: their kernel addresses an
+// element's codes by 32-bit offsets.
+static pa_status check_chain_ids(pa_engine *e, const int32_t *ids, int32_t n)
+{
+    const pa_status st = check_ids(e, ids, n);
+    if (st != PA_OK) return st;
+    for (int i = 0; i < n; i++)
+        if (wide_codes(e->tm.S, ((int64_t)e->n_pat[ids[i]] + 63) / 64 * 64))
+            return fail(e, PA_E_INPUT, "element " + std::to_string(ids[i]) + " is too long for the chains: its leaf codes take 4 GiB or more");
     return PA_OK;
 }
 
@@ -1922,7 +1938,7 @@ pa_status gt_plan_run(pa_engine *e, GtPlan *p, const int32_t *lens0, const int32
         A.ll_out2 = (double *)p->out2.p;
     }
     // the engine's arenas as they are now
-    A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab;
+    A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab; A.wide = e->wide;
     A.n_elems = (int)e->elems.size();
     A.site = e->d_site;
     A.queue = e->d_queue;
@@ -2162,7 +2178,7 @@ extern "C" pa_status pa_loglik_noalloc(pa_engine *e, const int32_t *d_ids, int32
     const int grid = (int)std::min<size_t>({(size_t)n, (size_t)loglik_grid_max(e, fp64, BS, LoglikUse::Score), usable / slot});
     LoglikArgs A;
     memset(&A, 0, sizeof A);
-    A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab;
+    A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab; A.wide = e->wide;
     A.n_elems = (int)e->elems.size();
     A.work = d_ids;
     A.n_work = n;
@@ -2176,6 +2192,13 @@ extern "C" pa_status pa_loglik_noalloc(pa_engine *e, const int32_t *d_ids, int32
     HIPCHK(e, launch_reset(A.queue, st));          // a fill kernel, not a memset: callers may capture the stream
     HIPCHK(e, launch_loglik(e->M, A, fp64, BS, grid, st));
     return PA_OK;
+}
+
+extern "C" int32_t pa_wide_codes(int32_t S, int64_t Ppad) { return wide_codes(S, Ppad); }
+extern "C" void pa_engine_force_wide(pa_engine *e, int32_t on)
+{
+    e->wide_forced = on != 0;
+    e->wide = e->wide_forced || wide_codes(e->tm.S, e->max_ppad);
 }
 
 extern "C" pa_status pa_release_scratch(pa_engine *e)
@@ -2193,7 +2216,7 @@ extern "C" pa_status pa_run_chains(pa_engine *e, const int32_t *ids, int32_t n, 
 {
     if (!e || !ids || !cfg || n < 0) return fail(e, PA_E_INPUT, "null argument");
     if (n == 0) return PA_OK;
-    pa_status st = check_ids(e, ids, n);
+    pa_status st = check_chain_ids(e, ids, n);
     if (st != PA_OK) return st;
     if ((st = upload(e)) != PA_OK) return st;
     HIPCHK(e, hipSetDevice(e->device));
@@ -2314,7 +2337,7 @@ extern "C" pa_status pa_batch_create(pa_engine *e, const int32_t *ids, int32_t n
     if (out) *out = nullptr;
     if (!e || !ids || !cfg || !out || n <= 0) return fail(e, PA_E_INPUT, "null argument or empty batch");
     if (cfg->mode != PA_RUN_BATCHED) return fail(e, PA_E_INPUT, "a prepared batch is one batched launch (PA_RUN_BATCHED)");
-    pa_status st = check_ids(e, ids, n);
+    pa_status st = check_chain_ids(e, ids, n);
     if (st != PA_OK) return st;
     if ((st = upload(e)) != PA_OK) return st;
     HIPCHK(e, hipSetDevice(e->device));
@@ -2637,7 +2660,7 @@ extern "C" pa_status pa_autotune(pa_engine *e, const int32_t *ids, int32_t n, in
                                  int32_t states, pa_tuning *out)
 {
     if (!e || !ids || n <= 0) return fail(e, PA_E_INPUT, "null argument");
-    pa_status st = check_ids(e, ids, n);
+    pa_status st = check_chain_ids(e, ids, n);
     if (st != PA_OK) return st;
     if ((st = upload(e)) != PA_OK) return st;
     if (states <= 1) states = 8;
@@ -2928,7 +2951,7 @@ extern "C" pa_status pa_serve_submit(pa_server *s, const int32_t *ids, int32_t n
 {
     if (!s || (!ids && n > 0) || n < 0) return PA_E_INPUT;
     pa_engine *e = s->e;
-    pa_status st = check_ids(e, ids, n);
+    pa_status st = check_chain_ids(e, ids, n);
     if (st != PA_OK) return st;
     const double now = pa_serve_clock();
     for (int i = 0; i < n; i++) {
@@ -3089,7 +3112,7 @@ static pa_status lane_launch(pa_server *s, Lane &L, bool others_busy)
         HIPCHK(e, hipMemcpyAsync(L.d_llen, L.h_llen, sizeof(double) * (size_t)nl * N, hipMemcpyHostToDevice, L.st));
         LoglikArgs A;
         memset(&A, 0, sizeof A);
-        A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab;
+        A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab; A.wide = e->wide;
         A.n_elems = (int)e->elems.size();
         A.work = L.d_lids; A.n_work = nl; A.queue = L.d_queue;
         A.scratch = base + scr_c; A.slot_bytes = (int64_t)loglik_slot(s);

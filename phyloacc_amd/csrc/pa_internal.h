@@ -93,3 +93,9 @@ pa_status element_set_trees(pa_engine *e, const int32_t *ids, int n, const int32
 pa_status engine_stream(pa_engine *e, hipStream_t *st);
 
 }  // namespace pa
+
+// For tests: whether an element of S species and Ppad padded patterns has wide
+// codes (wide_codes), and an engine whose likelihood launches all go to the
+// kernels for such elements.
+extern "C" int32_t pa_wide_codes(int32_t S, int64_t Ppad);
+extern "C" void pa_engine_force_wide(pa_engine *e, int32_t on);

@@ -34,6 +34,7 @@ struct LoglikArgs {
     int n_work;
     int *queue;               // work counter, reset before each launch
     const uint8_t *codes;     // arenas
+    int wide;                 // some element's codes are beyond a 32-bit offset (wide_codes)
     const int32_t *wts;
     const int32_t *tab;
     int n_elems;              // elements in the arenas: ids outside [0, n_elems) score NaN
@@ -159,6 +160,10 @@ inline LoglikUse loglik_use(const LoglikArgs &A)
 }
 // Workgroups resident on one CU (registers, LDS, launch bound).
 int loglik_blocks_per_cu(int fp64, int BS, int N, LoglikUse use);
+// A launch over arenas with wide codes takes WIDE_BLOCK threads whatever BS
+// says (the one size that such kernels are built for).
+constexpr int WIDE_BLOCK = 256;
+inline bool wide_codes(int S, int64_t Ppad) { return S * Ppad >= (int64_t)1 << 32; }
 hipError_t launch_loglik(const ModelDev &M, const LoglikArgs &A, int fp64, int BS, int grid, hipStream_t st);
 
 // Size of the device scratch array of the allocation-free likelihood entry

@@ -21,11 +21,33 @@ __device__ __forceinline__ Buf make_buf(T *base, int bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc((void *)(T *)base, 0, bytes, 0x00027000);
 }
-__device__ __forceinline__ int code_bytes(int S, int Ppad)
-{
-    const uint64_t n = (uint64_t)S * (uint32_t)Ppad;
-    return (int)(uint32_t)(n < 0xffffffffu ? n : 0xffffffffu);
-}
+
+// An element's leaf codes, S rows of Ppad.  A row's word is what a step keeps
+// of it: its byte offset, which a load takes as it is, or (WIDE) the row's
+// number, for codes of 4 GiB or more, beyond a 32-bit offset.  The kernels
+// that score are built for both (host: wide_codes); the wide ones spend the
+// scalar instructions of a 64-bit address on every load.
+template <bool WIDE>
+struct CodeRows;
+template <>
+struct CodeRows<false> {
+    Buf buf;
+    uint32_t Ppad;
+    __device__ __forceinline__ CodeRows(const GBL uint8_t *base, int S, int P) : buf(make_buf((GBL uint8_t *)base, (int)((uint32_t)S * (uint32_t)P))), Ppad((uint32_t)P) {}
+    __device__ __forceinline__ uint32_t row(int x) const { return (uint32_t)x * Ppad; }
+    __device__ __forceinline__ int at(uint32_t row, uint32_t p) const { return __builtin_amdgcn_raw_buffer_load_b8(buf, p, row, 0); }
+    // four codes of a row, a lane a row
+    __device__ __forceinline__ uint32_t four(int x, uint32_t p) const { return __builtin_amdgcn_raw_buffer_load_b32(buf, (uint32_t)x * Ppad + p, 0, 0); }
+};
+template <>
+struct CodeRows<true> {
+    const GBL uint8_t *base;
+    uint32_t Ppad;
+    __device__ __forceinline__ CodeRows(const GBL uint8_t *b, int S, int P) : base(b), Ppad((uint32_t)P) {}
+    __device__ __forceinline__ uint32_t row(int x) const { return (uint32_t)x; }
+    __device__ __forceinline__ int at(uint32_t row, uint32_t p) const { return base[(uint64_t)row * Ppad + p]; }
+    __device__ __forceinline__ uint32_t four(int x, uint32_t p) const { return *(const GBL uint32_t *)(base + ((uint64_t)(uint32_t)x * Ppad + p)); }
+};
 
 template <int... J, typename F>
 __device__ __forceinline__ void each_of(std::integer_sequence<int, J...>, F &&f) { (f(std::integral_constant<int, J>()), ...); }
@@ -64,7 +86,7 @@ __device__ __forceinline__ void buf_st4(Buf b, const V4<R> &v, uint32_t lane_off
 
 // One step of a pass, an internal node.  Four words:
 //   w0: type | SB_* bits | child A's slot << 14 | the slot the node is stored to << 23
-//   w1, w2: the code row offsets of children A and B (row 0 for a child that is no leaf)
+//   w1, w2: the code rows' words (CodeRows) of children A and B (row 0's, which is 0, for a child that is no leaf)
 //   w3: the children's matrices A | B << 10 (the node's id, + N for a proposal matrix) | child B's slot << 20
 // A child comes from its leaf code (L), its stored partial (S), or the result
 // of the step just before (P) or the one before that (P2), which the thread
@@ -81,7 +103,8 @@ static_assert(MAXN <= 512, "slots (below 2 I <= N) in nine bits, matrices (below
 
 // What a step's words say, the children in any order.
 struct StepDef {
-    int kind[2], miss_kid[2], mat[2], row[2], slot[2];   // SK_* source, missing, matrix, code row offset, stored slot
+    int kind[2], miss_kid[2], mat[2], slot[2];   // SK_* source, missing, matrix, stored slot
+    uint32_t row[2];                             // code row's word
     int slot_to;                                         // where the node is stored
     bool nostore;
     bool late = false;                                   // a stored child is the step three before (F = 4 below)
@@ -104,18 +127,18 @@ __device__ __forceinline__ void encode_step(LDS uint32_t *w, const StepDef &d)
            (d.nostore ? SB_NOSTORE : 0) | (d.late ? SB_LATE : 0) | (ma ? SB_MISS_A : 0) | (mb ? SB_MISS_B : 0) |
            ((uint32_t)ka << SB_KIND_A_SHIFT) | ((uint32_t)kb << SB_KIND_B_SHIFT) |
            ((uint32_t)(a ? d.slot[1] : d.slot[0]) << SB_SLOT_A_SHIFT) | ((uint32_t)d.slot_to << SB_SLOT_SHIFT);
-    w[1] = (uint32_t)(a ? d.row[1] : d.row[0]);
-    w[2] = (uint32_t)(a ? d.row[0] : d.row[1]);
+    w[1] = a ? d.row[1] : d.row[0];
+    w[2] = a ? d.row[0] : d.row[1];
     w[3] = (uint32_t)(a ? d.mat[1] : d.mat[0]) | ((uint32_t)(a ? d.mat[0] : d.mat[1]) << SB_MAT_B_SHIFT) |
            ((uint32_t)(a ? d.slot[0] : d.slot[1]) << SB_SLOT_B_SHIFT);
 }
 
 // The scalar arguments of a pass's pattern loop.
-template <typename R>
+template <typename R, bool WIDE = false>
 struct PassArgs {
     const LDS u32x4 *steps;
     const LDS R *PT;             // [2N][16]: the current matrices, then the proposal's
-    Buf codes;
+    CodeRows<WIDE> codes;
     int n, slots;                // steps; slots of a pattern block
 };
 
@@ -200,8 +223,8 @@ __device__ __forceinline__ ChildIn<R> slot_load(Buf blk, uint32_t slot, uint32_t
 // store.  F = 4 (with D = 4): stored partials are loaded four steps before
 // their use, for lists whose stored partials lie in HBM; a step marked
 // SB_LATE, whose child was stored after that, loads them again.
-template <typename R, bool AMB, int D, bool ALL, int F = 2>
-__device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL char *base, int blk_bytes, uint32_t p)
+template <typename R, bool AMB, int D, bool ALL, int F = 2, bool WIDE>
+__device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R, WIDE> &A, GBL char *base, int blk_bytes, uint32_t p)
 {
     const int n = A.n;
     const uint32_t lane = threadIdx.x & 63;
@@ -224,8 +247,8 @@ __device__ __forceinline__ ChildIn<R> prune_pattern(const PassArgs<R> &A, GBL ch
 #pragma unroll
         for (int i = 0; i < 4; i++) w[j][i] = (uint32_t)uni((int)nw[i]);
         nw = A.steps[k + 1 < n ? k + 1 : n];
-        cdA[j] = __builtin_amdgcn_raw_buffer_load_b8(A.codes, p, w[j][1], 0);
-        cdB[j] = __builtin_amdgcn_raw_buffer_load_b8(A.codes, p, w[j][2], 0);
+        cdA[j] = A.codes.at(w[j][1], p);
+        cdB[j] = A.codes.at(w[j][2], p);
     };
     // the stored partials of the step whose words are set j
     auto fetch_stored = [&](auto J) __attribute__((always_inline)) {

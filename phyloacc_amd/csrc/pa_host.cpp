@@ -549,9 +549,9 @@ struct pa_engine {
     void *d_ll_scratch = nullptr;
     size_t ll_scratch_bytes = 0;
     // a call's inputs and results: a pinned block and a device block of the
-    // same layout (CallBlock)
+    // same layout, which goes on behind it with what only kernels touch (CallBlock)
     char *h_io = nullptr, *d_io = nullptr;
-    size_t io_bytes = 0;
+    size_t io_bytes = 0, d_io_bytes = 0;
     bool io_busy = false;           // a call has started copies and not waited for them
     void *h_tab_stage = nullptr;    // pinned staging of accepted gene trees' node tables
     size_t h_tab_stage_bytes = 0;
@@ -1030,7 +1030,7 @@ static void release_ll_buffers(pa_engine *e)
     (void)hipHostFree(e->h_tab_stage);
     e->d_ll_scratch = e->h_tab_stage = nullptr;
     e->d_io = e->h_io = nullptr;
-    e->ll_scratch_bytes = e->io_bytes = e->h_tab_stage_bytes = 0;
+    e->ll_scratch_bytes = e->io_bytes = e->d_io_bytes = e->h_tab_stage_bytes = 0;
 }
 
 // A likelihood call's inputs and results in the engine's retained blocks:
@@ -1043,22 +1043,32 @@ struct CallBlock {
     size_t off = 0;
     explicit CallBlock(pa_engine *eng) : e(eng) {}
     static size_t up(size_t b) { return (b + 255) & ~(size_t)255; }
-    pa_status reserve(size_t bytes)
+    // Room for a layout of `bytes`, and device-only memory of dev_bytes (dev_only).  Pinning the host's side costs
+    // about as much as copying it, so what the host never reads is not part of the layout.
+    pa_status reserve(size_t bytes, size_t dev_bytes = 0)
     {
         // a call that failed half way may have left copies in flight
         if (e->io_busy) HIPCHK(e, hipStreamSynchronize(e->stream));
         e->io_busy = true;
-        if (bytes <= e->io_bytes) return PA_OK;
-        (void)hipFree(e->d_io);
-        (void)hipHostFree(e->h_io);
-        e->d_io = e->h_io = nullptr;
-        e->io_bytes = 0;
-        bytes = up(bytes + bytes / 4);
-        HIPCHK(e, hipMalloc(&e->d_io, bytes));
-        HIPCHK(e, hipHostMalloc(&e->h_io, bytes));
-        e->io_bytes = bytes;
+        if (bytes > e->io_bytes) {
+            (void)hipHostFree(e->h_io);
+            e->h_io = nullptr;
+            e->io_bytes = 0;
+            bytes = up(bytes + bytes / 4);
+            HIPCHK(e, hipHostMalloc(&e->h_io, bytes));
+            e->io_bytes = bytes;
+        }
+        if (e->io_bytes + up(dev_bytes) > e->d_io_bytes) {
+            (void)hipFree(e->d_io);
+            e->d_io = nullptr;
+            e->d_io_bytes = 0;
+            const size_t all = e->io_bytes + up(dev_bytes + dev_bytes / 4);
+            HIPCHK(e, hipMalloc(&e->d_io, all));
+            e->d_io_bytes = all;
+        }
         return PA_OK;
     }
+    char *dev_only() const { return e->d_io + e->io_bytes; }
     // the next `bytes` of the layout (within what was reserved): host and device addresses
     char *take(size_t bytes, char **dev)
     {
@@ -1445,7 +1455,7 @@ extern "C" pa_status pa_loglik(pa_engine *e, const int32_t *ids, int32_t n, cons
     for (int i = 0; i < n; i++) sorted[i] = ids[order[i]];
     st = run_kernel(e, sorted.data(), n, precision == PA_FP64, A, B, out, nullptr);
     if (st != PA_OK) return st;
-    if (e->ll_scratch_bytes + e->io_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
+    if (e->ll_scratch_bytes + e->d_io_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
     return PA_OK;
 }
 
@@ -1470,15 +1480,15 @@ extern "C" pa_status pa_loglik_gbgc(pa_engine *e, const int32_t *ids, int32_t n,
     const std::vector<int32_t> order = schedule(e, ids, n, PA_RUN_BATCHED);
     const size_t eig_bytes = (size_t)n * GB_CLASSES * GB_EIG_WORDS * 8;
     CallBlock K(e);
-    if ((st = K.reserve(call_room(e, ids, n) + (size_t)n * (8 * N + 24 + 4) + eig_bytes + 2048)) != PA_OK) return st;
+    if ((st = K.reserve(call_room(e, ids, n) + (size_t)n * (8 * N + 24 + 4) + 2048, eig_bytes)) != PA_OK) return st;
     LoglikArgs A;
     memset(&A, 0, sizeof A);
     // the selections first, so that the eigensystems are built while the rest is laid out
     const double *d_sel = K.put(sel, (size_t)n * 3);
     HIPCHK(e, hipMemcpyAsync(e->d_io, e->h_io, K.off, hipMemcpyHostToDevice, e->stream));
-    char *d_eig = e->d_io + e->io_bytes - CallBlock::up(eig_bytes);     // device only, behind the layout
-    HIPCHK(e, launch_gbgc_eig(e->Q0, d_sel, n, (double *)d_eig, e->stream));
-    A.gb_eig = (const double *)d_eig;
+    double *d_eig = (double *)K.dev_only();
+    HIPCHK(e, launch_gbgc_eig(e->Q0, d_sel, n, d_eig, e->stream));
+    A.gb_eig = d_eig;
     A.len_row = K.put(order.data(), n);
     A.Zin = K.put(Z, (size_t)n * N);
     A.Bin = K.put(B, (size_t)n * N);
@@ -1486,7 +1496,7 @@ extern "C" pa_status pa_loglik_gbgc(pa_engine *e, const int32_t *ids, int32_t n,
     for (int i = 0; i < n; i++) sorted[i] = ids[order[i]];
     st = run_kernel(e, sorted.data(), n, precision == PA_FP64, A, K, out, nullptr);
     if (st != PA_OK) return st;
-    if (e->ll_scratch_bytes + e->io_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
+    if (e->ll_scratch_bytes + e->d_io_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
     return PA_OK;
 }
 
@@ -1535,7 +1545,7 @@ static pa_status loglik_lengths_impl(pa_engine *e, const int32_t *ids, int32_t n
     // the lengths go up in the caller's row order; work position w reads row order[w]
     const size_t lbytes = dev_len ? 0 : (size_t)n * N * 8, eig_bytes = piA ? (size_t)n * (GB_EIG_WORDS + 4) * 8 : 0;
     CallBlock B(e);
-    if ((st = B.reserve(call_room(e, ids, n) + lbytes + eig_bytes + (size_t)n * (4 + 8 + 8) + 4096)) != PA_OK) return st;
+    if ((st = B.reserve(call_room(e, ids, n) + lbytes + (size_t)n * (4 + 8 + 8) + 4096, eig_bytes)) != PA_OK) return st;
     LoglikArgs A;
     memset(&A, 0, sizeof A);
     if (piA) {
@@ -1546,7 +1556,7 @@ static pa_status loglik_lengths_impl(pa_engine *e, const int32_t *ids, int32_t n
         double *pw = (double *)B.take((size_t)n * 8, &d);
         for (int i = 0; i < n; i++) pw[i] = piA[order[i]];
         HIPCHK(e, hipMemcpyAsync(e->d_io, e->h_io, B.off, hipMemcpyHostToDevice, e->stream));
-        double *d_eig = (double *)(e->d_io + e->io_bytes - CallBlock::up(eig_bytes));    // device only, behind the layout
+        double *d_eig = (double *)B.dev_only();
         HIPCHK(e, launch_gt_eig(inst, (const double *)d, n, d_eig, d_eig + (size_t)n * GB_EIG_WORDS, e->stream));
         A.el_eig = d_eig;
         A.el_pi = d_eig + (size_t)n * GB_EIG_WORDS;
@@ -1628,7 +1638,7 @@ static pa_status loglik_lengths_impl(pa_engine *e, const int32_t *ids, int32_t n
     if (st != PA_OK) return st;
     if (gx && gx->cand_score)
         HIPCHK(e, hipMemcpy(gx->cand_score, gb[11].p, (size_t)n * gx->cand_max * 8, hipMemcpyDeviceToHost));
-    if (e->ll_scratch_bytes + e->io_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
+    if (e->ll_scratch_bytes + e->d_io_bytes > PA_RETAIN_MAX) release_ll_buffers(e);
     return PA_OK;
 }
 

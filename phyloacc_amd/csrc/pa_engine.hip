@@ -268,11 +268,6 @@ __host__ __device__ inline size_t score_smem(int N)
     return (size_t)16 * N * sizeof(R) + (size_t)16 * (N / 2 + 2);
 }
 
-size_t score_smem_bytes(int N, int fp64)
-{
-    return (fp64 ? score_smem<double>(N) : score_smem<float>(N)) + sizeof(ModelDev) + sizeof(LoglikArgs) + 256;
-}
-
 size_t score_slot_bytes(int N, int S, int BS, int Pcap, int fp64)
 {
     return al((size_t)Pcap * 8, 256) + (size_t)(BS / 64) * block_bytes(score_slots(N - S), fp64 ? 8 : 4);
@@ -499,6 +494,7 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
 enum { MK_PATH = 1, MK_STALE = 2, MK_MISS = 4, MK_CHERRY = 8 };
 
 constexpr int CAND_CHUNK = 16;      // candidates whose matrices are built together
+constexpr int KEEP_CHUNKS = MAXN / 2 / 64;      // masks of 64 positions of the pruning order
 
 template <typename R>
 __host__ __device__ inline size_t keep_smem(int N, int BS, bool history)
@@ -509,10 +505,14 @@ __host__ __device__ inline size_t keep_smem(int N, int BS, bool history)
     return (size_t)16 * N * sizeof(R) + 16 * (I + 1) + al(3 * (size_t)N + 6 * I, 16) + (history ? 8 * (I + 2) + I * BS : 0);
 }
 
-size_t loglik_smem_bytes(int N, int fp64, LoglikUse use)
+// Dynamic and static LDS (the kernels' __shared__ variables) of a workgroup.
+size_t loglik_smem_bytes(int N, int fp64, int BS, LoglikUse use)
 {
-    return (fp64 ? keep_smem<double>(N, 256, false) : keep_smem<float>(N, 256, false)) + sizeof(ModelDev) + sizeof(LoglikArgs) +
-           (use == LoglikUse::Keep ? 0 : CAND_CHUNK * (16 + 4) * 8) + 256;
+    const size_t args = sizeof(ModelDev) + sizeof(LoglikArgs) + 8;
+    if (use == LoglikUse::Score) return (fp64 ? score_smem<double>(N) : score_smem<float>(N)) + args + 4 * 8;
+    const bool history = use == LoglikUse::History;
+    return (fp64 ? keep_smem<double>(N, BS, history) : keep_smem<float>(N, BS, history)) + args + 2 * KEEP_CHUNKS * 8 +
+           CAND_CHUNK * 4 * 8 + (use == LoglikUse::Candidates ? CAND_CHUNK * 16 * 8 : 0);
 }
 
 // Waves per SIMD the kernel is declared for: what holds its registers with few
@@ -558,8 +558,6 @@ __device__ __forceinline__ KeepLds<R> keep_lds(LDS char *base, int N, int S)
 // keep_steps returns the number of steps and adds to per what a pass that
 // stores the nodes it scores (all, or the path's) and reads all their children
 // would move per pattern.
-constexpr int KEEP_CHUNKS = MAXN / 2 / 64;
-
 template <typename R, int BS>
 __device__ __forceinline__ void keep_visits(const KeepLds<R> &k, LDS unsigned long long *visit, int n_int, bool path)
 {

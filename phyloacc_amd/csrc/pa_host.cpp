@@ -973,8 +973,7 @@ static int chain_grid_max(pa_engine *e, int fp64, int BS, int shape)
 static int loglik_grid_max(pa_engine *e, int fp64, int BS, LoglikUse use, int most = 8, size_t eig = 0)
 {
     const int N = e->tm.N;
-    return e->n_cu * fit_per_cu(e, (use == LoglikUse::Score ? score_smem_bytes(N, fp64) : loglik_smem_bytes(N, fp64, use)) + eig, BS,
-                                loglik_blocks_per_cu(fp64, BS, N, use), most);
+    return e->n_cu * fit_per_cu(e, loglik_smem_bytes(N, fp64, BS, use) + eig, BS, loglik_blocks_per_cu(fp64, BS, N, use), most);
 }
 
 // Scratch of one persistent launch of `grid` workgroups over elements of
@@ -1157,7 +1156,7 @@ static int score_block(pa_engine *e, const int32_t *work, int32_t n, int fp64, b
         total += e->n_pat[work[i]];
         longest = std::max(longest, (int)e->n_pat[work[i]]);
     }
-    if (total > (int64_t)600 * n || 8 * score_smem_bytes(e->tm.N, fp64) > e->lds_per_cu) return 256;
+    if (total > (int64_t)600 * n || 8 * loglik_smem_bytes(e->tm.N, fp64, 128, LoglikUse::Score) > e->lds_per_cu) return 256;
     if (prefixes && longest > total / (8 * cu)) return 256;
     return total <= (int64_t)160 * n && n > 64 * cu ? 64 : 128;
 }
@@ -1200,11 +1199,11 @@ static int split_elements(pa_engine *e, const int32_t *ids, int n, int BS, std::
 static pa_status run_kernel(pa_engine *e, const int32_t *ids, int32_t n, int fp64, LoglikArgs &A, CallBlock &B, double *res0, double *res1)
 {
     const int S = e->tm.S, N = e->tm.N;
-    const size_t smem = loglik_smem_bytes(N, fp64);
-    if (smem > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
     const LoglikUse use = loglik_use(A);
     const bool scores = use == LoglikUse::Score;
     const int BS = scores ? score_block(e, ids, n, fp64, A.pre_len != nullptr) : loglik_block(e, ids, n, fp64);
+    const size_t smem = loglik_smem_bytes(N, fp64, BS, use) + loglik_eig_bytes(A);
+    if (smem > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
     // a scoring workgroup's slot is small, so as many run as registers and LDS
     // allow (16 of 64 threads a CU)
     const int grid_max = loglik_grid_max(e, fp64, BS, use, scores ? 16 : 8, loglik_eig_bytes(A));
@@ -1852,6 +1851,7 @@ pa_status gt_launch(pa_engine *e, const int32_t *ids, int32_t n, const double *l
 // device; a run uploads the prefix lengths and launches, without waiting.
 struct GtPlan {
     int n = 0, fp64 = 0, BS = 0, grid = 0;
+    size_t lds = 0;
     std::vector<int32_t> pl;          // prefix lengths staged for the last run
     std::vector<int32_t> GG;          // sites per row
     DevBuf work, row, bo, pre, out, out2, eig, pi, cnt;
@@ -1880,7 +1880,8 @@ pa_status gt_plan_build(pa_engine *e, const int32_t *ids, int32_t n, const doubl
         p->GG[i] = e->elems[ids[i]].GG;
     }
     p->BS = loglik_block(e, sorted.data(), n, fp64);
-    if (loglik_smem_bytes(N, fp64) > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
+    p->lds = loglik_smem_bytes(N, fp64, p->BS, LoglikUse::Keep) + (piA ? GB_EIG_WORDS * 8 : 0);
+    if (p->lds > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
     p->grid = std::min(n, loglik_grid_max(e, fp64, p->BS, LoglikUse::Keep));
     HIPCHK(e, hipMalloc(&p->work.p, (size_t)n * 4));
     HIPCHK(e, hipMalloc(&p->row.p, (size_t)n * 4));
@@ -1960,7 +1961,7 @@ pa_status gt_plan_run(pa_engine *e, GtPlan *p, const int32_t *lens0, const int32
     HIPCHK(e, hipEventRecord(e->ll_t1, e->stream));
     e->ll_stats.grid = p->grid;
     e->ll_stats.block_threads = p->BS;
-    e->ll_stats.lds_bytes = (int32_t)loglik_smem_bytes(e->tm.N, p->fp64);
+    e->ll_stats.lds_bytes = (int32_t)p->lds;
     e->ll_stats.n_launches = 1;
     e->ll_stats.scratch_bytes = 0;
     return PA_OK;
@@ -2176,9 +2177,8 @@ extern "C" pa_status pa_loglik_noalloc(pa_engine *e, const int32_t *d_ids, int32
     if (n == 0) return PA_OK;
     HIPCHK(e, hipSetDevice(e->device));
     const int S = e->tm.S, N = e->tm.N, fp64 = precision == PA_FP64;
-    const size_t smem = loglik_smem_bytes(N, fp64);
-    if (smem > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
     const int BS = (e->mean_p <= 96) ? 64 : (e->mean_p <= 320 ? 128 : 256);
+    if (loglik_smem_bytes(N, fp64, BS, LoglikUse::Score) > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
     const size_t slot = loglik_slot_bytes(N, S, std::max(64, e->max_ppad), fp64);
     const size_t usable = NOALLOC_SCRATCH_BYTES - 256;
     if (slot > usable)
@@ -2941,7 +2941,7 @@ extern "C" pa_status pa_serve_create(pa_engine *e, const pa_serve_config *cfg, p
     s->shape = e->tune.shape;
     if (s->BS != 64 && s->BS != 128 && s->BS != 256) return fail(e, PA_E_INPUT, "block_threads must be 64, 128 or 256");
     const int N = e->tm.N, S = e->tm.S;
-    if (chain::chain_smem_bytes(N, S, s->BS, s->fp64) > e->lds_per_cu || loglik_smem_bytes(N, s->fp64) > e->lds_per_cu)
+    if (chain::chain_smem_bytes(N, S, s->BS, s->fp64) > e->lds_per_cu || loglik_smem_bytes(N, s->fp64, s->BS, LoglikUse::Score) > e->lds_per_cu)
         return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
     s->max_chains = cfg->max_chains > 0 ? cfg->max_chains : 4096;
     s->pool_bytes = cfg->hbm_budget_bytes > 0 ? (size_t)cfg->hbm_budget_bytes : ((size_t)4 << 30);

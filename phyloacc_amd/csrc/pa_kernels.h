@@ -137,8 +137,8 @@ hipError_t launch_gt_eig(const double *inst /*[6], host*/, const double *piA /*[
 // What a launch is for: log-likelihoods alone; resident partials; candidate
 // scores; a history draw.
 enum class LoglikUse { Score, Keep, Candidates, History };
-// LDS bytes of one workgroup (dynamic arrays + context + argument blocks).
-size_t loglik_smem_bytes(int N, int fp64, LoglikUse use = LoglikUse::Candidates);
+// LDS bytes of one workgroup of BS threads, without the eigensystems of loglik_eig_bytes.
+size_t loglik_smem_bytes(int N, int fp64, int BS, LoglikUse use);
 // Bytes of one workgroup's HBM slot for elements of up to Pcap (padded)
 // patterns: the partials (4 values each) and exponents of every internal node.
 size_t loglik_slot_bytes(int N, int S, int Pcap, int fp64);
@@ -149,10 +149,7 @@ size_t loglik_resident_bytes(int N, int S, int Ppad, int fp64);
 // (Pcap 0: none).  Never more than loglik_slot_bytes of the element's own
 // padded patterns, so a launch with such slots can score too.
 size_t score_slot_bytes(int N, int S, int BS, int Pcap, int fp64);
-// LDS bytes of one workgroup of a launch that only scores (no histories,
-// candidate scores or resident partials).
-size_t score_smem_bytes(int N, int fp64);
-// And the LDS of a launch whose work positions have eigensystems of their own.
+// LDS of the eigensystems of a launch whose work positions have their own.
 size_t loglik_eig_bytes(const LoglikArgs &A);
 inline LoglikUse loglik_use(const LoglikArgs &A)
 {

@@ -478,7 +478,8 @@ void pa_batch_destroy(pa_batch *b);
  * count) and the pattern-loop shape 0..PA_N_SHAPES-1, a pair (U nodes
  * pruned per round, K nodes per ancestral-sampling chunk): FP32 (2, 4),
  * (1, 4), (2, 8); FP64 (1, 2), (2, 2), (1, 4).  A pruning pass has no rounds
- * any more, so U is reported and changes nothing.  Neither changes any result
+ * any more, so U is reported and changes nothing: shape 1 is accepted and is
+ * shape 0's kernel.  Neither changes any result
  * (each chain is one workgroup's, and the shapes only regroup independent
  * loads).  round_nodes / chunk_nodes report U and K of the shape at the
  * precision the autotuner ran; rate: the element-MCMC iterations/s it
@@ -492,7 +493,7 @@ typedef struct {
 
 pa_status pa_set_tuning(pa_engine *e, const pa_tuning *t);
 pa_status pa_get_tuning(pa_engine *e, pa_tuning *t);
-/* Times every block size (64, 128, 256) and shape on the batch (or, with
+/* Times every block size (64, 128, 256) and shape (0 and 2) on the batch (or, with
  * sample > 0, on `sample` of its elements evenly spaced by pattern count)
  * with chains of `states` states (0: 8), times the three fastest again twice
  * at 2 * states and keeps the best of those (rate: its iterations per second

@@ -50,11 +50,11 @@ size_t chain_smem_bytes(int N, int S, int BS, int fp64);
 size_t chain_dyn_smem_bytes(int N, int S, int BS, int fp64);
 // Workgroups of the chain kernel resident on one CU (registers, LDS, launch bound).
 int chain_blocks_per_cu(int fp64, int BS, int N, int S, int shape = 0);
-// Pattern-loop shapes of the chain kernel (nodes per pruning round, nodes
-// per sampling chunk), 0 = the default; see Shape in pa_chain.hip.
+// Shapes of the chain kernel's sampler, 0 = the default, 1 the same kernel;
+// see Shape in pa_chain.hip.
 constexpr int N_SHAPES = 3;
-// Partials and exponents of one element of Ppad padded patterns: two buffers
-// per internal node; the exponents start at chain_exps_off.
+// Partials and exponents of one element of Ppad padded patterns, two slots per
+// internal node, by block of 64 patterns (block_bytes in pa_prune.h).
 size_t chain_part_bytes(int N, int S, int Ppad, int fp64);
 // Byte layout of one workgroup's HBM slot whose partial region holds elements
 // of up to Pcap (padded) patterns: off = {plin, logt, amb, parts}; returns its size.

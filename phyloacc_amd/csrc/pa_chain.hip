@@ -260,18 +260,17 @@ enum { KD_LEAF = 0, KD_STORED = 1, KD_CHERRY = 2 };
 enum { DB_KIND1_SHIFT = 2, DB_MISS0 = 1 << 4, DB_MISS1 = 1 << 5, DB_MISS_A0 = 1 << 6, DB_MISS_B0 = 1 << 7,
        DB_MISS_A1 = 1 << 8, DB_MISS_B1 = 1 << 9, DB_MISS = 1 << 10 };
 
-// Pattern-loop shapes the autotuner picks among.  U: patterns a thread takes
-// through a pass together (they share each step's matrices); K: internal
-// nodes whose partials one sampling chunk loads before drawing.  Shape 0 is
-// the default: two patterns in FP32 and one in FP64 fit the 128-register
-// budget of the chain kernel.
+// Shapes of the sampler's loop.  K: internal nodes whose partials and codes
+// are in flight at a time.  FP64 has half FP32's, its partials taking twice
+// the registers.  Shape 2 doubles K and was slower where it was measured: 373
+// against 355 ms for 50,000 elements of 43 species in FP32.  Shape 1 is shape
+// 0: they differed in how many nodes a pass pruned together, and a pass now
+// takes one node at a time.
 template <typename R, int SH>
 struct Shape;
 template <> struct Shape<float, 0> { static constexpr int K = 4; };
-template <> struct Shape<float, 1> { static constexpr int K = 4; };
 template <> struct Shape<float, 2> { static constexpr int K = 8; };
 template <> struct Shape<double, 0> { static constexpr int K = 2; };
-template <> struct Shape<double, 1> { static constexpr int K = 2; };
 template <> struct Shape<double, 2> { static constexpr int K = 4; };
 
 // The steps of a pass, written by one wave: a ballot per 64 internal nodes
@@ -1404,7 +1403,6 @@ static auto by_block(int BS, F &&f) -> decltype(f(std::integral_constant<int, 64
 template <typename R, typename F>
 static auto by_shape(int shape, F &&f) -> decltype(f(std::integral_constant<int, 0>()))
 {
-    if (shape == 1) return f(std::integral_constant<int, 1>());
     if (shape == 2) return f(std::integral_constant<int, 2>());
     return f(std::integral_constant<int, 0>());
 }

@@ -2637,7 +2637,7 @@ extern "C" pa_status pa_chain_summary(pa_engine *e, int32_t id, int32_t model, c
 
 // ------------------------------------------------------------- autotuner
 //
-// Batched chain launches use one block size and one pattern-loop shape.
+// Batched chain launches use one block size and one shape of the sampler's loop.
 // pa_autotune times each pair on the batch itself with short chains and
 // keeps the fastest for later calls with block_threads = 0.
 
@@ -2713,12 +2713,13 @@ extern "C" pa_status pa_autotune(pa_engine *e, const int32_t *ids, int32_t n, in
         if (r == PA_OK) *rate = (double)m * 3 * (T - 1) / (rs.elapsed_ms / 1e3);
         return r;
     };
-    // every (block, shape) once, then the three fastest again at twice the
-    // chain length, twice each, keeping each one's better time: neighbours
-    // that differ by a percent or two are then told apart reliably
+    // every block size and shape once (shape 1 is shape 0's kernel), then the
+    // three fastest again at twice the chain length, twice each, keeping each
+    // one's better time: neighbours that differ by a percent or two are then
+    // told apart reliably
     std::vector<std::pair<double, std::pair<int, int>>> first;
     for (int a = 0; a < 3 && st == PA_OK; a++)
-        for (int sh = 0; sh < chain::N_SHAPES && st == PA_OK; sh++) {
+        for (int sh = 0; sh < chain::N_SHAPES && st == PA_OK; sh += 2) {
             double rate = 0;
             if ((st = time_one(cand[a], sh, states, &rate)) == PA_OK) first.push_back({rate, {cand[a], sh}});
         }

@@ -570,7 +570,7 @@ class Engine:
         return d
 
     def autotune(self, ids, precision=PA_FP32, sample=0, states=8):
-        """Time every block size (64/128/256) and pattern-loop shape on the
+        """Time every block size (64/128/256) and sampler shape (0 and 2) on the
         batch (sample > 0: on that many elements evenly spaced by pattern
         count) with short chains; the fastest pair is kept for
         run_chains(block_threads=0) and Batch(block_threads=0)."""

@@ -46,8 +46,6 @@ struct ChainArgs {
 
 // LDS bytes of one workgroup (dynamic arrays + context + model constants).
 size_t chain_smem_bytes(int N, int S, int BS, int fp64);
-// Dynamic LDS bytes of one workgroup (the launch's dynamic allocation).
-size_t chain_dyn_smem_bytes(int N, int S, int BS, int fp64);
 // Workgroups of the chain kernel resident on one CU (registers, LDS, launch bound).
 int chain_blocks_per_cu(int fp64, int BS, int N, int S, int shape = 0);
 // Shapes of the chain kernel's sampler, 0 = the default, 1 the same kernel;

@@ -48,7 +48,7 @@ namespace chain {
 template <typename R>
 struct Ctx {
     // element
-    int S, N, I, GG, P, Ppad, root, n_nodes, n_int, n_up, n_down, has_amb;
+    int S, N, I, GG, P, Ppad, root, n_nodes, n_int, n_up, has_amb;
     const GBL uint8_t *codes;
     const GBL int32_t *wts, *site;
     // workgroup scratch in HBM
@@ -60,7 +60,7 @@ struct Ctx {
     // LDS arrays
     LDS int16_t *par, *nodes, *inodes, *porder, *upoff;
     LDS uint32_t *urec;    // [I] internal nodes by level: node | child 0 << 10 | child 1 << 20
-    LDS uint32_t *desc;    // [I][4] static pruning descriptor of each internal node (node_desc)
+    LDS uint32_t *desc;    // [I] static pruning descriptor of each internal node (node_desc)
     LDS uint32_t *steps;   // [I + 1][4] the steps of a pass (build_steps)
     LDS uint32_t *srec;    // [I + 1][2] the steps of the sampler (sample_steps)
     LDS uint8_t *flags, *fixZ, *dirty, *cur, *changed;
@@ -126,9 +126,7 @@ __host__ __device__ size_t smem_arrays(int N, int S, int BS, LDS char *base, CP<
         }
         o += szA;
     }
-    o = al(o, 16);      // descriptors are read as 16-byte vectors
-    if constexpr (BIND) c->desc = (LDS uint32_t *)(base + o);
-    o += (size_t)16 * (I > 0 ? I : 1);
+    PA_TAKE(desc, uint32_t, I > 0 ? I : 1);
     o = al(o, 8);       // sampler steps as 8-byte vectors
     PA_TAKE(srec, uint32_t, 2 * (I + 1));
     PA_TAKE(urec, uint32_t, I > 0 ? I : 1);
@@ -146,11 +144,6 @@ __host__ __device__ size_t smem_arrays(int N, int S, int BS, LDS char *base, CP<
     PA_TAKE(maxZ, int8_t, N);
 #undef PA_TAKE
     return al(o, 16);
-}
-
-size_t chain_dyn_smem_bytes(int N, int S, int BS, int fp64)
-{
-    return fp64 ? smem_arrays<double, false>(N, S, BS, nullptr, nullptr) : smem_arrays<float, false>(N, S, BS, nullptr, nullptr);
 }
 
 size_t chain_smem_bytes(int N, int S, int BS, int fp64)
@@ -253,12 +246,9 @@ enum { PR_FULL = 0, PR_DIRTY = 1, PR_PROP = 2 };
 enum { KD_LEAF = 0, KD_STORED = 1, KD_CHERRY = 2 };
 
 // Static pruning descriptor of an internal node, built when the element is
-// bound (node_desc): word 0 = its children x0 | x1 << 16; words 1 and 2 = the
-// two leaves of x0 (resp. x1) when that child is a cherry, yA | yB << 16;
-// word 3 = DB_* bits: each child's kind (KD_LEAF / KD_STORED / KD_CHERRY),
-// which children and cherry leaves are missing, and whether the node is.
-enum { DB_KIND1_SHIFT = 2, DB_MISS0 = 1 << 4, DB_MISS1 = 1 << 5, DB_MISS_A0 = 1 << 6, DB_MISS_B0 = 1 << 7,
-       DB_MISS_A1 = 1 << 8, DB_MISS_B1 = 1 << 9, DB_MISS = 1 << 10 };
+// bound (node_desc): its children x0 | x1 << 10 and DB_* bits: each child's
+// kind (KD_LEAF / KD_STORED / KD_CHERRY) and whether it is missing.
+enum { DB_KID = 0x3ff, DB_KID1_SHIFT = 10, DB_KIND0_SHIFT = 20, DB_KIND1_SHIFT = 22, DB_MISS0 = 1 << 24, DB_MISS1 = 1 << 25 };
 
 // Shapes of the sampler's loop.  K: internal nodes whose partials and codes
 // are in flight at a time.  FP64 has half FP32's, its partials taking twice
@@ -308,16 +298,15 @@ __device__ __forceinline__ void build_steps(CP<R> c, int mode, int cls)
         const int s1 = __shfl(s, l1 < 0 ? 0 : l1, 64), s2 = __shfl(s, l2 < 0 ? 0 : l2, 64);
         const int n1 = l1 >= 0 ? s1 : last1, n2 = l2 >= 0 ? s2 : (l1 >= 0 ? last1 : last2);
         if (v) {
-            const LDS uint32_t *dd = desc + 4 * (s - S);
-            const uint32_t d0 = dd[0], d3 = dd[3];
+            const uint32_t dd = desc[s - S];
             int kind[2], miss[2], m[2], slot[2] = {0, 0};
             uint32_t row[2] = {0, 0};
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                const int x = j ? (int)(d0 >> 16) : (int)(d0 & 0xffff);
-                const int k = j ? (d3 >> DB_KIND1_SHIFT) & 3 : d3 & 3;
+                const int x = (dd >> (j ? DB_KID1_SHIFT : 0)) & DB_KID;
+                const int k = (dd >> (j ? DB_KIND1_SHIFT : DB_KIND0_SHIFT)) & 3;
                 m[j] = x + ((prop && Z[x] == cls) ? N : 0);
-                miss[j] = (d3 & (j ? DB_MISS1 : DB_MISS0)) ? 1 : 0;
+                miss[j] = (dd & (j ? DB_MISS1 : DB_MISS0)) ? 1 : 0;
                 if (k == KD_LEAF) {
                     kind[j] = SK_LEAF;
                     row[j] = (uint32_t)x * (uint32_t)Ppad;
@@ -572,8 +561,8 @@ __device__ __noinline__ void sample_steps(CP<R> c)
     const int S = c->S, n_int = c->n_int;
     for (int t = threadIdx.x; t < n_int; t += BS) {
         const int s = c->inodes[n_int - 1 - t];
-        const LDS uint32_t *dd = c->desc + 4 * (s - S);
-        const int x0 = dd[0] & 0xffff, x1 = dd[0] >> 16;
+        const uint32_t dd = c->desc[s - S];
+        const int x0 = dd & DB_KID, x1 = (dd >> DB_KID1_SHIFT) & DB_KID;
         const int f = c->flags[s], f0 = c->flags[x0], f1 = c->flags[x1];
         uint32_t w0 = (uint32_t)s | ((f & NF_MISSING) ? SR_MISS : 0) | ((f & NF_CHERRY) ? SR_CHERRY : 0), w1 = 0;
         if (t > 0) {
@@ -1098,35 +1087,18 @@ __device__ __forceinline__ bool is_cherry(const int32_t *tab, int N, int S, int 
     return x >= S && x != root && tab[tab_ch0(N) + x] < S && tab[tab_ch1(N) + x] < S;
 }
 
-// The static pruning descriptor of internal node s (layout at DB_*): its
-// children, each child's kind and missing bit, a cherry child's two leaves
-// and their missing bits, and the node's own missing bit.
-__device__ __noinline__ void node_desc(LDS uint32_t *d, const int32_t *tab, int N, int S, int root, int s)
+// The static pruning descriptor of internal node s (layout at DB_*).
+__device__ __forceinline__ uint32_t node_desc(const int32_t *tab, int N, int S, int root, int s)
 {
-    const int32_t *ch0 = tab + tab_ch0(N), *ch1 = tab + tab_ch1(N), *fl = tab + tab_flags(N);
-    const int x[2] = {ch0[s], ch1[s]};
-    uint32_t w[2] = {0, 0};
-    uint32_t bits = (fl[s] & NF_MISSING) ? DB_MISS : 0;
+    const int x[2] = {tab[tab_ch0(N) + s], tab[tab_ch1(N) + s]};
+    uint32_t d = 0;
     for (int j = 0; j < 2; j++) {
-        const int xj = x[j];
-        if (xj < 0) continue;
-        int kind = KD_STORED;
-        if (xj < S) {
-            kind = KD_LEAF;
-        } else if (is_cherry(tab, N, S, root, xj)) {
-            kind = KD_CHERRY;
-            const int yA = ch0[xj], yB = ch1[xj];
-            w[j] = (uint32_t)yA | ((uint32_t)yB << 16);
-            if (fl[yA] & NF_MISSING) bits |= j ? DB_MISS_A1 : DB_MISS_A0;
-            if (fl[yB] & NF_MISSING) bits |= j ? DB_MISS_B1 : DB_MISS_B0;
-        }
-        bits |= (uint32_t)kind << (j ? DB_KIND1_SHIFT : 0);
-        if (fl[xj] & NF_MISSING) bits |= j ? DB_MISS1 : DB_MISS0;
+        if (x[j] < 0) continue;
+        const int kind = x[j] < S ? KD_LEAF : (is_cherry(tab, N, S, root, x[j]) ? KD_CHERRY : KD_STORED);
+        d |= (uint32_t)x[j] << (j ? DB_KID1_SHIFT : 0) | (uint32_t)kind << (j ? DB_KIND1_SHIFT : DB_KIND0_SHIFT);
+        if (tab[tab_flags(N) + x[j]] & NF_MISSING) d |= j ? DB_MISS1 : DB_MISS0;
     }
-    d[0] = (uint32_t)(x[0] < 0 ? 0 : x[0]) | ((uint32_t)(x[1] < 0 ? 0 : x[1]) << 16);
-    d[1] = w[0];
-    d[2] = w[1];
-    d[3] = bits;
+    return d;
 }
 
 template <typename R, int BS, int SH>
@@ -1137,7 +1109,7 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
     if (tid == 0) {
         c->S = M->S; c->N = N; c->I = M->I;
         c->GG = E.GG; c->P = E.P; c->Ppad = E.Ppad; c->root = E.root;
-        c->n_nodes = E.n_nodes; c->n_int = E.n_int; c->n_up = E.n_up; c->n_down = E.n_down; c->has_amb = E.has_amb;
+        c->n_nodes = E.n_nodes; c->n_int = E.n_int; c->n_up = E.n_up; c->has_amb = E.has_amb;
         c->codes = (const GBL uint8_t *)(A->codes + E.off_codes);
         c->wts = (const GBL int32_t *)(A->wts + E.off_w);
         c->site = (const GBL int32_t *)(A->site + E.off_site);
@@ -1170,7 +1142,7 @@ __device__ __noinline__ void bind_element(MP M, CP<R> c, const ChainArgs *A, int
         const int v = tab[tab_up(N) + q];
         c->urec[q] = (uint32_t)v | ((uint32_t)tab[tab_ch0(N) + v] << 10) | ((uint32_t)tab[tab_ch1(N) + v] << 20);
     }
-    for (int s = M->S + tid; s < N; s += BS) node_desc(c->desc + 4 * (s - M->S), tab, N, M->S, E.root, s);
+    for (int s = M->S + tid; s < N; s += BS) c->desc[s - M->S] = node_desc(tab, N, M->S, E.root, s);
     __syncthreads();
     sample_steps<R, BS>(c);
     // null-rate tables (rate 1), fixed for the element

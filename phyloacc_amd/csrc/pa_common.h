@@ -42,8 +42,8 @@ struct ModelDev {
 // Per-element descriptor.  Offsets index the engine's arenas.
 struct ElemDev {
     int GG, P, Ppad, root;
-    int n_nodes, n_int, n_up, n_down;   // n_up / n_down: number of levels
-    int has_amb, pad0, pad1, pad2;
+    int n_nodes, n_int, n_up;   // n_up: number of height levels
+    int has_amb;
     int64_t off_codes;   // uint8 [S][Ppad] leaf codes, pattern index fastest
     int64_t off_w;       // int32 [P] pattern weights
     int64_t off_site;    // int32 [GG] site -> pattern
@@ -52,13 +52,11 @@ struct ElemDev {
 
 // Node table layout (int32 words, per element; N = model N).
 //   ch0[N] ch1[N] par[N] flags[N] nodes[N] internal[N]
-//   up[N] up_off[N+1] down[N] down_off[N+1] tz[N] porder[N/2+1] dist2 (double, 2N words)
+//   up[N] up_off[N+1] porder[N/2+1] dist2 (double, 2N words)
 //   up: internal nodes of the element's tree by height (1, 2, ...);
 //       level h occupies up[up_off[h-1] .. up_off[h]).
-//   down: non-root nodes by depth (1, 2, ...), same convention.
 //   porder: the internal nodes in pruning order (post-order, the child with the
 //       larger subtree first, child 0 on ties), PO_* words.
-//   tz[s]: position of node s in the reverse post-order (root = 0), the Z-update draw slot.
 PA_TAB int tab_ch0(int N) { return 0; }
 PA_TAB int tab_ch1(int N) { return N; }
 PA_TAB int tab_par(int N) { return 2 * N; }
@@ -67,10 +65,7 @@ PA_TAB int tab_nodes(int N) { return 4 * N; }
 PA_TAB int tab_int(int N) { return 5 * N; }
 PA_TAB int tab_up(int N) { return 6 * N; }
 PA_TAB int tab_upoff(int N) { return 7 * N; }
-PA_TAB int tab_down(int N) { return 8 * N + 1; }
-PA_TAB int tab_downoff(int N) { return 9 * N + 1; }
-PA_TAB int tab_tz(int N) { return 10 * N + 2; }
-PA_TAB int tab_porder(int N) { return 11 * N + 2; }
+PA_TAB int tab_porder(int N) { return 8 * N + 1; }
 // behind everything the tree's shape decides, so that a new tree's table can
 // replace what lies before the lengths
 PA_TAB int tab_dist(int N) { return (tab_porder(N) + N / 2 + 2) & ~1; }   // even -> 8-byte aligned doubles

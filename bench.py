@@ -197,10 +197,11 @@ def main():
         blocks["reference_chain"] = reference_chain(E, w, keep, eng, rng)
         blocks["config2"] = config2_block(E, synth, args.seed)
         blocks["config4"] = serve(args, E, synth, None, 2000.0, 2000, args.lanes)
-        blocks["config5"] = gene_trees_block(
-            E, gt_w, traffic=measured_traffic(args, None, f"config=5 elements={gt_w.C} seed={args.seed} precision=fp32")[0])
+        key = f"config=5 elements={gt_w.C} seed={args.seed} precision=fp32"
+        blocks["config5"] = gene_trees_block(E, gt_w, traffic=measured_traffic(args, None, key)[0])
         if args.gt_sweeps > 0:
-            blocks["config5"]["gene_tree_moves"] = gt_moves_block(E, gt_w, args.gt_sweeps)
+            blocks["config5"]["gene_tree_moves"] = gt_moves_block(E, gt_w, args.gt_sweeps,
+                                                                  traffic=measured_traffic(args, None, key + " height moves")[0])
         del gt_w
         for k, v in blocks.items():
             log(f"{k}: {v}")
@@ -502,6 +503,16 @@ def measured_traffic(args, n_elements, key=None):
     return None, None
 
 
+def measured_rate(bound, traffic, ms):
+    """Roofline fields of a kernel whose passes keep partials on chip: the
+    counted bytes are those of a pass that stores every node it scores, which
+    it does not move, so the rate is of the measured traffic (None where no
+    summary covers the workload)."""
+    gbs = None if traffic is None else traffic / (ms * 1e-3) / 1e9
+    return {"bound": bound, "achieved": None if gbs is None else round(gbs, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": None if gbs is None else round(gbs / HBM_PEAK_GBS, 5), "traffic": traffic}
+
+
 def copy_probe(args):
     """A device-to-device copy of known size (a plain copy kernel), for
     scaling the HBM byte counters of a profiler run: FETCH_SIZE and
@@ -600,16 +611,18 @@ def gene_trees(args, E, synth):
     """Config 5 alone: the gene-tree block as a JSON line of its own."""
     from phyloacc_amd import synth as _s
     w = make_gt(_s, args.seed, args.elements or 20000, args.gt_cache)
-    tr, _ = measured_traffic(args, None, f"config=5 elements={w.C} seed={args.seed} precision={args.precision}")
+    key = f"config=5 elements={w.C} seed={args.seed} precision={args.precision}"
+    tr, _ = measured_traffic(args, None, key)
     out = gene_trees_block(E, w, args.steps, args.warmup, args.precision, tr, oracle=not args.no_cpu)
     out.update({"n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "higher_is_better": True,
                 "scaling": "weak", "vs_baseline": None})
     if args.gt_sweeps > 0:
-        out["gene_tree_moves"] = gt_moves_block(E, w, args.gt_sweeps, args.precision)
+        out["gene_tree_moves"] = gt_moves_block(E, w, args.gt_sweeps, args.precision,
+                                                measured_traffic(args, None, key + " height moves")[0])
     print(json.dumps(out))
 
 
-def gt_moves_block(E, w, sweeps=1, precision="fp32"):
+def gt_moves_block(E, w, sweeps=1, precision="fp32", traffic=None):
     """One PhyloAcc-GT sweep of the gene-tree moves over every element, as
     the reference's Gibbs orders them (src/PhyloAcc-GT/bpp_c.cpp:560-680):
     the history draw, one regraft (Sample_tree2) per element, the height move
@@ -693,10 +706,9 @@ def gt_moves_block(E, w, sweeps=1, precision="fp32"):
             "ms_per_sweep": round(tot / sweeps * 1e3, 1),
             "phase_ms": {k: round(v / sweeps * 1e3, 1) for k, v in phases.items()},
             "heights_kernel_ms": round(kernel_heights / sweeps, 1),
-            # the path passes' counted algorithmic bytes over their HIP-event time
-            "heights_kernel_roofline": {"bound": "hbm", "achieved": round(bytes_heights / (kernel_heights * 1e-3) / 1e9, 1),
-                                        "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                                        "frac": round(bytes_heights / (kernel_heights * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
+            # traffic of a path pass over its HIP-event time; bytes_per_sweep are the counted ones, of passes that
+            # store their path and read every child
+            "heights_kernel_roofline": {**measured_rate("hbm", traffic, kernel_heights / (sweeps * (N - S))),
                                         "bytes_per_sweep": bytes_heights / sweeps},
             # likelihood launches: history, two for the regraft, the session's
             # first full pass, one path pass per height move, the pi step
@@ -733,11 +745,7 @@ def gene_trees_block(E, w, steps=3, warmup=1, precision="fp32", traffic=None, or
         rates[name] = (len(ids) / float(np.mean(times)), float(np.mean(times)))
         if name == precision:
             ks = eng.loglik_stats()     # the last timed call's kernel
-            # the counted bytes are those of a pass that stores every node; the kernel moves
-            # fewer, so the rate is of the measured traffic where a summary covers the workload
-            ach = (traffic or ks["algorithmic_bytes"]) / (ks["elapsed_ms"] / 1e3) / 1e9
-            roof = {"bound": "hbm", "achieved": round(ach, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                    "frac": round(ach / HBM_PEAK_GBS, 5), "traffic": traffic, "kernel": "score_kernel",
+            roof = {**measured_rate("latency", traffic, ks["elapsed_ms"]), "kernel": "score_kernel",
                     "algorithmic_bytes_per_launch": ks["algorithmic_bytes"],
                     "kernel_ms": round(ks["elapsed_ms"], 3), "grid": ks["grid"], "block_threads": ks["block_threads"],
                     "lds_bytes": ks["lds_bytes"]}

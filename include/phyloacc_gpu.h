@@ -391,9 +391,9 @@ pa_status pa_release_scratch(pa_engine *e);
  * serving loops, harnesses that forbid hipMalloc).  ids [n], Z [n*N], rates
  * [n*2] and out [n] are DEVICE pointers, in the caller's order; the kernel
  * scores an id outside the engine's elements, or a filtered one, as NaN.
- * Scratch is the library's static device array of 256 MiB per GPU, every
- * workgroup slot sized for the engine's longest element: an engine whose
- * longest element needs more than the array holds is rejected with
+ * Scratch is the library's static device array of 256 MiB per GPU: an engine
+ * whose longest element's partials (internal nodes x padded patterns x 20 B in
+ * FP32, 36 B in FP64) are more than the array holds is rejected with
  * PA_E_INPUT.  The arenas must already be on the device (a pa_loglik or
  * pa_run_chains call after the last pa_elements_add), else PA_E_STATE.  The
  * launch is asynchronous on `stream` (a hipStream_t; NULL: the engine's
@@ -431,9 +431,11 @@ typedef struct {
 /* Launch statistics of one pa_run_chains call. */
 typedef struct {
     double elapsed_ms;          /* device time of the chain launches (HIP events on the engine stream) */
-    double algorithmic_bytes;   /* partial/code/weight bytes the passes must move (counted on device) */
+    double algorithmic_bytes;   /* partial/code/weight bytes of passes that store every node but the cherries that
+                                   they score and read back every child (counted on device); passes that keep partials
+                                   on chip move fewer */
     int32_t grid, block_threads;
-    int32_t lds_bytes;          /* LDS per workgroup */
+    int32_t lds_bytes;          /* LDS per workgroup of the kernel launched */
     int32_t n_launches;
     double scratch_bytes;       /* device scratch of the launch: workgroup slots + long elements' own regions */
 } pa_run_stats;

@@ -17,10 +17,10 @@
 //     cumulative exponent rides along as an int; GAPT marks all-gap subtrees
 //     (the reference's Tg >= num_base, src/PhyloAcc-ST/bpp_c.hpp:417-428);
 //   * a cherry (a non-root internal node whose children are both leaves) is
-//     never stored: its parent and the ancestral sampler recompute its
-//     scaled partial from the two leaf codes with the same operations, so
-//     results are unchanged and a pass saves the cherry's store, its reload
-//     and one dependent memory round trip;
+//     never stored: a pass that visits its parent computes it as the step just
+//     before, and the ancestral sampler from its two leaf codes, with the same
+//     operations, so results are unchanged and its store, its reload and one
+//     dependent memory round trip are saved;
 //   * per-branch 4x4 transition matrices of the current rate class live in
 //     LDS (read as broadcasts); FP64 is used for P(t) builds, log tables,
 //     emissions, the Z forward-backward, likelihood sums and MH ratios.
@@ -389,9 +389,8 @@ __device__ __forceinline__ double prune_patterns(MP M, CP<R> c, int mode)
 // and log_f_Xz, bpp_c.cpp:860-928).  FULL: every internal node of the tree
 // (missing nodes only record their GAPT flag) into the current buffer.
 // DIRTY: nodes with dirty[] set, in place.  PROP: dirty nodes into the other
-// buffer, with PTp for branches whose Z is cls.  Cherries are skipped: their
-// parent recomputes them (cherry_in) with the matrices the pass would have
-// used.  Returns the element's log-likelihood (FP64), identical on every
+// buffer, with PTp for branches whose Z is cls.  A cherry is a step of its
+// parent's visit, dirty or not, and is not stored.  Returns the element's log-likelihood (FP64), identical on every
 // thread.
 //
 // A pass is a chain of nodes, and what bounds it is the time of one link.
@@ -399,7 +398,7 @@ __device__ __forceinline__ double prune_patterns(MP M, CP<R> c, int mode)
 // first (pruning order), so that a node mostly follows its child: the
 // child's partial is still in registers, a cherry's always is, and only the
 // larger side of a fork of stored nodes is read back.  Each step's nodes,
-// sources and matrices come as two words (build_steps) that are read ahead of
+// sources and matrices come as four words (build_steps) that are read ahead of
 // their use, and the inputs of the step after next are in flight.  (By tree
 // level, with each node's descriptor read when its turn came, a step waited
 // for three dependent LDS round trips and the loads of both children.)

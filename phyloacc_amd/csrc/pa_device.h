@@ -1,7 +1,7 @@
 // pa_device.h -- device helpers shared by the chain kernel (pa_chain.hip)
-// and the log-likelihood kernel (pa_engine.hip): 4-vectors, the per-pattern
-// pruning steps (leaf rows, cherries recomputed from their leaf codes, child
-// messages) and wave-uniform values.  One copy, so the two kernels apply the
+// and the log-likelihood kernels (pa_engine.hip): 4-vectors, rows of branch
+// matrices, what a pattern's child contributes (leaf rows, child messages,
+// cherries from their leaf codes) and wave-uniform values.  One copy, so the two kernels apply the
 // same operations in the same order and their FP32 results agree bit for bit.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -67,7 +67,7 @@ __device__ __forceinline__ double block_sum(double v, LDS double *red)
 
 // Node flag set when an element is bound (above the element table's flags):
 // the node is a cherry (a non-root internal node whose children are both
-// leaves), whose partial is recomputed where it is read.
+// leaves), whose partial is not stored.
 constexpr uint8_t NF_CHERRY = 0x80;
 // Row j of P(t) = V diag(exp(lam t)) Vi, clamped at 0: out[i] = P_{j->i}.
 // Called by whole quads of lanes, lane j of a quad for row j of one matrix:

@@ -8,7 +8,8 @@
 // workgroups pull work from a device counter (persistent kernel).  Within a
 // workgroup:
 //   * each branch's 4x4 transition matrix P(t * rate of its class) is built
-//     in FP64 by one thread and stored in LDS in the partials' precision;
+//     in FP64 by a quad of lanes, a row a lane, and stored in LDS in the
+//     partials' precision;
 //   * the pass is a list of steps (pa_prune.h), a pattern a lane; a thread
 //     keeps its patterns through the whole pass, so no barrier is needed
 //     between tree nodes;

@@ -918,11 +918,20 @@ struct DevBuf {
 
 }  // namespace
 
-// Block size of a batched launch from the elements' mean pattern count.
-// Default block size (no tuning): by the mean pattern count (measured on the
-// 43-species workloads: 128 threads at a mean of 136 patterns, 256 at 299),
-// and 256 when the batch has fewer elements than four per CU, where more
-// threads per element is all the device can add.
+// Default block size of a batched chain launch (no tuning), by the elements'
+// mean pattern count; 256 when the batch has fewer elements than four per CU,
+// where more threads per element is all the device can add.  An element's
+// chains stay in one workgroup, so the block follows the long elements as much
+// as the mean: ms of a launch at 64, 128 and 256 threads, 43 species,
+//   50,000 Pareto elements (mean 136 patterns, up to 7,000), FP32 168 120 142
+//     FP64                                                      222 188 211
+//   10,000 of them, FP32                                        195 111  67
+//   5,000 log-normal elements (mean 311), FP32                  126  78  60
+//     FP64                                                      159 104  86
+//   8,000 elements of 30, 90, 180, 320 patterns (+- half), FP32
+//     13.4/14.1/19.3  19.7/18.1/22.9  30.2/25.2/30.1  44.5/34.4/41.1
+// The lines at 96 and 200 serve elements of spread lengths; a batch of even or
+// few elements gains by pa_autotune.
 static int block_for_mean(double meanP) { return meanP <= 96 ? 64 : (meanP <= 200 ? 128 : 256); }
 
 static int pick_block(pa_engine *e, const int32_t *work, int32_t n)

@@ -225,6 +225,17 @@ hipError_t launch_gbgc_eig(const double *Q0, const double *sel, int n, double *e
     return hipGetLastError();
 }
 
+// The log-likelihoods of work position w, by position and by caller row.
+__device__ __forceinline__ void write_scores(AP A, int w, int row, double s0, double s1)
+{
+    A->ll_out[w] = s0;
+    if (A->pre_len) A->ll_out2[w] = s1;
+    if (A->row_out0) {
+        A->row_out0[row] = s0;
+        if (A->pre_len) A->row_out1[row] = s1;
+    }
+}
+
 // Kernel arguments are copied to LDS once per workgroup: the device
 // functions take LDS pointers to them, which keeps the argument blocks out of
 // the private (scratch) segment.
@@ -424,14 +435,14 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
         ScoreItem item{it, 0, 0, -1};
         if (A->items) item = A->items[it];
         const int w = uni(item.w), part = uni(item.part);
-        // an id outside the arenas, or a filtered element (no patterns), scores NaN
+        // an id outside the arenas, or an element without patterns (filtered, or of no sites), scores NaN
         const int id = uni(A->work[w]);
+        const int row = A->len_row ? uni(A->len_row[w]) : w;
         if (id < 0 || id >= uni(A->n_elems) || A->elems[id].P <= 0) {
-            if (tid == 0) A->ll_out[w] = __builtin_nan("");
+            if (tid == 0) write_scores(A, w, row, __builtin_nan(""), __builtin_nan(""));
             __syncthreads();
             continue;
         }
-        const int row = A->len_row ? uni(A->len_row[w]) : w;
         const double *pw = A->el_pi ? A->el_pi + (size_t)w * 4 : nullptr;
         double pi[4];
         for (int j = 0; j < 4; j++) pi[j] = pw ? pw[j] : M->pi[j];
@@ -461,12 +472,7 @@ __global__ void __launch_bounds__(BS, 4) score_kernel(ModelDev Mk, LoglikArgs Ak
             if (part >= 0) {
                 A->part_sum[part] = s0;
             } else {
-                A->ll_out[w] = s0;
-                if (A->pre_len) A->ll_out2[w] = s1;
-                if (A->row_out0) {
-                    A->row_out0[row] = s0;
-                    if (A->pre_len) A->row_out1[row] = s1;
-                }
+                write_scores(A, w, row, s0, s1);
             }
             // and the root's partial, exponent and pattern weight
             if (A->counters) atomicAdd(A->counters, (unsigned long long)(P - first) * (per_sh + 4 * sizeof(R) + 8));
@@ -958,12 +964,12 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
         const int w = uni(work_sh);
         if (w >= uni(A->n_work)) break;
         const int id = uni(A->work[w]);
+        const int row = A->len_row ? uni(A->len_row[w]) : w;
         if (id < 0 || id >= uni(A->n_elems) || A->elems[id].P <= 0) {
-            if (tid == 0) A->ll_out[w] = __builtin_nan("");
+            if (tid == 0) write_scores(A, w, row, __builtin_nan(""), __builtin_nan(""));
             __syncthreads();
             continue;
         }
-        const int row = A->len_row ? uni(A->len_row[w]) : w;
         const double *pw = A->el_pi ? A->el_pi + (size_t)w * 4 : nullptr;
         double pi[4];
         for (int j = 0; j < 4; j++) pi[j] = pw ? pw[j] : M->pi[j];
@@ -1041,12 +1047,7 @@ __global__ void __launch_bounds__(BS, keep_waves(sizeof(R), USE)) keep_kernel(Mo
         if constexpr (USE == LoglikUse::Candidates)
             gt_candidates<R, BS, WIDE>(M, A, k, blocks, (const GBL uint8_t *)(A->codes + E.off_codes), site, (LDS double *)Pc, (LDS double *)red, w, row, S, I, E.Ppad, pi[0], pi[1], pi[2], pi[3]);
         if (tid == 0) {
-            A->ll_out[w] = s0;
-            if (A->pre_len) A->ll_out2[w] = s1;
-            if (A->row_out0) {
-                A->row_out0[row] = s0;
-                if (A->pre_len) A->row_out1[row] = s1;
-            }
+            write_scores(A, w, row, s0, s1);
             // and the root's partial, exponent and pattern weight
             if (A->counters) atomicAdd(A->counters, (unsigned long long)E.P * (per_sh + 4 * sizeof(R) + 8));
         }
